@@ -155,7 +155,8 @@ class Conv3d(Convolution):
                                         bool(relu), cache_packed=not self.training and w is weight)
         elif not training:
             w = weight if weight.dtype == input.feature.dtype else weight.to(input.feature.dtype)
-            out_feature = ext.rule_conv(input.feature, w.detach(), book, rule_size, oz_idx.shape[0],
+            # (the view itself, not a detached copy of it: the kept packed weight is looked up by the parameter behind it)
+            out_feature = ext.rule_conv(input.feature, w, book, rule_size, oz_idx.shape[0],
                                         cache_packed=not self.training and w is weight)
         else:
             out_feature = ConvFunction.apply(input.feature, weight, book, rule_size, tile_grid_shape,
