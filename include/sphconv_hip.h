@@ -145,6 +145,23 @@ int sph_rules_build_pack(const int32_t *z_idx, const int32_t *z_ptr, int in_rows
                          sph_dtype dt, const void *w, int KV, int kdim, int ndim, long stride_k,
                          long stride_kk, long stride_n, void *packed, void *stream);
 
+/* One weight to put in fragment order (see sph_weight_pack): B[k][kk][n] = w[k*stride_k + kk*stride_kk + n*stride_n].
+ * w_f32 != 0: w holds fp32 values (a master weight), rounded to dt (fp16 or bf16) on the way. */
+typedef struct sph_pack_desc {
+    sph_dtype dt; /* element type of the packed copy */
+    int32_t w_f32;
+    const void *w;
+    int32_t KV, kdim, ndim;
+    long stride_k, stride_kk, stride_n;
+    void *packed;
+} sph_pack_desc;
+/* sph_rules_build_pack with up to two weights (a training step wants the layer's weight for its forward pass and,
+ * transposed, for dgrad); npacks 0: sph_rules_build. */
+int sph_rules_build_packs(const int32_t *z_idx, const int32_t *z_ptr, int in_rows,
+                          const int32_t *oz_idx, const int32_t *oz_ptr, int out_rows,
+                          const sph_geom *g, int transposed, const sph_book *book,
+                          const int32_t *row_cols, const sph_pack_desc *packs, int npacks, void *stream);
+
 /* Replaces the output-coordinate half of get_rules (rules.cu:417-443, 461-462: prepareGridKernel, two
  * cumsums, roll/index_put/add and the device->host read), in two steps because the caller must size oz_idx:
  *  1. sph_outcoords_count: counts every output column's active bins into oz_ptr and scans them in place
@@ -209,6 +226,9 @@ size_t sph_weight_packed_bytes(sph_dtype dt, int KV, int kdim, int ndim);
  * where B[k][kk][n] = w[k*stride_k + kk*stride_kk + n*stride_n] (element strides). */
 int sph_weight_pack(sph_dtype dt, const void *w, int KV, int kdim, int ndim,
                     long stride_k, long stride_kk, long stride_n, void *packed, void *stream);
+
+/* Up to two weights in one launch. */
+int sph_weight_packs(const sph_pack_desc *packs, int npacks, void *stream);
 
 /* Optional epilogue applied to the accumulator before the store:
  *   y = acc * scale[c] + shift[c]   (each pointer may be null: 1 / 0)
@@ -278,10 +298,24 @@ size_t sph_init_tensor_workspace(int n, int B, int S0, int S1, int S2);
 int sph_init_tensor(const int32_t *indices, int n, int B, int S0, int S1, int S2, int32_t *z_idx,
                     int32_t *z_ptr, int32_t *permutation, int32_t *status, void *workspace,
                     size_t workspace_bytes, void *stream);
+/* sph_init_tensor and everything a sparse tensor wants beside it, in four launches: `row_cols` [n] (may be null): the
+ * column of every output row (sph_row_columns); `feature` (may be null) [n] rows of row_bytes, moved to `out_feature`
+ * (sph_permute_rows); `host_status` (may be null): two int32 the GPU can write and the host can read (pinned memory,
+ * 8-byte aligned) that receive the two status words in one 8-byte store, so that a host that has set them to -1
+ * before the call can wait for them without a copy.  Same workspace. */
+int sph_init_tensor_rows(const int32_t *indices, int n, int B, int S0, int S1, int S2, const void *feature,
+                         int row_bytes, int32_t *z_idx, int32_t *z_ptr, int32_t *permutation, int32_t *row_cols,
+                         void *out_feature, int32_t *status, int32_t *host_status, void *workspace,
+                         size_t workspace_bytes, void *stream);
 /* Replaces to_dense / to_dense_backward (tensor.cu:222-309): dense is
  * [B,S0,S1,S2,C]; only active cells are written (forward) / read (backward). */
 int sph_to_dense(const void *feature, const int32_t *z_idx, const int32_t *z_ptr, int rows,
                  int ncol, int S2, int row_bytes, void *dense, void *stream);
+/* The same with the channels in front, dense [B,C,S0,S1,S2] (what the reference makes of it with a permuted copy,
+ * sphconv/functional.py:81-106), zeros in the inactive cells included: `out` is fully overwritten.  elem_size 1, 2 or
+ * 4 bytes; ncol = B*S0*S1, cols_per_sample = S0*S1. */
+int sph_to_dense_channels_first(const void *feature, const int32_t *z_idx, const int32_t *z_ptr, int rows, int ncol,
+                                int cols_per_sample, int S2, int C, int elem_size, void *out, void *stream);
 int sph_to_dense_backward(const void *d_dense, const int32_t *z_idx, const int32_t *z_ptr,
                           int rows, int ncol, int S2, int row_bytes, void *d_feature,
                           void *stream);
@@ -312,7 +346,8 @@ int sph_xyz_to_rangevoxel(const float *points, int m, int ndim, int v_res, int h
  * in the reference's loop.  Outputs (all zero where unused): voxels [max_voxels, max_points, W]
  * (append_mode 0: the point's nfeat values, W = nfeat; 1: those plus (c0, c1, c2), W = nfeat + 3;
  * 2: (c0, c1, c2, intensity), W = nfeat), mask [max_voxels, max_points] (1.0 where a point sits),
- * coors [max_voxels, 3] = (bin of c2, of c1, of c0), num_points [max_voxels], voxel_num [1] (device).
+ * coors [max_voxels, 3] = (bin of c2, of c1, of c0), num_points [max_voxels], voxel_num [1] (device memory, or pinned
+ * host memory that a host which set it to -1 may watch: it is written once, before the kernel that fills the voxels).
  * cell_in (optional, [n] int64): take these cells ((bin2*g1 + bin1)*g0 + bin0, negative = skip)
  * instead of computing them; cell_out (optional): receives the cells.  `workspace`: device memory
  * of sph_points_to_voxel_workspace(n, g0, g1, g2) bytes, 256-byte aligned; nothing is allocated. */
@@ -322,6 +357,15 @@ int sph_points_to_voxel(const float *points, int n, int nfeat, int system, float
                         int max_voxels, int append_mode, float *voxels, float *mask, int32_t *coors,
                         int32_t *num_points, int32_t *voxel_num, const long long *cell_in,
                         long long *cell_out, void *workspace, size_t workspace_bytes, void *stream);
+
+/* Mean of the points of every voxel (SimpleVoxel, sphconv/vfe.py:210-228): voxels [nv, max_points, width] with zeros in
+ * unused slots, out [nv, nf] = the sum of their first nf values over the slots / num_points. */
+int sph_voxel_mean(const float *voxels, const int32_t *num_points, int nv, int max_points, int width, int nf,
+                   float *out, void *stream);
+/* Coordinates of a batch (merge_batch_torch, sphconv/datagen.py:53-74): parts (host array of device pointers) of
+ * rows[b] x 3 int32 -> out [sum of rows, 4] = (b, the part's three). */
+#define SPH_MAX_BATCH_PARTS 64
+int sph_batch_coordinates(const int32_t *const *parts, const int32_t *rows, int nparts, int32_t *out, void *stream);
 
 #ifdef __cplusplus
 }

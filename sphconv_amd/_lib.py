@@ -1,5 +1,5 @@
-"""ctypes binding of ``libsphconv_hip.so`` (the C ABI declared in
-``include/sphconv_hip.h``).  PyTorch is used only to own device memory and the
+"""Binding of ``libsphconv_hip.so`` (the C ABI declared in ``include/sphconv_hip.h``): ctypes signatures of every
+entry point, and the host extension through which the calls on the convolution path go.  PyTorch is used only to own device memory and the
 current HIP stream; every computation on the path happens inside the library.
 
 There is no CPU fallback: if the library is missing or a call fails, an
@@ -43,8 +43,15 @@ class Epilogue(C.Structure):
     _fields_ = [("scale", C.c_void_p), ("shift", C.c_void_p), ("relu", C.c_int32)]
 
 
+class PackDesc(C.Structure):
+    _fields_ = [("dt", C.c_int32), ("w_f32", C.c_int32), ("w", C.c_void_p), ("KV", C.c_int32), ("kdim", C.c_int32),
+                ("ndim", C.c_int32), ("stride_k", C.c_long), ("stride_kk", C.c_long), ("stride_n", C.c_long),
+                ("packed", C.c_void_p)]
+
+
 _lib = None
-ABI_VERSION = 7       # sph_abi_version() of the library these signatures describe
+_host = None
+ABI_VERSION = 8       # sph_abi_version() of the library these signatures describe
 
 _I, _P, _L, _Z = C.c_int, C.c_void_p, C.c_long, C.c_size_t
 _SIGNATURES = {
@@ -57,6 +64,8 @@ _SIGNATURES = {
     "sph_rules_build": (_I, [_P, _P, _I, _P, _P, _I, C.POINTER(Geom), _I, C.POINTER(Book), _P, _P]),
     "sph_rules_build_pack": (_I, [_P, _P, _I, _P, _P, _I, C.POINTER(Geom), _I, C.POINTER(Book), _P, _I, _P, _I, _I, _I, _L,
                                   _L, _L, _P, _P]),
+    "sph_rules_build_packs": (_I, [_P, _P, _I, _P, _P, _I, C.POINTER(Geom), _I, C.POINTER(Book), _P, C.POINTER(PackDesc), _I,
+                                   _P]),
     "sph_row_columns": (_I, [_P, _I, _I, _P, _P]),
     "sph_outcoords_blocks": (_I, [C.POINTER(Geom)]),
     "sph_outcoords_scratch_ints": (_I, [C.POINTER(Geom)]),
@@ -69,6 +78,7 @@ _SIGNATURES = {
     "sph_rules_from_padded": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _P, C.POINTER(Book), _P]),
     "sph_weight_packed_bytes": (_Z, [_I, _I, _I, _I]),
     "sph_weight_pack": (_I, [_I, _P, _I, _I, _I, _L, _L, _L, _P, _P]),
+    "sph_weight_packs": (_I, [C.POINTER(PackDesc), _I, _P]),
     "sph_conv_apply": (_I, [_I, _P, _I, _I, _P, _I, C.POINTER(Book), C.POINTER(Epilogue), _P, _P]),
     "sph_rules_conv": (_I, [_P, _P, _I, _P, _P, _I, C.POINTER(Geom), C.POINTER(Book), _I, _P, _I, _P, _I, _P, _I,
                             C.POINTER(Epilogue), _P, _P]),
@@ -76,13 +86,17 @@ _SIGNATURES = {
     "sph_conv_wgrad": (_I, [_I, _P, _I, _I, _P, _I, C.POINTER(Book), _P, _P, _I, _P]),
     "sph_init_tensor_workspace": (_Z, [_I, _I, _I, _I, _I]),
     "sph_init_tensor": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _Z, _P]),
+    "sph_init_tensor_rows": (_I, [_P, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _P]),
     "sph_permute_rows": (_I, [_P, _P, _I, _I, _I, _P, _P]),
     "sph_points_to_voxel_workspace": (_Z, [_I, _I, _I, _I]),
     "sph_points_to_voxel": (_I, [_P, _I, _I, _I, C.c_float, C.c_float, C.c_float, C.c_float, C.c_float, C.c_float, _I, _I,
                                  _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _P]),
+    "sph_voxel_mean": (_I, [_P, _P, _I, _I, _I, _I, _P, _P]),
+    "sph_batch_coordinates": (_I, [C.POINTER(C.c_void_p), C.POINTER(C.c_int32), _I, _P, _P]),
     "sph_xyz_to_rangevoxel": (_I, [_P, _I, _I, _I, _I, _I, C.c_float, C.c_float, C.c_float, C.c_float, C.c_float,
                                    C.c_float, _I, _P, _P, _P, _P, _P, _P]),
     "sph_to_dense": (_I, [_P, _P, _P, _I, _I, _I, _I, _P, _P]),
+    "sph_to_dense_channels_first": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P]),
     "sph_to_dense_backward": (_I, [_P, _P, _P, _I, _I, _I, _I, _P, _P]),
 }
 EXPORTS = tuple(_SIGNATURES)
@@ -106,6 +120,23 @@ def lib():
                                % (LIB_PATH, handle.sph_abi_version(), ABI_VERSION))
         _lib = handle
     return _lib
+
+
+def host():
+    """The host extension (``csrc/host.cpp``): the calls of the C ABI with their allocations and structs, in C++."""
+    global _host
+    if _host is None:
+        lib()                                            # says what is missing, and loads what the extension links to
+        try:
+            from . import _host as ext
+        except ImportError as e:
+            raise SphconvError("_host.so is not built or does not load (run `make -C sphconv_amd/csrc`): %s" % e) from e
+        if ext.abi_version() != ABI_VERSION:
+            raise SphconvError("_host.so has ABI version %d, this package needs %d: rebuild it (make -C sphconv_amd/csrc)"
+                               % (ext.abi_version(), ABI_VERSION))
+        ext.set_error(SphconvError)
+        _host = ext
+    return _host
 
 
 def check(rc: int):

@@ -30,9 +30,9 @@ namespace {
 // ---------------------------------------------------------------------------
 // Weight packing (layout and element copy: pack.h)
 // ---------------------------------------------------------------------------
-__global__ void pack_weight_kernel(SphPackJob p)
+__global__ void pack_weight_kernel(SphPackJobs p)
 {
-    sph_pack_element(p, (long)blockIdx.x * blockDim.x + threadIdx.x);
+    sph_pack_fragments(p, (int)(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
 constexpr int kMetaGroups = 32; // groups whose indices are staged in LDS at a time
@@ -1409,9 +1409,23 @@ SPH_EXPORT int sph_weight_pack(sph_dtype dt, const void *w, int KV, int kdim, in
 {
     int rc = sph_pack_args_ok("sph_weight_pack", dt, w, packed, KV, kdim, ndim);
     if (rc) return rc;
-    const SphPackJob p = sph_pack_job(dt, w, KV, kdim, ndim, stride_k, stride_kk, stride_n, packed);
-    hipLaunchKernelGGL(pack_weight_kernel, dim3((unsigned)((p.total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, p);
+    SPH_REQUIRE((uintptr_t)packed % 16 == 0, SPH_ERR_ARG, "sph_weight_pack: packed weight must be 16-byte aligned");
+    SphPackJobs p;
+    p.job[0] = sph_pack_job(dt, w, KV, kdim, ndim, stride_k, stride_kk, stride_n, packed);
+    p.job[1].total = 0;
+    hipLaunchKernelGGL(pack_weight_kernel, dim3(sph_div_up(p.job[0].total, 64)), dim3(64), 0, (hipStream_t)stream, p);
     return sph_check_launch("sph_weight_pack");
+}
+
+SPH_EXPORT int sph_weight_packs(const sph_pack_desc *packs, int npacks, void *stream)
+{
+    SphPackJobs p;
+    int rc = sph_pack_jobs("sph_weight_packs", packs, npacks, &p);
+    if (rc) return rc;
+    const int total = sph_pack_total(p.job);
+    if (total == 0) return SPH_OK;
+    hipLaunchKernelGGL(pack_weight_kernel, dim3(sph_div_up(total, 64)), dim3(64), 0, (hipStream_t)stream, p);
+    return sph_check_launch("sph_weight_packs");
 }
 
 SPH_EXPORT int sph_conv_apply(sph_dtype dt, const void *feature, int feature_rows, int kdim,

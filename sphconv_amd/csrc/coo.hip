@@ -5,25 +5,25 @@
 // ascending S2 -- one legal, deterministic serialisation of the reference's output
 // (its order inside a fiber is the order in which atomics happen to land).
 //
-// No sort: a row's place is the start of its column (a scan of per-column counts) plus its rank
-// inside the column, and the rank needs no order of arrival.
-// Shallow grids (S2 <= 128, the usual case):
-//   1. coo_count_kernel    slot = atomicAdd(count[column]) per row (arrival order, only used
-//                          to park the row inside its column's segment)
-//   2. sum-scan (scan.h)   counts -> z_ptr (inclusive)
-//   3. coo_scatter_kernel  (s2, row) -> segment position start + slot
-//   4. coo_rank_kernel     every row counts the entries of its column with a smaller s2:
-//                          that rank is its final position, whatever the arrival order was
-// Deep grids (S2 > 128), where a full column would make that walk long: one bit per cell instead,
-//   1. coo_mark_kernel     count[column]++ and the cell's bit set in the column's bitmap (a bit
-//                          that was set already is a duplicate coordinate: status[1])
-//   2. sum-scan            counts -> z_ptr
-//   3. coo_place_kernel    rank = set bits of the column below s2 (popcounts of up to S2/64 words)
-// (the reference keeps four bytes per cell for the same purpose, tensor.cu:21-36; a bitmap of more
-// than 1 GiB -- 8.6e9 cells -- falls back to the walk, which needs memory by rows only).
-// Four to six launches, none from a library.
-// The feature rows are then moved with sph_permute_rows.  No memory is allocated:
-// segments, bitmaps and the scan's state live in the caller's workspace.
+// No sort: a row's place is the start of its column plus its rank inside the column, and one bit per cell says both:
+//   1. coo_clear_kernel  zeroes the bitmap, the scan's state and the status words (one launch)
+//   2. coo_mark_kernel   every row sets its cell's bit in its column's bitmap (one 64-bit atomic without a result:
+//                        nothing waits for it)
+//   3. sum-scan (scan.h) of the columns' bit counts, made from the bitmap as they are read -> z_ptr
+//   4. coo_place_kernel  rank = set bits of the column below s2 (popcounts of up to S2/64 words); writes z_idx, the
+//                        permutation, the row's column, moves the feature row and reports the status.  Rows that
+//                        share a cell set one bit between them: their number is what the bits are short of the rows.
+// (the reference keeps four bytes per cell for the same purpose, tensor.cu:21-36.)
+// What bounds it: the random accesses, one atomic and one feature row per input row.  623 k rows in random order on a
+// 4x64x2048x64 grid, 16 fp16 channels: 118 us in eight launches with per-column counters, slots, a scatter into segments
+// and a walk of each row's segment; four launches now.
+// A bitmap of more than 1 GiB (8.6e9 cells) falls back to that walk, which needs memory by rows only:
+//   coo_count_kernel    slot = atomicAdd(count[column]) per row (arrival order, only used to park the row inside its
+//                       column's segment); sum-scan -> z_ptr
+//   coo_scatter_kernel  (s2, row) -> segment position start + slot
+//   coo_rank_kernel     every row counts the entries of its column with a smaller s2: that rank is its final
+//                       position, whatever the arrival order was
+// No memory is allocated: bitmap or segments and the scan's state live in the caller's workspace.
 #include "common.h"
 
 #include <cstring>
@@ -33,8 +33,6 @@
 namespace {
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-constexpr int kRankMaxDepth = 128; // S2 up to which a row's rank is found by walking its column's segment
 
 inline size_t sum_scan_bytes(int ncol) { return sph_scan::state_bytes(ncol); }
 
@@ -56,7 +54,7 @@ inline RankLayout rank_layout(int n, int ncol)
     return l;
 }
 
-constexpr size_t kBitmapMaxBytes = (size_t)1 << 30; // deep grids whose bitmap would be larger are ranked by the walk
+constexpr size_t kBitmapMaxBytes = (size_t)1 << 30; // grids whose bitmap would be larger are ranked by the walk
 
 struct BitLayout {
     size_t bits, bits_bytes, temp, temp_bytes, total;
@@ -77,7 +75,7 @@ inline BitLayout bit_layout(int ncol, int S2)
 
 inline bool by_bitmap(int ncol, int S2)
 {
-    return S2 > kRankMaxDepth && (double)ncol * ((S2 + 63) / 64) * 8.0 <= (double)kBitmapMaxBytes;
+    return (double)ncol * ((S2 + 63) / 64) * 8.0 <= (double)kBitmapMaxBytes;
 }
 
 __global__ void fill_zero_kernel(int32_t *p, int n)
@@ -86,46 +84,94 @@ __global__ void fill_zero_kernel(int32_t *p, int n)
     if (i < n) p[i] = 0;
 }
 
-// Deep grids, step 1: the row is counted in its column and marks its cell.
-__global__ void coo_mark_kernel(const int32_t *idx, int n, int B, int S0, int S1, int S2, int words, int32_t *counts,
-                                unsigned long long *bits, int32_t *status)
+// bitmap and scan state, which follow each other in the workspace (n16 16-byte words), and the status words
+__global__ __launch_bounds__(256) void coo_clear_kernel(uint4 *p, long n16, int32_t *status)
+{
+    const long step = (long)gridDim.x * 256;
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n16; i += step) p[i] = make_uint4(0, 0, 0, 0);
+    if (blockIdx.x == 0 && threadIdx.x < 2) status[threadIdx.x] = 0;
+}
+
+__global__ void copy_status_kernel(const int32_t *status, int32_t *host_status)
+{
+    if (threadIdx.x == 0) *(unsigned long long *)host_status = *(const unsigned long long *)status;
+}
+
+struct CooGrid {
+    int B, S0, S1, S2, words; // words: 64-bit words of a column's bitmap
+};
+__device__ __forceinline__ bool coo_inside(const int4 &c, const CooGrid &g)
+{
+    return (unsigned)c.x < (unsigned)g.B && (unsigned)c.y < (unsigned)g.S0 && (unsigned)c.z < (unsigned)g.S1 &&
+           (unsigned)c.w < (unsigned)g.S2;
+}
+
+__global__ __launch_bounds__(256) void coo_mark_kernel(const int32_t *idx, int n, CooGrid g, unsigned long long *bits, int32_t *status)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int4 c = ((const int4 *)idx)[i]; // (b, s0, s1, s2)
-    const bool ok = (unsigned)c.x < (unsigned)B && (unsigned)c.y < (unsigned)S0 && (unsigned)c.z < (unsigned)S1 &&
-                    (unsigned)c.w < (unsigned)S2;
-    if (!ok) {
+    if (!coo_inside(c, g)) {
         atomicAdd(&status[0], 1);
         return;
     }
-    const int col = (c.x * S0 + c.y) * S1 + c.z;
-    atomicAdd(&counts[col], 1);
-    const unsigned long long bit = 1ull << (c.w & 63);
-    const unsigned long long old = atomicOr(&bits[(size_t)col * words + (c.w >> 6)], bit);
-    if (old & bit) atomicAdd(&status[1], 1);
+    const int col = (c.x * g.S0 + c.y) * g.S1 + c.z;
+    atomicOr(&bits[(size_t)col * g.words + (c.w >> 6)], 1ull << (c.w & 63));
 }
 
-// Deep grids, step 3: place = start of the column + number of its cells below the row's.
-__global__ void coo_place_kernel(const int32_t *idx, int n, int B, int S0, int S1, int S2, int words, const int32_t *z_ptr,
-                                 const unsigned long long *bits, int32_t *z_idx, int32_t *permutation)
+// rows of a column, from its bitmap (what the scan reads)
+struct ColumnRows {
+    const unsigned long long *bits;
+    int words;
+    __device__ __forceinline__ int operator()(long col) const
+    {
+        int n = 0;
+        for (int w = 0; w < words; w++) n += __popcll(bits[(size_t)col * words + w]);
+        return n;
+    }
+};
+
+struct CooRows {
+    const int32_t *z_ptr;
+    const unsigned long long *bits;
+    int32_t *z_idx, *permutation, *row_cols; // row_cols may be null
+    const char *feature;                     // null: no rows to move
+    char *out;
+    int32_t *status, *host_status;           // host_status (may be null): the same two words where the host reads them
+};
+
+// gpr threads per row, one 16-byte (G) granule of its features each; gpr = 1 without features
+template <typename G>
+__global__ __launch_bounds__(256) void coo_place_kernel(const int32_t *idx, int n, CooGrid g, CooRows r, int gpr)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    if (t == 0) {
+        const int outside = r.status[0], ncol = g.B * g.S0 * g.S1;
+        const int dup = n - outside - r.z_ptr[ncol - 1];
+        r.status[1] = dup;
+        if (r.host_status) {
+            // one 8-byte store: the host may be watching the pair
+            *(unsigned long long *)r.host_status = ((unsigned long long)(unsigned)dup << 32) | (unsigned)outside;
+        }
+    }
+    const int i = gpr == 1 ? (int)t : (int)(t / gpr);
+    const int q = gpr == 1 ? 0 : (int)(t - (long)i * gpr);
     if (i >= n) return;
     const int4 c = ((const int4 *)idx)[i];
-    const bool ok = (unsigned)c.x < (unsigned)B && (unsigned)c.y < (unsigned)S0 && (unsigned)c.z < (unsigned)S1 &&
-                    (unsigned)c.w < (unsigned)S2;
-    if (!ok) return;
-    const int col = (c.x * S0 + c.y) * S1 + c.z;
-    const unsigned long long *cb = bits + (size_t)col * words;
+    if (!coo_inside(c, g)) return;
+    const int col = (c.x * g.S0 + c.y) * g.S1 + c.z;
+    const unsigned long long *cb = r.bits + (size_t)col * g.words;
     const int wz = c.w >> 6;
     int rank = __popcll(cb[wz] & ((1ull << (c.w & 63)) - 1ull));
     for (int w = 0; w < wz; w++) rank += __popcll(cb[w]);
-    const int pos = (col ? z_ptr[col - 1] : 0) + rank;
-    if ((unsigned)pos < (unsigned)n) {
-        z_idx[pos] = c.w;
-        permutation[i] = pos;
+    const int pos = (col ? r.z_ptr[col - 1] : 0) + rank;
+    if ((unsigned)pos >= (unsigned)n) return;
+    if (q == 0) {
+        r.z_idx[pos] = c.w;
+        r.permutation[i] = pos;
+        if (r.row_cols) r.row_cols[pos] = col;
     }
+    if (r.feature) ((G *)r.out)[(long)pos * gpr + q] = ((const G *)r.feature)[(long)i * gpr + q];
 }
 
 __global__ void coo_count_kernel(const int32_t *idx, int n, int B, int S0, int S1, int S2, int32_t *counts, int32_t *slot,
@@ -196,7 +242,7 @@ SPH_EXPORT size_t sph_init_tensor_workspace(int n, int B, int S0, int S1, int S2
     return rank_layout(n, B * S0 * S1).total;
 }
 
-// count, scan, scatter, rank by a walk of the column's segment (shallow grids; deep ones whose bitmap would not fit)
+// count, scan, scatter, rank by a walk of the column's segment (grids whose bitmap would not fit)
 static int init_tensor_by_rank(const int32_t *indices, int n, int B, int S0, int S1, int S2, int32_t *z_idx, int32_t *z_ptr,
                                int32_t *permutation, int32_t *status, void *workspace, size_t workspace_bytes,
                                hipStream_t st)
@@ -228,45 +274,78 @@ static int init_tensor_by_rank(const int32_t *indices, int n, int B, int S0, int
     return sph_check_launch("sph_init_tensor(rank)");
 }
 
+// Granules of a row up to which the place kernel moves the features itself (each granule's thread finds the row's
+// place again, from cached words); longer rows are moved by sph_permute_rows.
+constexpr int kPlaceGranules = 16;
+
+SPH_EXPORT int sph_init_tensor_rows(const int32_t *indices, int n, int B, int S0, int S1, int S2, const void *feature,
+                                    int row_bytes, int32_t *z_idx, int32_t *z_ptr, int32_t *permutation, int32_t *row_cols,
+                                    void *out_feature, int32_t *status, int32_t *host_status, void *workspace,
+                                    size_t workspace_bytes, void *stream)
+{
+    const char *who = "sph_init_tensor";
+    SPH_REQUIRE(n >= 0 && B > 0 && S0 > 0 && S1 > 0 && S2 > 0, SPH_ERR_ARG, "%s: bad sizes", who);
+    SPH_REQUIRE((double)B * S0 * S1 < 2147483648.0, SPH_ERR_UNSUPPORTED, "%s: more than 2^31 columns", who);
+    SPH_REQUIRE(z_ptr && status && workspace && (n == 0 || (indices && z_idx && permutation)), SPH_ERR_ARG, "%s: null pointer", who);
+    SPH_REQUIRE((uintptr_t)indices % 16 == 0 && (uintptr_t)workspace % 256 == 0 && (uintptr_t)host_status % 8 == 0, SPH_ERR_ARG,
+                "%s: indices must be 16-byte aligned, the workspace 256-byte aligned, the host's status words 8-byte aligned", who);
+    SPH_REQUIRE(!feature || (out_feature && row_bytes > 0), SPH_ERR_ARG, "%s: feature rows without a place to go", who);
+    const int ncol = B * S0 * S1;
+    hipStream_t st = (hipStream_t)stream;
+    const bool move = feature && n > 0;
+    int rc;
+    if (!by_bitmap(ncol, S2)) {
+        rc = init_tensor_by_rank(indices, n, B, S0, S1, S2, z_idx, z_ptr, permutation, status, workspace, workspace_bytes, st);
+        if (rc) return rc;
+        if (row_cols && n > 0 && (rc = sph_row_columns(z_ptr, ncol, n, row_cols, stream))) return rc;
+        if (move && (rc = sph_permute_rows(feature, permutation, n, row_bytes, 0, out_feature, stream))) return rc;
+        if (host_status) hipLaunchKernelGGL(copy_status_kernel, dim3(1), dim3(64), 0, st, (const int32_t *)status, host_status);
+        return sph_check_launch(who);
+    }
+    const BitLayout l = bit_layout(ncol, S2);
+    SPH_REQUIRE(l.total != 0, SPH_ERR_LAUNCH, "%s: temporary storage query failed", who);
+    SPH_REQUIRE(workspace_bytes >= l.total, SPH_ERR_ARG, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, l.total);
+    char *ws = (char *)workspace;
+    CooGrid g{B, S0, S1, S2, l.words};
+    CooRows r{z_ptr, (const unsigned long long *)(ws + l.bits), z_idx, permutation, row_cols, nullptr, nullptr, status, host_status};
+    const long n16 = (long)(l.total / 16);
+    hipLaunchKernelGGL(coo_clear_kernel, dim3((unsigned)(n16 < 256L * 2048 ? (n16 + 255) / 256 : 2048)), dim3(256), 0, st,
+                       (uint4 *)workspace, n16, status);
+    const dim3 block(256);
+    if (n > 0)
+        hipLaunchKernelGGL(coo_mark_kernel, dim3(sph_div_up(n, 256)), block, 0, st, indices, n, g, (unsigned long long *)(ws + l.bits), status);
+    const hipError_t e = sph_scan::launch_from<sph_scan::Plus, true>(sph_scan::FromFunction<ColumnRows>{ColumnRows{r.bits, l.words}}, z_ptr,
+                                                                     (long)ncol, ws + l.temp, 0, st, nullptr, /*clear_state=*/false);
+    if (e != hipSuccess) {
+        sph_set_error("%s: scan: %s", who, hipGetErrorString(e));
+        return SPH_ERR_LAUNCH;
+    }
+    const uintptr_t al = (uintptr_t)feature | (uintptr_t)out_feature | (uintptr_t)row_bytes;
+    const int gran = al % 16 == 0 ? 16 : (al % 4 == 0 ? 4 : (al % 2 == 0 ? 2 : 1));
+    const bool here = move && row_bytes / gran <= kPlaceGranules;
+    int gpr = 1;
+    if (here) {
+        r.feature = (const char *)feature;
+        r.out = (char *)out_feature;
+        gpr = row_bytes / gran;
+    }
+    const dim3 grid((unsigned)(((long)n * gpr + 255) / 256 + (n == 0)));
+    switch (here ? gran : 16) {
+    case 16: hipLaunchKernelGGL(coo_place_kernel<uint4>, grid, block, 0, st, indices, n, g, r, gpr); break;
+    case 4: hipLaunchKernelGGL(coo_place_kernel<uint32_t>, grid, block, 0, st, indices, n, g, r, gpr); break;
+    case 2: hipLaunchKernelGGL(coo_place_kernel<uint16_t>, grid, block, 0, st, indices, n, g, r, gpr); break;
+    default: hipLaunchKernelGGL(coo_place_kernel<uint8_t>, grid, block, 0, st, indices, n, g, r, gpr); break;
+    }
+    rc = sph_check_launch(who);
+    if (rc) return rc;
+    if (move && !here) return sph_permute_rows(feature, permutation, n, row_bytes, 0, out_feature, stream);
+    return SPH_OK;
+}
+
 SPH_EXPORT int sph_init_tensor(const int32_t *indices, int n, int B, int S0, int S1, int S2, int32_t *z_idx,
                                int32_t *z_ptr, int32_t *permutation, int32_t *status, void *workspace,
                                size_t workspace_bytes, void *stream)
 {
-    SPH_REQUIRE(n >= 0 && B > 0 && S0 > 0 && S1 > 0 && S2 > 0, SPH_ERR_ARG, "sph_init_tensor: bad sizes");
-    SPH_REQUIRE((double)B * S0 * S1 < 2147483648.0, SPH_ERR_UNSUPPORTED, "sph_init_tensor: more than 2^31 columns");
-    SPH_REQUIRE(z_ptr && status && workspace && (n == 0 || (indices && z_idx && permutation)), SPH_ERR_ARG,
-                "sph_init_tensor: null pointer");
-    SPH_REQUIRE((uintptr_t)indices % 16 == 0 && (uintptr_t)workspace % 256 == 0, SPH_ERR_ARG,
-                "sph_init_tensor: indices must be 16-byte aligned, the workspace 256-byte aligned");
-    const int ncol = B * S0 * S1;
-    if (!by_bitmap(ncol, S2))
-        return init_tensor_by_rank(indices, n, B, S0, S1, S2, z_idx, z_ptr, permutation, status, workspace, workspace_bytes,
-                                   (hipStream_t)stream);
-    const BitLayout l = bit_layout(ncol, S2);
-    SPH_REQUIRE(l.total != 0, SPH_ERR_LAUNCH, "sph_init_tensor: temporary storage query failed");
-    SPH_REQUIRE(workspace_bytes >= l.total, SPH_ERR_ARG, "sph_init_tensor: workspace of %zu bytes, %zu needed",
-                workspace_bytes, l.total);
-    hipStream_t st = (hipStream_t)stream;
-    char *ws = (char *)workspace;
-    unsigned long long *bits = (unsigned long long *)(ws + l.bits);
-    const int bit_ints = (int)(l.bits_bytes / sizeof(int32_t)); // at most 2^28
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((ncol + 255) / 256), dim3(256), 0, st, z_ptr, ncol);
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, st, status, 2);
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((bit_ints + 255) / 256), dim3(256), 0, st, (int32_t *)bits, bit_ints);
-    int rc = sph_check_launch("sph_init_tensor(fill)");
-    if (rc || n == 0) return rc;
-    const dim3 grid((n + 255) / 256), block(256);
-    hipLaunchKernelGGL(coo_mark_kernel, grid, block, 0, st, indices, n, B, S0, S1, S2, l.words, z_ptr, bits, status);
-    rc = sph_check_launch("sph_init_tensor(mark)");
-    if (rc) return rc;
-    hipError_t e = sph_scan::launch<sph_scan::Plus, true>(z_ptr, z_ptr, ncol, ws + l.temp, 0, st);
-    if (e != hipSuccess) {
-        sph_set_error("sph_init_tensor: scan: %s", hipGetErrorString(e));
-        return SPH_ERR_LAUNCH;
-    }
-    hipLaunchKernelGGL(coo_place_kernel, grid, block, 0, st, indices, n, B, S0, S1, S2, l.words, (const int32_t *)z_ptr,
-                       (const unsigned long long *)bits, z_idx, permutation);
-    rc = sph_check_launch("sph_init_tensor(place)");
-    if (rc) return rc;
-    return SPH_OK;
+    return sph_init_tensor_rows(indices, n, B, S0, S1, S2, nullptr, 0, z_idx, z_ptr, permutation, nullptr, nullptr, status,
+                                nullptr, workspace, workspace_bytes, stream);
 }

@@ -235,7 +235,7 @@ SPH_EXPORT int sph_rules_conv(const int32_t *z_idx, const int32_t *z_ptr, int in
     b.by_q01 = fast_div((uint32_t)b.Q.n0 * (uint32_t)b.Q.n1);
     b.cap = a.cap;
     b.book = *book;
-    b.pack.total = 0;
+    b.pack.job[0].total = b.pack.job[1].total = 0;
     b.tile_blocks = 0;
     b.long_fibers = 0;
     const int nt = sph_book_tiles(out_rows);

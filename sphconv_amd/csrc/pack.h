@@ -11,10 +11,11 @@
 struct SphPackJob {
     const void *w;
     void *packed;
-    int elem_size;          // 1, 2 or 4 bytes
+    int elem_size;          // 1, 2 or 4 bytes of an element of the packed copy
+    int narrow;             // 0: w holds elements of that size; 1 / 2: w is fp32, rounded to fp16 / bf16 on the way
     int KV, kdim, ndim, nsteps, ntn;
     long sk, skk, sn;       // element strides of w over (k, kk, n)
-    long total;             // elements of the packed copy
+    int total;              // 16-byte fragments of the packed copy
 };
 
 static inline int sph_elem_size(sph_dtype dt) { return dt == SPH_F32 ? 4 : (dt == SPH_I8 ? 1 : 2); }
@@ -28,14 +29,15 @@ static inline int sph_pad_waves(int ndim)
 // MFMA super steps (64 bytes of every row each) of a contraction over kdim elements
 static inline int sph_num_steps(sph_dtype dt, int kdim) { return sph_div_up(kdim, 4 * sph_frag_elems(dt)); }
 static inline SphPackJob sph_pack_job(sph_dtype dt, const void *w, int KV, int kdim, int ndim, long sk, long skk,
-                                      long sn, void *packed)
+                                      long sn, void *packed, int w_f32 = 0)
 {
     SphPackJob p;
     p.w = w; p.packed = packed; p.elem_size = sph_elem_size(dt);
+    p.narrow = !w_f32 || dt == SPH_F32 ? 0 : (dt == SPH_F16 ? 1 : 2);
     p.KV = KV; p.kdim = kdim; p.ndim = ndim;
     p.nsteps = sph_num_steps(dt, kdim); p.ntn = sph_pad_waves(ndim);
     p.sk = sk; p.skk = skk; p.sn = sn;
-    p.total = (long)KV * p.nsteps * p.ntn * 64 * sph_frag_elems(dt);
+    p.total = KV * p.nsteps * p.ntn * 64;
     return p;
 }
 // argument checks shared by the entry points that pack; returns 0 or an error code (message set)
@@ -49,32 +51,61 @@ static inline int sph_pack_args_ok(const char *who, sph_dtype dt, const void *w,
     return SPH_OK;
 }
 
-#ifdef __HIPCC__
-template <typename T>
-__device__ __forceinline__ void sph_pack_elements(const SphPackJob &p, long i)
+// Up to two jobs share a launch: a training step wants the weight for its forward pass and, transposed, for dgrad.
+struct SphPackJobs {
+    SphPackJob job[2]; // total == 0: no job
+};
+static inline int sph_pack_total(const SphPackJob *jobs) { return jobs[0].total + jobs[1].total; }
+static inline int sph_pack_jobs(const char *who, const sph_pack_desc *d, int n, SphPackJobs *out)
 {
-    constexpr int KW = 16 / (int)sizeof(T);
-    if (i >= p.total) return;
-    const int j = (int)(i % KW);
-    long t = i / KW;
-    const int lane = (int)(t % 64);
-    t /= 64;
-    const int nt = (int)(t % p.ntn);
-    t /= p.ntn;
-    const int st = (int)(t % p.nsteps);
-    const int k = (int)(t / p.nsteps);
-    const int kk = st * 4 * KW + KW * (lane >> 4) + j;
-    const int n = nt * 16 + (lane & 15);
-    T v = (T)0;
-    if (kk < p.kdim && n < p.ndim) v = ((const T *)p.w)[k * p.sk + kk * p.skk + n * p.sn];
-    ((T *)p.packed)[i] = v;
+    out->job[0].total = out->job[1].total = 0;
+    if (n < 0 || n > 2 || (n > 0 && !d)) { sph_set_error("%s: 0 to 2 weights can be packed, not %d", who, n); return SPH_ERR_ARG; }
+    for (int i = 0; i < n; i++) {
+        int rc = sph_pack_args_ok(who, d[i].dt, d[i].w, d[i].packed, d[i].KV, d[i].kdim, d[i].ndim);
+        if (rc) return rc;
+        if (d[i].w_f32 && d[i].dt == SPH_I8) { sph_set_error("%s: an fp32 weight has no int8 copy", who); return SPH_ERR_ARG; }
+        if ((uintptr_t)d[i].packed % 16) { sph_set_error("%s: packed weight must be 16-byte aligned", who); return SPH_ERR_ARG; }
+        out->job[i] = sph_pack_job(d[i].dt, d[i].w, d[i].KV, d[i].kdim, d[i].ndim, d[i].stride_k, d[i].stride_kk,
+                                   d[i].stride_n, d[i].packed, d[i].w_f32);
+    }
+    return SPH_OK;
 }
 
-// element i of the job, whatever its type
-__device__ __forceinline__ void sph_pack_element(const SphPackJob &p, long i)
+#ifdef __HIPCC__
+// Fragment i of the job.  T: element of the packed copy, S: element of w.  A lane's 16 bytes are put together in
+// registers and stored at once (one division chain per 16 bytes instead of one per element); the 16 lanes of a column
+// tile read neighbouring columns (forward weights) or 16 bytes of one column each (transposed ones).
+template <typename T, typename S>
+__device__ __forceinline__ void sph_pack_fragment_as(const SphPackJob &p, int i)
 {
-    if (p.elem_size == 2) sph_pack_elements<uint16_t>(p, i);
-    else if (p.elem_size == 4) sph_pack_elements<uint32_t>(p, i);
-    else sph_pack_elements<uint8_t>(p, i);
+    constexpr int KW = 16 / (int)sizeof(T);
+    const int lane = i & 63;
+    int t = i >> 6;
+    const int nt = t % p.ntn;
+    t /= p.ntn;
+    const int st = t % p.nsteps, k = t / p.nsteps;
+    const int kk0 = st * 4 * KW + KW * (lane >> 4), n = nt * 16 + (lane & 15);
+    const S *src = (const S *)p.w + k * p.sk + kk0 * p.skk + n * p.sn;
+    union { T e[KW]; uint4 v; } u;
+#pragma unroll
+    for (int j = 0; j < KW; j++) u.e[j] = (kk0 + j < p.kdim && n < p.ndim) ? (T)src[j * p.skk] : (T)0;
+    ((uint4 *)p.packed)[i] = u.v;
+}
+
+// fragment i of the job, whatever its types (a permutation of elements, so equal types go by their size)
+__device__ __forceinline__ void sph_pack_fragment(const SphPackJob &p, int i)
+{
+    if (i >= p.total) return;
+    if (p.narrow == 1) sph_pack_fragment_as<_Float16, float>(p, i);
+    else if (p.narrow == 2) sph_pack_fragment_as<__bf16, float>(p, i);
+    else if (p.elem_size == 2) sph_pack_fragment_as<uint16_t, uint16_t>(p, i);
+    else if (p.elem_size == 4) sph_pack_fragment_as<uint32_t, uint32_t>(p, i);
+    else sph_pack_fragment_as<uint8_t, uint8_t>(p, i);
+}
+
+__device__ __forceinline__ void sph_pack_fragments(const SphPackJobs &p, int i)
+{
+    if (i < p.job[0].total) sph_pack_fragment(p.job[0], i);
+    else sph_pack_fragment(p.job[1], i - p.job[0].total);
 }
 #endif

@@ -26,7 +26,7 @@ __global__ __launch_bounds__(kThreads) void build_book_kernel(BuildArgs a)
     if ((int)blockIdx.x >= a.tile_blocks) {
         // a weight rides along with the rule generation: the copy needs a launch of its own
         // otherwise, which costs more than the copy
-        sph_pack_element(a.pack, (long)(blockIdx.x - a.tile_blocks) * kThreads + tid);
+        sph_pack_fragments(a.pack, (int)(blockIdx.x - a.tile_blocks) * kThreads + tid);
         return;
     }
     const int tile = sph_xcd_tile(blockIdx.x, (a.q_rows + R - 1) / R);
@@ -395,7 +395,7 @@ void sph_set_error(const char *fmt, ...)
 }
 
 SPH_EXPORT const char *sph_last_error(void) { return g_err; }
-SPH_EXPORT int sph_abi_version(void) { return 7; }
+SPH_EXPORT int sph_abi_version(void) { return 8; }
 SPH_EXPORT int sph_book_tiles(int rows) { return rows <= 0 ? 0 : sph_div_up(rows, R); }
 SPH_EXPORT int sph_book_cap(int KV) { return KV * (R / SPH_GROUP); }
 
@@ -418,7 +418,7 @@ SPH_EXPORT int sph_num_tiles(const sph_geom *g, int T0, int T1)
 
 static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_ptr, int in_rows, const int32_t *oz_idx,
                        const int32_t *oz_ptr, int out_rows, const sph_geom *g, int transposed, const sph_book *book,
-                       const int32_t *row_cols, const SphPackJob *pack, void *stream)
+                       const int32_t *row_cols, const SphPackJobs *pack, void *stream)
 {
     SPH_REQUIRE(sph_geom_ok(g), SPH_ERR_ARG, "%s: bad geometry (kernel volume <= %d)", who, SPH_MAX_KV);
     SPH_REQUIRE(book_ok(book), SPH_ERR_ARG, "%s: bad book", who);
@@ -448,11 +448,10 @@ static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_p
     const int nt = sph_book_tiles(book->rows);
     a.tile_blocks = book->rows > 0 ? sph_xcd_grid(nt) : 0;
     int pack_blocks = 0;
+    a.pack.job[0].total = a.pack.job[1].total = 0;
     if (pack) {
         a.pack = *pack;
-        pack_blocks = (int)((pack->total + kThreads - 1) / kThreads);
-    } else {
-        a.pack.total = 0;
+        pack_blocks = sph_div_up(sph_pack_total(pack->job), kThreads);
     }
     if (a.tile_blocks + pack_blocks == 0) return SPH_OK;
     size_t lds = (size_t)R * KV * sizeof(int32_t) + emit_scratch_bytes(KV);
@@ -489,8 +488,22 @@ SPH_EXPORT int sph_rules_build_pack(const int32_t *z_idx, const int32_t *z_ptr, 
 {
     int rc = sph_pack_args_ok("sph_rules_build_pack", dt, w, packed, KV, kdim, ndim);
     if (rc) return rc;
-    const SphPackJob p = sph_pack_job(dt, w, KV, kdim, ndim, stride_k, stride_kk, stride_n, packed);
+    SphPackJobs p;
+    p.job[0] = sph_pack_job(dt, w, KV, kdim, ndim, stride_k, stride_kk, stride_n, packed);
+    p.job[1].total = 0;
     return rules_build("sph_rules_build_pack", z_idx, z_ptr, in_rows, oz_idx, oz_ptr, out_rows, g, transposed, book,
+                       row_cols, &p, stream);
+}
+
+SPH_EXPORT int sph_rules_build_packs(const int32_t *z_idx, const int32_t *z_ptr, int in_rows,
+                                     const int32_t *oz_idx, const int32_t *oz_ptr, int out_rows,
+                                     const sph_geom *g, int transposed, const sph_book *book,
+                                     const int32_t *row_cols, const sph_pack_desc *packs, int npacks, void *stream)
+{
+    SphPackJobs p;
+    int rc = sph_pack_jobs("sph_rules_build_packs", packs, npacks, &p);
+    if (rc) return rc;
+    return rules_build("sph_rules_build_packs", z_idx, z_ptr, in_rows, oz_idx, oz_ptr, out_rows, g, transposed, book,
                        row_cols, &p, stream);
 }
 

@@ -418,8 +418,8 @@ struct BuildArgs {
     ConvParams cv;
     int cap;
     sph_book book;
-    // optional passenger: workgroups behind the tile workgroups pack a weight (total == 0: none)
-    SphPackJob pack;
+    // optional passengers: workgroups behind the tile workgroups pack one or two weights (total == 0: none)
+    SphPackJobs pack;
     int tile_blocks;
     // gathered-side fibers are long (several entries on average) and their bins fit a 64-bit mask:
     // join through per-column occupancy masks instead of walking a fiber once per row

@@ -40,11 +40,35 @@ static __global__ void clear_state_kernel(int *state, int nints)
     if (i < nints) state[i] = 0;
 }
 
+// What is scanned: an array in memory (16-byte loads where it is aligned), or any function object load(i) that makes
+// element i on the fly (an intermediate array less to write and read).
+struct FromArray {
+    const int32_t *in;
+    __device__ __forceinline__ void tile(long base, long n, int identity, int (&v)[kItems]) const
+    {
+        if (base + kItems <= n && ((uintptr_t)in & 15) == 0) {
+            const int4 a = *(const int4 *)(in + base), b = *(const int4 *)(in + base + 4);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
+#pragma unroll
+            for (int i = 0; i < kItems; i++) v[i] = base + i < n ? in[base + i] : identity;
+        }
+    }
+};
+template <class F> struct FromFunction {
+    F load;
+    __device__ __forceinline__ void tile(long base, long n, int identity, int (&v)[kItems]) const
+    {
+#pragma unroll
+        for (int i = 0; i < kItems; i++) v[i] = base + i < n ? load(base + i) : identity;
+    }
+};
+
 // out[i] = op(in[0], ..., in[i]) (INCLUSIVE) or op(init, in[0], ..., in[i-1]) (exclusive; init counts first).
 // *total (may be null; any address the GPU can write, e.g. pinned host memory) receives op over all n elements
 // (and init, for an exclusive scan).
-template <class OP, bool INCLUSIVE>
-__global__ __launch_bounds__(kThreads) void scan_kernel(const int32_t *in, int32_t *out, long n, int *state, int init,
+template <class OP, bool INCLUSIVE, class IN>
+__global__ __launch_bounds__(kThreads) void scan_kernel(IN in, int32_t *out, long n, int *state, int init,
                                                         int32_t *total)
 {
     __shared__ int s_ticket;
@@ -58,13 +82,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const int32_t *in, int32
     const long base = (long)t * kTile + (long)tid * kItems;
 
     int v[kItems];
-    if (base + kItems <= n && ((uintptr_t)in & 15) == 0) {
-        const int4 a = *(const int4 *)(in + base), b = *(const int4 *)(in + base + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-#pragma unroll
-        for (int i = 0; i < kItems; i++) v[i] = base + i < n ? in[base + i] : OP::identity();
-    }
+    in.tile(base, n, OP::identity(), v);
     // inclusive scan of the thread's items, then of the threads' totals over the wave
 #pragma unroll
     for (int i = 1; i < kItems; i++) v[i] = OP::op(v[i - 1], v[i]);
@@ -149,17 +167,23 @@ inline int state_ints(long n) { return 2 + 2 * tiles(n > 0 ? n : 1); }
 
 // Enqueues the scan of n elements on st; state: state_bytes(n) bytes of device memory, 8-byte aligned.
 // clear_state = false: a kernel enqueued before on the same stream has already zeroed the first state_ints(n) ints.
-template <class OP, bool INCLUSIVE>
-inline hipError_t launch(const int32_t *in, int32_t *out, long n, void *state, int init, hipStream_t st,
-                         int32_t *total = nullptr, bool clear_state = true)
+template <class OP, bool INCLUSIVE, class IN>
+inline hipError_t launch_from(const IN &in, int32_t *out, long n, void *state, int init, hipStream_t st,
+                              int32_t *total = nullptr, bool clear_state = true)
 {
     if (n <= 0) return hipSuccess;
     const int nt = tiles(n), nints = state_ints(n);
     if (clear_state)
         hipLaunchKernelGGL(clear_state_kernel, dim3((nints + 255) / 256), dim3(256), 0, st, (int *)state, nints);
-    hipLaunchKernelGGL((scan_kernel<OP, INCLUSIVE>), dim3(nt), dim3(kThreads), 0, st, in, out, n, (int *)state, init,
+    hipLaunchKernelGGL((scan_kernel<OP, INCLUSIVE, IN>), dim3(nt), dim3(kThreads), 0, st, in, out, n, (int *)state, init,
                        total);
     return hipGetLastError();
+}
+template <class OP, bool INCLUSIVE>
+inline hipError_t launch(const int32_t *in, int32_t *out, long n, void *state, int init, hipStream_t st,
+                         int32_t *total = nullptr, bool clear_state = true)
+{
+    return launch_from<OP, INCLUSIVE>(FromArray{in}, out, n, state, init, st, total, clear_state);
 }
 
 } // namespace sph_scan

@@ -127,3 +127,56 @@ SPH_EXPORT int sph_to_dense_backward(const void *d_dense, const int32_t *z_idx, 
 #undef CALL
     return sph_check_launch("sph_to_dense_backward");
 }
+
+// ---------------------------------------------------------------------------
+// Channels-first densify in one pass over the dense tensor: a fill, then every row's elements to their cells.  (Dense
+// rows first and a permuted copy behind them moved the dense tensor three times.)
+// ---------------------------------------------------------------------------
+static __global__ __launch_bounds__(256) void zero16_kernel(char *p, size_t bytes)
+{
+    const size_t step = (size_t)gridDim.x * 256 * 16;
+    size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 16;
+    for (; i + 16 <= bytes; i += step) *(uint4 *)(p + i) = make_uint4(0, 0, 0, 0);
+    if (i < bytes)
+        for (size_t j = i; j < bytes; j++) p[j] = 0;
+}
+
+// thread = (row, eight channels): consecutive threads take consecutive rows, whose cells lie next to each other along S2
+template <typename T>
+static __global__ __launch_bounds__(256) void dense_cf_kernel(const T *feature, const int32_t *z_idx, const int32_t *z_ptr, int rows,
+                                                              int ncol, int cols_per_sample, int S2, int C, T *out)
+{
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= rows) return;
+    const int col = column_of_row(z_ptr, ncol, r), z = z_idx[r];
+    if (col >= ncol || (unsigned)z >= (unsigned)S2) return;
+    const int b = col / cols_per_sample;
+    const size_t plane = (size_t)cols_per_sample * S2;
+    T *dst = out + (size_t)b * C * plane + (size_t)(col - b * cols_per_sample) * S2 + z;
+    const T *src = feature + (size_t)r * C;
+    const int c1 = min(C, (int)(blockIdx.y + 1) * 8);
+    for (int c = blockIdx.y * 8; c < c1; c++) dst[(size_t)c * plane] = src[c];
+}
+
+SPH_EXPORT int sph_to_dense_channels_first(const void *feature, const int32_t *z_idx, const int32_t *z_ptr, int rows, int ncol,
+                                           int cols_per_sample, int S2, int C, int elem_size, void *out, void *stream)
+{
+    const char *who = "sph_to_dense_channels_first";
+    SPH_REQUIRE(rows >= 0 && ncol > 0 && S2 > 0 && C > 0 && cols_per_sample > 0 && ncol % cols_per_sample == 0 &&
+                    (elem_size == 1 || elem_size == 2 || elem_size == 4), SPH_ERR_ARG, "%s: bad size", who);
+    SPH_REQUIRE(out && (uintptr_t)out % 16 == 0 && (rows == 0 || (feature && z_idx && z_ptr)), SPH_ERR_ARG,
+                "%s: null pointer or output not 16-byte aligned", who);
+    hipStream_t st = (hipStream_t)stream;
+    const size_t bytes = (size_t)ncol * S2 * C * elem_size;
+    const size_t want = (bytes + 4095) / 4096;
+    hipLaunchKernelGGL(zero16_kernel, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, st, (char *)out, bytes);
+    if (rows > 0) {
+        const dim3 grid((unsigned)sph_div_up(rows, 256), (unsigned)sph_div_up(C, 8)), block(256);
+#define CALL(T) hipLaunchKernelGGL(dense_cf_kernel<T>, grid, block, 0, st, (const T *)feature, z_idx, z_ptr, rows, ncol, cols_per_sample, S2, C, (T *)out)
+        if (elem_size == 4) CALL(uint32_t);
+        else if (elem_size == 2) CALL(uint16_t);
+        else CALL(uint8_t);
+#undef CALL
+    }
+    return sph_check_launch(who);
+}

@@ -11,13 +11,13 @@
 //                          the cell of every point; a point inside the grid enters its cell into a hash
 //                          table (open addressing, at most half full), counts itself there and offers
 //                          its index as the cell's first point (atomic minimum)
-//   3. vox_mark_kernel     marks the points that open a cell, in point order, behind the cells' counts
-//   4. one exclusive sum   over [counts of the table's slots | marks of the points]: a slot's segment
-//                          of the point list, and (minus the points inside) every mark's voxel number
-//   5. vox_scatter_kernel  writes every point into its cell's segment (in any order); the point
+//   3. one exclusive sum   over [counts of the table's slots | 1 for every point that opens a cell]: a slot's
+//                          segment of the point list, and (minus the points inside) every such point's voxel
+//                          number; the second half is made as it is read
+//   4. vox_scatter_kernel  writes every point into its cell's segment (in any order); the point
 //                          that would open voxel number max_voxels is where the reference's loop
 //                          stops: every later point is dropped
-//   6. vox_write_kernel    a point's place in its voxel = the number of smaller point indices in its
+//   5. vox_write_kernel    a point's place in its voxel = the number of smaller point indices in its
 //                          segment (counted until max_points are found: such a point is dropped);
 //                          segments of more than 256 points are walked by the whole wave, 64 entries at a time
 // Which slot a cell gets, and the order inside a segment, depend on the order the atomics land in;
@@ -143,25 +143,31 @@ __global__ __launch_bounds__(256) void vox_insert_kernel(const float *points, in
     slot_of[i] = (int32_t)slot;
 }
 
-__global__ __launch_bounds__(256) void vox_mark_kernel(const int32_t *slot_of, const int32_t *first, int n, int32_t *mark)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int s = slot_of[i];
-    mark[i] = s >= 0 && first[s] == i;
-}
+// what the scan reads: the counts of the table's slots, then 1 for every point that opens a cell, made on the fly
+struct CountsThenMarks {
+    const int32_t *count, *slot_of, *first;
+    long T;
+    __device__ __forceinline__ int operator()(long i) const
+    {
+        if (i < T) return count[i];
+        const int p = (int)(i - T), s = slot_of[p];
+        return s >= 0 && first[s] == p;
+    }
+};
 
 // sum[0..T): first place of every slot's segment; sum[T + i] - sum[T]: marks in front of point i; *total: all of it
-__global__ __launch_bounds__(256) void vox_scatter_kernel(const int32_t *slot_of, const int32_t *sum, const int32_t *mark,
+__global__ __launch_bounds__(256) void vox_scatter_kernel(const int32_t *slot_of, const int32_t *sum, const int32_t *first,
                                                           const int32_t *total, int n, long T, int max_voxels,
                                                           int32_t *count, int32_t *seg, int32_t *stop, int32_t *voxel_num)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int s = slot_of[i];
-    if (s >= 0) seg[sum[s] + atomicSub(&count[s], 1) - 1] = i;
     const int inside = sum[T];
-    if (mark[i] && sum[T + i] - inside == max_voxels) *stop = i; // exactly one such point, if any
+    if (s >= 0) {
+        seg[sum[s] + atomicSub(&count[s], 1) - 1] = i;
+        if (first[s] == i && sum[T + i] - inside == max_voxels) *stop = i; // exactly one such point, if any
+    }
     if (i == 0) *voxel_num = min(*total - inside, max_voxels);
 }
 
@@ -240,7 +246,7 @@ inline VoxLayout vox_layout(int n)
     size_t o = 0;
     l.keys = o; o += al256((size_t)l.T * 8);
     l.first = o; o += al256((size_t)l.T * 4);
-    l.count = o; o += al256(((size_t)l.T + nn) * 4); // the slots' counts, then the points' marks
+    l.count = o; o += al256((size_t)l.T * 4);
     l.sum = o; o += al256(((size_t)l.T + nn) * 4);
     l.slot_of = o; o += al256(nn * 4);
     l.seg = o; o += al256(nn * 4);
@@ -291,7 +297,7 @@ SPH_EXPORT int sph_points_to_voxel(const float *points, int n, int nfeat, int sy
     unsigned long long *keys = (unsigned long long *)(ws + l.keys);
     int32_t *first = (int32_t *)(ws + l.first), *count = (int32_t *)(ws + l.count), *sum = (int32_t *)(ws + l.sum);
     int32_t *slot_of = (int32_t *)(ws + l.slot_of), *seg = (int32_t *)(ws + l.seg), *stop = (int32_t *)(ws + l.stop);
-    int32_t *total = stop + 1, *mark = count + l.T;
+    int32_t *total = stop + 1;
 
     const int width = append_mode == 1 ? nfeat + 3 : nfeat;
     const long nv = (long)max_voxels * max_points;
@@ -305,7 +311,7 @@ SPH_EXPORT int sph_points_to_voxel(const float *points, int n, int nfeat, int sy
     fill(mask, nv, 0);
     fill(coors, 3L * max_voxels, 0);
     fill(num_points, (long)max_voxels, 0);
-    fill(voxel_num, 1L, 0);
+    if (n == 0) fill(voxel_num, 1L, 0); // else it is written once, by the scatter kernel: the host may be watching it
     if (n > 0) {
         fill(keys, 2 * l.T, -1);
         fill(first, l.T, INT_MAX);
@@ -318,19 +324,84 @@ SPH_EXPORT int sph_points_to_voxel(const float *points, int n, int nfeat, int sy
     if (rc || n == 0) return rc;
     hipLaunchKernelGGL(vox_insert_kernel, dim3(blocks(n)), dim3(256), 0, st, points, n, q, cell_in, l.tbits, keys, first,
                        count, slot_of, cell_out);
-    hipLaunchKernelGGL(vox_mark_kernel, dim3(blocks(n)), dim3(256), 0, st, (const int32_t *)slot_of, (const int32_t *)first,
-                       n, mark);
     rc = sph_check_launch("sph_points_to_voxel(cells)");
     if (rc) return rc;
-    const hipError_t e = sph_scan::launch<sph_scan::Plus, false>(count, sum, l.T + n, ws + l.state, 0, st, total, false);
+    const hipError_t e = sph_scan::launch_from<sph_scan::Plus, false>(
+        sph_scan::FromFunction<CountsThenMarks>{CountsThenMarks{count, slot_of, first, l.T}}, sum, l.T + n, ws + l.state, 0, st, total, false);
     if (e != hipSuccess) {
         sph_set_error("sph_points_to_voxel: scan: %s", hipGetErrorString(e));
         return SPH_ERR_LAUNCH;
     }
     hipLaunchKernelGGL(vox_scatter_kernel, dim3(blocks(n)), dim3(256), 0, st, (const int32_t *)slot_of, (const int32_t *)sum,
-                       (const int32_t *)mark, (const int32_t *)total, n, l.T, max_voxels, count, seg, stop, voxel_num);
+                       (const int32_t *)first, (const int32_t *)total, n, l.T, max_voxels, count, seg, stop, voxel_num);
     hipLaunchKernelGGL(vox_write_kernel, dim3(blocks(n)), dim3(256), 0, st, points, n, q, (const unsigned long long *)keys,
                        (const int32_t *)first, (const int32_t *)slot_of, (const int32_t *)sum, (const int32_t *)seg, l.T,
                        (const int32_t *)stop, voxels, mask, coors, num_points);
     return sph_check_launch("sph_points_to_voxel");
+}
+
+// ---------------------------------------------------------------------------
+// What follows the voxeliser on the way to a sparse tensor: the mean of a voxel's points (SimpleVoxel,
+// sphconv/vfe.py:210-228) and the batch's coordinates (merge_batch_torch, sphconv/datagen.py:53-74).  As tensor
+// operations these are three and two or more launches of a few microseconds each for 24 000 voxels.
+// ---------------------------------------------------------------------------
+static __global__ __launch_bounds__(256) void voxel_mean_kernel(const float *voxels, const int32_t *num, int nv, int max_points,
+                                                                int width, int nf, float *out)
+{
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    const long v = t / nf;
+    const int f = (int)(t - v * nf);
+    if (v >= nv) return;
+    const float *p = voxels + v * max_points * width + f;
+    float s = 0.f;
+    for (int j = 0; j < max_points; j++) s += p[(long)j * width];
+    out[t] = __fdiv_rn(s, (float)num[v]);
+}
+
+SPH_EXPORT int sph_voxel_mean(const float *voxels, const int32_t *num_points, int nv, int max_points, int width, int nf,
+                              float *out, void *stream)
+{
+    SPH_REQUIRE(nv >= 0 && max_points > 0 && nf > 0 && width >= nf, SPH_ERR_ARG, "sph_voxel_mean: bad sizes");
+    if (nv == 0) return SPH_OK;
+    SPH_REQUIRE(voxels && num_points && out, SPH_ERR_ARG, "sph_voxel_mean: null pointer");
+    hipLaunchKernelGGL(voxel_mean_kernel, dim3(blocks((long)nv * nf)), dim3(256), 0, (hipStream_t)stream, voxels, num_points, nv,
+                       max_points, width, nf, out);
+    return sph_check_launch("sph_voxel_mean");
+}
+
+namespace {
+struct CoordParts {
+    const int32_t *p[SPH_MAX_BATCH_PARTS]; // [rows, 3] each
+    int first[SPH_MAX_BATCH_PARTS + 1];    // first output row of every part
+    int n;
+};
+} // namespace
+
+static __global__ __launch_bounds__(256) void batch_coordinates_kernel(CoordParts c, int4 *out)
+{
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= c.first[c.n]) return;
+    int b = 0;
+    while (r >= c.first[b + 1]) b++;
+    const int32_t *p = c.p[b] + 3L * (r - c.first[b]);
+    out[r] = make_int4(b, p[0], p[1], p[2]);
+}
+
+SPH_EXPORT int sph_batch_coordinates(const int32_t *const *parts, const int32_t *rows, int nparts, int32_t *out, void *stream)
+{
+    SPH_REQUIRE(parts && rows && nparts > 0 && nparts <= SPH_MAX_BATCH_PARTS && (uintptr_t)out % 16 == 0, SPH_ERR_ARG,
+                "sph_batch_coordinates: 1 to %d parts and a 16-byte aligned output", SPH_MAX_BATCH_PARTS);
+    CoordParts c;
+    c.n = nparts;
+    c.first[0] = 0;
+    for (int b = 0; b < nparts; b++) {
+        SPH_REQUIRE(rows[b] >= 0 && (rows[b] == 0 || parts[b]), SPH_ERR_ARG, "sph_batch_coordinates: null part");
+        c.p[b] = parts[b];
+        c.first[b + 1] = c.first[b] + rows[b];
+    }
+    const int total = c.first[nparts];
+    if (total == 0) return SPH_OK;
+    SPH_REQUIRE(out, SPH_ERR_ARG, "sph_batch_coordinates: null output");
+    hipLaunchKernelGGL(batch_coordinates_kernel, dim3(blocks(total)), dim3(256), 0, (hipStream_t)stream, c, (int4 *)out);
+    return sph_check_launch("sph_batch_coordinates");
 }
