@@ -23,6 +23,8 @@ class Convolution(SphModule):
     """Holds the weight ``[K0,K1,K2,iC,oC]`` (conv.py:43-72).  As in the reference,
     a bias parameter can be created but is not applied by ``forward``."""
 
+    is_convolution = True
+
     def __init__(self, in_channels: int, out_channels: int, kernel_size, stride, padding, dilation,
                  groups: int, tile_size: List[int], bias: bool, subm: bool, name: Optional[str],
                  indice_key: Optional[str] = None, **kwargs):
@@ -141,32 +143,37 @@ class Conv3d(Convolution):
         in_shape = [input.D, input.W, input.H]
         out_shape = in_shape if self.subm else out_spatial(in_shape, self.kernel_size, self.stride,
                                                             self.padding, self.dilation)
-        weight = self.weight.view(-1, self.in_channels, self.out_channels)
-        training = torch.is_grad_enabled() and (weight.requires_grad or input.feature.requires_grad)
+        feature, weight = input.feature, self.weight
+        grad = torch.is_grad_enabled()
+        training = grad and (weight.requires_grad or feature.requires_grad)
         oz_idx, oz_ptr, book, rule_size, tile_grid_shape = self._rules(
             input, out_shape, ahead, keep=training or self.indice_key is not None, training=training)
-        self.rule_book = book if isinstance(book, RuleBook) else None
-        if epilogue is not None:
-            if training:
-                raise RuntimeError("a fused epilogue has no backward: call under torch.no_grad()")
-            scale, shift, relu = epilogue
-            w = weight if weight.dtype == input.feature.dtype else weight.to(input.feature.dtype)
-            out_feature = ext.rule_conv(input.feature, w, book, rule_size, oz_idx.shape[0], scale, shift,
-                                        bool(relu), cache_packed=not self.training and w is weight)
-        elif not training:
-            w = weight if weight.dtype == input.feature.dtype else weight.to(input.feature.dtype)
-            # (the view itself, not a detached copy of it: the kept packed weight is looked up by the parameter behind it)
-            out_feature = ext.rule_conv(input.feature, w, book, rule_size, oz_idx.shape[0],
-                                        cache_packed=not self.training and w is weight)
+        native = isinstance(book, RuleBook)
+        self.__dict__["rule_book"] = book if native else None      # a plain attribute: no need to ask nn.Module
+        if epilogue is not None and training:
+            raise RuntimeError("a fused epilogue has no backward: call under torch.no_grad()")
+        rows = oz_idx.shape[0]
+        if training:
+            out_feature = ConvFunction.apply(feature, weight.view(-1, self.in_channels, self.out_channels), book,
+                                             rule_size, tile_grid_shape, rows)
         else:
-            out_feature = ConvFunction.apply(input.feature, weight, book, rule_size, tile_grid_shape,
-                                             oz_idx.shape[0])
-        out = SparseConvTensor(out_feature, out_shape, input.B, z_ptr=oz_ptr, z_idx=oz_idx)
-        out.rule_cache = input.rule_cache
+            scale, shift, relu = epilogue if epilogue is not None else (None, None, False)
+            keep = not self.training and not grad and weight.dtype == feature.dtype
+            packed = ext._kept_packed(weight, ext.L.stream()) if keep and native else None
+            if packed is not None:
+                out_feature = ext._conv_packed(feature, packed, self.in_channels, self.out_channels, book, rows, scale,
+                                               shift, bool(relu))
+            else:
+                # (the view itself, not a detached copy of it: the kept packed weight is looked up by the parameter
+                # behind it)
+                w = weight.view(-1, self.in_channels, self.out_channels)
+                if w.dtype != feature.dtype:
+                    w = w.to(feature.dtype)
+                out_feature = ext.rule_conv(feature, w, book, rule_size, rows, scale, shift, bool(relu), cache_packed=keep)
         # the rows' columns, where known: the input's own for a submanifold layer, a by-product of the
         # output-coordinate kernels for a strided one
-        out.row_cols = book.out_row_cols if isinstance(book, RuleBook) else None
-        return out
+        return SparseConvTensor._of(out_feature, out_shape, input.B, oz_idx, oz_ptr,
+                                    book.out_row_cols if native else None, input.rule_cache)
 
 
 SparseConv3d = Conv3d

@@ -2,6 +2,7 @@
 import numpy as np
 import torch
 
+from . import _lib as L
 from .vfe import SimpleVoxel
 from .voxelize import VoxelGeneratorV3
 
@@ -13,6 +14,7 @@ _CONCATENATED = frozenset(("voxels", "voxel", "num_points", "num_gt", "voxel_lab
 # points per voxel, voxel budget
 _POINT_RANGE = (6, -40, -3, 70.4, 40, 1)
 _SPHERE_RANGE = (6, -45, 87.5, 70.4, 45, 100)
+_MAX_PARTS = 64                        # SPH_MAX_BATCH_PARTS of the header
 _POINTS_PER_VOXEL, _MAX_VOXELS = 2, 24000
 
 
@@ -26,6 +28,10 @@ def merge_batch_torch(batch_list):
     merged = {}
     for name in names:
         parts = [example[name] for example in batch_list if name in example]
+        if name == "coordinates" and len(parts) <= _MAX_PARTS and all(
+                c.is_cuda and c.dtype == torch.int32 and c.dim() == 2 and c.shape[1] == 3 and c.is_contiguous() for c in parts):
+            merged[name] = L.host().batch_coordinates(parts)                               # one kernel
+            continue
         if name == "coordinates":
             parts = [torch.cat([torch.full((c.shape[0], 1), b, dtype=c.dtype, device=c.device), c], dim=1)
                      for b, c in enumerate(parts)]

@@ -27,6 +27,19 @@ class ConvFunction(torch.autograd.Function):
         if packed is not None and weight.dtype != feature.dtype:
             packed = None                       # packed in the weight's type, the kernel needs the feature's
         book.keep = True                        # backward walks the book
+        ctx.packed_t = None
+        ic, oc = weight.shape[1], weight.shape[2]
+        if packed is None and ctx.needs_input_grad[0] and feature.is_cuda and (weight.dtype == feature.dtype or weight.dtype == torch.float32) \
+                and weight.is_contiguous() and feature.shape[1] == ic and book.kv == weight.shape[0]:
+            # the weight is put in order for the forward pass and for dgrad at once (an fp32 master weight is rounded
+            # to the features' type on the way), by the rule kernel's own launch where the book is still to be built
+            # by one of its own; autograd refuses a weight that was changed in place before backward
+            w = weight.detach()
+            if not book.built and not book.goes_in_one_launch(ic, oc, feature.element_size()):
+                packed, ctx.packed_t = book._build_for_training(w, feature.dtype)
+            else:
+                packed, ctx.packed_t = ext.L.host().pack_weight_both(w, book.mirrored(), ext.L.dtype_code(feature.dtype))
+            return ext._conv_packed(feature, packed, ic, oc, book, outNNZ)
         return ext.rule_conv(feature, weight, book, None, outNNZ, packed=packed)
 
     @staticmethod
@@ -38,13 +51,15 @@ class ConvFunction(torch.autograd.Function):
             d_out = d_out.to(feature.dtype)
         d_feature = d_weight = None
         if ctx.needs_input_grad[0]:
-            w = weight if weight.dtype == feature.dtype else weight.to(feature.dtype)
+            ic, oc = weight.shape[1], weight.shape[2]
             # contraction over oC with W[k]^T: packed straight from [KV,iC,oC], no permuted copy
-            buf, reverse = ext._dgrad_buffers(book, d_out, w.shape[2], w.shape[1])
+            buf, reverse = ext._dgrad_buffers(book, d_out, oc, ic)
             if buf is None:
                 buf = book.transposed()
-            packed = ext._packed_weight(w, True, reverse)
-            d_feature = ext._apply(d_out, packed, w.shape[2], w.shape[1], buf)
+            packed = ctx.packed_t
+            if packed is None:
+                packed = ext._packed_weight(weight if weight.dtype == feature.dtype else weight.to(feature.dtype), True, reverse)
+            d_feature = ext._apply(d_out, packed, oc, ic, buf)
         if ctx.needs_input_grad[1]:
             # an fp32 master weight gets its gradient straight from the fp32 reduction, not through a 16-bit type
             want_f32 = weight.dtype == torch.float32
@@ -60,6 +75,8 @@ class ToDenseFunction(torch.autograd.Function):
     def forward(ctx, feature, z_idx, z_ptr, shape: List[int]):
         ctx.save_for_backward(z_idx, z_ptr)
         B, C, S0, S1, S2 = shape
+        if feature.is_cuda and feature.element_size() <= 4:
+            return ext.L.host().to_dense_channels_first(feature, z_idx, z_ptr, B, C, S0, S1, S2)
         res = torch.zeros((B, S0, S1, S2, C), device=feature.device, dtype=feature.dtype)
         ext.to_dense(feature, z_idx, z_ptr, S2, res)
         return res.permute(0, 4, 1, 2, 3).contiguous()
@@ -75,14 +92,14 @@ class InitTensorFunction(torch.autograd.Function):
     """COO rows -> per-column compressed rows (functional.py:109-131)."""
 
     @staticmethod
-    def forward(ctx, raw_feature, indices_bzyx, batchsize: int, spatial_shape: List[int]):
-        feature_out, z_idx, z_ptr, permutation = ext.init_tensor(raw_feature, indices_bzyx, batchsize,
-                                                                  spatial_shape)
+    def forward(ctx, raw_feature, indices_bzyx, batchsize: int, spatial_shape: List[int], with_columns: bool = False):
+        """``with_columns``: also return the column of every row (no reference counterpart)."""
+        feature_out, z_idx, z_ptr, permutation, cols = ext._init_tensor(raw_feature, indices_bzyx, batchsize, spatial_shape)
         ctx.save_for_backward(permutation)
-        ctx.mark_non_differentiable(z_idx, z_ptr)
-        return feature_out, z_idx, z_ptr
+        ctx.mark_non_differentiable(z_idx, z_ptr, cols)
+        return (feature_out, z_idx, z_ptr, cols) if with_columns else (feature_out, z_idx, z_ptr)
 
     @staticmethod
-    def backward(ctx, d_featureOut, d_zidx, d_zptr):
+    def backward(ctx, d_featureOut, *_):
         permutation, = ctx.saved_tensors
-        return ext.init_tensor_backward(d_featureOut, permutation), None, None, None
+        return ext.init_tensor_backward(d_featureOut, permutation), None, None, None, None

@@ -14,21 +14,26 @@ class SphModule(nn.Module):
     """Marker base class: modules derived from it receive the SparseConvTensor
     itself inside :class:`Sequential`; any other module receives ``.feature``."""
 
+    is_convolution = False
+
 
 def is_sph_module(module) -> bool:
     return isinstance(module, SphModule)
 
 
 def is_sparse_conv(module) -> bool:
-    from .conv import Convolution
-    return isinstance(module, Convolution)
+    return isinstance(module, SphModule) and module.is_convolution
 
 
 def _bn_affine(bn: nn.BatchNorm1d):
     """Evaluation-mode BatchNorm1d as y = x*scale + shift (fp32 [C]); computed once per state of
     the module's tensors (their version counters) and kept on the module."""
-    tensors = (bn.running_mean, bn.running_var, bn.weight, bn.bias)
-    key = tuple((t.data_ptr(), t._version, t.dtype) if t is not None else None for t in tensors) + (bn.eps,)
+    key = [bn.eps]
+    for t in (bn.running_mean, bn.running_var, bn.weight, bn.bias):
+        if t is not None:
+            key += (t.data_ptr(), t._version, t.dtype)
+        else:
+            key.append(None)
     cached = getattr(bn, "_sph_affine", None)
     if cached is not None and cached[0] == key:
         return cached[1], cached[2]
@@ -118,6 +123,8 @@ class Sequential(SphModule):
         from .tensor import SparseConvTensor
         mods = list(self._modules.items())
         only = [m for _, m in mods]
+        conv = [is_sparse_conv(m) for m in only]
+        profiling = torch.autograd._profiler_enabled()
         skip = 0
         ahead = {}      # index of a strided convolution -> its count on the way
 
@@ -127,13 +134,13 @@ class Sequential(SphModule):
                 return
             for j in range(first, len(only)):
                 m = only[j]
-                if is_sparse_conv(m) and not m.subm:
+                if conv[j] and not m.subm:
                     if hasattr(m, "count_ahead"):
                         h = m.count_ahead(input)
                         if h is not None:
                             ahead[j] = h
                     return
-                if is_sph_module(m) and not is_sparse_conv(m):
+                if not conv[j] and is_sph_module(m):
                     return          # a module that may change the coordinates
 
         start_count(0)
@@ -145,7 +152,7 @@ class Sequential(SphModule):
                 assert isinstance(input, SparseConvTensor)
                 # a range costs 5 us of host time per module: only for a profiler that is there to see it
                 with (torch.autograd.profiler.record_function("sphconv:{}:{}".format(type(module).__name__, name))
-                      if torch.autograd._profiler_enabled() else _NO_RANGE):
+                      if profiling else _NO_RANGE):
                     skip, bn, relu = self._fusable_tail(only, i)
                     kw = {"ahead": ahead.pop(i)} if i in ahead else {}
                     if skip:
@@ -153,7 +160,7 @@ class Sequential(SphModule):
                         input = module(input, epilogue=(scale, shift, relu), **kw)
                     else:
                         input = module(input, **kw)
-                    if is_sparse_conv(module) and not module.subm:
+                    if conv[i] and not module.subm:
                         start_count(i + 1)      # new coordinates: the next strided layer can start counting
             elif isinstance(input, SparseConvTensor):
                 input.feature = module(input.feature)

@@ -41,6 +41,7 @@ class ScanPipeline:
             raise L.SphconvError("weight holds %d offsets, kernel %s has %d" % (self.kv, self.kernel,
                                  self.kernel[0] * self.kernel[1] * self.kernel[2]))
         self.batch, self.shape = int(batch), [int(v) for v in shape]
+        self._z_shape = (self.batch, self.shape[0], self.shape[1])
         self.max_voxels = int(max_voxels)
         self.dt = L.dtype_code(self.weight.dtype)
         dev = self.weight.device
@@ -97,7 +98,7 @@ class ScanPipeline:
             raise L.SphconvError("scan of %d voxels, pipeline sized for %d" % (n, self.max_voxels))
         if feature.shape != (n, self.ic) or feature.dtype != self.weight.dtype or not feature.is_contiguous():
             raise L.SphconvError("feature must be contiguous [%d,%d] %s" % (n, self.ic, self.weight.dtype))
-        _check_index_tensors(z_idx, z_ptr, self.batch, self.shape)
+        _check_index_tensors(z_idx, z_ptr, self._z_shape)
         slot = self._next
         self._next = (slot + 1) % len(self._streams)
         side = self._streams[slot]

@@ -15,9 +15,8 @@ from . import _lib as L
 
 
 class _Buffers:
-    """Device arrays of one book (forward or transposed), carved out of ONE allocation
-    (a single caching-allocator call per book); the named tensors are views made on
-    first access."""
+    """Device arrays of one book (forward or transposed), carved out of ONE allocation by the host extension; the
+    named tensors are views made on first access."""
 
     _FIELDS = ("tile_ngrp", "tile_koff", "grp_k", "grp_gather", "grp_owner", "tile_nbr")
 
@@ -25,40 +24,32 @@ class _Buffers:
         """``by_row`` also keeps the pairs by stationary row (``tile_nbr`` [NT,KV,128]), the form the
         convolution walks when neighbourhoods are dense; with it, ``groups=False`` leaves the groups out
         (forward-only use: the rule kernel then writes a fifth of the bytes)."""
-        lib = L.lib()
         self.rows, self.kv = int(rows), int(kv)
-        self.ntiles = lib.sph_book_tiles(self.rows)
-        self.cap = lib.sph_book_cap(self.kv)
         self.by_row = bool(by_row)
         self.groups = bool(groups) or not self.by_row
-        nt = max(self.ntiles, 1)
-        g = 1 if self.groups else 0
-        sizes = (nt * 4, nt * (self.kv + 1) * 2, g * nt * self.cap * 4, g * nt * self.cap * L.GROUP * 4,
-                 g * nt * self.cap * L.GROUP * 4, nt * self.kv * L.TILE_ROWS * 4 if by_row else 0)
-        self._off = []
-        total = 0
-        for sz in sizes:
-            self._off.append(total)
-            total += (sz + 255) & ~255
-        self._sizes = sizes
-        self.storage = torch.empty(total, dtype=torch.uint8, device=device)
-        base = self.storage.data_ptr()
-        ptrs = [base + o for o in self._off]
-        if not self.groups:
-            ptrs[2] = ptrs[3] = ptrs[4] = None
-        self._struct = L.Book(*ptrs[:5], self.rows, self.kv, ptrs[5] if by_row else None, 0)
-        self._views = {}
+        if not isinstance(device, torch.device):
+            device = torch.device(device)
+        self.native = L.host().BookBuffers(self.rows, self.kv, device, self.by_row, self.groups)
+        self._struct = None
+        self._views = None
 
     def struct(self) -> L.Book:
+        """The book as the C ABI takes it (the extension's own struct: what is set here, its calls see)."""
+        if self._struct is None:
+            self._struct = L.Book.from_address(self.native.address)
         return self._struct
 
     def __getattr__(self, name):
+        if name in ("storage", "ntiles", "cap"):
+            return getattr(self.native, name)
         # views of the single allocation, typed and shaped like the C arrays
         if name in _Buffers._FIELDS:
+            if self._views is None:
+                self._views = {}
             v = self._views.get(name)
             if v is None:
-                i = _Buffers._FIELDS.index(name)
-                raw = self.storage[self._off[i]:self._off[i] + self._sizes[i]]
+                first, size = self.native.range(_Buffers._FIELDS.index(name))
+                raw = self.storage[first:first + size]
                 v = raw.view(torch.int16 if name == "tile_koff" else torch.int32)
                 if name == "tile_koff":
                     v = v.view(max(self.ntiles, 1), self.kv + 1)
@@ -82,7 +73,41 @@ class _Buffers:
         return int(((own >= 0) & used).sum().item())
 
 
-_NO_EPILOGUE = L.Epilogue(None, None, 0)
+
+class _Geometry:
+    """One convolution geometry: the C struct and what Python wants to know of it.  Made once per geometry and shared
+    by every book that has it (a network meets a few dozen)."""
+
+    __slots__ = ("native", "batch", "in_shape", "out_shape", "kernel", "stride", "padding", "dilation", "kv", "in_cells",
+                 "out_cells", "steps", "odd_same", "z_shape")
+
+    def __init__(self, batch, in_shape, out_shape, kernel, stride, padding, dilation):
+        self.batch = batch
+        self.in_shape, self.out_shape, self.kernel = list(in_shape), list(out_shape), list(kernel)
+        self.stride, self.padding, self.dilation = list(stride), list(padding), list(dilation)
+        self.kv = kernel[0] * kernel[1] * kernel[2]
+        self.in_cells = max(batch * in_shape[0] * in_shape[1] * in_shape[2], 1)
+        self.out_cells = max(batch * out_shape[0] * out_shape[1] * out_shape[2], 1)
+        self.steps = stride[0] * stride[1] * stride[2]
+        self.z_shape = (batch, in_shape[0], in_shape[1])
+        # odd kernel, stride 1, padding K//2: a submanifold book is then its own transpose, offsets mirrored
+        self.odd_same = all(k % 2 == 1 for k in kernel) and self.steps == 1 and all(p == k // 2 for p, k in zip(padding, kernel))
+        self.native = L.host().Geometry(batch, self.in_shape, self.out_shape, self.kernel, self.stride, self.padding,
+                                        self.dilation)
+
+
+_GEOMETRIES = {}
+
+
+def _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation) -> _Geometry:
+    key = (batch, *in_shape, *out_shape, *kernel, *stride, *padding, *dilation)
+    g = _GEOMETRIES.get(key)
+    if g is None:
+        if len(_GEOMETRIES) >= 4096:                     # a program with ever new shapes: start over
+            _GEOMETRIES.clear()
+        g = _Geometry(int(batch), *(tuple(int(v) for v in x) for x in (in_shape, out_shape, kernel, stride, padding, dilation)))
+        _GEOMETRIES[key] = g
+    return g
 
 # Estimated pairs per stationary row from which a book also keeps its pairs by row (and the
 # convolution walks that form).  float("inf") never does, 0 always.
@@ -100,30 +125,43 @@ class RuleBook:
 
     def __init__(self, z_idx, z_ptr, oz_idx, oz_ptr, batch, in_shape, out_shape, kernel, stride,
                  padding, dilation, subm, row_cols=None, out_row_cols=None):
+        self._take(_geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation), z_idx, z_ptr, oz_idx, oz_ptr,
+                   subm, row_cols, out_row_cols)
+
+    @classmethod
+    def _of(cls, geometry, z_idx, z_ptr, oz_idx, oz_ptr, subm, row_cols, out_row_cols) -> "RuleBook":
+        rb = cls.__new__(cls)
+        rb._take(geometry, z_idx, z_ptr, oz_idx, oz_ptr, subm, row_cols, out_row_cols)
+        return rb
+
+    def _take(self, geometry, z_idx, z_ptr, oz_idx, oz_ptr, subm, row_cols, out_row_cols):
+        self._geometry = geometry
         self.z_idx, self.z_ptr = z_idx, z_ptr
         self.oz_idx, self.oz_ptr = oz_idx, oz_ptr
         # optional: the column of every input / output row (what init_tensor and the output-coordinate kernels know
         # when they write the rows); the rule kernel then need not search z_ptr for them
         self.row_cols, self.out_row_cols = row_cols, out_row_cols
-        self.batch = int(batch)
-        self.in_shape = [int(v) for v in in_shape]
-        self.out_shape = [int(v) for v in out_shape]
-        self.kernel = [int(v) for v in kernel]
-        self.stride = [int(v) for v in stride]
-        self.padding = [int(v) for v in padding]
-        self.dilation = [int(v) for v in dilation]
         self.subm = bool(subm)
-        self.kv = self.kernel[0] * self.kernel[1] * self.kernel[2]
-        self.in_rows = int(z_idx.shape[0]) if z_idx is not None else 0
-        self.out_rows = int(oz_idx.shape[0]) if oz_idx is not None else 0
+        self.kv = geometry.kv
+        self.in_rows = z_idx.shape[0] if z_idx is not None else 0
+        self.out_rows = oz_idx.shape[0] if oz_idx is not None else 0
         self._fwd: Optional[_Buffers] = None   # built on first use (see ``fwd``)
         self._bwd: Optional[_Buffers] = None
         self.keep = True                       # a fused rules + forward launch also writes the book (``fused_forward``)
         # (input channels, output channels, element size) of the forward pass a lazy book is made for, when no
         # gradient will be asked of it: lets a book that goes by rows leave its groups out (see ``_build``)
         self.forward_only: Optional[tuple] = None
-        self._padded = {}
+        self._padded = None
         self._from_padded = None     # (rules, rule_size) when built from reference-format tensors
+
+    # the geometry's numbers (None / 0 for a book made from padded tensors, which has none)
+    batch = property(lambda self: self._geometry.batch if self._geometry is not None else 0)
+    in_shape = property(lambda self: self._geometry.in_shape if self._geometry is not None else None)
+    out_shape = property(lambda self: self._geometry.out_shape if self._geometry is not None else None)
+    kernel = property(lambda self: self._geometry.kernel if self._geometry is not None else None)
+    stride = property(lambda self: self._geometry.stride if self._geometry is not None else None)
+    padding = property(lambda self: self._geometry.padding if self._geometry is not None else None)
+    dilation = property(lambda self: self._geometry.dilation if self._geometry is not None else None)
 
     # -- construction -----------------------------------------------------
     @property
@@ -148,12 +186,10 @@ class RuleBook:
     def _pairs_per_row(self, transposed: bool) -> float:
         """Pairs a stationary row can expect: kernel volume x occupancy of the gathered side's grid
         (a stride thins the offsets that can pair with an input row)."""
-        rows, shape = (self.out_rows, self.out_shape) if transposed else (self.in_rows, self.in_shape)
-        cells = max(self.batch * shape[0] * shape[1] * shape[2], 1)
-        est = self.kv * rows / cells
+        g = self._geometry
         if transposed:
-            est /= self.stride[0] * self.stride[1] * self.stride[2]
-        return est
+            return g.kv * self.out_rows / g.out_cells / g.steps
+        return g.kv * self.in_rows / g.in_cells
 
     def _rows_kernel_takes(self, weight, weight_transposed: bool) -> bool:
         """Whether ``sph_conv_apply`` can walk this layer by stationary row (rows of 16-byte multiples up
@@ -184,37 +220,29 @@ class RuleBook:
                 by_row = est >= BY_ROW_MIN_PAIRS * BY_ROW_FORWARD_ONLY
             groups = not (by_row and forward_only)
         buf = _Buffers(rows, self.kv, self.z_ptr.device, by_row, groups)
-        buf.struct().middle_run = int(self.subm)     # every row pairs with itself at the middle offset
-        g, b = self.geom(), buf.struct()
-        lib = L.lib()
-        hint = _row_cols_ptr(self.row_cols if transposed else self.out_row_cols, rows)
+        buf.native.middle_run = int(self.subm)       # every row pairs with itself at the middle offset
+        hint = self.row_cols if transposed else self.out_row_cols
+        where = (self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, transposed, buf.native, hint)
         if weight is None:
-            rc = lib.sph_rules_build(self.z_idx.data_ptr(), self.z_ptr.data_ptr(), self.in_rows,
-                                     self.oz_idx.data_ptr(), self.oz_ptr.data_ptr(), self.out_rows,
-                                     C.byref(g), int(transposed), C.byref(b), hint, L.stream())
-            if rc:
-                L.check(rc)
+            L.host().rules_build(*where)
             return buf
         w = weight.detach()
         if not w.is_contiguous():
             w = w.contiguous()
         if not w.is_cuda or w.dim() != 3:
             raise L.SphconvError("weight must be a GPU tensor [KV,iC,oC]")
-        kv, wa, wb = w.shape
-        kdim, ndim = (wb, wa) if weight_transposed else (wa, wb)
-        skk, sn = (1, wb) if weight_transposed else (wb, 1)
-        dt = L.dtype_code(w.dtype)
-        nbytes = lib.sph_weight_packed_bytes(dt, kv, kdim, ndim)
-        if nbytes == 0:
-            raise L.SphconvError("cannot pack weight of shape %s" % (tuple(w.shape),))
-        packed = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
-        rc = lib.sph_rules_build_pack(self.z_idx.data_ptr(), self.z_ptr.data_ptr(), self.in_rows,
-                                      self.oz_idx.data_ptr(), self.oz_ptr.data_ptr(), self.out_rows,
-                                      C.byref(g), int(transposed), C.byref(b), hint, dt, w.data_ptr(), kv, kdim, ndim,
-                                      wa * wb, skk, sn, packed.data_ptr(), L.stream())
-        if rc:
-            L.check(rc)
-        return buf, packed
+        return buf, L.host().rules_build_pack(*where, w, int(bool(weight_transposed)), False, L.dtype_code(w.dtype))
+
+    def _build_for_training(self, weight, dtype):
+        """The forward book and, by the same launch, the layer's weight (its own type or fp32, rounded to ``dtype``)
+        in fragment order for the forward pass and for dgrad; -> the two copies."""
+        by_row = self._pairs_per_row(False) >= BY_ROW_MIN_PAIRS
+        buf = _Buffers(self.out_rows, self.kv, self.z_ptr.device, by_row, True)
+        buf.native.middle_run = int(self.subm)
+        both = L.host().rules_build_pack(self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, False,
+                                         buf.native, self.out_row_cols, weight, 2, self.mirrored(), L.dtype_code(dtype))
+        self._fwd = buf
+        return both
 
     @classmethod
     def build_subm(cls, z_idx, z_ptr, batch, shape, kernel, padding=None,
@@ -226,10 +254,10 @@ class RuleBook:
         ``row_cols`` (optional, int32 [NNZ]): the column of every row (``SparseConvTensor.row_cols``).
         ``lazy``: launch nothing yet; the pairs are generated by the first use -- by ``rule_conv`` in the same
         launch as the convolution where the library has that kernel (:meth:`fused_forward`)."""
-        _check_index_tensors(z_idx, z_ptr, batch, shape)
-        pad = [int(k) // 2 for k in kernel] if padding is None else [int(v) for v in padding]
-        rb = cls(z_idx, z_ptr, z_idx, z_ptr, batch, shape, shape, kernel, (1, 1, 1), pad, dilation, True,
-                 row_cols, row_cols)
+        pad = [int(k) // 2 for k in kernel] if padding is None else padding
+        geometry = _geometry(batch, shape, shape, kernel, (1, 1, 1), pad, dilation)
+        _check_index_tensors(z_idx, z_ptr, geometry.z_shape)
+        rb = cls._of(geometry, z_idx, z_ptr, z_idx, z_ptr, True, row_cols, row_cols)
         if lazy:
             return rb
         if weight is None:
@@ -241,81 +269,34 @@ class RuleBook:
     @classmethod
     def count_ahead(cls, z_idx, z_ptr, batch, in_shape, out_shape, kernel, stride, padding, dilation=(1, 1, 1)):
         """First half of :meth:`build`, to be enqueued as soon as a strided layer's INPUT coordinates exist:
-        the output rows per column are counted and scanned, the row count goes to pinned host memory, and an
-        event marks the place in the stream.  Pass the returned object to ``build(..., ahead=)`` when the layer
+        the output rows per column are counted and scanned, the row count goes to pinned host memory, and the
+        coordinates are written behind it.  Pass the returned object to ``build(..., ahead=)`` when the layer
         itself is reached: whatever the caller has enqueued in between (the convolutions of the layers before)
         keeps the GPU busy while the host reads the count, instead of the GPU waiting for the host."""
-        _check_index_tensors(z_idx, z_ptr, batch, in_shape)
-        lib = L.lib()
-        dev = z_ptr.device
-        g = L.make_geom(batch, in_shape, out_shape, kernel, stride, padding, dilation)
-        if min(int(v) for v in out_shape) <= 0:
-            raise L.SphconvError("empty output grid %s" % (list(out_shape),))
-        nints = lib.sph_outcoords_scratch_ints(C.byref(g))
-        if nints < 0:
-            L.check(nints)
-        oz_ptr = torch.empty((int(batch), int(out_shape[0]), int(out_shape[1])), dtype=torch.int32, device=dev)
-        # scratch and the pinned word are this call's own: other strided layers may be generated before build()
-        scratch = torch.empty(max(nints + (nints & 1), 2), dtype=torch.int32, device=dev)
-        total = _pinned_word()
-        stream = torch.cuda.current_stream(dev)
-        L.check(lib.sph_outcoords_count(L.ptr(z_idx), L.ptr(z_ptr), int(z_idx.shape[0]), C.byref(g), L.ptr(oz_ptr),
-                                        L.ptr(scratch), total.data_ptr(), stream.cuda_stream))
-        event = torch.cuda.Event()
-        event.record(stream)
-        key = (z_idx.data_ptr(), z_ptr.data_ptr(), int(batch), tuple(int(v) for v in in_shape),
-               tuple(int(v) for v in out_shape), tuple(int(v) for v in kernel), tuple(int(v) for v in stride),
-               tuple(int(v) for v in padding), tuple(int(v) for v in dilation))
-        return _CountAhead(key, oz_ptr, scratch, total, event, stream.cuda_stream)
+        geometry = _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation)
+        _check_index_tensors(z_idx, z_ptr, geometry.z_shape)
+        if min(geometry.out_shape) <= 0:
+            raise L.SphconvError("empty output grid %s" % geometry.out_shape)
+        return _CountAhead(geometry, z_idx, z_ptr)
 
     @classmethod
     def build(cls, z_idx, z_ptr, batch, in_shape, out_shape, kernel, stride, padding,
               dilation=(1, 1, 1), weight=None, ahead=None, row_cols=None, lazy=False):
         """Strided rules (replaces get_rules, rules.cu:405-486): output coordinates
         (oz_ptr inclusive scan, oz_idx ascending per column) and pairs.  One wait for the
-        output row count, as in the reference (rules.cu:461): the count kernel writes it to pinned
-        host memory, so the wait is a stream synchronisation and no copy.  ``ahead``: what
-        :meth:`count_ahead` returned for the same arguments on the same stream; the wait is then for its
-        event only."""
-        _check_index_tensors(z_idx, z_ptr, batch, in_shape)
-        lib = L.lib()
-        dev = z_ptr.device
-        g = L.make_geom(batch, in_shape, out_shape, kernel, stride, padding, dilation)
-        if min(int(v) for v in out_shape) <= 0:
-            raise L.SphconvError("empty output grid %s" % (list(out_shape),))
-        n_in = int(z_idx.shape[0])
-        stream = torch.cuda.current_stream(dev)
-        if ahead is not None:
-            key = (z_idx.data_ptr(), z_ptr.data_ptr(), int(batch), tuple(int(v) for v in in_shape),
-                   tuple(int(v) for v in out_shape), tuple(int(v) for v in kernel), tuple(int(v) for v in stride),
-                   tuple(int(v) for v in padding), tuple(int(v) for v in dilation))
-            if ahead.key != key or ahead.stream != stream.cuda_stream:
-                raise L.SphconvError("count_ahead() was called for another layer, tensor or stream")
-            oz_ptr, scratch, total = ahead.oz_ptr, ahead.scratch, ahead.total
-            ahead.event.synchronize()
-        else:
-            nints = lib.sph_outcoords_scratch_ints(C.byref(g))
-            if nints < 0:
-                L.check(nints)
-            oz_ptr = torch.empty((int(batch), int(out_shape[0]), int(out_shape[1])), dtype=torch.int32, device=dev)
-            scratch, total = _outcoords_workspace(dev, nints)
-            try:
-                # one launch: counts, their scan into oz_ptr, and the row count written straight to pinned host memory
-                L.check(lib.sph_outcoords_count(L.ptr(z_idx), L.ptr(z_ptr), n_in, C.byref(g), L.ptr(oz_ptr),
-                                                L.ptr(scratch), total.data_ptr(), stream.cuda_stream))
-                stream.synchronize()             # the one wait of a strided layer (the reference's is rules.cu:461)
-            except Exception:
-                _WORKSPACES.pop(_workspace_key(dev), None)   # whatever failed, the next call starts from fresh buffers
-                raise
-        out_rows = int(total[0])
-        oz_idx = torch.empty(out_rows, dtype=torch.int32, device=dev)
-        out_cols = torch.empty(out_rows, dtype=torch.int32, device=dev)   # the output rows' columns, a by-product
-        L.check(lib.sph_outcoords_fill(L.ptr(z_idx), L.ptr(z_ptr), n_in, C.byref(g), L.ptr(scratch),
-                                       L.ptr(oz_ptr), L.ptr(oz_idx), out_rows, L.ptr(out_cols), L.stream()))
-        if ahead is not None:
-            _release_pinned_word(total)
-        rb = cls(z_idx, z_ptr, oz_idx, oz_ptr, batch, in_shape, out_shape, kernel, stride, padding,
-                 dilation, False, row_cols, out_cols)
+        output row count, as in the reference (rules.cu:461): the scan kernel writes it to pinned
+        host memory and the host waits for that store alone -- behind it the kernel that writes the coordinates is
+        enqueued already, so the GPU is not idle meanwhile.  ``ahead``: what :meth:`count_ahead` returned for the same
+        arguments on the same stream."""
+        geometry = _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation)
+        if ahead is None:
+            ahead = cls.count_ahead(z_idx, z_ptr, batch, in_shape, out_shape, kernel, stride, padding, dilation)
+        elif ahead.geometry is not geometry or ahead.z_idx.data_ptr() != z_idx.data_ptr() \
+                or ahead.z_ptr.data_ptr() != z_ptr.data_ptr() or ahead.native.stream != L.stream():
+            raise L.SphconvError("count_ahead() was called for another layer, tensor or stream")
+        # the rows' columns are a by-product of the coordinates
+        oz_idx, oz_ptr, out_cols = ahead.native.finish()
+        rb = cls._of(geometry, z_idx, z_ptr, oz_idx, oz_ptr, False, row_cols, out_cols)
         if lazy:                                     # output coordinates now, pairs with the first use
             return rb
         if weight is None:
@@ -334,9 +315,8 @@ class RuleBook:
         if rules.dtype != torch.int32 or rule_size.dtype != torch.int32:
             raise L.SphconvError("rules and rule_size must be int32")
         rb = cls.__new__(cls)
+        rb._geometry = None
         rb.z_idx = rb.z_ptr = rb.oz_idx = rb.oz_ptr = None
-        rb.batch = 0
-        rb.in_shape = rb.out_shape = rb.kernel = rb.stride = rb.padding = rb.dilation = None
         rb.subm = False
         rb.kv = int(rules.shape[1])
         rb.in_rows, rb.out_rows = int(in_rows), int(out_rows)
@@ -345,7 +325,7 @@ class RuleBook:
         rb.keep = True
         rb.forward_only = None
         rb.row_cols = rb.out_row_cols = None
-        rb._padded = {}
+        rb._padded = None
         rb._from_padded = (rules.contiguous(), rule_size.contiguous())
         rb.fwd = rb._convert(False)
         return rb
@@ -368,45 +348,31 @@ class RuleBook:
     # 2457 tiles 68.6 / 66.9, 5957 tiles 140 / 142).
     FUSED_MAX_TILES = 1024
 
-    def fused_forward(self, feature: torch.Tensor, packed: torch.Tensor, kdim: int, ndim: int, epilogue=None,
-                      out: Optional[torch.Tensor] = None, buffers: Optional[_Buffers] = None):
+    def goes_in_one_launch(self, kdim: int, ndim: int, element_size: int) -> bool:
+        """Whether this book's pairs are better made by the launch that convolves them (``fused_forward``)."""
+        row_bytes, rows = kdim * element_size, self.out_rows
+        return (self._fwd is None and self._from_padded is None and 0 < rows <= self.FUSED_MAX_TILES * L.TILE_ROWS
+                and self.kv <= 32 and ndim <= 64 and row_bytes % 16 == 0 and row_bytes <= 128
+                and self._pairs_per_row(False) < BY_ROW_MIN_PAIRS * BY_ROW_FORWARD_ONLY)
+
+    def fused_forward(self, feature: torch.Tensor, packed: torch.Tensor, kdim: int, ndim: int, scale=None, shift=None,
+                      relu: bool = False):
         """Pairs and forward convolution of this (not yet built) book in ONE launch (``sph_rules_conv``): replaces
         get_rules_subm / get_rules' pair half + rule_conv (rules.cu:326-486, rule_conv.cu:286-336) where the
         reference launches three kernels.  Returns the output rows, or None when this layer is better served by
         the two kernels (dense neighbourhoods that go by rows, more than FUSED_MAX_TILES tiles, shapes the
         library's fused kernel does not take).  With ``self.keep`` the book is written too and the object counts
         as built afterwards; without, only the output exists and a later use of the book generates it."""
-        if self._fwd is not None or self._from_padded is not None:
+        if not self.goes_in_one_launch(kdim, ndim, feature.element_size()):
             return None
-        lib = L.lib()
-        es = feature.element_size()
-        ntiles = lib.sph_book_tiles(self.out_rows)
-        if self.out_rows == 0 or ntiles > self.FUSED_MAX_TILES or self.kv > 32 or ndim > 64 \
-                or (kdim * es) % 16 or kdim * es > 128 or self._pairs_per_row(False) >= BY_ROW_MIN_PAIRS * BY_ROW_FORWARD_ONLY:
-            return None
-        if not feature.is_contiguous():
-            feature = feature.contiguous()
-        if buffers is not None:
-            buf = buffers
-        elif self.keep:
-            buf = _Buffers(self.out_rows, self.kv, self.z_ptr.device)
-        else:
-            buf = _scratch_book(self.out_rows, self.kv, self.z_ptr.device)   # nobody keeps it: the stream's own
-        buf.struct().middle_run = int(self.subm)
-        if out is None:
-            out = torch.empty((self.out_rows, ndim), dtype=feature.dtype, device=feature.device)
-        g = self.geom()
-        epi = epilogue if epilogue is not None else _NO_EPILOGUE
-        rc = lib.sph_rules_conv(self.z_idx.data_ptr(), self.z_ptr.data_ptr(), self.in_rows, self.oz_idx.data_ptr(),
-                                self.oz_ptr.data_ptr(), self.out_rows, C.byref(g), C.byref(buf.struct()), int(self.keep),
-                                _row_cols_ptr(self.out_row_cols, self.out_rows), L.dtype_code(feature.dtype),
-                                feature.data_ptr(), int(kdim), packed.data_ptr(), int(ndim), C.byref(epi), out.data_ptr(),
-                                L.stream())
-        if rc == L.ERR_UNSUPPORTED:
-            return None
-        if rc:
-            L.check(rc)
-        if self.keep:
+        rows = self.out_rows
+        dev = self.z_ptr.device
+        # a book nobody keeps is the stream's own
+        buf = _Buffers(rows, self.kv, dev) if self.keep else _scratch_book(rows, self.kv, dev)
+        buf.native.middle_run = int(self.subm)
+        out = L.host().rules_conv(self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, buf.native,
+                                  int(self.keep), self.out_row_cols, feature, packed, kdim, ndim, scale, shift, relu)
+        if out is not None and self.keep:
             self._fwd = buf
         return out
 
@@ -426,9 +392,7 @@ class RuleBook:
     def mirrored(self) -> bool:
         """True if the book is its own transpose up to mirroring the offsets (k <-> KV-1-k): submanifold,
         stride 1, odd kernel, padding K//2 -- then dgrad runs on the forward book with reversed weights."""
-        return bool(self.subm and self.kernel is not None and self.oz_idx is self.z_idx
-                    and all(k % 2 == 1 for k in self.kernel) and all(s == 1 for s in self.stride)
-                    and all(p == k // 2 for p, k in zip(self.padding, self.kernel)))
+        return self.subm and self._geometry is not None and self.oz_idx is self.z_idx and self._geometry.odd_same
 
     def transposed(self) -> _Buffers:
         """Book stationary on input rows (what dgrad gathers through when the book is not mirrored)."""
@@ -447,6 +411,8 @@ class RuleBook:
         if self._from_padded is not None:
             return self._from_padded
         key = (int(tile_size[0]), int(tile_size[1]))
+        if self._padded is None:
+            self._padded = {}
         if key not in self._padded:
             lib = L.lib()
             g, b = self.geom(), self.grouped().struct()
@@ -471,58 +437,14 @@ class RuleBook:
         return [-(-self.out_shape[0] // int(tile_size[0])), -(-self.out_shape[1] // int(tile_size[1]))]
 
 
-# Scratch of the output-coordinate kernels, kept per (device, stream), and one pinned host int that receives
-# the output row count.
-_WORKSPACES = {}
-
-
-def _workspace_key(dev):
-    dev = torch.device(dev)
-    index = dev.index if dev.index is not None else torch.cuda.current_device()
-    return (index, torch.cuda.current_stream(index).cuda_stream)
-
-
-# The scratch holds 8 bytes per output column and 64 bins (up to 128 MB, see sph_outcoords_count): it scales with
-# the dense column grid, not with the number of voxels.  Up to this many int32 entries it is kept per (device,
-# stream) between calls; a larger one belongs to its call and goes back to the allocator with it.
-_WORKSPACE_KEEP_INTS = 1 << 24      # 64 MB
-
-
-def _outcoords_workspace(dev, nints: int):
-    key = _workspace_key(dev)
-    ws = _WORKSPACES.get(key)
-    if nints > _WORKSPACE_KEEP_INTS:
-        total = ws[1] if ws is not None else torch.zeros(1, dtype=torch.int32).pin_memory()
-        if ws is None:
-            _WORKSPACES[key] = (torch.empty(1 << 16, dtype=torch.int32, device=dev), total)
-        return torch.empty(nints + (nints & 1), dtype=torch.int32, device=dev), total
-    if ws is None or ws[0].numel() < nints:
-        scratch = torch.empty(max(nints + (nints & 1), 1 << 16), dtype=torch.int32, device=dev)
-        total = ws[1] if ws is not None else torch.zeros(1, dtype=torch.int32).pin_memory()
-        ws = (scratch, total)
-        _WORKSPACES[key] = ws
-    return ws
-
-
 class _CountAhead:
     """Output-row counts of a strided layer on their way (RuleBook.count_ahead)."""
 
-    def __init__(self, key, oz_ptr, scratch, total, event, stream):
-        self.key, self.oz_ptr, self.scratch, self.total, self.event, self.stream = key, oz_ptr, scratch, total, event, stream
+    __slots__ = ("geometry", "z_idx", "z_ptr", "native")
 
-
-# Pinned host words that receive row counts; handed out one per count in flight and taken back when read
-# (pinning memory costs a system call, so they are never freed).
-_PINNED_WORDS = []
-
-
-def _pinned_word():
-    return _PINNED_WORDS.pop() if _PINNED_WORDS else torch.zeros(1, dtype=torch.int32).pin_memory()
-
-
-def _release_pinned_word(word):
-    if len(_PINNED_WORDS) < 64:
-        _PINNED_WORDS.append(word)
+    def __init__(self, geometry, z_idx, z_ptr):
+        self.geometry, self.z_idx, self.z_ptr = geometry, z_idx, z_ptr
+        self.native = L.host().OutCoords(z_idx, z_ptr, geometry.native)
 
 
 # Scratch books of one-launch calls that keep no book (the kernel still wants one for tiles with more groups than
@@ -540,7 +462,7 @@ def _scratch_book(rows: int, kv: int, device) -> "_Buffers":
         buf = _Buffers(max(rows, 1 << 17), kv, device)
         buf.capacity = buf.rows
         _SCRATCH_BOOKS[key] = buf
-    buf.struct().rows = rows
+    buf.native.rows = rows
     return buf
 
 
@@ -559,13 +481,13 @@ def row_columns(z_ptr: torch.Tensor, rows: int) -> torch.Tensor:
     return out
 
 
-def _check_index_tensors(z_idx, z_ptr, batch, shape):
+def _check_index_tensors(z_idx, z_ptr, want):
+    """``want`` = (B, S0, S1)."""
     if z_idx.dtype != torch.int32 or z_ptr.dtype != torch.int32:
         raise L.SphconvError("z_idx and z_ptr must be int32")
     if z_idx.dim() != 1:
         raise L.SphconvError("z_idx must be [NNZ]")
-    want = (int(batch), int(shape[0]), int(shape[1]))
-    if tuple(z_ptr.shape) != want:
+    if z_ptr.shape != want:
         raise L.SphconvError("z_ptr must be [B,S0,S1] = %s, got %s" % (want, tuple(z_ptr.shape)))
     if not (z_idx.is_contiguous() and z_ptr.is_contiguous()):
         raise L.SphconvError("z_idx and z_ptr must be contiguous")

@@ -13,7 +13,6 @@ unchanged with ``sphconv_amd.sphconv_cuda``.  Differences, all additive:
 * float16 / bfloat16 features (fp32 accumulate) and int8 (:func:`rule_conv_int8`);
 * bad arguments raise ``SphconvError`` / ``ValueError`` instead of aborting.
 """
-import ctypes as C
 import weakref
 from typing import List, Optional, Sequence
 
@@ -67,22 +66,20 @@ def _packed_weight(weight: torch.Tensor, transpose: bool, reverse: bool = False,
         hit = _PACKED_CACHE.get(cache_key)
         if hit is not None and hit[0]() is base and hit[1] == state:
             return hit[2]
-    lib = L.lib()
-    kv, a, b = w.shape
-    kdim, ndim = (b, a) if transpose else (a, b)
-    skk, sn = (1, b) if transpose else (b, 1)
-    dt = L.dtype_code(w.dtype)
-    nbytes = lib.sph_weight_packed_bytes(dt, kv, kdim, ndim)
-    if nbytes == 0:
-        raise L.SphconvError("cannot pack weight of shape %s" % (tuple(w.shape),))
-    packed = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
-    first, sk = L.ptr(w), a * b
-    if reverse:                                  # start at the last offset and walk backwards
-        first, sk = first + (kv - 1) * a * b * w.element_size(), -a * b
-    L.check(lib.sph_weight_pack(dt, first, kv, kdim, ndim, sk, skk, sn, L.ptr(packed), L.stream()))
+    packed = L.host().pack_weight(w, transpose, reverse, L.dtype_code(w.dtype))
     if cache_key is not None:
         _PACKED_CACHE[cache_key] = (weakref.ref(base, lambda _r, k=cache_key: _PACKED_CACHE.pop(k, None)), state, packed)
     return packed
+
+
+def _kept_packed(weight: torch.Tensor, stream: int) -> Optional[torch.Tensor]:
+    """The kept fragment-ordered copy of ``weight`` (the parameter itself, of any shape) for the forward pass, if there
+    is one and the weight has not changed since; None otherwise."""
+    hit = _PACKED_CACHE.get((id(weight), False, False, stream))
+    if hit is None or hit[0]() is not weight:
+        return None
+    version, address, _, dtype = hit[1]
+    return hit[2] if version == weight._version and address == weight.data_ptr() and dtype == weight.dtype else None
 
 
 def _dgrad_buffers(book: RuleBook, d_out: torch.Tensor, kdim: int, ndim: int):
@@ -90,8 +87,7 @@ def _dgrad_buffers(book: RuleBook, d_out: torch.Tensor, kdim: int, ndim: int):
     its own transpose with the offsets mirrored (the pair (k, in=i, out=j) has the twin (KV-1-k, in=j,
     out=i)): the forward book serves, with the weight's offsets reversed, and no transposed book is built."""
     if book.mirrored():
-        fake_w = torch.empty((book.kv, kdim, ndim), dtype=d_out.dtype, device="meta")
-        return _conv_buffers(book, d_out, fake_w, False), True
+        return _conv_buffers(book, d_out, kdim, ndim, False), True
     return None, False
 
 
@@ -101,25 +97,8 @@ def _as_book(rules, rule_size, in_rows: int, out_rows: int) -> RuleBook:
     return RuleBook.from_padded(rules, rule_size, in_rows, out_rows)
 
 
-_NO_EPILOGUE = L.Epilogue(None, None, 0)
-
-
-def _apply(feature, packed, kdim, ndim, buffers, scale=None, shift=None, relu=False, out_dtype=None):
-    if not feature.is_contiguous():
-        feature = feature.contiguous()
-    if not feature.is_cuda:
-        raise L.SphconvError("expected a GPU tensor, got device %s" % feature.device)
-    out = torch.empty((buffers.rows, ndim), dtype=out_dtype or feature.dtype, device=feature.device)
-    if scale is None and shift is None and not relu:
-        epi = _NO_EPILOGUE
-    else:
-        epi = L.Epilogue(L.ptr(scale), L.ptr(shift), int(bool(relu)))
-    rc = L.lib().sph_conv_apply(L.dtype_code(feature.dtype), feature.data_ptr(), feature.shape[0], kdim,
-                                packed.data_ptr(), ndim, C.byref(buffers.struct()), C.byref(epi),
-                                out.data_ptr(), L.stream())
-    if rc:
-        L.check(rc)
-    return out
+def _apply(feature, packed, kdim, ndim, buffers, scale=None, shift=None, relu=False):
+    return L.host().conv_apply(feature, packed, kdim, ndim, buffers.native, scale, shift, relu)
 
 
 # ---- tensor.h ---------------------------------------------------------------
@@ -128,38 +107,24 @@ def init_tensor(feature: torch.Tensor, indicesBZYX: torch.Tensor, batchSize: int
                 spatialShape: Sequence[int]) -> List[torch.Tensor]:
     """tensor.cu:78-127 -> [outFeature, zIndices, zPtr, permutation].  Rows of a
     fiber are ordered by ascending S2 (one legal order of the reference's output).
-    One 8-byte device->host read checks the coordinates (the reference checks nothing:
+    Two counts the last kernel reports to the host check the coordinates (the reference checks nothing:
     coordinates outside the grid or duplicated ones corrupt its output)."""
     if indicesBZYX.dtype != torch.int32 or indicesBZYX.dim() != 2 or indicesBZYX.shape[1] != 4:
         raise ValueError("indices must be int32 [NNZ,4] (b,s0,s1,s2)")
     if feature.dim() != 2 or feature.shape[0] != indicesBZYX.shape[0]:
         raise ValueError("feature must be [NNZ,C]")
-    S0, S1, S2 = (int(v) for v in spatialShape)
-    B = int(batchSize)
-    n = feature.shape[0]
-    dev = feature.device
-    lib = L.lib()
-    idx = indicesBZYX.contiguous()
-    z_idx = torch.empty(n, dtype=torch.int32, device=dev)
-    z_ptr = torch.empty((B, S0, S1), dtype=torch.int32, device=dev)
-    permutation = torch.empty(n, dtype=torch.int32, device=dev)
-    status = torch.empty(2, dtype=torch.int32, device=dev)
-    nbytes = lib.sph_init_tensor_workspace(n, B, S0, S1, S2)
-    if nbytes == 0:
-        raise L.SphconvError("bad batch size / spatial shape %s" % ([B, S0, S1, S2],))
-    work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    L.check(lib.sph_init_tensor(L.ptr(idx), n, B, S0, S1, S2, L.ptr(z_idx), L.ptr(z_ptr), L.ptr(permutation),
-                                L.ptr(status), L.ptr(work), nbytes, L.stream()))
-    outside, dup = (int(v) for v in status.tolist())
+    return _init_tensor(feature, indicesBZYX, batchSize, spatialShape)[:4]
+
+
+def _init_tensor(feature, indices, batch, shape):
+    """-> [outFeature, zIndices, zPtr, permutation, columns of the rows]"""
+    S0, S1, S2 = shape
+    out, z_idx, z_ptr, permutation, cols, outside, dup = L.host().init_tensor(feature, indices, batch, S0, S1, S2)
     if outside:
-        raise ValueError("voxel coordinate outside batch/spatial shape %s" % ([B, S0, S1, S2],))
+        raise ValueError("voxel coordinate outside batch/spatial shape %s" % ([int(batch), int(S0), int(S1), int(S2)],))
     if dup:
         raise ValueError("duplicate voxel coordinates")
-    feature = feature.contiguous()
-    out = torch.empty_like(feature)
-    L.check(lib.sph_permute_rows(L.ptr(feature), L.ptr(permutation), n,
-                                 feature.shape[1] * feature.element_size(), 0, L.ptr(out), L.stream()))
-    return [out, z_idx, z_ptr, permutation]
+    return [out, z_idx, z_ptr, permutation, cols]
 
 
 def init_tensor_backward(d_featureOut: torch.Tensor, permutation: torch.Tensor) -> torch.Tensor:
@@ -266,25 +231,27 @@ def rule_conv(feature: torch.Tensor, weight: torch.Tensor, rules, ruleSize, outN
                                                            weight.shape[1], weight.shape[2]):
         raise L.SphconvError("packed weight of %d bytes does not belong to a weight of shape %s"
                              % (packed.numel(), tuple(weight.shape)))
+    return _conv_packed(feature, packed, weight.shape[1], weight.shape[2], book, outNNZ, scale, shift, relu)
+
+
+def _conv_packed(feature, packed, kdim: int, ndim: int, book, outNNZ: int, scale=None, shift=None, relu: bool = False):
+    """The convolution of ``rule_conv`` once its weight is in fragment order."""
+    if book.out_rows != int(outNNZ):
+        raise L.SphconvError("rules hold %d output rows, call says %d" % (book.out_rows, int(outNNZ)))
     if not book.built and feature.is_cuda and feature.shape[0] == book.in_rows:
-        epi = None
-        if scale is not None or shift is not None or relu:
-            epi = L.Epilogue(L.ptr(scale), L.ptr(shift), int(bool(relu)))
-        out = book.fused_forward(feature, packed, weight.shape[1], weight.shape[2], epi)
+        out = book.fused_forward(feature, packed, kdim, ndim, scale, shift, relu)
         if out is not None:
             return out
-    return _apply(feature, packed, weight.shape[1], weight.shape[2], _conv_buffers(book, feature, weight, False),
-                  scale, shift, relu)
+    return _apply(feature, packed, kdim, ndim, _conv_buffers(book, feature, kdim, ndim, False), scale, shift, relu)
 
 
-def _conv_buffers(book, feature, weight, transposed: bool):
+def _conv_buffers(book, feature, kdim: int, ndim: int, transposed: bool):
     """The book's buffers for one convolution call; a book kept by rows only gets its groups built
     when this call cannot go by rows."""
     buf = book.transposed() if transposed else book.fwd
     if buf.groups:
         return buf
     es = feature.element_size()
-    kdim, ndim = weight.shape[1], weight.shape[2]
     by_rows = (kdim * es) % 16 == 0 and kdim * es <= 128 and (ndim * es) % 16 == 0 and feature.data_ptr() % 16 == 0 \
         and feature.shape[0] > 0
     return buf if by_rows else book.grouped(transposed)
@@ -301,10 +268,10 @@ def rule_conv_int8(feature: torch.Tensor, weight: torch.Tensor, scale: torch.Ten
     packed = _packed_weight(weight, False)
     scale = scale.to(torch.float32).contiguous()
     if not book.built and feature.is_cuda and feature.shape[0] == book.in_rows:
-        out = book.fused_forward(feature, packed, weight.shape[1], weight.shape[2], L.Epilogue(L.ptr(scale), None, 0))
+        out = book.fused_forward(feature, packed, weight.shape[1], weight.shape[2], scale)
         if out is not None:
             return out
-    return _apply(feature, packed, weight.shape[1], weight.shape[2], _conv_buffers(book, feature, weight, False), scale)
+    return _apply(feature, packed, weight.shape[1], weight.shape[2], _conv_buffers(book, feature, weight.shape[1], weight.shape[2], False), scale)
 
 
 def rule_conv_d_feature(feature: torch.Tensor, weight: torch.Tensor, rules, ruleSize,
@@ -316,7 +283,7 @@ def rule_conv_d_feature(feature: torch.Tensor, weight: torch.Tensor, rules, rule
     book = _as_book(rules, ruleSize, int(outNNZ), feature.shape[0])
     buf, reverse = _dgrad_buffers(book, feature, weight.shape[1], weight.shape[2])
     if buf is None:
-        buf = _conv_buffers(book, feature, weight, True)
+        buf = _conv_buffers(book, feature, weight.shape[1], weight.shape[2], True)
     packed = _packed_weight(weight, False, reverse)
     return _apply(feature, packed, weight.shape[1], weight.shape[2], buf)
 
@@ -330,18 +297,9 @@ def rule_conv_d_weight(feature: torch.Tensor, d_featureOut: torch.Tensor, rules,
     d_out = d_featureOut.contiguous()
     if d_out.dtype != feature.dtype:
         d_out = d_out.to(feature.dtype)
-    lib = L.lib()
-    ic, oc = feature.shape[1], d_out.shape[1]
-    n = lib.sph_wgrad_partial_elems(book.kv, ic, oc, book.out_rows)
-    partial = torch.empty(max(n, 1), dtype=torch.float32, device=feature.device)
     if out_dtype not in (None, feature.dtype, torch.float32):
         raise L.SphconvError("d_weight comes in the features' type or in float32, not %s" % out_dtype)
-    f32 = out_dtype == torch.float32
-    dw = torch.empty((book.kv, ic, oc), dtype=torch.float32 if f32 else feature.dtype, device=feature.device)
-    b = book.grouped().struct()
-    L.check(lib.sph_conv_wgrad(L.dtype_code(feature.dtype), L.ptr(feature), feature.shape[0], ic,
-                               L.ptr(d_out), oc, C.byref(b), L.ptr(partial), L.ptr(dw), int(f32), L.stream()))
-    return dw
+    return L.host().conv_wgrad(feature, d_out, book.grouped().native, out_dtype == torch.float32)
 
 
 def rule_conv_backward(d_featureOut: torch.Tensor, feature: torch.Tensor, weight: torch.Tensor, rules,

@@ -4,6 +4,7 @@ from typing import List, Optional
 
 import torch
 
+from . import sphconv_cuda as ext
 from .functional import InitTensorFunction, ToDenseFunction
 
 
@@ -44,10 +45,22 @@ class SparseConvTensor(SparseTensorBase):
         assert raw_feature.device == indices.device
         super().__init__(batch_size, s0, s1, s2, raw_feature.shape[-1], raw_feature.device,
                          raw_feature.dtype, indices.dtype, None, None, None)
-        self.feature, self.z_idx, self.z_ptr = InitTensorFunction.apply(
-            raw_feature, indices, self.B, [self.D, self.W, self.H])
-        if self.z_ptr.is_cuda:
-            self.with_row_cols()
+        if torch.is_grad_enabled() and raw_feature.requires_grad:
+            self.feature, self.z_idx, self.z_ptr, self.row_cols = InitTensorFunction.apply(
+                raw_feature, indices, self.B, [self.D, self.W, self.H], True)
+        else:
+            self.feature, self.z_idx, self.z_ptr, _, self.row_cols = ext._init_tensor(
+                raw_feature, indices, self.B, [self.D, self.W, self.H])
+
+    @classmethod
+    def _of(cls, feature, shape, batch, z_idx, z_ptr, row_cols, rule_cache) -> "SparseConvTensor":
+        """A tensor of ready parts (what a convolution returns)."""
+        x = cls.__new__(cls)
+        x.rule_cache, x.row_cols, x.requires_grad = rule_cache, row_cols, False
+        x.B, (x.D, x.W, x.H) = batch, shape
+        x.C, x.device, x.dtype, x.itype = feature.shape[-1], feature.device, feature.dtype, z_idx.dtype
+        x.feature, x.z_idx, x.z_ptr = feature, z_idx, z_ptr
+        return x
 
     def with_row_cols(self):
         """Computes ``row_cols`` from ``z_ptr`` (one small kernel) if the tensor does not have it yet."""

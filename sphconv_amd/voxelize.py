@@ -4,7 +4,8 @@ sphconv/utils/voxel_generator.py, sphconv/utils/coord_transform.py, include/poin
 ``points_to_voxel_v2`` keeps the reference's arguments and result dictionary
 (voxelize.py:126-214); the coordinate transform, the binning and the voxel numbering in
 order of first appearance run in one C call (``sph_points_to_voxel``)."""
-import ctypes as C
+import contextlib
+import functools
 from typing import List, Optional
 
 import numpy as np
@@ -29,6 +30,18 @@ def system_range(coors_range, sphere_coors_range, coord_system: str) -> np.ndarr
     raise ValueError("unknown coord_system %r (one of %s)" % (coord_system, sorted(COORD_SYSTEMS)))
 
 
+@functools.lru_cache(maxsize=64)
+def _bins(coors_range, sphere_coors_range, coord_system: str, grid):
+    """(range of the system coordinates, voxel sizes) in float32, as the reference's float instantiation computes them
+    (point2voxel.h:436-439); one pair per geometry, which a program keeps."""
+    f32 = np.float32
+    rng = system_range(coors_range, sphere_coors_range, coord_system).astype(f32)
+    return rng, [f32((rng[3 + i] - rng[i]) / f32(grid[i])) for i in range(3)]
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
 def points_to_voxel_v2(points, voxel_size, coors_range, sphere_coors_range, coor_to_voxelidx=None,
                        max_points=1, max_voxels=30000, pad_output=False,
                        resolution_HWD: Optional[List[int]] = None, coord_system: Optional[str] = None,
@@ -36,7 +49,7 @@ def points_to_voxel_v2(points, voxel_size, coors_range, sphere_coors_range, coor
     """voxelize.py:126-214.  ``points`` [N,>=4] float32 (numpy or
     torch) -> dict with ``voxels`` [max_voxels,max_points,W], ``coordinates`` [max_voxels,3] int32,
     ``num_points_per_voxel`` [max_voxels] int32, ``voxel_point_mask`` [max_voxels,max_points,1] (GPU
-    tensors, zero beyond ``voxel_num``) and ``voxel_num`` (int; one 4-byte device->host read).
+    tensors, zero beyond ``voxel_num``) and ``voxel_num`` (int; the host waits for the kernel that knows it).
     ``coor_to_voxelidx`` (the reference's dense scratch map) is accepted and not used; ``voxel_size``
     only without ``resolution_HWD`` (then: log-spherical bins of that size, coordinates (theta, phi, r),
     and no appended columns are filled: point2voxel.h:387-390 copies the point as it is).
@@ -60,40 +73,24 @@ def points_to_voxel_v2(points, voxel_size, coors_range, sphere_coors_range, coor
     else:
         pad_cols = 0
         coord_system = coord_system or "spherical"
-        rng = system_range(coors_range, sphere_coors_range, coord_system).astype(np.float32)
         grid = [int(v) for v in resolution_HWD]
-        # float32 voxel sizes, as the reference's float instantiation computes them (point2voxel.h:436-439)
-        vs = [f32((rng[3 + i] - rng[i]) / f32(grid[i])) for i in range(3)]
+        rng, vs = _bins(tuple(map(float, coors_range)), tuple(map(float, sphere_coors_range)), coord_system, tuple(grid))
     if isinstance(points, np.ndarray):
         points = torch.from_numpy(np.ascontiguousarray(points, dtype=np.float32))
     dev = points.device if points.is_cuda else torch.device("cuda", torch.cuda.current_device())
     pts = points.to(device=dev, dtype=torch.float32).contiguous()
     n, nfeat = pts.shape
-    width = nfeat + 3 if append_mode == 1 else nfeat
-    lib = L.lib()
-    voxels = torch.empty((max_voxels, max_points, width), dtype=torch.float32, device=dev)
-    mask = torch.empty((max_voxels, max_points), dtype=torch.float32, device=dev)
-    coors = torch.empty((max_voxels, 3), dtype=torch.int32, device=dev)
-    num = torch.empty((max_voxels,), dtype=torch.int32, device=dev)
-    voxel_num = torch.empty(1, dtype=torch.int32, device=dev)
-    nbytes = lib.sph_points_to_voxel_workspace(n, grid[0], grid[1], grid[2])
-    if nbytes == 0:
-        raise L.SphconvError("bad resolution %s, or more than 2^29 points (%d)" % (grid, n))
-    work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     cell_out = torch.empty(n, dtype=torch.int64, device=dev) if return_cells else None
     if cells is not None:
         cells = cells.to(device=dev, dtype=torch.int64).contiguous()
-    with torch.cuda.device(dev):
-        L.check(lib.sph_points_to_voxel(L.ptr(pts) if n else None, n, nfeat, COORD_SYSTEMS[coord_system],
-                                        float(rng[0]), float(rng[1]), float(rng[2]), float(vs[0]), float(vs[1]),
-                                        float(vs[2]), grid[0], grid[1], grid[2], int(max_points), int(max_voxels),
-                                        int(append_mode), L.ptr(voxels), L.ptr(mask), L.ptr(coors), L.ptr(num),
-                                        L.ptr(voxel_num), L.ptr(cells), L.ptr(cell_out), L.ptr(work), nbytes,
-                                        L.stream()))
+    # (entering a device context costs 3 us: only for points on another GPU)
+    with torch.cuda.device(dev) if dev.index != torch.cuda.current_device() else _SAME_DEVICE:
+        voxels, mask, coors, num, voxel_num = L.host().points_to_voxel(
+            pts, COORD_SYSTEMS[coord_system], [float(v) for v in rng[:3]], [float(v) for v in vs], grid, int(max_points), int(max_voxels), int(append_mode), cells, cell_out)
     if pad_cols:
         voxels = torch.nn.functional.pad(voxels, (0, pad_cols))
     res = {"voxels": voxels, "coordinates": coors, "num_points_per_voxel": num,
-           "voxel_point_mask": mask.reshape(-1, max_points, 1), "voxel_num": int(voxel_num.item())}
+           "voxel_point_mask": mask, "voxel_num": voxel_num}
     if return_cells:
         res["cells"] = cell_out
     return res
