@@ -185,6 +185,32 @@ __global__ __launch_bounds__(kWave * (1 + kRunHelpers)) __attribute__((amdgpu_wa
     }
 }
 
+// A grid that the chip holds at once lasts as long as one tile's chain of groups, so the S waves of a workgroup share the
+// tile's groups: each adds its share into accumulators of its own (up to 64 output columns), and the copies are summed as
+// the tile is written, in the waves' order.  S is the most that still lets every tile be resident (LDS); see
+// split_waves().  A tile whose groups are few is all set-up and store; one of a denser stage (70 to 100 groups) is where
+// this counts.
+template <sph_dtype DT, int NS, int CT, bool MASKED, int S>
+__global__ __launch_bounds__(kWave * S) __attribute__((amdgpu_waves_per_eu(1))) void conv_wave_split_kernel(ConvArgs a, int nwtot)
+{
+    extern __shared__ __attribute__((aligned(16))) uint32_t s_acc[]; // [S][R + 1][LDW]
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = tid / kWave;
+    const int tile = sph_xcd_tile(blockIdx.x, (a.book.rows + R - 1) / R);
+    const int r0 = tile * R;
+    if (r0 >= a.book.rows) return;
+    const int nrows = min(R, a.book.rows - r0);
+    const int ngrp = min(max(a.book.tile_ngrp[tile], 0), a.cap);
+    int base, n;
+    group_share(ngrp, S, wave, base, n);
+    BookMeta meta(a.book, a.cap, tile, n, r0, nrows, a.feat_rows);
+    meta.base = base;
+    conv_wave_groups<DT, NS, CT, MASKED>(a, nwtot, meta, n, s_acc + wave * (R + 1) * (nwtot * 16 + 4), 0, lane, true);
+    lds_barrier();
+    conv_wave_store<DT, CT, S>(a, nwtot, s_acc, 0, r0, nrows, tid, kWave * S);
+}
+
 // ---------------------------------------------------------------------------
 // Walk by stationary row (book.tile_nbr): for dense neighbourhoods.
 //
@@ -1180,11 +1206,25 @@ int launch_conv_ns(const ConvArgs &a, int ntiles, hipStream_t st)
     return sph_check_launch("sph_conv_apply");
 }
 
+template <sph_dtype DT, int NS, int CT, bool MASKED, int S>
+int launch_conv_split(const ConvArgs &a, int nwtot, int ntiles, size_t lds, hipStream_t st)
+{
+    int rc = set_lds(conv_wave_split_kernel<DT, NS, CT, MASKED, S>, lds);
+    if (rc) return rc;
+    hipLaunchKernelGGL((conv_wave_split_kernel<DT, NS, CT, MASKED, S>), dim3(sph_xcd_grid(ntiles)), dim3(kWave * S), lds, st, a, nwtot);
+    return sph_check_launch("sph_conv_apply");
+}
+
 template <sph_dtype DT, int NS, int CT, bool MASKED>
 int launch_conv_wave(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
 {
     size_t lds = (size_t)(R + 1) * (nwtot * 16 + 4) * sizeof(uint32_t); // + scratch row
     const int waves = (nwtot + CT - 1) / CT;
+    if (waves == 1) {
+        const int s = split_waves(ntiles, lds, 0);
+        if (s == 4) return launch_conv_split<DT, NS, CT, MASKED, 4>(a, nwtot, ntiles, 4 * lds, st);
+        if (s == 2) return launch_conv_split<DT, NS, CT, MASKED, 2>(a, nwtot, ntiles, 2 * lds, st);
+    }
     if constexpr (NS <= 2 && !(DT == SPH_F32 && NS == 2 && CT == 4)) {
         // one wave's worth of columns, rows of up to 128 bytes: helper waves for the middle offset's run (fp32 rows
         // of 128 bytes into 64 columns do not fit the registers three waves per SIMD leave)

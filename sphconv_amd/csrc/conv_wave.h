@@ -183,6 +183,7 @@ constexpr int kRsrcFlags = 0x00020000; // raw buffer descriptor, 32-bit data for
 struct BookMeta {
     __amdgpu_buffer_rsrc_t r_gat, r_own, r_gk;
     int cap, ngrp, r0, nrows, feat_rows, KV;
+    int base = 0;        // the wave's share of the tile's groups starts here (a multiple of kBlk): its group 0 is the tile's `base`
     int skip_lo, skip_n; // groups [skip_lo, skip_lo + skip_n) of the book are somebody else's: group g >= skip_lo is the book's g + skip_n
     __device__ __forceinline__ BookMeta(const sph_book &book, int cap_, int tile, int ngrp_, int r0_, int nrows_, int feat_rows_,
                                         int skip_lo_ = 0, int skip_n_ = 0)
@@ -197,10 +198,10 @@ struct BookMeta {
     __device__ __forceinline__ void load(int g0, int lane, int &gi, int &ow, int &kk) const
     {
         // lane l: entry l % 16 of group g0 + l / 16, inside this tile's capacity
-        const int slot = (book_group(g0 + (lane >> 4)) * SPH_GROUP + (lane & 15)) * 4;
+        const int slot = (book_group(base + g0 + (lane >> 4)) * SPH_GROUP + (lane & 15)) * 4;
         gi = __builtin_amdgcn_raw_buffer_load_b32(r_gat, slot, 0, 0);
         ow = __builtin_amdgcn_raw_buffer_load_b32(r_own, slot, 0, 0);
-        kk = __builtin_amdgcn_raw_buffer_load_b32(r_gk, book_group(g0 + (lane & (kBlk - 1))) * 4, 0, 0);
+        kk = __builtin_amdgcn_raw_buffer_load_b32(r_gk, book_group(base + g0 + (lane & (kBlk - 1))) * 4, 0, 0);
     }
     __device__ __forceinline__ void finish(int g0, int lane, int &gi, int &ow, int &kk) const
     {
@@ -228,16 +229,17 @@ struct LdsMeta {
     const int32_t *gat;
     const unsigned char *own, *gk;
     int room, ngrp;
+    int base = 0; // as in BookMeta
     __device__ __forceinline__ void load(int g0, int lane, int &gi, int &ow, int &kk) const
     {
-        const int gs = min(g0, room - kBlk);
+        const int gs = min(base + g0, room - kBlk);
         gi = gat[gs * SPH_GROUP + lane];
         ow = own[gs * SPH_GROUP + lane];
         kk = gk[gs + (lane & (kBlk - 1))];
     }
     __device__ __forceinline__ void finish(int g0, int lane, int &gi, int &ow, int &kk) const
     {
-        const bool inside = g0 <= room - kBlk;
+        const bool inside = base + g0 <= room - kBlk;
         const bool ok = inside && g0 + (lane >> 4) < ngrp && gi >= 0;
         gi = ok ? gi : -1;
         ow = ok ? ow : -1;
@@ -463,12 +465,41 @@ __device__ __forceinline__ void conv_run_store(const ConvArgs &a, int nwtot, con
     }
 }
 
+// Waves that share a tile's groups: the most of 4, 2 and 1 whose accumulator copies (acc_bytes each, beside `other` bytes
+// of LDS) leave room for all tiles at once on the chip's 256 CUs of 160 KB.
+inline int split_waves(int ntiles, size_t acc_bytes, size_t other)
+{
+    for (int s = 4; s > 1; s /= 2) {
+        const size_t wg = s * acc_bytes + other + 1024; // + static LDS and its rounding
+        if (wg <= 160 * 1024 && ntiles <= 256 * (int)(160 * 1024 / wg)) return s;
+    }
+    return 1;
+}
+
+// Share `part` of `parts` of a tile's n groups, in whole blocks of kBlk: its first group and how many there are.
+__device__ __forceinline__ void group_share(int n, int parts, int part, int &base, int &count)
+{
+    const int per = ((n + parts - 1) / parts + kBlk - 1) & ~(kBlk - 1);
+    base = min(part * per, n);
+    count = min(per, n - base);
+    base = part * per;
+    count = max(count, 0);
+}
+
 // Epilogue: columns [col0, col0 + CT*16) of the tile's rows [0, nrows) from s_acc to out rows r0.., by the
-// threads t, t + nthr, ... (a wave alone: t = lane, nthr = 64).
-template <sph_dtype DT, int CT>
+// threads t, t + nthr, ... (a wave alone: t = lane, nthr = 64).  COPIES > 1: the tile is the sum of that many copies,
+// one behind the other in s_acc (waves that shared the groups), added in their order.
+template <sph_dtype DT, int CT, int COPIES = 1>
 __device__ __forceinline__ void conv_wave_store(const ConvArgs &a, int nwtot, const uint32_t *s_acc, int col0, int r0, int nrows,
                                                 int t, int nthr)
 {
+    typedef typename Traits<DT>::acc4 acc4;
+    auto sum4 = [&](int at) {
+        acc4 v = *(const acc4 *)&s_acc[at];
+#pragma unroll
+        for (int c = 1; c < COPIES; c++) v += *(const acc4 *)&s_acc[at + c * (R + 1) * (nwtot * 16 + 4)];
+        return __builtin_bit_cast(int4v, v);
+    };
     typedef typename Traits<DT>::elem elem;
     const int LDW = nwtot * 16 + 4;
     constexpr int VE = 16 / (int)sizeof(elem);
@@ -490,7 +521,7 @@ __device__ __forceinline__ void conv_wave_store(const ConvArgs &a, int nwtot, co
                     const int row = min(row0 + q * rstep, nrows - 1);
 #pragma unroll
                     for (int j = 0; j < VE / 4; j++)
-                        f[q][j] = *(const float4v *)&s_acc[row * LDW + col0 + ch * VE + j * 4];
+                        f[q][j] = __builtin_bit_cast(float4v, sum4(row * LDW + col0 + ch * VE + j * 4));
                 }
 #pragma unroll
                 for (int q = 0; q < UR; q++) {
@@ -521,7 +552,7 @@ __device__ __forceinline__ void conv_wave_store(const ConvArgs &a, int nwtot, co
                     const int row = min(row0 + q * rstep, nrows - 1);
 #pragma unroll
                     for (int j = 0; j < VE / 4; j++)
-                        f[q][j] = *(const int4v *)&s_acc[row * LDW + col0 + ch * VE + j * 4];
+                        f[q][j] = sum4(row * LDW + col0 + ch * VE + j * 4);
                 }
 #pragma unroll
                 for (int q = 0; q < UR; q++) {
@@ -542,7 +573,8 @@ __device__ __forceinline__ void conv_wave_store(const ConvArgs &a, int nwtot, co
     } else {
         for (int i = t; i < nrows * ncols; i += nthr) {
             int row = i / ncols, c = i - row * ncols;
-            out[(long)row * a.ndim + c] = to_elem<DT>(epilogue_value<DT>(a, s_acc[row * LDW + col0 + c], col0 + c));
+            const int at = row * LDW + col0 + c;
+            out[(long)row * a.ndim + c] = to_elem<DT>(epilogue_value<DT>(a, (uint32_t)sum4(at & ~3)[c & 3], col0 + c));
         }
     }
 }

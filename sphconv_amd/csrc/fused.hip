@@ -30,9 +30,10 @@ struct FusedArgs {
     int small_wg;   // two-wave workgroups (four fit a CU) whatever the tile count: for callers with scans in flight
 };
 
-inline size_t fused_region_a(int KV, int nwtot)
+inline size_t fused_acc(int nwtot) { return (size_t)(R + 1) * (nwtot * 16 + 4) * sizeof(uint32_t); }
+inline size_t fused_region_a(int KV, int nwtot, int split)
 {
-    const size_t acc = (size_t)(R + 1) * (nwtot * 16 + 4) * sizeof(uint32_t);
+    const size_t acc = split * fused_acc(nwtot);
     const size_t tab = (size_t)R * KV * sizeof(int32_t) + emit_scratch_bytes(KV);
     return ((acc > tab ? acc : tab) + 15) & ~(size_t)15;
 }
@@ -41,8 +42,10 @@ inline size_t fused_region_b() { return compact_bytes(); }
 
 // NT threads per workgroup: 256 (four waves: more hands for the rule generation, at most three workgroups per CU
 // by registers) or 128 (two waves: four workgroups per CU, for grids of more tiles than three per CU hold).
-template <sph_dtype DT, int NS, int CT, bool MASKED, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? 3 : 2))) void rules_conv_kernel(FusedArgs fa, int region_a)
+// S > 1: that many waves share the tile's groups instead, each with accumulators of its own (conv_wave_split_kernel), for
+// grids that leave the LDS for the copies.
+template <sph_dtype DT, int NS, int CT, bool MASKED, int NT, int S>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(S > 1 ? 1 : (NT == 256 ? 3 : 2)))) void rules_conv_kernel(FusedArgs fa, int region_a)
 {
     extern __shared__ __attribute__((aligned(16))) uint32_t s_mem[];
     constexpr int NW = NT / kWave;
@@ -79,7 +82,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? 
     const bool fits = ci.fits;
     if (fits && fa.write_book) {
         // the book is wanted too (a shared indice_key, a backward pass): region B holds all of it
-        if (b.book.tile_nbr) emit_nbr_store(s_nbr, KV, tile, b.book, tid, NT);
+        if (b.book.tile_nbr) {
+            emit_nbr_store(s_nbr, KV, tile, b.book, tid, NT);
+            lds_barrier(); // region A becomes the accumulators below
+        }
         compact_store<NT>(cg, ci, kc, r0, KV, tile, b.cap, b.book);
     }
     if (!fits) {
@@ -98,7 +104,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? 
     //    zero the rows that offset does not reach) while wave 0 requests its first rows and fragments;
     // 4. wave 0 adds the other groups one after the other.
     const int LDW = fa.nwtot * 16 + 4;
-    if (fits) {
+    if constexpr (S > 1) {
+        if (wave < S) {
+            int base, n;
+            group_share(ngrp, S, wave, base, n);
+            uint32_t *acc = s_mem + wave * (R + 1) * LDW;
+            if (fits) {
+                LdsMeta meta{m_gat, m_own, m_gk, kFusedGroups, n};
+                meta.base = base;
+                conv_wave_groups<DT, NS, CT, MASKED>(a, fa.nwtot, meta, n, acc, 0, lane, true);
+            } else {
+                BookMeta meta(b.book, b.cap, tile, n, r0, nrows, a.feat_rows);
+                meta.base = base;
+                conv_wave_groups<DT, NS, CT, MASKED>(a, fa.nwtot, meta, n, acc, 0, lane, true);
+            }
+        }
+    } else if (fits) {
         if (wave == 0) {
             const LdsMeta meta{m_gat, m_own, m_gk, kFusedGroups, n0};
             conv_wave_groups<DT, NS, CT, MASKED>(a, fa.nwtot, meta, n0, s_mem, 0, lane, false, 1);
@@ -119,23 +140,23 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? 
     lds_barrier();
 
     // 5. the tile goes to global memory once, by all threads, with the epilogue fused
-    conv_wave_store<DT, CT>(a, fa.nwtot, s_mem, 0, r0, nrows, tid, NT);
+    conv_wave_store<DT, CT, S>(a, fa.nwtot, s_mem, 0, r0, nrows, tid, NT);
 }
 
-template <sph_dtype DT, int NS, int CT, bool MASKED, int NT>
+template <sph_dtype DT, int NS, int CT, bool MASKED, int NT, int S>
 int launch_fused_nt(const FusedArgs &fa, int ntiles, hipStream_t st)
 {
-    const size_t ra = fused_region_a(fa.b.book.KV, fa.nwtot);
+    const size_t ra = fused_region_a(fa.b.book.KV, fa.nwtot, S);
     const size_t lds = ra + fused_region_b();
     if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void *)rules_conv_kernel<DT, NS, CT, MASKED, NT>,
+        hipError_t e = hipFuncSetAttribute((const void *)rules_conv_kernel<DT, NS, CT, MASKED, NT, S>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             sph_set_error("sph_rules_conv: hipFuncSetAttribute(%zu bytes of LDS): %s", lds, hipGetErrorString(e));
             return SPH_ERR_LAUNCH;
         }
     }
-    hipLaunchKernelGGL((rules_conv_kernel<DT, NS, CT, MASKED, NT>), dim3(sph_xcd_grid(ntiles)), dim3(NT), lds, st, fa, (int)ra);
+    hipLaunchKernelGGL((rules_conv_kernel<DT, NS, CT, MASKED, NT, S>), dim3(sph_xcd_grid(ntiles)), dim3(NT), lds, st, fa, (int)ra);
     return sph_check_launch("sph_rules_conv");
 }
 
@@ -144,8 +165,13 @@ int launch_fused(const FusedArgs &fa, int ntiles, hipStream_t st)
 {
     // three workgroups of 256 threads per CU hold 768 tiles at once, four of 128 threads 1024 (and fp32 rows of 128
     // bytes into 64 columns do not fit the registers three workgroups leave a wave)
-    if (fa.small_wg || ntiles > 768 || (DT == SPH_F32 && NS == 2 && CT == 4)) return launch_fused_nt<DT, NS, CT, MASKED, 128>(fa, ntiles, st);
-    return launch_fused_nt<DT, NS, CT, MASKED, 256>(fa, ntiles, st);
+    if (!fa.small_wg) {
+        const int s = split_waves(ntiles, fused_acc(fa.nwtot), fused_region_b());
+        if (s == 4) return launch_fused_nt<DT, NS, CT, MASKED, 256, 4>(fa, ntiles, st);
+        if (s == 2) return launch_fused_nt<DT, NS, CT, MASKED, 256, 2>(fa, ntiles, st);
+    }
+    if (fa.small_wg || ntiles > 768 || (DT == SPH_F32 && NS == 2 && CT == 4)) return launch_fused_nt<DT, NS, CT, MASKED, 128, 1>(fa, ntiles, st);
+    return launch_fused_nt<DT, NS, CT, MASKED, 256, 1>(fa, ntiles, st);
 }
 
 template <sph_dtype DT, int NS, int CT>
