@@ -126,6 +126,7 @@ class Conv3d(Convolution):
                                   self.kernel_size, self.stride, self.padding, self.dilation, ahead=ahead,
                                   row_cols=row_cols, lazy=True)
         book.keep = bool(keep)
+        book.cluster = getattr(input, "cluster", 1.0)
         if not training:
             book.forward_only = (self.in_channels, self.out_channels, input.feature.element_size())
         entry = (book.oz_idx, book.oz_ptr, book, None, get_tile_grid_shape(out_shape, self.tile_size))
@@ -173,7 +174,8 @@ class Conv3d(Convolution):
         # the rows' columns, where known: the input's own for a submanifold layer, a by-product of the
         # output-coordinate kernels for a strided one
         return SparseConvTensor._of(out_feature, out_shape, input.B, oz_idx, oz_ptr,
-                                    book.out_row_cols if native else None, input.rule_cache)
+                                    book.out_row_cols if native else None, input.rule_cache,
+                                    getattr(input, "cluster", 1.0) if self.subm or not native else book._geometry.cluster)
 
 
 SparseConv3d = Conv3d

@@ -79,7 +79,7 @@ class _Geometry:
     by every book that has it (a network meets a few dozen)."""
 
     __slots__ = ("native", "batch", "in_shape", "out_shape", "kernel", "stride", "padding", "dilation", "kv", "in_cells",
-                 "out_cells", "steps", "odd_same", "z_shape")
+                 "out_cells", "steps", "odd_same", "z_shape", "cluster")
 
     def __init__(self, batch, in_shape, out_shape, kernel, stride, padding, dilation):
         self.batch = batch
@@ -90,6 +90,13 @@ class _Geometry:
         self.out_cells = max(batch * out_shape[0] * out_shape[1] * out_shape[2], 1)
         self.steps = stride[0] * stride[1] * stride[2]
         self.z_shape = (batch, in_shape[0], in_shape[1])
+        # Outputs an input row makes, as an output row meets them (size-biased mean): an input reaches floor or ceil
+        # of K / stride outputs on each axis, neighbours of one another -- 1 to 8, 4.6 as an output row sees it, for a
+        # 3x3x3 kernel of stride 2.
+        self.cluster = 1.0
+        for k, s in zip(kernel, stride):
+            reach = [len(range(r, k, s)) for r in range(s)]
+            self.cluster *= sum(c * c for c in reach) / max(sum(reach), 1)
         # odd kernel, stride 1, padding K//2: a submanifold book is then its own transpose, offsets mirrored
         self.odd_same = all(k % 2 == 1 for k in kernel) and self.steps == 1 and all(p == k // 2 for p, k in zip(padding, kernel))
         self.native = L.host().Geometry(batch, self.in_shape, self.out_shape, self.kernel, self.stride, self.padding,
@@ -151,6 +158,9 @@ class RuleBook:
         # (input channels, output channels, element size) of the forward pass a lazy book is made for, when no
         # gradient will be asked of it: lets a book that goes by rows leave its groups out (see ``_build``)
         self.forward_only: Optional[tuple] = None
+        # rows that lie together in the gathered side's grid whatever its occupancy (``_Geometry.cluster`` of the layer
+        # that made them; 1: nothing known)
+        self.cluster = 1.0
         self._padded = None
         self._from_padded = None     # (rules, rule_size) when built from reference-format tensors
 
@@ -185,11 +195,13 @@ class RuleBook:
 
     def _pairs_per_row(self, transposed: bool) -> float:
         """Pairs a stationary row can expect: kernel volume x occupancy of the gathered side's grid
-        (a stride thins the offsets that can pair with an input row)."""
+        (a stride thins the offsets that can pair with an input row), and the rest of a row's cluster where the
+        gathered rows are the outputs of a strided layer: one scan's second encoder stage holds 4.1 pairs per row by
+        its occupancy and about eight in fact (grouped 41 us per layer, by rows 22)."""
         g = self._geometry
         if transposed:
             return g.kv * self.out_rows / g.out_cells / g.steps
-        return g.kv * self.in_rows / g.in_cells
+        return g.kv * self.in_rows / g.in_cells + self.cluster - 1.0
 
     def _rows_kernel_takes(self, weight, weight_transposed: bool) -> bool:
         """Whether ``sph_conv_apply`` can walk this layer by stationary row (rows of 16-byte multiples up
@@ -325,6 +337,7 @@ class RuleBook:
         rb.keep = True
         rb.forward_only = None
         rb.row_cols = rb.out_row_cols = None
+        rb.cluster = 1.0
         rb._padded = None
         rb._from_padded = (rules.contiguous(), rule_size.contiguous())
         rb.fwd = rb._convert(False)

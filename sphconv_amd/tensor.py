@@ -32,6 +32,7 @@ class SparseConvTensor(SparseTensorBase):
         # of convolutions carry it; ``with_row_cols()`` adds it to a tensor made from bare z_idx / z_ptr.
         self.row_cols = row_cols
         self.requires_grad = False
+        self.cluster = 1.0     # see RuleBook.cluster: set by strided layers on what they return
         s0, s1, s2 = (int(v) for v in spatial_shape_DWH)
         if z_idx is not None and z_ptr is not None:
             super().__init__(batch_size, s0, s1, s2, raw_feature.shape[-1], raw_feature.device,
@@ -53,10 +54,10 @@ class SparseConvTensor(SparseTensorBase):
                 raw_feature, indices, self.B, [self.D, self.W, self.H])
 
     @classmethod
-    def _of(cls, feature, shape, batch, z_idx, z_ptr, row_cols, rule_cache) -> "SparseConvTensor":
+    def _of(cls, feature, shape, batch, z_idx, z_ptr, row_cols, rule_cache, cluster) -> "SparseConvTensor":
         """A tensor of ready parts (what a convolution returns)."""
         x = cls.__new__(cls)
-        x.rule_cache, x.row_cols, x.requires_grad = rule_cache, row_cols, False
+        x.rule_cache, x.row_cols, x.requires_grad, x.cluster = rule_cache, row_cols, False, cluster
         x.B, (x.D, x.W, x.H) = batch, shape
         x.C, x.device, x.dtype, x.itype = feature.shape[-1], feature.device, feature.dtype, z_idx.dtype
         x.feature, x.z_idx, x.z_ptr = feature, z_idx, z_ptr
