@@ -120,53 +120,6 @@ __device__ unsigned long long column_mask(const OutArgs &a, int b, int o0, int o
     return mask;
 }
 
-// The same walk for the first NCH chunks of 64 bins at once (O2 <= 64 * NCH): the fibers are read once, not once
-// per chunk.  The chunk of a bin is matched against constants, so the masks stay in registers.
-template <int NCH>
-__device__ __forceinline__ void column_masks(const OutArgs &a, int b, int o0, int o1, int part, int step,
-                                             unsigned long long (&mask)[NCH])
-{
-#pragma unroll
-    for (int c = 0; c < NCH; c++) mask[c] = 0;
-    const int K01 = a.cv.K0 * a.cv.K1;
-    const bool pow2 = (a.cv.s2 & (a.cv.s2 - 1)) == 0;
-    const int sh2 = __ffs(a.cv.s2) - 1;
-    for (int k01 = part; k01 < K01; k01 += step) {
-        const int k0 = k01 / a.cv.K1, k1 = k01 - k0 * a.cv.K1;
-        int x0 = o0 * a.cv.s0 - a.cv.p0 + k0;
-        int x1 = o1 * a.cv.s1 - a.cv.p1 + k1;
-        if (x0 < 0 || x0 >= a.S.n0 || x1 < 0 || x1 >= a.S.n1) continue;
-        int pc = (b * a.S.n0 + x0) * a.S.n1 + x1;
-        int ps, pe;
-        fiber_range(a.z_ptr, pc, a.in_rows, ps, pe);
-        for (int e0 = ps; e0 < pe; e0 += 4) {
-            int z[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) z[q] = a.z_idx[min(e0 + q, pe - 1)];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                if (e0 + q >= pe) continue;
-                for (int k2 = 0; k2 < a.cv.K2; k2++) {
-                    int t = z[q] + a.cv.p2 - k2;
-                    int o2;
-                    if (pow2) {
-                        if (t < 0 || (t & (a.cv.s2 - 1))) continue;
-                        o2 = t >> sh2;
-                    } else {
-                        if (t < 0 || t % a.cv.s2) continue;
-                        o2 = t / a.cv.s2;
-                    }
-                    if (o2 >= a.O.n2) continue;
-                    const unsigned long long bit = 1ull << (o2 & 63);
-                    const int ch = o2 >> 6;
-#pragma unroll
-                    for (int c = 0; c < NCH; c++) mask[c] |= ch == c ? bit : 0ull;
-                }
-            }
-        }
-    }
-}
-
 constexpr int kMaskChunks = 8;                   // chunks of 64 bins (O2 <= 512) up to which every column's masks are kept
 constexpr long kMaskWordsMax = 1L << 24;         // ... and 64-bit mask words (128 MB) up to which they are kept at all
 __host__ __device__ inline int mask_chunks(int O2) { return (O2 + 63) >> 6; }
@@ -192,36 +145,15 @@ __device__ __forceinline__ unsigned long long or_reduce16(unsigned long long m)
     return ((unsigned long long)hi << 32) | lo;
 }
 
-// Active bins of one output column, counted by its 16 lanes in one walk over the fibers that reach it; the
-// masks of its nchunk <= NCH chunks go to masks[oc * nchunk + chunk] (masks may be null).
-template <int NCH>
-__device__ __forceinline__ int count_column(const OutArgs &a, int b, int o0, int o1, int part, unsigned long long *masks,
-                                            int oc, int nchunk)
-{
-    unsigned long long m[NCH];
-    column_masks<NCH>(a, b, o0, o1, part, kColLanes, m);
-    int cnt = 0;
-#pragma unroll
-    for (int c = 0; c < NCH; c++) {
-        m[c] = or_reduce16(m[c]);
-        cnt += __popcll(m[c]);
-        if (masks && part == 0 && c < nchunk) masks[(long)oc * nchunk + c] = m[c];
-    }
-    return cnt;
-}
-
 // Scratch of the output-coordinate kernels: the state of the scan of the counts (sph_scan, one 64-bit word per
 // tile of 2048 columns) at its head, the columns' bin masks behind it.
 inline long scan_state_ints(long ncol) { return (long)(sph_scan::state_bytes(ncol) / 4); }
 
-// Per-column counts.  16 lanes share an output column (one input column (k0, k1) each, K0*K1 = 9 of them busy
-// for a 3x3x3 kernel), so the fibers that reach a column are walked side by side and small grids still fill
-// the chip.  The counts go to oz_ptr, which sph_scan then scans in place: a scan folded into this kernel
-// (workgroups numbered by a ticket, decoupled look-back) was measured slower than the two kernels, because
-// every workgroup then pays an atomic on the one ticket counter and same-address device-scope atomics queue
-// at about 20 ns each, while the counting wants thousands of small workgroups (131 072 columns: 74 us with
-// 2048 workgroups of 64 columns, 31 us with 256 of 512 columns, against 19 us here + 6 us of scan).
-// `masks` (O2 <= 512 only, else null) keeps each column's bin masks for the fill kernel.
+// Per-column counts; they go to oz_ptr, which sph_scan then scans in place (a scan folded into a count kernel was
+// measured slower: every workgroup then pays an atomic on the one ticket counter, and same-address device-scope atomics
+// queue at about 20 ns each).  `masks` (O2 <= 512 only, else null) keeps each column's bin masks for the fill kernel.
+// This one serves grids of more than 512 bins and kernels too wide for the LDS of outcoords_count_tile_kernel: 16 lanes
+// share an output column and walk the fibers that reach it, once per 64 bins.
 __global__ __launch_bounds__(kCountThreads) void outcoords_count_kernel(OutArgs a, int32_t *counts,
                                                                         unsigned long long *masks, int *scan_state,
                                                                         int scan_state_n)
@@ -239,24 +171,128 @@ __global__ __launch_bounds__(kCountThreads) void outcoords_count_kernel(OutArgs 
     const int rem = oc - b * (a.O.n0 * a.O.n1);
     const int o0 = rem / a.O.n1, o1 = rem % a.O.n1;
     int cnt = 0;
-    if (nchunk == 1) {
-        cnt = count_column<1>(a, b, o0, o1, part, masks, oc, nchunk);
-    } else if (nchunk <= 2) {
-        cnt = count_column<2>(a, b, o0, o1, part, masks, oc, nchunk);
-    } else if (nchunk <= 4) {
-        cnt = count_column<4>(a, b, o0, o1, part, masks, oc, nchunk);
-    } else if (nchunk <= kMaskChunks) {
-        cnt = count_column<kMaskChunks>(a, b, o0, o1, part, masks, oc, nchunk);
-    } else { // deeper grids: one walk per chunk, nothing kept
-        for (int ch = 0; ch < nchunk; ch++) cnt += __popcll(or_reduce16(column_mask(a, b, o0, o1, ch, part, kColLanes)));
+    for (int ch = 0; ch < nchunk; ch++) {
+        const unsigned long long m = or_reduce16(column_mask(a, b, o0, o1, ch, part, kColLanes));
+        cnt += __popcll(m);
+        if (masks && part == 0) masks[(long)oc * nchunk + ch] = m;
     }
     if (part == 0) counts[oc] = cnt;
 }
 
-// oz_ptr holds the inclusive scan of the counts; one thread writes the bins of one column.
+// The usual kernel: a workgroup takes `tc` neighbouring output columns of
+// one (b, o0) line, turns each of the K0 x ((tc - 1) * s1 + K1) input columns that reach them into the bins it covers on
+// the output side, once, and every output column ORs K0 * K1 of those words.  With 16 lanes per output column walking
+// the fibers themselves every fiber was walked by each of the two to nine columns it reaches, by lanes of which seven of
+// sixteen had none, and a bin was found by trying every k2: 19.3 us at the 131 072 output columns of four scans (64x2048x64,
+// 3x3x3, stride 2), instruction bound; this way 8.3 us, half of it the chain of dependent loads of the longest fibers.
+// NCH: words of 64 bins per column (O2 <= 64 * NCH).
+template <int NCH>
+__global__ __launch_bounds__(kThreads) void outcoords_count_tile_kernel(OutArgs a, int32_t *counts, unsigned long long *masks,
+                                                                        int *scan_state, int scan_state_n, int tc, int tiles1)
+{
+    extern __shared__ unsigned long long s_words[]; // [NCH][K0 * W]
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0)
+        for (int i = tid; i < scan_state_n; i += kThreads) scan_state[i] = 0;
+    const int nchunk = mask_chunks(a.O.n2);
+    const int t1 = blockIdx.x % tiles1, line = blockIdx.x / tiles1;
+    const int o0 = line % a.O.n0, b = line / a.O.n0;
+    const int o1_0 = t1 * tc, n1 = min(tc, a.O.n1 - o1_0);
+    const int W = (n1 - 1) * a.cv.s1 + a.cv.K1, n_in = a.cv.K0 * W;
+    const int x0_0 = o0 * a.cv.s0 - a.cv.p0, x1_0 = o1_0 * a.cv.s1 - a.cv.p1;
+    const bool pow2 = (a.cv.s2 & (a.cv.s2 - 1)) == 0;
+    const int sh2 = __ffs(a.cv.s2) - 1;
+    for (int it = tid; it < n_in; it += kThreads) {
+        const int k0 = it / W, x0 = x0_0 + k0, x1 = x1_0 + it - k0 * W;
+        unsigned long long m[NCH];
+#pragma unroll
+        for (int c = 0; c < NCH; c++) m[c] = 0;
+        if (x0 >= 0 && x0 < a.S.n0 && x1 >= 0 && x1 < a.S.n1) {
+            int ps, pe;
+            fiber_range(a.z_ptr, (b * a.S.n0 + x0) * a.S.n1 + x1, a.in_rows, ps, pe);
+            for (int e0 = ps; e0 < pe; e0 += 4) {
+                int z[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) z[q] = a.z_idx[min(e0 + q, pe - 1)]; // (the last one again: the same bins)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    // bins o2 with 0 <= z + p2 - o2 * s2 < K2
+                    const int t = z[q] + a.cv.p2, t0 = t - a.cv.K2 + a.cv.s2;
+                    int hi, lo;
+                    if (pow2) { hi = t >> sh2; lo = t0 >> sh2; }
+                    else { hi = t < 0 ? -1 : t / a.cv.s2; lo = t0 < 0 ? 0 : t0 / a.cv.s2; }
+                    lo = max(lo, 0);
+                    hi = min(hi, a.O.n2 - 1);
+                    if (NCH == 1) {
+                        if (lo <= hi) m[0] |= (2ull << hi) - (1ull << lo);
+                    } else {
+                        for (int o2 = lo; o2 <= hi; o2++) {
+                            const unsigned long long bit = 1ull << (o2 & 63);
+                            const int ch = o2 >> 6;
+#pragma unroll
+                            for (int c = 0; c < NCH; c++) m[c] |= ch == c ? bit : 0ull;
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NCH; c++) s_words[c * n_in + it] = m[c];
+    }
+    lds_barrier();
+    for (int j = tid; j < n1; j += kThreads) {
+        const long oc = (long)line * a.O.n1 + o1_0 + j;
+        int cnt = 0;
+#pragma unroll
+        for (int c = 0; c < NCH; c++) {
+            if (c >= nchunk) break;
+            unsigned long long m = 0;
+            for (int k0 = 0; k0 < a.cv.K0; k0++)
+                for (int k1 = 0; k1 < a.cv.K1; k1++) m |= s_words[c * n_in + k0 * W + j * a.cv.s1 + k1];
+            cnt += __popcll(m);
+            if (masks) masks[oc * nchunk + c] = m;
+        }
+        counts[oc] = cnt;
+    }
+}
+
+// Bins of every column from the kept masks, written as they lie: a workgroup's 256 columns put their bins into LDS at
+// the rows' places (kFillWindow rows at a time), and the rows go to memory in order, a row's bin and its column side by
+// side: 7.3 us for the 1.63 million rows of four scans (64x2048x64, stride 2).  (A thread per column that writes its own rows
+// stores a line in a dozen pieces: 16.7 us.)
+constexpr int kFillWindow = 8192;
+__global__ __launch_bounds__(kThreads) void outcoords_fill_tile_kernel(int ncol, int nchunk, const int32_t *oz_ptr, int32_t *oz_idx,
+                                                                       int out_rows, const unsigned long long *masks, int32_t *row_cols)
+{
+    __shared__ uint16_t s_z[kFillWindow];
+    __shared__ unsigned char s_c[kFillWindow];
+    const int tid = threadIdx.x, c0 = blockIdx.x * kThreads, c = c0 + tid;
+    const int c_last = min(c0 + kThreads, ncol) - 1;
+    const int first = c0 ? clampi(oz_ptr[c0 - 1], 0, out_rows) : 0, last = clampi(oz_ptr[c_last], 0, out_rows);
+    const int start = c <= c_last ? (c ? clampi(oz_ptr[c - 1], 0, out_rows) : 0) : last;
+    for (int w = first; w < last; w += kFillWindow) {
+        if (c <= c_last) {
+            int at = start - w;
+            for (int ch = 0; ch < nchunk; ch++)
+                for (unsigned long long m = masks[(long)c * nchunk + ch]; m; m &= m - 1, at++)
+                    if ((unsigned)at < (unsigned)kFillWindow) {
+                        s_z[at] = (uint16_t)(ch * 64 + __ffsll((long long)m) - 1);
+                        s_c[at] = (unsigned char)tid;
+                    }
+        }
+        lds_barrier();
+        const int n = min(kFillWindow, last - w);
+        for (int i = tid; i < n; i += kThreads) {
+            oz_idx[w + i] = s_z[i];
+            if (row_cols) row_cols[w + i] = c0 + s_c[i];
+        }
+        lds_barrier();
+    }
+}
+
+// oz_ptr holds the inclusive scan of the counts; one thread writes the bins of one column (grids that keep no masks).
 __global__ __launch_bounds__(kThreads) void outcoords_fill_kernel(OutArgs a, const int32_t *oz_ptr, int32_t *oz_idx,
-                                                                  int out_rows, const unsigned long long *masks,
-                                                                  int32_t *row_cols)
+                                                                  int out_rows, int32_t *row_cols)
 {
     const int ncol = a.B * a.O.n0 * a.O.n1;
     const int oc = blockIdx.x * kThreads + threadIdx.x;
@@ -269,7 +305,7 @@ __global__ __launch_bounds__(kThreads) void outcoords_fill_kernel(OutArgs a, con
     int o0 = rem / a.O.n1, o1 = rem % a.O.n1;
     int nchunk = (a.O.n2 + 63) >> 6;
     for (int ch = 0; ch < nchunk; ch++) {
-        unsigned long long m = masks ? masks[(long)oc * nchunk + ch] : column_mask(a, b, o0, o1, ch, 0, 1);
+        unsigned long long m = column_mask(a, b, o0, o1, ch, 0, 1);
         while (m) {
             int bit = __ffsll((long long)m) - 1;
             if (pos < out_rows) {
@@ -556,8 +592,28 @@ static int outcoords_count(const char *who, const int32_t *z_idx, const int32_t 
     SPH_REQUIRE(z_ptr && oz_ptr && scratch && in_rows >= 0 && (in_rows == 0 || z_idx), SPH_ERR_ARG, "%s: null argument", who);
     SPH_REQUIRE((uintptr_t)scratch % 8 == 0, SPH_ERR_ARG, "%s: scratch must be 8-byte aligned", who);
     const long ncol = (long)g->B * g->O[0] * g->O[1];
-    const unsigned nblocks = (unsigned)((ncol + kCountCols - 1) / kCountCols);
-    hipLaunchKernelGGL(outcoords_count_kernel, dim3(nblocks), dim3(kCountThreads), 0, (hipStream_t)stream,
+    // Output columns per workgroup: as many as leave the chip two workgroups per CU (fewer fibers are then read twice), and
+    // fit 32 KB of words.
+    const int nchunk = mask_chunks(g->O[2]), nch = nchunk <= 1 ? 1 : (nchunk <= 2 ? 2 : (nchunk <= 4 ? 4 : kMaskChunks));
+    const long lines = (long)g->B * g->O[0];
+    auto words = [&](int tc) { return (size_t)nch * g->K[0] * ((size_t)(tc - 1) * g->stride[1] + g->K[1]) * 8; };
+    int tc = 128;
+    while (tc > 16 && (lines * sph_div_up(g->O[1], tc) < 512 || words(tc) > 32 * 1024)) tc /= 2;
+    const long tiles = lines * sph_div_up(g->O[1], tc);
+    if (nchunk <= kMaskChunks && words(tc) <= 32 * 1024 && tiles < 2147483647L) {
+        const OutArgs oa = out_args(z_idx, z_ptr, in_rows, g);
+        unsigned long long *masks = outcoords_masks(g, scratch);
+        const int tiles1 = sph_div_up(g->O[1], tc), ns = sph_scan::state_ints(ncol);
+#define SPH_COUNT(N)                                                                                                      \
+    hipLaunchKernelGGL(outcoords_count_tile_kernel<N>, dim3((unsigned)tiles), dim3(kThreads), words(tc), (hipStream_t)stream, oa, \
+                       oz_ptr, masks, (int *)scratch, ns, tc, tiles1)
+        if (nch == 1) SPH_COUNT(1);
+        else if (nch == 2) SPH_COUNT(2);
+        else if (nch == 4) SPH_COUNT(4);
+        else SPH_COUNT(kMaskChunks);
+#undef SPH_COUNT
+    } else
+        hipLaunchKernelGGL(outcoords_count_kernel, dim3((unsigned)((ncol + kCountCols - 1) / kCountCols)), dim3(kCountThreads), 0, (hipStream_t)stream,
                        out_args(z_idx, z_ptr, in_rows, g), oz_ptr, outcoords_masks(g, scratch), (int *)scratch,
                        sph_scan::state_ints(ncol));
     int rc = sph_check_launch(who);
@@ -642,9 +698,13 @@ SPH_EXPORT int sph_outcoords_fill(const int32_t *z_idx, const int32_t *z_ptr, in
     SPH_REQUIRE(z_ptr && oz_ptr && scratch && out_rows >= 0 && (out_rows == 0 || oz_idx) &&
                     (in_rows == 0 || z_idx), SPH_ERR_ARG, "sph_outcoords_fill: null argument");
     const int nb = sph_outcoords_blocks(g);
+    if (const unsigned long long *masks = outcoords_masks(g, (int32_t *)scratch)) {
+        hipLaunchKernelGGL(outcoords_fill_tile_kernel, dim3(nb), dim3(kThreads), 0, (hipStream_t)stream, g->B * g->O[0] * g->O[1],
+                           mask_chunks(g->O[2]), (const int32_t *)oz_ptr, oz_idx, out_rows, masks, row_cols);
+        return sph_check_launch("sph_outcoords_fill");
+    }
     hipLaunchKernelGGL(outcoords_fill_kernel, dim3(nb), dim3(kThreads), 0, (hipStream_t)stream,
-                       out_args(z_idx, z_ptr, in_rows, g), (const int32_t *)oz_ptr, oz_idx, out_rows,
-                       (const unsigned long long *)outcoords_masks(g, (int32_t *)scratch), row_cols);
+                       out_args(z_idx, z_ptr, in_rows, g), (const int32_t *)oz_ptr, oz_idx, out_rows, row_cols);
     return sph_check_launch("sph_outcoords_fill");
 }
 
