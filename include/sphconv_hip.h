@@ -278,6 +278,11 @@ size_t sph_wgrad_partial_elems(int KV, int iC, int oC, int out_rows);
 int sph_conv_wgrad(sph_dtype dt, const void *feature, int in_rows, int iC, const void *d_out,
                    int oC, const sph_book *fwd_book, float *partial, void *d_weight,
                    int d_weight_f32, void *stream);
+/* The same sum from the TRANSPOSED book (stationary on the input rows; partial: sph_wgrad_partial_elems of its rows), for
+ * a layer with fewer input than output rows whose transposed book exists anyway: the same pairs lie in fewer, fuller
+ * groups there. */
+int sph_conv_wgrad_transposed(sph_dtype dt, const void *feature, int iC, const void *d_out, int out_rows, int oC,
+                              const sph_book *t_book, float *partial, void *d_weight, int d_weight_f32, void *stream);
 
 /* ---- tensor construction / densify (tensor.cu) ------------------------- */
 

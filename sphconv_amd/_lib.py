@@ -83,6 +83,7 @@ _SIGNATURES = {
     "sph_rules_conv": (_I, [_P, _P, _I, _P, _P, _I, C.POINTER(Geom), C.POINTER(Book), _I, _P, _I, _P, _I, _P, _I,
                             C.POINTER(Epilogue), _P, _P]),
     "sph_wgrad_partial_elems": (_Z, [_I, _I, _I, _I]),
+    "sph_conv_wgrad_transposed": (_I, [_I, _P, _I, _P, _I, _I, C.POINTER(Book), _P, _P, _I, _P]),
     "sph_conv_wgrad": (_I, [_I, _P, _I, _I, _P, _I, C.POINTER(Book), _P, _P, _I, _P]),
     "sph_init_tensor_workspace": (_Z, [_I, _I, _I, _I, _I]),
     "sph_init_tensor": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _Z, _P]),

@@ -700,6 +700,7 @@ struct WgradArgs {
     const char *dout;
     int out_rows, oC;
     sph_book book;
+    const int32_t *list_in, *list_out; // the book's two lists: input rows and output rows of the groups
     int cap, ntiles, nchunk;
     float *partial;
     int *flags;      // wave kernel: one per partial slot, 1 = the slot was written
@@ -746,8 +747,8 @@ __global__ __launch_bounds__(kWgThreads) void wgrad_kernel(WgradArgs a)
                 int vi = -1, vo = -1;
                 if (g < g1) {
                     long slot = ((long)t * a.cap + g) * SPH_GROUP + (tid & (SPH_GROUP - 1));
-                    vi = a.book.grp_gather[slot];
-                    vo = a.book.grp_owner[slot];
+                    vi = a.list_in[slot];
+                    vo = a.list_out[slot];
                 }
                 if ((unsigned)vi >= (unsigned)a.in_rows || (unsigned)vo >= (unsigned)a.out_rows) vi = vo = -1;
                 s_in[tid] = vi;
@@ -825,6 +826,10 @@ __global__ void wgrad_reduce_kernel(const float *partial, int KV, int nchunk, in
 // LDS reads (16-bit types) or strided 4-byte reads (fp32).  The block lives in registers;
 // the workgroup's four blocks are summed through LDS into one fp32 partial, and
 // wgrad_slot_reduce_kernel adds the written slots in a fixed order.
+// The book is the layer's forward one or its transposed one (list_in, list_out): a strided layer on scattered voxels has
+// its pairs in 3.1 times fewer tiles stationary on the input rows, with groups more than twice as full (64->64 fp32 on
+// eight 64x512x512 scans, stride 2: 117 us from the forward book, 59 us from the transposed one with the empty fours left out;
+// 24->40 bf16: 52 -> 38 us).  Chunks of 32 or 16 tiles, for more workgroups, were slower (62 and 65 us).
 // What bounds it (64->64 fp16, 8 waves per CU): LDS traffic (8 KiB staged and 8 KiB read
 // back per batch and wave) and the MFMAs, about equally.
 // ---------------------------------------------------------------------------
@@ -993,7 +998,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_wave_kernel(WgradArgs a)
         const int fl = GPB * b + (pr >> 4);                 // group within the slice
         valid = s0 + fl < s1;
         const int base = __shfl(bases, fl & (kWave - 1), kWave);
-        return (lane < 32 ? a.book.grp_gather : a.book.grp_owner)[base + (pr & 15)];
+        return (lane < 32 ? a.list_in : a.list_out)[base + (pr & 15)];
     };
     // Row loads are unconditional (clamped to row 0; in_rows and out_rows are positive here)
     // so that several batches stay in flight; slots without a pair are zeroed when the rows
@@ -1025,16 +1030,32 @@ __global__ __launch_bounds__(256, 2) void wgrad_wave_kernel(WgradArgs a)
             if (dstG[it] >= 0) *(int4v *)(xg + dstG[it]) = ((ok >> pairG[it]) & 1) ? rg[it] : int4v{0, 0, 0, 0};
     };
     const char *fragA = xa + wgrad_frag_offset<DT>(rsA, lane), *fragG = xg + wgrad_frag_offset<DT>(rsG, lane);
-    auto multiply = [&]() {
+    // `ok`: pairs of the staged batch that exist.  fp32 takes the pairs four at a time and leaves out the fours behind the
+    // last of them (a group's pairs come first, its padding behind): at 32 cycles an MFMA the padding was most of what
+    // the kernel did on a strided layer's books, whose groups hold five pairs of sixteen.
+    auto multiply = [&](unsigned ok) {
         int4v fa[MI], fb[NI];
 #pragma unroll
         for (int i = 0; i < MI; i++) fa[i] = wgrad_frag<DT>(fragA + i * 16 * E, rsA);
 #pragma unroll
         for (int i = 0; i < NI; i++) fb[i] = wgrad_frag<DT>(fragG + i * 16 * E, rsG);
+        if constexpr (E == 4) {
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+            for (int s = 0; s < 4; s++) {
+                if (!(ok >> (4 * s))) break; // wave-uniform
 #pragma unroll
-            for (int j = 0; j < NI; j++) acc[i][j] = mfma_step<DT>(fa[i], fb[j], acc[i][j]);
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int j = 0; j < NI; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float4v, fa[i])[s],
+                                                                         __builtin_bit_cast(float4v, fb[j])[s], acc[i][j], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NI; j++) acc[i][j] = mfma_step<DT>(fa[i], fb[j], acc[i][j]);
+        }
     };
 
     // Per slice, this wave owns batches wave, wave+4, ... (at most NB).  All their index
@@ -1055,7 +1076,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_wave_kernel(WgradArgs a)
         for (int j = 0; j < NB; j++)
             idx[j] = (valid[j] && (unsigned)idx[j] < (unsigned)(lane < 32 ? a.in_rows : a.out_rows)) ? idx[j] : -1;
         int4v ra[DEPTH][MI], rg[DEPTH][NI];
-        unsigned ok[DEPTH];
+        unsigned ok[DEPTH], staged = 0;
 #pragma unroll
         for (int j = 0; j < DEPTH - 1; j++)
             if (j < NB) ok[j] = gather(idx[j], ra[j], rg[j]);
@@ -1064,13 +1085,14 @@ __global__ __launch_bounds__(256, 2) void wgrad_wave_kernel(WgradArgs a)
             if (wave + 4 * j < nbatch) {     // wave-uniform
                 if (j + DEPTH - 1 < NB)
                     ok[(j + DEPTH - 1) % DEPTH] = gather(idx[j + DEPTH - 1], ra[(j + DEPTH - 1) % DEPTH], rg[(j + DEPTH - 1) % DEPTH]);
-                if (j > 0) multiply();            // batch j-1, from LDS
+                if (j > 0) multiply(staged);      // batch j-1, from LDS
                 asm volatile("" ::: "memory");    // keep the staging writes behind the transposing reads
                 stage(ok[j % DEPTH], ra[j % DEPTH], rg[j % DEPTH]);
+                staged = ok[j % DEPTH] & (unsigned)((1ull << PB) - 1);
                 asm volatile("" ::: "memory");
             }
         }
-        if (wave < nbatch) multiply();            // the last staged batch
+        if (wave < nbatch) multiply(staged);      // the last staged batch
     }
 
     // Sum the four waves' blocks through LDS (over the staging areas), pairwise: (0+2, 1+3),
@@ -1523,27 +1545,30 @@ SPH_EXPORT size_t sph_wgrad_partial_elems(int KV, int iC, int oC, int out_rows)
     return general > fast ? general : fast;
 }
 
-SPH_EXPORT int sph_conv_wgrad(sph_dtype dt, const void *feature, int in_rows, int iC, const void *d_out,
-                              int oC, const sph_book *fwd_book, float *partial, void *d_weight, int d_weight_f32,
-                              void *stream)
+// `book`: stationary on the output rows, or on the input rows (`transposed`); other_rows: the rows its groups gather
+static int conv_wgrad(sph_dtype dt, const void *feature, int iC, const void *d_out, int oC, const sph_book *book, int other_rows,
+                      bool transposed, float *partial, void *d_weight, int d_weight_f32, void *stream)
 {
-    SPH_REQUIRE(book_ok(fwd_book) && book_has_groups(fwd_book), SPH_ERR_ARG, "sph_conv_wgrad: bad book (it must hold its groups)");
+    SPH_REQUIRE(book_ok(book) && book_has_groups(book), SPH_ERR_ARG, "sph_conv_wgrad: bad book (it must hold its groups)");
     SPH_REQUIRE(partial && d_weight, SPH_ERR_ARG, "sph_conv_wgrad: null pointer");
     SPH_REQUIRE(dt == SPH_F32 || dt == SPH_F16 || dt == SPH_BF16, SPH_ERR_UNSUPPORTED,
                 "sph_conv_wgrad: dtype %d has no weight gradient", (int)dt);
     SPH_REQUIRE(iC > 0 && iC <= 128 && oC > 0 && oC <= 128, SPH_ERR_UNSUPPORTED,
                 "sph_conv_wgrad: channels %d->%d not in 1..128", iC, oC);
-    SPH_REQUIRE((in_rows == 0 || feature) && (fwd_book->rows == 0 || d_out), SPH_ERR_ARG, "sph_conv_wgrad: null pointer");
+    const int in_rows = transposed ? book->rows : other_rows, out_rows = transposed ? other_rows : book->rows;
+    SPH_REQUIRE((in_rows == 0 || feature) && (out_rows == 0 || d_out), SPH_ERR_ARG, "sph_conv_wgrad: null pointer");
     WgradArgs a;
     a.feat = (const char *)feature;
     a.in_rows = in_rows;
     a.iC = iC;
     a.dout = (const char *)d_out;
-    a.out_rows = fwd_book->rows;
+    a.out_rows = out_rows;
     a.oC = oC;
-    a.book = *fwd_book;
-    a.cap = sph_book_cap(fwd_book->KV);
-    a.ntiles = sph_book_tiles(fwd_book->rows);
+    a.book = *book;
+    a.list_in = transposed ? book->grp_owner : book->grp_gather;
+    a.list_out = transposed ? book->grp_gather : book->grp_owner;
+    a.cap = sph_book_cap(book->KV);
+    a.ntiles = sph_book_tiles(book->rows);
     a.nchunk = wgrad_chunks(a.ntiles);
     a.partial = partial;
     a.nslots = 0;
@@ -1556,4 +1581,17 @@ SPH_EXPORT int sph_conv_wgrad(sph_dtype dt, const void *feature, int in_rows, in
     case SPH_F16: return launch_wgrad<SPH_F16>(a, d_weight, d_weight_f32 != 0, st);
     default: return launch_wgrad<SPH_BF16>(a, d_weight, d_weight_f32 != 0, st);
     }
+}
+
+SPH_EXPORT int sph_conv_wgrad(sph_dtype dt, const void *feature, int in_rows, int iC, const void *d_out,
+                              int oC, const sph_book *fwd_book, float *partial, void *d_weight, int d_weight_f32,
+                              void *stream)
+{
+    return conv_wgrad(dt, feature, iC, d_out, oC, fwd_book, in_rows, false, partial, d_weight, d_weight_f32, stream);
+}
+
+SPH_EXPORT int sph_conv_wgrad_transposed(sph_dtype dt, const void *feature, int iC, const void *d_out, int out_rows, int oC,
+                                         const sph_book *t_book, float *partial, void *d_weight, int d_weight_f32, void *stream)
+{
+    return conv_wgrad(dt, feature, iC, d_out, oC, t_book, out_rows, true, partial, d_weight, d_weight_f32, stream);
 }

@@ -373,15 +373,20 @@ py::object rules_conv(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz
     return py::cast(out);
 }
 
-Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf, bool f32)
+Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf, bool transposed, bool f32)
 {
     const Tensor feature = feature_.contiguous(), d_out = d_out_.contiguous();
     const int ic = (int)feature.size(1), oc = (int)d_out.size(1);
     const int64_t n = (int64_t)sph_wgrad_partial_elems(buf.kv, ic, oc, buf.book.rows);
     const Tensor partial = at::empty({n > 0 ? n : 1}, feature.options().dtype(at::kFloat).requires_grad(false));
     const Tensor dw = at::empty({buf.kv, ic, oc}, feature.options().dtype(f32 ? at::kFloat : feature.scalar_type()).requires_grad(false));
-    check(sph_conv_wgrad((sph_dtype)dtype_code(feature.scalar_type()), ptr(feature), (int)feature.size(0), ic, ptr(d_out), oc, &buf.book,
-                         (float *)partial.data_ptr(), dw.data_ptr(), f32, stream()));
+    const sph_dtype dt = (sph_dtype)dtype_code(feature.scalar_type());
+    if (transposed)
+        check(sph_conv_wgrad_transposed(dt, ptr(feature), ic, ptr(d_out), (int)d_out.size(0), oc, &buf.book, (float *)partial.data_ptr(),
+                                        dw.data_ptr(), f32, stream()));
+    else
+        check(sph_conv_wgrad(dt, ptr(feature), (int)feature.size(0), ic, ptr(d_out), oc, &buf.book, (float *)partial.data_ptr(),
+                             dw.data_ptr(), f32, stream()));
     return dw;
 }
 

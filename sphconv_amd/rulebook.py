@@ -413,6 +413,10 @@ class RuleBook:
             self._bwd = self._convert(True) if self._from_padded is not None else self._build(True)
         return self._bwd
 
+    def transposed_groups_built(self) -> bool:
+        """True if the transposed book exists, with its groups."""
+        return self._bwd is not None and self._bwd.groups
+
     def num_pairs(self) -> int:
         return self.fwd.num_pairs()
 

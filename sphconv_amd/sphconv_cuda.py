@@ -299,7 +299,10 @@ def rule_conv_d_weight(feature: torch.Tensor, d_featureOut: torch.Tensor, rules,
         d_out = d_out.to(feature.dtype)
     if out_dtype not in (None, feature.dtype, torch.float32):
         raise L.SphconvError("d_weight comes in the features' type or in float32, not %s" % out_dtype)
-    return L.host().conv_wgrad(feature, d_out, book.grouped().native, out_dtype == torch.float32)
+    # From the book with fewer tiles, if dgrad has made the transposed one: the same pairs lie in fewer, fuller groups
+    # there (a strided layer on scattered voxels has more output than input rows, its forward groups five pairs of 16).
+    transposed = book.transposed_groups_built() and book.in_rows < book.out_rows
+    return L.host().conv_wgrad(feature, d_out, book.grouped(transposed).native, transposed, out_dtype == torch.float32)
 
 
 def rule_conv_backward(d_featureOut: torch.Tensor, feature: torch.Tensor, weight: torch.Tensor, rules,
