@@ -56,6 +56,12 @@ inline RankLayout rank_layout(int n, int ncol)
 
 constexpr size_t kBitmapMaxBytes = (size_t)1 << 30; // grids whose bitmap would be larger are ranked by the walk
 
+// Columns per thread of the scan of the columns' bit counts.  With eight, 32 768 columns of eight words are sixteen
+// workgroups that fetch 128 KB each: 12.8 us.  So the columns of deep grids go one to a thread as long as the workgroups
+// stay few (they take a number each, one after the other, at 20 ns).
+constexpr int kWideScanCols = 65536;
+inline int scan_items(int ncol, int words) { return words > 1 && ncol <= kWideScanCols ? 1 : sph_scan::kItems; }
+
 struct BitLayout {
     size_t bits, bits_bytes, temp, temp_bytes, total;
     int words; // 64-bit words per column
@@ -68,7 +74,7 @@ inline BitLayout bit_layout(int ncol, int S2)
     l.bits = 0;
     l.bits_bytes = (size_t)ncol * l.words * sizeof(unsigned long long);
     l.temp = align256(l.bits_bytes);
-    l.temp_bytes = sum_scan_bytes(ncol);
+    l.temp_bytes = sph_scan::state_bytes(ncol, scan_items(ncol, l.words));
     l.total = l.temp_bytes ? l.temp + align256(l.temp_bytes) : 0;
     return l;
 }
@@ -120,16 +126,32 @@ __global__ __launch_bounds__(256) void coo_mark_kernel(const int32_t *idx, int n
 }
 
 // rows of a column, from its bitmap (what the scan reads)
+template <int WORDS> // words per column where that is known to the compiler: their loads are then in flight together; 0: any
 struct ColumnRows {
     const unsigned long long *bits;
     int words;
     __device__ __forceinline__ int operator()(long col) const
     {
         int n = 0;
-        for (int w = 0; w < words; w++) n += __popcll(bits[(size_t)col * words + w]);
+        if constexpr (WORDS > 0) {
+            const unsigned long long *p = bits + (size_t)col * WORDS;
+#pragma unroll
+            for (int w = 0; w < WORDS; w++) n += __popcll(p[w]);
+        } else {
+            for (int w = 0; w < words; w++) n += __popcll(bits[(size_t)col * words + w]);
+        }
         return n;
     }
 };
+
+template <int WORDS>
+inline hipError_t scan_columns(const unsigned long long *bits, int words, int32_t *z_ptr, int ncol, void *state, hipStream_t st)
+{
+    const sph_scan::FromFunction<ColumnRows<WORDS>> rows{ColumnRows<WORDS>{bits, words}};
+    const sph_scan::ToArray out{z_ptr, nullptr};
+    if (scan_items(ncol, words) == 1) return sph_scan::launch_from<sph_scan::Plus, 1>(rows, out, ncol, state, st, /*clear_state=*/false);
+    return sph_scan::launch_from<sph_scan::Plus, sph_scan::kItems>(rows, out, ncol, state, st, /*clear_state=*/false);
+}
 
 struct CooRows {
     const int32_t *z_ptr;
@@ -262,7 +284,7 @@ static int init_tensor_by_rank(const int32_t *indices, int n, int B, int S0, int
     hipLaunchKernelGGL(coo_count_kernel, grid, block, 0, st, indices, n, B, S0, S1, S2, z_ptr, slot, status);
     rc = sph_check_launch("sph_init_tensor(count)");
     if (rc) return rc;
-    hipError_t e = sph_scan::launch<sph_scan::Plus, true>(z_ptr, z_ptr, ncol, ws + l.temp, 0, st);
+    hipError_t e = sph_scan::launch(z_ptr, z_ptr, ncol, ws + l.temp, st);
     if (e != hipSuccess) {
         sph_set_error("sph_init_tensor: scan: %s", hipGetErrorString(e));
         return SPH_ERR_LAUNCH;
@@ -314,8 +336,14 @@ SPH_EXPORT int sph_init_tensor_rows(const int32_t *indices, int n, int B, int S0
     const dim3 block(256);
     if (n > 0)
         hipLaunchKernelGGL(coo_mark_kernel, dim3(sph_div_up(n, 256)), block, 0, st, indices, n, g, (unsigned long long *)(ws + l.bits), status);
-    const hipError_t e = sph_scan::launch_from<sph_scan::Plus, true>(sph_scan::FromFunction<ColumnRows>{ColumnRows{r.bits, l.words}}, z_ptr,
-                                                                     (long)ncol, ws + l.temp, 0, st, nullptr, /*clear_state=*/false);
+    hipError_t e;
+    switch (l.words) {
+    case 1: e = scan_columns<1>(r.bits, 1, z_ptr, ncol, ws + l.temp, st); break;
+    case 2: e = scan_columns<2>(r.bits, 2, z_ptr, ncol, ws + l.temp, st); break;
+    case 4: e = scan_columns<4>(r.bits, 4, z_ptr, ncol, ws + l.temp, st); break;
+    case 8: e = scan_columns<8>(r.bits, 8, z_ptr, ncol, ws + l.temp, st); break;
+    default: e = scan_columns<0>(r.bits, l.words, z_ptr, ncol, ws + l.temp, st); break;
+    }
     if (e != hipSuccess) {
         sph_set_error("%s: scan: %s", who, hipGetErrorString(e));
         return SPH_ERR_LAUNCH;

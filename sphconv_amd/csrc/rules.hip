@@ -619,8 +619,7 @@ static int outcoords_count(const char *who, const int32_t *z_idx, const int32_t 
     int rc = sph_check_launch(who);
     if (rc) return rc;
     // counts -> inclusive scan in place; the last tile also writes the row count
-    hipError_t e = sph_scan::launch<sph_scan::Plus, true>(oz_ptr, oz_ptr, ncol, scratch, 0, (hipStream_t)stream, total,
-                                                          /*clear_state=*/false);
+    hipError_t e = sph_scan::launch(oz_ptr, oz_ptr, ncol, scratch, (hipStream_t)stream, total, /*clear_state=*/false);
     if (e != hipSuccess) {
         sph_set_error("%s: scan: %s", who, hipGetErrorString(e));
         return SPH_ERR_LAUNCH;

@@ -8,15 +8,14 @@
 // loop:
 //   1. vox_clear_kernel    zeroes the outputs and resets the workspace (one launch)
 //   2. vox_insert_kernel   system coordinates (float32, operation by operation as numpy does it) and
-//                          the cell of every point; a point inside the grid enters its cell into a hash
-//                          table (open addressing, at most half full), counts itself there and offers
-//                          its index as the cell's first point (atomic minimum)
-//   3. one exclusive sum   over [counts of the table's slots | 1 for every point that opens a cell]: a slot's
-//                          segment of the point list, and (minus the points inside) every such point's voxel
-//                          number; the second half is made as it is read
-//   4. vox_scatter_kernel  writes every point into its cell's segment (in any order); the point
-//                          that would open voxel number max_voxels is where the reference's loop
-//                          stops: every later point is dropped
+//                          the cell of every point; the cells of a workgroup's points meet in a table in LDS, and each
+//                          of them enters a hash table (open addressing, at most half full), with the number of its
+//                          points and the smallest of their indices (atomic sum and minimum)
+//   3. one scan            over the points: those that open a cell count as one voxel and as their cell's number of
+//                          points, so the sums in front of one are its voxel number and the start of its cell's segment
+//                          of the point list; they go to the cell's record.  The point that would open voxel number
+//                          max_voxels is where the reference's loop stops: every later point is dropped
+//   4. vox_scatter_kernel  writes every point into its cell's segment (in any order)
 //   5. vox_write_kernel    a point's place in its voxel = the number of smaller point indices in its
 //                          segment (counted until max_points are found: such a point is dropped);
 //                          segments of more than 256 points are walked by the whole wave, 64 entries at a time
@@ -95,98 +94,150 @@ constexpr int kFills = 10;
 constexpr int kFillBlocks = 128;  // workgroups per range
 constexpr int kLongSegment = 256; // longer segments are walked by the wave together
 
-// up to kFills ranges of 32-bit words, each set to its value: blockIdx.y = range
+// up to kFills ranges of 32-bit words, each set to its value (or to two values in turn: an even number of words, aligned
+// to 16 bytes): blockIdx.y = range
 struct VoxFills {
     int32_t *p[kFills];
     long words[kFills];
-    int32_t value[kFills];
+    int32_t value[kFills], odd_value[kFills];
 };
 
 __global__ __launch_bounds__(256) void vox_clear_kernel(VoxFills f)
 {
     int32_t *p = f.p[blockIdx.y];
     const long n = f.words[blockIdx.y];
-    const int32_t v = f.value[blockIdx.y];
+    const int32_t v = f.value[blockIdx.y], w = f.odd_value[blockIdx.y];
     const long t = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
     if (((uintptr_t)p & 15) == 0) {
-        const int4 v4 = make_int4(v, v, v, v);
+        const int4 v4 = make_int4(v, w, v, w);
         for (long i = t; i < n / 4; i += step) ((int4 *)p)[i] = v4;
-        if (t < (n & 3)) p[(n & ~3L) + t] = v;
+        if (t < (n & 3)) p[(n & ~3L) + t] = (t & 1) ? w : v;
     } else {
         for (long i = t; i < n; i += step) p[i] = v;
     }
 }
 
-// tbits = log2 of the table's slots
-__global__ __launch_bounds__(256) void vox_insert_kernel(const float *points, int n, VoxParams q, const long long *cell_in,
-                                                         int tbits, unsigned long long *keys, int32_t *first,
-                                                         int32_t *count, int32_t *slot_of, long long *cell_out)
+// tbits = log2 of the table's slots.  slot_place[i]: the point's slot (-1: outside the grid) and its place in the slot's
+// segment, the places given in the order of arrival: from the front (>= 0) to the points of the workgroup that brought the
+// cell, from the back (-1, -2, ...) to all others.
+// Device-wide atomics bound it (about 24 per ns over the chip), so there are few: what a workgroup's points have in common
+// is settled in LDS, and the workgroup that brings a cell needs one, the compare-and-swap, and stores its points' number
+// and smallest index where nobody else does (`brought`); the others add to `later` (smallest index, number).  123 k points
+// in 24 k cells: 17.4 us with three atomics per point, 13.6 us this way.
+constexpr int kInsertThreads = 512, kInsertSlots = 1024; // (at most half full too)
+__global__ __launch_bounds__(kInsertThreads) void vox_insert_kernel(const float *points, int n, VoxParams q, const long long *cell_in,
+                                                                    int tbits, unsigned long long *keys, int2 *brought,
+                                                                    int2 *later, int2 *slot_place, long long *cell_out)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint64_t key = point_cell(points, i, q, cell_in);
-    if (cell_out) cell_out[i] = key == q.cells ? -1 : (long long)key;
-    if (key == q.cells) {
-        slot_of[i] = -1;
-        return;
+    __shared__ unsigned long long s_key[kInsertSlots];
+    __shared__ int s_first[kInsertSlots], s_count[kInsertSlots], s_slot[kInsertSlots], s_base[kInsertSlots];
+    const int i = blockIdx.x * kInsertThreads + threadIdx.x;
+    for (int e = threadIdx.x; e < kInsertSlots; e += kInsertThreads) {
+        s_key[e] = kEmptyKey;
+        s_first[e] = INT_MAX;
+        s_count[e] = 0;
     }
-    const unsigned mask = (1u << tbits) - 1u;
-    unsigned slot = (unsigned)((key * 0x9E3779B97F4A7C15ull) >> (64 - tbits));
-    // the table has at least twice as many slots as there are points: a free one is always met
-    for (;;) {
-        const unsigned long long seen = atomicCAS(&keys[slot], (unsigned long long)kEmptyKey, (unsigned long long)key);
-        if (seen == kEmptyKey || seen == key) break;
-        slot = (slot + 1) & mask;
+    __syncthreads();
+    const uint64_t key = i < n ? point_cell(points, i, q, cell_in) : (uint64_t)q.cells;
+    if (cell_out && i < n) cell_out[i] = key == q.cells ? -1 : (long long)key;
+    const bool inside = key != q.cells;
+    const uint64_t hash = key * 0x9E3779B97F4A7C15ull;
+    int e = 0, place = 0;
+    bool opens = false; // the first of the workgroup's points to bring this cell
+    if (inside) {
+        e = (int)(hash >> (64 - 10));
+        for (;;) {
+            const unsigned long long seen = atomicCAS(&s_key[e], (unsigned long long)kEmptyKey, (unsigned long long)key);
+            opens = seen == kEmptyKey;
+            if (opens || seen == key) break;
+            e = (e + 1) & (kInsertSlots - 1);
+        }
+        place = atomicAdd(&s_count[e], 1);
+        atomicMin(&s_first[e], i);
     }
-    atomicAdd(&count[slot], 1);
-    atomicMin(&first[slot], i);
-    slot_of[i] = (int32_t)slot;
+    __syncthreads();
+    if (opens) {
+        const unsigned mask = (1u << tbits) - 1u;
+        unsigned slot = (unsigned)(hash >> (64 - tbits));
+        unsigned long long seen;
+        // the table has at least twice as many slots as there are points: a free one is always met
+        for (;;) {
+            seen = atomicCAS(&keys[slot], (unsigned long long)kEmptyKey, (unsigned long long)key);
+            if (seen == kEmptyKey || seen == key) break;
+            slot = (slot + 1) & mask;
+        }
+        if (seen == kEmptyKey) {
+            brought[slot] = make_int2(s_first[e], s_count[e]);
+            s_base[e] = -1;
+        } else {
+            atomicMin(&later[slot].x, s_first[e]);
+            s_base[e] = atomicAdd(&later[slot].y, s_count[e]);
+        }
+        s_slot[e] = (int)slot;
+    }
+    __syncthreads();
+    if (i < n) slot_place[i] = inside ? make_int2(s_slot[e], s_base[e] < 0 ? place : ~(s_base[e] + place)) : make_int2(-1, 0);
 }
 
-// what the scan reads: the counts of the table's slots, then 1 for every point that opens a cell, made on the fly
-struct CountsThenMarks {
-    const int32_t *count, *slot_of, *first;
-    long T;
-    __device__ __forceinline__ int operator()(long i) const
+// What the scan reads: per point that opens a cell one voxel (upper half) and the cell's points (lower 30 bits).
+constexpr int kPairShift = 30;
+constexpr int kPointItems = 4; // points per thread of the scan
+struct OpenedCells {
+    const int2 *brought, *later, *slot_place;
+    __device__ __forceinline__ unsigned long long operator()(long i) const
     {
-        if (i < T) return count[i];
-        const int p = (int)(i - T), s = slot_of[p];
-        return s >= 0 && first[s] == p;
+        const int s = slot_place[i].x;
+        if (s < 0) return 0ull;
+        const int2 b = brought[s], l = later[s];
+        return min(b.x, l.x) == (int)i ? (1ull << kPairShift) + (unsigned)(b.y + l.y) : 0ull;
     }
 };
+// ... and where the sums go: rec[slot] = (first and last + 1 of its segment, its voxel number, the point that opened it)
+struct CellRecords {
+    const int2 *slot_place;
+    int4 *rec;
+    int32_t *stop, *voxel_num;
+    int max_voxels;
+    template <int ITEMS>
+    __device__ __forceinline__ void tile(long base, long, unsigned long long before, const unsigned long long (&incl)[ITEMS]) const
+    {
+        constexpr unsigned long long kLow = (1ull << kPairShift) - 1;
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const unsigned long long excl = j ? incl[j - 1] : before;
+            if (incl[j] == excl) continue;
+            const int i = (int)(base + j), vid = (int)(excl >> kPairShift);
+            rec[slot_place[i].x] = make_int4((int)(excl & kLow), (int)(incl[j] & kLow), vid, i);
+            if (vid == max_voxels) *stop = i; // exactly one such point, if any
+        }
+    }
+    __device__ __forceinline__ void all(unsigned long long sum) const { *voxel_num = min((int)(sum >> kPairShift), max_voxels); }
+};
 
-// sum[0..T): first place of every slot's segment; sum[T + i] - sum[T]: marks in front of point i; *total: all of it
-__global__ __launch_bounds__(256) void vox_scatter_kernel(const int32_t *slot_of, const int32_t *sum, const int32_t *first,
-                                                          const int32_t *total, int n, long T, int max_voxels,
-                                                          int32_t *count, int32_t *seg, int32_t *stop, int32_t *voxel_num)
+__global__ __launch_bounds__(256) void vox_scatter_kernel(const int2 *slot_place, const int4 *rec, int n, int32_t *seg)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int s = slot_of[i];
-    const int inside = sum[T];
-    if (s >= 0) {
-        seg[sum[s] + atomicSub(&count[s], 1) - 1] = i;
-        if (first[s] == i && sum[T + i] - inside == max_voxels) *stop = i; // exactly one such point, if any
-    }
-    if (i == 0) *voxel_num = min(*total - inside, max_voxels);
+    const int2 sp = slot_place[i];
+    if (sp.x < 0) return;
+    const int4 r = rec[sp.x];
+    seg[(sp.y >= 0 ? r.x : r.y) + sp.y] = i;
 }
 
 __global__ __launch_bounds__(256) void vox_write_kernel(const float *points, int n, VoxParams q, const unsigned long long *keys,
-                                                        const int32_t *first, const int32_t *slot_of, const int32_t *sum,
-                                                        const int32_t *seg, long T, const int32_t *stop, float *voxels,
-                                                        float *mask, int32_t *coors, int32_t *num_points)
+                                                        const int2 *slot_place, const int4 *rec, const int32_t *seg,
+                                                        const int32_t *stop, float *voxels, float *mask, int32_t *coors,
+                                                        int32_t *num_points)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const int s = i < n ? slot_of[i] : -1;
+    const int s = i < n ? slot_place[i].x : -1;
     int vid = 0, h = 0, s0 = 0, s1 = 0;
     bool live = s >= 0;
     if (live) {
-        h = first[s];
-        vid = sum[T + h] - sum[T];
+        const int4 r = rec[s];
+        s0 = r.x; s1 = r.y; vid = r.z; h = r.w;
         live = vid < q.max_voxels && i < *stop;
-        s0 = sum[s];
-        s1 = sum[s + 1]; // slot T - 1 ends where the marks begin: sum[T] = points inside
     }
     // place among the cell's points = smaller indices in the segment
     int rank = 0;
@@ -231,7 +282,7 @@ __global__ __launch_bounds__(256) void vox_write_kernel(const float *points, int
 struct VoxLayout {
     int tbits;
     long T; // slots of the table: a power of two, at least twice the points
-    size_t keys, first, count, sum, slot_of, seg, stop, state, state_words, total;
+    size_t keys, later, brought, rec, slot_place, seg, stop, state, state_words, total;
 };
 
 inline size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -245,15 +296,15 @@ inline VoxLayout vox_layout(int n)
     l.T = 1L << l.tbits;
     size_t o = 0;
     l.keys = o; o += al256((size_t)l.T * 8);
-    l.first = o; o += al256((size_t)l.T * 4);
-    l.count = o; o += al256((size_t)l.T * 4);
-    l.sum = o; o += al256(((size_t)l.T + nn) * 4);
-    l.slot_of = o; o += al256(nn * 4);
+    l.later = o; o += al256((size_t)l.T * 8);
+    l.brought = o; o += al256((size_t)l.T * 8);
+    l.rec = o; o += al256((size_t)l.T * 16);
+    l.slot_place = o; o += al256(nn * 8);
     l.seg = o; o += al256(nn * 4);
-    l.stop = o; o += 256;                            // stop, total
+    l.stop = o; o += 256;
     l.state = o;
-    l.state_words = (size_t)sph_scan::state_ints(l.T + (long)nn);
-    o += al256(sph_scan::state_bytes(l.T + (long)nn));
+    l.state_words = (size_t)sph_scan::state_ints((long)nn, kPointItems);
+    o += al256(sph_scan::state_bytes((long)nn, kPointItems));
     l.total = o;
     return l;
 }
@@ -295,48 +346,52 @@ SPH_EXPORT int sph_points_to_voxel(const float *points, int n, int nfeat, int sy
     hipStream_t st = (hipStream_t)stream;
     char *ws = (char *)workspace;
     unsigned long long *keys = (unsigned long long *)(ws + l.keys);
-    int32_t *first = (int32_t *)(ws + l.first), *count = (int32_t *)(ws + l.count), *sum = (int32_t *)(ws + l.sum);
-    int32_t *slot_of = (int32_t *)(ws + l.slot_of), *seg = (int32_t *)(ws + l.seg), *stop = (int32_t *)(ws + l.stop);
-    int32_t *total = stop + 1;
+    int2 *later = (int2 *)(ws + l.later), *brought = (int2 *)(ws + l.brought);
+    int32_t *seg = (int32_t *)(ws + l.seg), *stop = (int32_t *)(ws + l.stop);
+    int2 *slot_place = (int2 *)(ws + l.slot_place);
+    int4 *rec = (int4 *)(ws + l.rec);
 
     const int width = append_mode == 1 ? nfeat + 3 : nfeat;
     const long nv = (long)max_voxels * max_points;
     VoxFills f;
     int nf = 0;
+    auto fill_pairs = [&](void *p, long pairs, int32_t v, int32_t w) {
+        f.p[nf] = (int32_t *)p; f.words[nf] = 2 * pairs; f.value[nf] = v; f.odd_value[nf] = w;
+        nf++;
+    };
     auto fill = [&](void *p, long words, int32_t v) {
-        f.p[nf] = (int32_t *)p; f.words[nf] = words; f.value[nf] = v;
+        f.p[nf] = (int32_t *)p; f.words[nf] = words; f.value[nf] = f.odd_value[nf] = v;
         nf++;
     };
     fill(voxels, nv * width, 0);
     fill(mask, nv, 0);
     fill(coors, 3L * max_voxels, 0);
     fill(num_points, (long)max_voxels, 0);
-    if (n == 0) fill(voxel_num, 1L, 0); // else it is written once, by the scatter kernel: the host may be watching it
+    if (n == 0) fill(voxel_num, 1L, 0); // else it is written once, by the scan: the host may be watching it
     if (n > 0) {
         fill(keys, 2 * l.T, -1);
-        fill(first, l.T, INT_MAX);
-        fill(count, l.T, 0);
+        fill_pairs(later, l.T, INT_MAX, 0);
         fill(stop, 1L, n);
         fill(ws + l.state, (long)l.state_words, 0);
     }
     hipLaunchKernelGGL(vox_clear_kernel, dim3(kFillBlocks, nf), dim3(256), 0, st, f);
     int rc = sph_check_launch("sph_points_to_voxel(clear)");
     if (rc || n == 0) return rc;
-    hipLaunchKernelGGL(vox_insert_kernel, dim3(blocks(n)), dim3(256), 0, st, points, n, q, cell_in, l.tbits, keys, first,
-                       count, slot_of, cell_out);
+    hipLaunchKernelGGL(vox_insert_kernel, dim3(sph_div_up(n, kInsertThreads)), dim3(kInsertThreads), 0, st, points, n, q, cell_in,
+                       l.tbits, keys, brought, later, slot_place, cell_out);
     rc = sph_check_launch("sph_points_to_voxel(cells)");
     if (rc) return rc;
-    const hipError_t e = sph_scan::launch_from<sph_scan::Plus, false>(
-        sph_scan::FromFunction<CountsThenMarks>{CountsThenMarks{count, slot_of, first, l.T}}, sum, l.T + n, ws + l.state, 0, st, total, false);
+    const hipError_t e = sph_scan::launch_from<sph_scan::PlusPair, kPointItems>(
+        sph_scan::FromFunction<OpenedCells>{OpenedCells{brought, later, slot_place}}, CellRecords{slot_place, rec, stop, voxel_num, max_voxels},
+        (long)n, ws + l.state, st, /*clear_state=*/false);
     if (e != hipSuccess) {
         sph_set_error("sph_points_to_voxel: scan: %s", hipGetErrorString(e));
         return SPH_ERR_LAUNCH;
     }
-    hipLaunchKernelGGL(vox_scatter_kernel, dim3(blocks(n)), dim3(256), 0, st, (const int32_t *)slot_of, (const int32_t *)sum,
-                       (const int32_t *)first, (const int32_t *)total, n, l.T, max_voxels, count, seg, stop, voxel_num);
+    hipLaunchKernelGGL(vox_scatter_kernel, dim3(blocks(n)), dim3(256), 0, st, (const int2 *)slot_place, (const int4 *)rec, n, seg);
     hipLaunchKernelGGL(vox_write_kernel, dim3(blocks(n)), dim3(256), 0, st, points, n, q, (const unsigned long long *)keys,
-                       (const int32_t *)first, (const int32_t *)slot_of, (const int32_t *)sum, (const int32_t *)seg, l.T,
-                       (const int32_t *)stop, voxels, mask, coors, num_points);
+                       (const int2 *)slot_place, (const int4 *)rec, (const int32_t *)seg, (const int32_t *)stop, voxels, mask, coors,
+                       num_points);
     return sph_check_launch("sph_points_to_voxel");
 }
 
