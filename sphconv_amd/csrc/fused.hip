@@ -69,7 +69,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(S > 1 ? 1 : 
     __shared__ unsigned long long s_cov[2];
 
     // 1. the tile's pairs: the table of (row, offset) -> gathered row
-    tile_table<false, false, NT>(b, tile, s_nbr, nullptr);
+    tile_table<false, false, true, true, NT>(b, tile, s_nbr, nullptr);
     // 2. the groups, from the table straight to region B (compact_groups).  Those of the middle offset (in a
     // submanifold layer: every row's pair with itself, a run of eight full groups) go to the waves that would
     // otherwise wait, and are the first the tile is given: stored, not added.  Region B keeps them behind the
@@ -264,6 +264,7 @@ SPH_EXPORT int sph_rules_conv(const int32_t *z_idx, const int32_t *z_ptr, int in
     b.pack.job[0].total = b.pack.job[1].total = 0;
     b.tile_blocks = 0;
     b.long_fibers = 0;
+    b.lines = join_lines(b, false);
     const int nt = sph_book_tiles(out_rows);
     hipStream_t st = (hipStream_t)stream;
     switch (dt) {

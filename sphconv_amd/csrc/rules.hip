@@ -18,7 +18,8 @@ namespace {
 
 // Book builder: one workgroup per tile of R stationary rows (tile_table, then emit_groups); workgroups behind
 // the tiles' pack a weight.
-template <bool TRANSPOSED>
+// LINES: the kernel for joins by lines alone; else the one for masks and columns (long fibers, wide kernels).
+template <bool TRANSPOSED, bool LINES>
 __global__ __launch_bounds__(kThreads) void build_book_kernel(BuildArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) int32_t s_nbr[]; // [R * KV], emit scratch, masks of the mask join
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(kThreads) void build_book_kernel(BuildArgs a)
     const int KV = a.cv.K0 * a.cv.K1 * a.cv.K2;
     const int r0 = tile * R;
     if (r0 >= a.q_rows) return; // grid is padded to a multiple of the XCD count
-    tile_table<TRANSPOSED, true, kThreads>(a, tile, s_nbr, (char *)(s_nbr + R * KV) + emit_scratch_bytes(KV));
+    tile_table<TRANSPOSED, !LINES, LINES, !LINES, kThreads>(a, tile, s_nbr, (char *)(s_nbr + R * KV) + emit_scratch_bytes(KV));
     emit_groups<kThreads>(s_nbr, min(R, a.q_rows - r0), r0, KV, tile, a.cap, emit_scratch_at(s_nbr + R * KV, KV), a.book);
 }
 
@@ -496,13 +497,14 @@ static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_p
     const size_t lds_masks = (size_t)kMaskCols * (g->K[0] * g->K[1]) * (sizeof(unsigned long long) + sizeof(int32_t));
     a.long_fibers = a.P.n2 <= 64 && (long)a.p_rows >= 4 * p_cols && lds + lds_masks <= 64 * 1024;
     if (a.long_fibers) lds += lds_masks;
+    a.lines = join_lines(a, transposed != 0);
     hipStream_t st = (hipStream_t)stream;
-    int rc = transposed ? allow_lds(build_book_kernel<true>, lds, who) : allow_lds(build_book_kernel<false>, lds, who);
+    const bool by_lines = a.lines && !a.long_fibers;
+    void (*kernel)(BuildArgs) = transposed ? (by_lines ? build_book_kernel<true, true> : build_book_kernel<true, false>)
+                                           : (by_lines ? build_book_kernel<false, true> : build_book_kernel<false, false>);
+    const int rc = allow_lds(kernel, lds, who);
     if (rc) return rc;
-    if (!transposed)
-        hipLaunchKernelGGL(build_book_kernel<false>, dim3(a.tile_blocks + pack_blocks), dim3(kThreads), lds, st, a);
-    else
-        hipLaunchKernelGGL(build_book_kernel<true>, dim3(a.tile_blocks + pack_blocks), dim3(kThreads), lds, st, a);
+    hipLaunchKernelGGL(kernel, dim3(a.tile_blocks + pack_blocks), dim3(kThreads), lds, st, a);
     return sph_check_launch(who);
 }
 

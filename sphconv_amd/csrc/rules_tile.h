@@ -424,6 +424,7 @@ struct BuildArgs {
     // gathered-side fibers are long (several entries on average) and their bins fit a 64-bit mask:
     // join through per-column occupancy masks instead of walking a fiber once per row
     int long_fibers;
+    int lines;             // columns a row can pair with on one line of the gathered grid, if the join goes by lines (1 to 3), else 0
     FastDiv by_q1, by_q01; // division by Q.n1 and by Q.n0 * Q.n1
     // optional: column of every stationary row (q_rows entries; what the producer of the coordinates knew when it
     // wrote them).  Null: the columns are searched for in q_ptr.  Every entry is checked against q_ptr before it is
@@ -431,14 +432,24 @@ struct BuildArgs {
     const int32_t *q_rowcol;
 };
 
+// Columns a row can pair with on a line, where the join can go by lines: at most three of them, and the gathered grid's
+// arrays within the reach of a buffer descriptor.  (Wider kernels take the join by columns.)
+inline int join_lines(const BuildArgs &a, bool transposed)
+{
+    const int c = transposed ? (a.cv.K1 + a.cv.s1 - 1) / a.cv.s1 : a.cv.K1;
+    const bool reach = (double)a.B * a.P.n0 * a.P.n1 < 5e8 && a.p_rows < 500000000 && a.P.n2 < (1 << 22) && a.cv.s2 < (1 << 22);
+    return c <= 3 && reach ? c : 0;
+}
+
 constexpr int kMaskCols = 32;  // distinct columns of a tile the mask join provides for
 constexpr int kMaskWalk = 16;  // fiber entries fetched together when a mask is built
 
 // Fills s_nbr[row of the tile * KV + k] = gathered row or -1 for tile `tile` (which must hold at least one row) by
 // the whole workgroup of kThreads threads; returns behind a barrier.  s_masks: LDS for the mask join (used when
 // a.long_fibers; kMaskCols * K0 * K1 * 12 bytes, 8-byte aligned).
-// MASKS = false leaves the mask join (and its 3 KB of static LDS) out of the kernel.
-template <bool TRANSPOSED, bool MASKS, int NT>
+// MASKS, LINES, COLUMNS: the joins the kernel holds (a.long_fibers and a.lines choose among them): a join that is left out
+// costs neither registers nor, the mask join, its 3 KB of static LDS.
+template <bool TRANSPOSED, bool MASKS, bool LINES, bool COLUMNS, int NT>
 __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t *s_nbr, void *s_masks)
 {
     __shared__ int s_col[R];
@@ -464,32 +475,43 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
     // With a table of the rows' columns the search is one coalesced load; every entry is checked against the two
     // pointers that bound its column (for a submanifold layer the join below asks for the same two), and one entry
     // that fails sends the whole tile to the search.
-    bool hinted = false;
-    if (a.q_rowcol) {
+    // The entries are believed before they are checked: the join's first loads go out with the check's.
+    bool search = a.q_rowcol == nullptr, checked = false;
+    int my_c = -1, hint_e = 0, hint_s = 0;
+    bool hint_inside = true;
+    if (!search) {
         for (int i = tid; i < R * KV / 4; i += NT) ((int4 *)s_nbr)[i] = make_int4(-1, -1, -1, -1);
+        int c = my_rl < nrows ? a.q_rowcol[r0 + my_rl] : 0;
+        hint_inside = (unsigned)c < (unsigned)q_ncol;
+        c = hint_inside ? c : 0;
+        hint_e = a.q_ptr[c];
+        hint_s = c ? a.q_ptr[c - 1] : 0;
+        my_c = my_rl < nrows ? c : -1;
+    }
+    // by all threads; behind it the table is clear, and the rows' columns are in s_col
+    auto check_hint = [&]() -> bool {
         const int r = r0 + my_rl;
-        int c = my_rl < nrows ? a.q_rowcol[r] : 0;
-        const bool inside = (unsigned)c < (unsigned)q_ncol;
-        c = inside ? c : 0;
-        const int pe = a.q_ptr[c], ps = c ? a.q_ptr[c - 1] : 0;
-        const bool good = my_rl >= nrows || (inside && ps <= r && r < pe);
+        const bool good = my_rl >= nrows || (hint_inside && hint_s <= r && r < hint_e);
         const unsigned long long bad = __ballot(!good);
-        if (tid < R) s_col[tid] = my_rl < nrows ? c : -1;
+        if (tid < R) s_col[tid] = my_c;
         if ((tid & (kWave - 1)) == 0) s_first[(NT / kWave) + tid / kWave] = bad != 0; // the half the search's first round leaves alone
         lds_barrier();
         int any_bad = 0;
 #pragma unroll
         for (int w = 0; w < (NT / kWave); w++) any_bad |= s_first[(NT / kWave) + w];
-        hinted = !any_bad;
-    }
+        checked = true;
+        search = any_bad != 0;
+        return !search;
+    };
+    if constexpr (!LINES) if (!search) check_hint(); // (nothing to overlap it with)
+    for (;;) { // once, or twice where the table of the rows' columns was wrong
     constexpr int kWalk = 2 * NT; // columns per walk step, two consecutive ones per thread
-    int c_first = q_ncol;
-    if (!hinted)
-        c_first = block_upper_bound<NT>(a.q_ptr, q_ncol, r0, kWalk, s_first, [&]() {
+    if (search) {
+        const int c_first = block_upper_bound<NT>(a.q_ptr, q_ncol, r0, kWalk, s_first, [&]() {
             for (int i = tid; i < R * KV / 4; i += NT) ((int4 *)s_nbr)[i] = make_int4(-1, -1, -1, -1); // R * KV is a multiple of 4
             for (int i = tid; i < R; i += NT) s_col[i] = -1;
         });
-    bool done = (c_first >= q_ncol);
+        bool done = (c_first >= q_ncol);
     for (int cb = c_first, step = 0; !done; cb += kWalk, step ^= 1) { // the steps alternate between two flags: one barrier each
         const int last = min(cb + kWalk - 1, q_ncol - 1);
         const int c = cb + 2 * tid;
@@ -507,8 +529,11 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
         lds_barrier();
         done = s_flag[step] != 0;
     }
+        my_c = my_rl < nrows ? s_col[my_rl] : -1;
+        checked = true;
+        search = false;
+    }
     // the row's column -> (batch, S0, S1), by every thread for its own row
-    const int my_c = my_rl < nrows ? s_col[my_rl] : -1;
     const bool my_ok = my_c >= 0;
     const int my_b = (int)div_by((uint32_t)max(my_c, 0), a.by_q01);
     const int my_rem = max(my_c, 0) - my_b * (a.Q.n0 * a.Q.n1);
@@ -521,6 +546,7 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
     // leaves the 64 bins sends the whole tile to the general join below.
     bool by_masks = false;
     if constexpr (MASKS) if (a.long_fibers) {
+        if constexpr (LINES) if (!checked && !check_hint()) continue;
         unsigned long long *s_cmask = (unsigned long long *)s_masks; // [K01][ncols], ncols <= kMaskCols
         int *s_cstart = (int *)(s_cmask + kMaskCols * K01);
         __shared__ int s_b[R], s_c0[R], s_c1[R], s_z[R];
@@ -625,7 +651,117 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
         }
     }
 
-    // 2. join.  item = (k01, row), consecutive lanes take consecutive rows.  Per pass a
+    // 2b. join by lines.  item = (line of the gathered grid, row): the columns a row can pair with on one line lie next to
+    // each other (at most three of them, else 2c), so the four pointers that bound them are neighbours, and so are all the
+    // entries of their fibers: an entry's column is found by comparing its position with the pointers in between.  The
+    // waves of a thread group take the same lines, so everything but the row's own numbers is scalar.  Per pass a thread
+    // issues the pointer loads of all its items, then the first entries, and only then compares.
+    // What bounds the rule kernel on large books is the vector ALU (90 % busy between ramp and tail, some 600 instructions
+    // per wave, a third of them here), on small ones the chain of loads.  Against the join by columns, with two pointer and
+    // three entry loads per column: 5890 tiles of a submanifold layer 35.3 us either way, 920 tiles of a transposed book of
+    // stride 2, where two lines of three at most can pair and mostly one column of theirs, 17.1 -> 12.2 us, ten tiles with
+    // the convolution behind it 11.3 -> 10.8 us.
+    if constexpr (LINES) if (!by_masks && (!COLUMNS || a.lines)) {
+        const int C = a.lines, p_ncol = a.B * a.P.n0 * a.P.n1;
+        const __amdgpu_buffer_rsrc_t r_ptr = __builtin_amdgcn_make_buffer_rsrc((void *)a.p_ptr, 0, p_ncol * 4, 0x00020000);
+        const __amdgpu_buffer_rsrc_t r_idx = __builtin_amdgcn_make_buffer_rsrc((void *)a.p_idx, 0, a.p_rows * 4, 0x00020000);
+        const int K12 = a.cv.K1 * a.cv.K2;
+        // line j: coordinate y0 + j * dy on the first axis, table offset slot + j * dslot_line; its columns ya, ya + 1, ..
+        int y0, ya, slot, rem0 = 0, lo;
+        const int dy = TRANSPOSED ? -1 : 1, dslot_line = TRANSPOSED ? a.cv.s0 * K12 : K12;
+        const int dslot = TRANSPOSED ? -a.cv.s1 * a.cv.K2 : a.cv.K2;
+        const int nlines = TRANSPOSED ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0;
+        if (!TRANSPOSED) {
+            y0 = my_c0 * a.cv.s0 - a.cv.p0;
+            ya = my_c1 * a.cv.s1 - a.cv.p1;
+            slot = my_rl * KV;
+            lo = max(0, -ya);
+        } else { // k_d = x_d + p_d - y_d * s_d: the highest column and the first line have the smallest offsets
+            const int t0 = my_c0 + a.cv.p0, t1 = my_c1 + a.cv.p1;
+            int yb;
+            if (((a.cv.s0 & (a.cv.s0 - 1)) | (a.cv.s1 & (a.cv.s1 - 1))) == 0) {
+                y0 = t0 >> (__ffs(a.cv.s0) - 1);
+                yb = t1 >> (__ffs(a.cv.s1) - 1);
+            } else {
+                y0 = t0 / a.cv.s0;
+                yb = t1 / a.cv.s1;
+            }
+            rem0 = t0 - y0 * a.cv.s0;
+            ya = yb - (C - 1);
+            const int k1a = t1 - ya * a.cv.s1; // offset of column ya: the only one that can be too large
+            slot = my_rl * KV + rem0 * K12 + k1a * a.cv.K2;
+            lo = max(k1a >= a.cv.K1 ? 1 : 0, -ya);
+        }
+        const int hi = min(C, a.P.n1 - ya);
+        const bool row_ok = my_ok && lo < hi;
+        const bool lo1 = lo >= 1, lo2 = lo >= 2, hi1 = hi <= 1, hi2 = hi <= 2;
+        const int off_z = TRANSPOSED ? my_zz + a.cv.p2 : a.cv.p2 - my_zz * a.cv.s2; // k2 = off_z +- v
+        const int pc0 = (my_b * a.P.n0 + y0) * a.P.n1 + ya;
+        constexpr int kLines = NT >= 256 ? 2 : 3;
+        const int grp = __builtin_amdgcn_readfirstlane(tid / R);
+        for (int j0 = grp; j0 < nlines || j0 == grp; j0 += kLines * (NT / R)) { // (every thread meets the check below)
+            int p[kLines][4];
+            bool ok[kLines];
+#pragma unroll
+            for (int i = 0; i < kLines; i++) {
+                const int j = j0 + i * (NT / R), y = y0 + j * dy;
+                ok[i] = row_ok && j < nlines && (unsigned)y < (unsigned)a.P.n0 && (!TRANSPOSED || rem0 + j * a.cv.s0 < a.cv.K0);
+                const int b = ok[i] ? (pc0 + j * dy * a.P.n1 - 1) * 4 : 0x7ffffff0 - 16; // none: beyond the array, zeros
+#pragma unroll
+                for (int q = 0; q < 4; q++) p[i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_ptr, max(b + 4 * q, 0), 0, 0);
+            }
+            if (!checked && !check_hint()) break;
+            int st[kLines], n[kLines], d1[kLines], d2[kLines], v[kLines][8];
+#pragma unroll
+            for (int i = 0; i < kLines; i++) {
+                const int j = j0 + i * (NT / R);
+                int s = lo2 ? p[i][2] : (lo1 ? p[i][1] : p[i][0]), e = hi1 ? p[i][1] : (hi2 ? p[i][2] : p[i][3]);
+                if (pc0 + j * dy * a.P.n1 - 1 + lo < 0) s = 0; // the grid's first column
+                s = clampi(s, 0, a.p_rows);
+                e = clampi(e, 0, a.p_rows);
+                d1[i] = lo1 ? 0 : (hi1 ? 0x7fffffff : p[i][1] - s);
+                d2[i] = lo2 ? 0 : (hi2 ? 0x7fffffff : p[i][2] - s);
+                st[i] = s;
+                n[i] = ok[i] ? e - s : 0;
+                if (!__any(n[i] > 0)) continue;
+                const int at = n[i] > 0 ? s * 4 : 0x7ffffff0 - 32;
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, at + 4 * q, 0, 0);
+                if (__any(n[i] > 4)) {
+#pragma unroll
+                    for (int q = 4; q < 8; q++) v[i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, at + 4 * q, 0, 0);
+                }
+            }
+            auto pair = [&](int i, int at, int e, int z) { // entry e of the line's, with S2 coordinate z
+                const int k2 = TRANSPOSED ? off_z - __mul24(z, a.cv.s2) : off_z + z;
+                const int w = at + (e >= d1[i] ? dslot : 0) + (e >= d2[i] ? dslot : 0) + k2;
+                if (e < n[i] && (unsigned)k2 < (unsigned)a.cv.K2) s_nbr[w] = st[i] + e;
+            };
+#pragma unroll
+            for (int i = 0; i < kLines; i++) {
+                if (!__any(n[i] > 0)) continue;
+                const int at = slot + (j0 + i * (NT / R)) * dslot_line;
+#pragma unroll
+                for (int q = 0; q < 4; q++) pair(i, at, q, v[i][q]);
+                if (!__any(n[i] > 4)) continue;
+#pragma unroll
+                for (int q = 4; q < 8; q++) pair(i, at, q, v[i][q]);
+                for (int e = 8; __any(n[i] > e); e += 4) { // longer fibers: four entries per round, their loads in flight together
+                    int u[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) u[q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, (st[i] + e + q) * 4, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) pair(i, at, e + q, u[q]);
+                }
+            }
+        }
+        if (search) continue;
+        break;
+    }
+    if constexpr (!COLUMNS) break;
+    if constexpr (LINES) if (!checked && !check_hint()) continue;
+
+    // 2c. join by columns.  item = (k01, row), consecutive lanes take consecutive rows.  Per pass a
     // thread first issues the two fiber-bound loads of all its items, then the first
     // three S2 coordinates of every fiber, and only then compares; longer fibers finish
     // in a loop.
@@ -709,6 +845,8 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
                 }
             }
         }
+    }
+    break;
     }
     lds_barrier();
 }
