@@ -9,9 +9,9 @@ import torch.nn as nn
 from . import sphconv_cuda as ext
 from .functional import ConvFunction
 from .modules import SphModule
-from .rulebook import RuleBook
+from .rulebook import RuleBook, layer_geometry
 from .tensor import SparseConvTensor
-from .utils import _calculate_fan_in_and_fan_out, _triple, kaiming_uniform_, out_spatial
+from .utils import _calculate_fan_in_and_fan_out, _triple, kaiming_uniform_
 
 
 def get_tile_grid_shape(out_spatial_shape_DWH: List[int], tile_size: List[int]) -> List[int]:
@@ -102,12 +102,14 @@ class Conv3d(Convolution):
         same coordinates.  None when there is nothing to do ahead."""
         if self.subm or input.find_rule(self.indice_key) is not None or not input.z_ptr.is_cuda:
             return None
-        in_shape = [input.D, input.W, input.H]
-        out_shape = out_spatial(in_shape, self.kernel_size, self.stride, self.padding, self.dilation)
-        return RuleBook.count_ahead(input.z_idx, input.z_ptr, input.B, in_shape, out_shape, self.kernel_size,
-                                    self.stride, self.padding, self.dilation)
+        return RuleBook._count(self._layer(input)[0], input.z_idx, input.z_ptr)
 
-    def _rules(self, input: SparseConvTensor, out_shape, ahead=None, keep: bool = True, training: bool = True):
+    def _layer(self, input):
+        """Geometry and output shape of this layer on ``input``'s grid."""
+        return layer_geometry(input.B, input.D, input.W, input.H, tuple(self.kernel_size), tuple(self.stride),
+                              tuple(self.padding), tuple(self.dilation), self.subm)
+
+    def _rules(self, input: SparseConvTensor, geometry, out_shape, ahead=None, keep: bool = True, training: bool = True):
         """Rule book of this layer on ``input``, shared through ``rule_cache`` when an
         ``indice_key`` is set (conv.py:159-177).  A book that is not cached yet is returned unbuilt (for a strided
         layer with its output coordinates): ``rule_conv`` generates its pairs in the launch that convolves them
@@ -116,15 +118,11 @@ class Conv3d(Convolution):
         cached = input.find_rule(self.indice_key)
         if cached is not None:
             return cached
-        in_shape = [input.D, input.W, input.H]
         row_cols = getattr(input, "row_cols", None)
         if self.subm:
-            book = RuleBook.build_subm(input.z_idx, input.z_ptr, input.B, in_shape, self.kernel_size,
-                                       self.padding, self.dilation, row_cols=row_cols, lazy=True)
+            book = RuleBook._subm(geometry, input.z_idx, input.z_ptr, row_cols)
         else:
-            book = RuleBook.build(input.z_idx, input.z_ptr, input.B, in_shape, out_shape,
-                                  self.kernel_size, self.stride, self.padding, self.dilation, ahead=ahead,
-                                  row_cols=row_cols, lazy=True)
+            book = RuleBook._strided(geometry, input.z_idx, input.z_ptr, ahead, row_cols)
         book.keep = bool(keep)
         book.cluster = getattr(input, "cluster", 1.0)
         if not training:
@@ -141,14 +139,15 @@ class Conv3d(Convolution):
         coordinates (no reference counterpart either)."""
         assert self.in_channels == input.C, \
             "input channel does not match Expect: {}, got {}".format(self.in_channels, input.C)
-        in_shape = [input.D, input.W, input.H]
-        out_shape = in_shape if self.subm else out_spatial(in_shape, self.kernel_size, self.stride,
-                                                            self.padding, self.dilation)
-        feature, weight = input.feature, self.weight
+        geometry, out_shape = self._layer(input)
+        # (a parameter straight from the module's table: asking the module takes longer than the rest of this line)
+        feature, weight = input.feature, self._parameters.get("weight")
+        if weight is None:
+            weight = self.weight
         grad = torch.is_grad_enabled()
         training = grad and (weight.requires_grad or feature.requires_grad)
         oz_idx, oz_ptr, book, rule_size, tile_grid_shape = self._rules(
-            input, out_shape, ahead, keep=training or self.indice_key is not None, training=training)
+            input, geometry, out_shape, ahead, keep=training or self.indice_key is not None, training=training)
         native = isinstance(book, RuleBook)
         self.__dict__["rule_book"] = book if native else None      # a plain attribute: no need to ask nn.Module
         if epilogue is not None and training:

@@ -161,6 +161,13 @@ struct Geometry {
         }
     }
     uintptr_t address() const { return (uintptr_t)&g; }
+    // whether the compressed coordinates of a tensor are what the rule kernels take on this geometry
+    bool takes(const Tensor &z_idx, const Tensor &z_ptr) const
+    {
+        return z_idx.scalar_type() == at::kInt && z_ptr.scalar_type() == at::kInt && z_idx.dim() == 1 && z_ptr.dim() == 3 &&
+               z_ptr.size(0) == g.B && z_ptr.size(1) == g.S[0] && z_ptr.size(2) == g.S[1] && z_idx.is_contiguous() &&
+               z_ptr.is_contiguous() && z_idx.is_cuda() && z_ptr.is_cuda();
+    }
 };
 
 // Device arrays of one book, carved out of one allocation.
@@ -478,6 +485,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     py::class_<Geometry>(m, "Geometry")
         .def(py::init<int, const std::vector<int> &, const std::vector<int> &, const std::vector<int> &, const std::vector<int> &,
                       const std::vector<int> &, const std::vector<int> &>())
+        .def("takes", &Geometry::takes)
         .def_property_readonly("address", &Geometry::address);
     py::class_<BookBuffers>(m, "BookBuffers")
         .def(py::init([](int rows, int kv, py::object dev, bool by_row, bool groups) {

@@ -28,13 +28,15 @@ def is_sparse_conv(module) -> bool:
 def _bn_affine(bn: nn.BatchNorm1d):
     """Evaluation-mode BatchNorm1d as y = x*scale + shift (fp32 [C]); computed once per state of
     the module's tensors (their version counters) and kept on the module."""
+    # (straight from the module's tables: asking the module four times takes longer than the key)
+    p, b = bn._parameters, bn._buffers
     key = [bn.eps]
-    for t in (bn.running_mean, bn.running_var, bn.weight, bn.bias):
+    for t in (b["running_mean"], b["running_var"], p["weight"], p["bias"]):
         if t is not None:
             key += (t.data_ptr(), t._version, t.dtype)
         else:
             key.append(None)
-    cached = getattr(bn, "_sph_affine", None)
+    cached = bn.__dict__.get("_sph_affine")
     if cached is not None and cached[0] == key:
         return cached[1], cached[2]
     scale, shift = _bn_affine_now(bn)
@@ -107,11 +109,12 @@ class Sequential(SphModule):
         conv = mods[i]
         if not (self.fuse_eval and is_sparse_conv(conv)) or torch.is_grad_enabled():
             return 0, None, False
-        if conv.weight.dtype not in (torch.float16, torch.bfloat16, torch.float32):
+        weight = conv._parameters.get("weight")
+        if (conv.weight if weight is None else weight).dtype not in (torch.float16, torch.bfloat16, torch.float32):
             return 0, None, False
         n, bn, relu = 0, None, False
         nxt = mods[i + 1] if i + 1 < len(mods) else None
-        if (type(nxt) is nn.BatchNorm1d and not nxt.training and nxt.running_mean is not None
+        if (type(nxt) is nn.BatchNorm1d and not nxt.training and nxt._buffers["running_mean"] is not None
                 and nxt.num_features == conv.out_channels):
             bn, n = nxt, 1
             nxt = mods[i + 2] if i + 2 < len(mods) else None

@@ -12,6 +12,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from . import _lib as L
+from .utils import out_spatial
 
 
 class _Buffers:
@@ -115,6 +116,24 @@ def _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation) -> 
         g = _Geometry(int(batch), *(tuple(int(v) for v in x) for x in (in_shape, out_shape, kernel, stride, padding, dilation)))
         _GEOMETRIES[key] = g
     return g
+
+# A layer's geometry and output shape by what the layer and its input hold, so that a forward pass does not work them out
+# again (shapes are a list comprehension with divisions, the geometry's key twenty numbers).
+_LAYERS = {}
+
+
+def layer_geometry(batch, D, W, H, kernel, stride, padding, dilation, subm):
+    """-> (geometry, output shape) of a layer on a ``[batch, D, W, H]`` grid."""
+    key = (batch, D, W, H, kernel, stride, padding, dilation, subm)
+    hit = _LAYERS.get(key)
+    if hit is None:
+        shape = [D, W, H]
+        out = shape if subm else out_spatial(shape, kernel, stride, padding, dilation)
+        if len(_LAYERS) >= 4096:
+            _LAYERS.clear()
+        hit = _LAYERS[key] = (_geometry(batch, shape, out, kernel, (1, 1, 1) if subm else stride, padding, dilation), tuple(out))
+    return hit
+
 
 # Estimated pairs per stationary row from which a book also keeps its pairs by row (and the
 # convolution walks that form).  float("inf") never does, 0 always.
@@ -268,8 +287,7 @@ class RuleBook:
         launch as the convolution where the library has that kernel (:meth:`fused_forward`)."""
         pad = [int(k) // 2 for k in kernel] if padding is None else padding
         geometry = _geometry(batch, shape, shape, kernel, (1, 1, 1), pad, dilation)
-        _check_index_tensors(z_idx, z_ptr, geometry.z_shape)
-        rb = cls._of(geometry, z_idx, z_ptr, z_idx, z_ptr, True, row_cols, row_cols)
+        rb = cls._subm(geometry, z_idx, z_ptr, row_cols)
         if lazy:
             return rb
         if weight is None:
@@ -285,11 +303,34 @@ class RuleBook:
         coordinates are written behind it.  Pass the returned object to ``build(..., ahead=)`` when the layer
         itself is reached: whatever the caller has enqueued in between (the convolutions of the layers before)
         keeps the GPU busy while the host reads the count, instead of the GPU waiting for the host."""
-        geometry = _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation)
-        _check_index_tensors(z_idx, z_ptr, geometry.z_shape)
+        return cls._count(_geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation), z_idx, z_ptr)
+
+    @classmethod
+    def _subm(cls, geometry, z_idx, z_ptr, row_cols) -> "RuleBook":
+        """A submanifold book, not built yet."""
+        if not geometry.native.takes(z_idx, z_ptr):
+            _check_index_tensors(z_idx, z_ptr, geometry.z_shape)          # says what is wrong
+        return cls._of(geometry, z_idx, z_ptr, z_idx, z_ptr, True, row_cols, row_cols)
+
+    @classmethod
+    def _count(cls, geometry, z_idx, z_ptr) -> "_CountAhead":
+        if not geometry.native.takes(z_idx, z_ptr):
+            _check_index_tensors(z_idx, z_ptr, geometry.z_shape)          # says what is wrong
         if min(geometry.out_shape) <= 0:
             raise L.SphconvError("empty output grid %s" % geometry.out_shape)
         return _CountAhead(geometry, z_idx, z_ptr)
+
+    @classmethod
+    def _strided(cls, geometry, z_idx, z_ptr, ahead, row_cols) -> "RuleBook":
+        """A strided layer's book: its output coordinates now, its pairs not built yet."""
+        if ahead is None:
+            ahead = cls._count(geometry, z_idx, z_ptr)
+        elif ahead.geometry is not geometry or ahead.z_idx.data_ptr() != z_idx.data_ptr() \
+                or ahead.z_ptr.data_ptr() != z_ptr.data_ptr() or ahead.native.stream != L.stream():
+            raise L.SphconvError("count_ahead() was called for another layer, tensor or stream")
+        # the rows' columns are a by-product of the coordinates
+        oz_idx, oz_ptr, out_cols = ahead.native.finish()
+        return cls._of(geometry, z_idx, z_ptr, oz_idx, oz_ptr, False, row_cols, out_cols)
 
     @classmethod
     def build(cls, z_idx, z_ptr, batch, in_shape, out_shape, kernel, stride, padding,
@@ -301,14 +342,7 @@ class RuleBook:
         enqueued already, so the GPU is not idle meanwhile.  ``ahead``: what :meth:`count_ahead` returned for the same
         arguments on the same stream."""
         geometry = _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation)
-        if ahead is None:
-            ahead = cls.count_ahead(z_idx, z_ptr, batch, in_shape, out_shape, kernel, stride, padding, dilation)
-        elif ahead.geometry is not geometry or ahead.z_idx.data_ptr() != z_idx.data_ptr() \
-                or ahead.z_ptr.data_ptr() != z_ptr.data_ptr() or ahead.native.stream != L.stream():
-            raise L.SphconvError("count_ahead() was called for another layer, tensor or stream")
-        # the rows' columns are a by-product of the coordinates
-        oz_idx, oz_ptr, out_cols = ahead.native.finish()
-        rb = cls._of(geometry, z_idx, z_ptr, oz_idx, oz_ptr, False, row_cols, out_cols)
+        rb = cls._strided(geometry, z_idx, z_ptr, ahead, row_cols)
         if lazy:                                     # output coordinates now, pairs with the first use
             return rb
         if weight is None:
