@@ -5,6 +5,7 @@ current HIP stream; every computation on the path happens inside the library.
 There is no CPU fallback: if the library is missing or a call fails, an
 exception is raised.
 """
+import contextlib
 import ctypes as C
 import os
 
@@ -163,9 +164,21 @@ def ptr(t):
     return t.data_ptr()
 
 
-def stream():
-    """Raw handle of torch's current HIP stream on the current device."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+def stream(device=None):
+    """Raw handle of torch's current HIP stream on ``device`` (None: the current device)."""
+    index = device.index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+_IS_CURRENT = contextlib.nullcontext()
+
+
+def on_device(device):
+    """Context for calls of the C ABI on tensors of ``device``: kernels are launched on the current device, and on that
+    device's stream.  (Entering a device context costs 3 us: only where the device is not the current one.)"""
+    if device.type != "cuda" or device.index is None or device.index == torch.cuda.current_device():
+        return _IS_CURRENT
+    return torch.cuda.device(device)
 
 
 def make_geom(batch, in_shape, out_shape, kernel, stride, padding, dilation=(1, 1, 1)) -> Geom:

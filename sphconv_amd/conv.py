@@ -159,7 +159,7 @@ class Conv3d(Convolution):
         else:
             scale, shift, relu = epilogue if epilogue is not None else (None, None, False)
             keep = not self.training and not grad and weight.dtype == feature.dtype
-            packed = ext._kept_packed(weight, ext.L.stream()) if keep and native else None
+            packed = ext._kept_packed(weight) if keep and native else None
             if packed is not None:
                 out_feature = ext._conv_packed(feature, packed, self.in_channels, self.out_channels, book, rows, scale,
                                                shift, bool(relu))

@@ -8,6 +8,7 @@
 // (which kernel form a book takes, what is kept) stays in Python; this file holds no state beyond pinned words.
 #include <torch/extension.h>
 
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -57,7 +58,19 @@ template <typename T = void> T *ptr(const Tensor &t)
 }
 template <typename T = void> T *ptr(const OptTensor &t) { return t ? ptr<T>(*t) : nullptr; }
 
-void *stream() { return (void *)c10::hip::getCurrentHIPStream().stream(); }
+// The device of a call's tensors, current while the call allocates and launches, and torch's current stream on it.  A
+// kernel is launched on a stream that came from here and nowhere else: torch's own operations follow their tensors'
+// device, so a launch on the stream of whatever device happens to be current would not be ordered with what made its inputs.
+struct OnDevice {
+    c10::DeviceGuard guard;
+    hipStream_t stream;
+    explicit OnDevice(const Tensor &t) : guard(of(t)), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+    static c10::Device of(const Tensor &t)
+    {
+        if (!t.is_cuda()) raise("expected a GPU tensor, got device " + t.device().str());
+        return t.device();
+    }
+};
 
 Tensor bytes(size_t n, const Tensor &like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte).requires_grad(false)); }
 Tensor ints(int64_t n, const Tensor &like) { return at::empty({n}, like.options().dtype(at::kInt).requires_grad(false)); }
@@ -104,7 +117,7 @@ class HostWord {
     bool seen = false;
 
 public:
-    HostWord() : w(pinned().take()), st((hipStream_t)stream()) { __atomic_store_n(w, (int64_t)-1, __ATOMIC_SEQ_CST); }
+    explicit HostWord(const OnDevice &here) : w(pinned().take()), st(here.stream) { __atomic_store_n(w, (int64_t)-1, __ATOMIC_SEQ_CST); }
     HostWord(const HostWord &) = delete;
     HostWord &operator=(const HostWord &) = delete;
     ~HostWord()
@@ -244,18 +257,20 @@ sph_pack_desc describe_pack(const Tensor &w, bool transpose, bool reverse, int d
 
 Tensor pack_weight(const Tensor &w, bool transpose, bool reverse, int dt)
 {
+    const OnDevice here(w);
     Tensor packed;
     const sph_pack_desc d = describe_pack(w, transpose, reverse, dt, packed);
-    check(sph_weight_packs(&d, 1, stream()));
+    check(sph_weight_packs(&d, 1, here.stream));
     return packed;
 }
 
 // the copies for the forward pass and for dgrad in one launch
 std::pair<Tensor, Tensor> pack_weight_both(const Tensor &w, bool reverse, int dt)
 {
+    const OnDevice here(w);
     Tensor f, t;
     const sph_pack_desc d[2] = {describe_pack(w, false, false, dt, f), describe_pack(w, true, reverse, dt, t)};
-    check(sph_weight_packs(d, 2, stream()));
+    check(sph_weight_packs(d, 2, here.stream));
     return {f, t};
 }
 
@@ -263,10 +278,11 @@ std::pair<Tensor, Tensor> pack_weight_both(const Tensor &w, bool reverse, int dt
 void rules_build(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz_idx, const Tensor &oz_ptr, const Geometry &geom,
                  bool transposed, BookBuffers &buf, const OptTensor &row_cols)
 {
+    const OnDevice here(z_ptr);
     const int in_rows = (int)z_idx.size(0), out_rows = (int)oz_idx.size(0);
     check(sph_rules_build((const int32_t *)z_idx.data_ptr(), (const int32_t *)z_ptr.data_ptr(), in_rows, (const int32_t *)oz_idx.data_ptr(),
                           (const int32_t *)oz_ptr.data_ptr(), out_rows, &geom.g, transposed, &buf.book,
-                          row_table(row_cols, transposed ? in_rows : out_rows), stream()));
+                          row_table(row_cols, transposed ? in_rows : out_rows), here.stream));
 }
 
 // ... with one weight (kind 0: as it is; 1: transposed) or both forms (2; reverse: dgrad's offsets mirrored) packed by
@@ -275,6 +291,7 @@ py::object rules_build_pack(const Tensor &z_idx, const Tensor &z_ptr, const Tens
                             bool transposed, BookBuffers &buf, const OptTensor &row_cols, const Tensor &weight, int kind, bool reverse,
                             int dt)
 {
+    const OnDevice here(z_ptr);
     const int in_rows = (int)z_idx.size(0), out_rows = (int)oz_idx.size(0);
     Tensor p[2];
     sph_pack_desc d[2];
@@ -283,7 +300,7 @@ py::object rules_build_pack(const Tensor &z_idx, const Tensor &z_ptr, const Tens
     if (n == 2) d[1] = describe_pack(weight, true, reverse, dt, p[1]);
     check(sph_rules_build_packs((const int32_t *)z_idx.data_ptr(), (const int32_t *)z_ptr.data_ptr(), in_rows,
                                 (const int32_t *)oz_idx.data_ptr(), (const int32_t *)oz_ptr.data_ptr(), out_rows, &geom.g, transposed,
-                                &buf.book, row_table(row_cols, transposed ? in_rows : out_rows), d, n, stream()));
+                                &buf.book, row_table(row_cols, transposed ? in_rows : out_rows), d, n, here.stream));
     if (n == 2) return py::make_tuple(p[0], p[1]);
     return py::cast(p[0]);
 }
@@ -300,7 +317,8 @@ struct OutCoords {
     HostWord total;
     long bound;
     bool filled = false;
-    OutCoords(Tensor zi, Tensor zp, py::object g) : z_idx(std::move(zi)), z_ptr(std::move(zp)), geom(g.cast<const Geometry *>()), geom_owner(g)
+    OutCoords(const OnDevice &here, Tensor zi, Tensor zp, py::object g)
+        : z_idx(std::move(zi)), z_ptr(std::move(zp)), geom(g.cast<const Geometry *>()), geom_owner(g), total(here)
     {
         const sph_geom &q = geom->g;
         const int n = sph_outcoords_scratch_ints(&q);
@@ -315,10 +333,11 @@ struct OutCoords {
                                   total.address(), total.on()));
         if (most * 8 <= kAheadBytes) {
             bound = (long)most;
-            fill(bound);
+            fill(here, bound);
         }
     }
-    void fill(long rows)
+    // (on the stream of the count, which `here`'s device is that of)
+    void fill(const OnDevice &here, long rows)
     {
         oz_idx = ints(rows, z_ptr);
         cols = ints(rows, z_ptr);
@@ -332,7 +351,7 @@ struct OutCoords {
     {
         const long rows = (long)total.wait(false);
         if (rows < 0 || (filled && rows > bound)) raise("the output coordinates of a strided layer are inconsistent");
-        if (!filled) fill(rows);
+        if (!filled) fill(OnDevice(z_ptr), rows);
         else if (rows < bound) {
             oz_idx = oz_idx.narrow(0, 0, rows);
             cols = cols.narrow(0, 0, rows);
@@ -354,11 +373,12 @@ const sph_epilogue *epilogue(sph_epilogue &e, const OptTensor &scale, const OptT
 Tensor conv_apply(const Tensor &feature_, const Tensor &packed, int kdim, int ndim, BookBuffers &buf, const OptTensor &scale,
                   const OptTensor &shift, bool relu)
 {
+    const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous();
     const Tensor out = at::empty({buf.book.rows, ndim}, feature.options().requires_grad(false));
     sph_epilogue e;
     check(sph_conv_apply((sph_dtype)dtype_code(feature.scalar_type()), ptr(feature), (int)feature.size(0), kdim, packed.data_ptr(), ndim,
-                         &buf.book, epilogue(e, scale, shift, relu), out.data_ptr(), stream()));
+                         &buf.book, epilogue(e, scale, shift, relu), out.data_ptr(), here.stream));
     return out;
 }
 
@@ -367,6 +387,7 @@ py::object rules_conv(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz
                       BookBuffers &buf, int flags, const OptTensor &row_cols, const Tensor &feature_, const Tensor &packed, int kdim,
                       int ndim, const OptTensor &scale, const OptTensor &shift, bool relu)
 {
+    const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous();
     const int out_rows = (int)oz_idx.size(0);
     const Tensor out = at::empty({out_rows, ndim}, feature.options().requires_grad(false));
@@ -374,7 +395,7 @@ py::object rules_conv(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz
     const int rc = sph_rules_conv((const int32_t *)z_idx.data_ptr(), (const int32_t *)z_ptr.data_ptr(), (int)z_idx.size(0),
                                   (const int32_t *)oz_idx.data_ptr(), (const int32_t *)oz_ptr.data_ptr(), out_rows, &geom.g, &buf.book,
                                   flags, row_table(row_cols, out_rows), (sph_dtype)dtype_code(feature.scalar_type()), ptr(feature), kdim,
-                                  packed.data_ptr(), ndim, epilogue(e, scale, shift, relu), out.data_ptr(), stream());
+                                  packed.data_ptr(), ndim, epilogue(e, scale, shift, relu), out.data_ptr(), here.stream);
     if (rc == SPH_ERR_UNSUPPORTED) return py::none();
     check(rc);
     return py::cast(out);
@@ -382,6 +403,7 @@ py::object rules_conv(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz
 
 Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf, bool transposed, bool f32)
 {
+    const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous(), d_out = d_out_.contiguous();
     const int ic = (int)feature.size(1), oc = (int)d_out.size(1);
     const int64_t n = (int64_t)sph_wgrad_partial_elems(buf.kv, ic, oc, buf.book.rows);
@@ -390,10 +412,10 @@ Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf
     const sph_dtype dt = (sph_dtype)dtype_code(feature.scalar_type());
     if (transposed)
         check(sph_conv_wgrad_transposed(dt, ptr(feature), ic, ptr(d_out), (int)d_out.size(0), oc, &buf.book, (float *)partial.data_ptr(),
-                                        dw.data_ptr(), f32, stream()));
+                                        dw.data_ptr(), f32, here.stream));
     else
         check(sph_conv_wgrad(dt, ptr(feature), (int)feature.size(0), ic, ptr(d_out), oc, &buf.book, (float *)partial.data_ptr(),
-                             dw.data_ptr(), f32, stream()));
+                             dw.data_ptr(), f32, here.stream));
     return dw;
 }
 
@@ -401,6 +423,7 @@ Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf
 // -> out feature, z_idx, z_ptr, permutation, row_cols, coordinates outside the grid, duplicated coordinates
 py::tuple init_tensor(const Tensor &feature_, const Tensor &indices_, int B, int S0, int S1, int S2)
 {
+    const OnDevice here(indices_);
     const Tensor indices = indices_.contiguous(), feature = feature_.contiguous();
     const int n = (int)indices.size(0);
     const size_t nbytes = sph_init_tensor_workspace(n, B, S0, S1, S2);
@@ -411,7 +434,7 @@ py::tuple init_tensor(const Tensor &feature_, const Tensor &indices_, int B, int
     Tensor z_ptr = at::empty({B, S0, S1}, indices.options());
     Tensor out = at::empty_like(feature, feature.options().requires_grad(false));
     const Tensor work = bytes(nbytes, indices);
-    HostWord word;
+    HostWord word(here);
     check(sph_init_tensor_rows(ptr<int32_t>(indices), n, B, S0, S1, S2, ptr(feature),
                                (int)(feature.size(1) * feature.element_size()), ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), ptr<int32_t>(perm),
                                ptr<int32_t>(cols), ptr(out), ptr<int32_t>(status), word.address(), ptr(work), nbytes, word.on()));
@@ -421,11 +444,12 @@ py::tuple init_tensor(const Tensor &feature_, const Tensor &indices_, int B, int
 
 Tensor to_dense_channels_first(const Tensor &feature_, const Tensor &z_idx, const Tensor &z_ptr, int B, int C, int S0, int S1, int S2)
 {
+    const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous();
     if (feature.size(1) != C || z_ptr.numel() != (int64_t)B * S0 * S1) raise("rows and pointers do not match the dense shape");
     const Tensor out = at::empty({B, C, S0, S1, S2}, feature.options().requires_grad(false));
     check(sph_to_dense_channels_first(ptr(feature), ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), (int)feature.size(0), B * S0 * S1, S0 * S1,
-                                      S2, C, (int)feature.element_size(), out.data_ptr(), stream()));
+                                      S2, C, (int)feature.element_size(), out.data_ptr(), here.stream));
     return out;
 }
 
@@ -435,6 +459,7 @@ py::tuple points_to_voxel(const Tensor &points, int system, const std::vector<do
                           const std::vector<int> &grid, int max_points, int max_voxels, int append_mode, const OptTensor &cells,
                           const OptTensor &cell_out)
 {
+    const OnDevice here(points);
     const int n = (int)points.size(0), nfeat = (int)points.size(1), width = append_mode == 1 ? nfeat + 3 : nfeat;
     const size_t nbytes = sph_points_to_voxel_workspace(n, grid[0], grid[1], grid[2]);
     if (nbytes == 0)
@@ -445,7 +470,7 @@ py::tuple points_to_voxel(const Tensor &points, int system, const std::vector<do
     Tensor coors = at::empty({max_voxels, 3}, points.options().dtype(at::kInt));
     Tensor num = at::empty({max_voxels}, points.options().dtype(at::kInt));
     const Tensor work = bytes(nbytes, points);
-    HostWord word;
+    HostWord word(here);
     check(sph_points_to_voxel(n ? ptr<float>(points) : nullptr, n, nfeat, system, (float)lo[0], (float)lo[1], (float)lo[2], (float)vs[0],
                               (float)vs[1], (float)vs[2], grid[0], grid[1], grid[2], max_points, max_voxels, append_mode,
                               ptr<float>(voxels), ptr<float>(mask), ptr<int32_t>(coors), ptr<int32_t>(num), word.address(),
@@ -455,14 +480,17 @@ py::tuple points_to_voxel(const Tensor &points, int system, const std::vector<do
 
 Tensor voxel_mean(const Tensor &voxels, const Tensor &num, int nf)
 {
+    const OnDevice here(voxels);
     const Tensor out = at::empty({voxels.size(0), nf}, voxels.options());
     check(sph_voxel_mean(ptr<float>(voxels), ptr<int32_t>(num), (int)voxels.size(0), (int)voxels.size(1), (int)voxels.size(2), nf,
-                         (float *)out.data_ptr(), stream()));
+                         (float *)out.data_ptr(), here.stream));
     return out;
 }
 
 Tensor batch_coordinates(const std::vector<Tensor> &parts)
 {
+    if (parts.empty()) raise("no coordinates to join");
+    const OnDevice here(parts[0]);
     std::vector<const int32_t *> p;
     std::vector<int32_t> rows;
     int64_t total = 0;
@@ -472,7 +500,7 @@ Tensor batch_coordinates(const std::vector<Tensor> &parts)
         total += t.size(0);
     }
     const Tensor out = at::empty({total, 4}, parts[0].options());
-    check(sph_batch_coordinates(p.data(), rows.data(), (int)parts.size(), (int32_t *)out.data_ptr(), stream()));
+    check(sph_batch_coordinates(p.data(), rows.data(), (int)parts.size(), (int32_t *)out.data_ptr(), here.stream));
     return out;
 }
 
@@ -503,7 +531,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
         .def_property_readonly("address", &BookBuffers::address)
         .def("range", [](const BookBuffers &b, int i) { return std::make_pair(b.off[i], b.size[i]); });
     py::class_<OutCoords>(m, "OutCoords")
-        .def(py::init<Tensor, Tensor, py::object>())
+        .def(py::init([](Tensor z_idx, Tensor z_ptr, py::object geometry) {
+            const OnDevice here(z_ptr);
+            return new OutCoords(here, std::move(z_idx), std::move(z_ptr), std::move(geometry));
+        }))
         .def_property_readonly("stream", &OutCoords::on)
         .def("finish", &OutCoords::finish);
     m.def("pack_weight", &pack_weight);

@@ -64,7 +64,7 @@ def xyz2RangeVoxel(points,
     thick = torch.empty((1, v_res, h_res), dtype=torch.int32, device=device)
     winner = torch.empty(v_res * h_res, dtype=torch.int32, device=device)
     idx = torch.empty((m, 3), dtype=torch.int32, device=device) if return_indices else None
-    with torch.cuda.device(device):
+    with L.on_device(pts.device):
         L.check(L.lib().sph_xyz_to_rangevoxel(L.ptr(pts) if m else None, m, ndim, int(v_res), int(h_res), int(d_res),
                                               v0, h0, dtheta, dphi, d0, dr, int(bool(log)), L.ptr(winner),
                                               L.ptr(feature), L.ptr(depth), L.ptr(thick), L.ptr(idx), L.stream()))

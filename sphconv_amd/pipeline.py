@@ -44,7 +44,7 @@ class ScanPipeline:
         self._z_shape = (self.batch, self.shape[0], self.shape[1])
         self.max_voxels = int(max_voxels)
         self.dt = L.dtype_code(self.weight.dtype)
-        dev = self.weight.device
+        dev = self._device = self.weight.device
         lib = L.lib()
         pad = [k // 2 for k in self.kernel]
         self._geom = L.make_geom(self.batch, self.shape, self.shape, self.kernel, (1, 1, 1), pad)
@@ -78,9 +78,10 @@ class ScanPipeline:
             raise L.SphconvError("weight must stay [%d,%d,%d] %s" % (self.kv, self.ic, self.oc, self.weight.dtype))
         self.weight = weight.detach().contiguous()
         w = self.weight
-        L.check(self._lib.sph_weight_pack(self.dt, w.data_ptr(), self.kv, self.ic, self.oc, self.ic * self.oc, self.oc, 1,
-                                          self._packed.data_ptr(), L.stream()))
-        self._packed_ready.record(torch.cuda.current_stream())
+        with L.on_device(self._device):
+            L.check(self._lib.sph_weight_pack(self.dt, w.data_ptr(), self.kv, self.ic, self.oc, self.ic * self.oc, self.oc,
+                                              1, self._packed.data_ptr(), L.stream()))
+            self._packed_ready.record(torch.cuda.current_stream())
         self._packed_seen = [False] * len(self._streams)
 
     @property
@@ -103,7 +104,7 @@ class ScanPipeline:
         self._next = (slot + 1) % len(self._streams)
         side = self._streams[slot]
         if wait_inputs:
-            side.wait_stream(torch.cuda.current_stream())   # the inputs were produced on the caller's stream
+            side.wait_stream(torch.cuda.current_stream(self._device))   # the inputs were produced on the caller's stream
         if not self._packed_seen[slot]:
             side.wait_event(self._packed_ready)              # the packed weight was made on another stream
             self._packed_seen[slot] = True
@@ -119,16 +120,17 @@ class ScanPipeline:
         hint = _row_cols_ptr(row_cols, n)
         zi, zp = z_idx.data_ptr(), z_ptr.data_ptr()
         rc = L.ERR_UNSUPPORTED
-        if self.fused and lib.sph_book_tiles(n) <= self._fused_max_tiles:
-            rc = lib.sph_rules_conv(zi, zp, n, zi, zp, n, C.byref(self._geom), C.byref(book._struct),
-                                    L.FUSED_IN_FLIGHT if len(self._streams) >= 3 else 0, hint, self.dt,
-                                    feature.data_ptr(), self.ic, self._packed.data_ptr(), self.oc, C.byref(self._epi),
-                                    self._out[slot].data_ptr(), st)
-        if rc == L.ERR_UNSUPPORTED:
-            rc = lib.sph_rules_build(zi, zp, n, zi, zp, n, C.byref(self._geom), 0, C.byref(book._struct), hint, st)
-            if rc == 0:
-                rc = lib.sph_conv_apply(self.dt, feature.data_ptr(), n, self.ic, self._packed.data_ptr(), self.oc,
-                                        C.byref(book._struct), C.byref(self._epi), self._out[slot].data_ptr(), st)
+        with L.on_device(self._device):
+            if self.fused and lib.sph_book_tiles(n) <= self._fused_max_tiles:
+                rc = lib.sph_rules_conv(zi, zp, n, zi, zp, n, C.byref(self._geom), C.byref(book._struct),
+                                        L.FUSED_IN_FLIGHT if len(self._streams) >= 3 else 0, hint, self.dt,
+                                        feature.data_ptr(), self.ic, self._packed.data_ptr(), self.oc, C.byref(self._epi),
+                                        self._out[slot].data_ptr(), st)
+            if rc == L.ERR_UNSUPPORTED:
+                rc = lib.sph_rules_build(zi, zp, n, zi, zp, n, C.byref(self._geom), 0, C.byref(book._struct), hint, st)
+                if rc == 0:
+                    rc = lib.sph_conv_apply(self.dt, feature.data_ptr(), n, self.ic, self._packed.data_ptr(), self.oc,
+                                            C.byref(book._struct), C.byref(self._epi), self._out[slot].data_ptr(), st)
         if rc:
             L.check(rc)
         self._done[slot].record(side)
@@ -147,7 +149,7 @@ class ScanPipeline:
 
     def wait(self, slot: int):
         """Makes the caller's current stream wait for the scan last submitted to ``slot``."""
-        torch.cuda.current_stream().wait_event(self._done[slot])
+        torch.cuda.current_stream(self._device).wait_event(self._done[slot])
 
     def synchronize(self):
         for s in self._streams:

@@ -326,7 +326,7 @@ class RuleBook:
         if ahead is None:
             ahead = cls._count(geometry, z_idx, z_ptr)
         elif ahead.geometry is not geometry or ahead.z_idx.data_ptr() != z_idx.data_ptr() \
-                or ahead.z_ptr.data_ptr() != z_ptr.data_ptr() or ahead.native.stream != L.stream():
+                or ahead.z_ptr.data_ptr() != z_ptr.data_ptr() or ahead.native.stream != L.stream(z_ptr.device):
             raise L.SphconvError("count_ahead() was called for another layer, tensor or stream")
         # the rows' columns are a by-product of the coordinates
         oz_idx, oz_ptr, out_cols = ahead.native.finish()
@@ -383,10 +383,11 @@ class RuleBook:
         buf = _Buffers(rows, self.kv, rules.device)
         nbr = torch.empty(max(rows, 1) * self.kv, dtype=torch.int32, device=rules.device)
         b = buf.struct()
-        L.check(L.lib().sph_rules_from_padded(L.ptr(rules), L.ptr(rule_size), int(rules.shape[0]),
-                                              self.kv, int(rules.shape[3]), self.in_rows,
-                                              self.out_rows, int(transposed), L.ptr(nbr),
-                                              C.byref(b), L.stream()))
+        with L.on_device(rules.device):
+            L.check(L.lib().sph_rules_from_padded(L.ptr(rules), L.ptr(rule_size), int(rules.shape[0]),
+                                                  self.kv, int(rules.shape[3]), self.in_rows,
+                                                  self.out_rows, int(transposed), L.ptr(nbr),
+                                                  C.byref(b), L.stream()))
         return buf
 
     # Tiles up to which one launch for rules + forward beats two (three workgroups of four waves, or four of two,
@@ -471,15 +472,17 @@ class RuleBook:
             ntile = lib.sph_num_tiles(C.byref(g), *key)
             nbr = torch.empty(max(self.out_rows, 1) * self.kv, dtype=torch.int32, device=dev)
             rule_size = torch.empty((ntile, self.kv), dtype=torch.int32, device=dev)
-            L.check(lib.sph_rules_to_padded_count(C.byref(b), L.ptr(self.oz_ptr), C.byref(g), key[0],
-                                                  key[1], L.ptr(nbr), L.ptr(rule_size), L.stream()))
+            with L.on_device(dev):
+                L.check(lib.sph_rules_to_padded_count(C.byref(b), L.ptr(self.oz_ptr), C.byref(g), key[0],
+                                                      key[1], L.ptr(nbr), L.ptr(rule_size), L.stream()))
             n_max = lib.sph_tile_n_max(C.byref(g), key[0], key[1], self.in_rows)
             longest = int(rule_size.max().item()) if rule_size.numel() else 0
             n_max = max(n_max, (longest + 15) & ~15, 16)
             rules = torch.empty((ntile, self.kv, 2, n_max), dtype=torch.int32, device=dev)
-            L.check(lib.sph_rules_to_padded_fill(L.ptr(self.oz_ptr), C.byref(g), key[0], key[1],
-                                                 L.ptr(nbr), self.out_rows, self.kv, n_max,
-                                                 L.ptr(rules), L.stream()))
+            with L.on_device(dev):
+                L.check(lib.sph_rules_to_padded_fill(L.ptr(self.oz_ptr), C.byref(g), key[0], key[1],
+                                                     L.ptr(nbr), self.out_rows, self.kv, n_max,
+                                                     L.ptr(rules), L.stream()))
             self._padded[key] = (rules, rule_size)
         return self._padded[key]
 
@@ -505,7 +508,7 @@ _SCRATCH_BOOKS = {}
 
 
 def _scratch_book(rows: int, kv: int, device) -> "_Buffers":
-    key = (device.index, L.stream(), kv)
+    key = (device.index, L.stream(device), kv)
     buf = _SCRATCH_BOOKS.get(key)
     if buf is None or buf.capacity < rows:
         if len(_SCRATCH_BOOKS) >= 64:
@@ -528,7 +531,8 @@ def _row_cols_ptr(row_cols, rows: int):
 def row_columns(z_ptr: torch.Tensor, rows: int) -> torch.Tensor:
     """int32 [rows]: the column (index into the flattened ``z_ptr``) of every row."""
     out = torch.empty(int(rows), dtype=torch.int32, device=z_ptr.device)
-    L.check(L.lib().sph_row_columns(L.ptr(z_ptr), z_ptr.numel(), int(rows), L.ptr(out), L.stream()))
+    with L.on_device(z_ptr.device):
+        L.check(L.lib().sph_row_columns(L.ptr(z_ptr), z_ptr.numel(), int(rows), L.ptr(out), L.stream()))
     return out
 
 

@@ -61,7 +61,7 @@ def _packed_weight(weight: torch.Tensor, transpose: bool, reverse: bool = False,
     cache_key = None
     if cache and not torch.is_grad_enabled() and w.data_ptr() == weight.data_ptr():
         base = weight._base if weight._base is not None else weight
-        cache_key = (id(base), bool(transpose), bool(reverse), L.stream())
+        cache_key = (id(base), bool(transpose), bool(reverse), L.stream(w.device))
         state = (base._version, w.data_ptr(), tuple(w.shape), w.dtype)
         hit = _PACKED_CACHE.get(cache_key)
         if hit is not None and hit[0]() is base and hit[1] == state:
@@ -72,10 +72,10 @@ def _packed_weight(weight: torch.Tensor, transpose: bool, reverse: bool = False,
     return packed
 
 
-def _kept_packed(weight: torch.Tensor, stream: int) -> Optional[torch.Tensor]:
+def _kept_packed(weight: torch.Tensor) -> Optional[torch.Tensor]:
     """The kept fragment-ordered copy of ``weight`` (the parameter itself, of any shape) for the forward pass, if there
     is one and the weight has not changed since; None otherwise."""
-    hit = _PACKED_CACHE.get((id(weight), False, False, stream))
+    hit = _PACKED_CACHE.get((id(weight), False, False, L.stream(weight.device)))
     if hit is None or hit[0]() is not weight:
         return None
     version, address, _, dtype = hit[1]
@@ -131,8 +131,9 @@ def init_tensor_backward(d_featureOut: torch.Tensor, permutation: torch.Tensor) 
     """tensor.cu:147-162: d_feature[n] = d_featureOut[permutation[n]]."""
     d = d_featureOut.contiguous()
     out = torch.empty_like(d)
-    L.check(L.lib().sph_permute_rows(L.ptr(d), L.ptr(permutation.contiguous()), d.shape[0],
-                                     d.shape[1] * d.element_size(), 1, L.ptr(out), L.stream()))
+    with L.on_device(d.device):
+        L.check(L.lib().sph_permute_rows(L.ptr(d), L.ptr(permutation.contiguous()), d.shape[0],
+                                         d.shape[1] * d.element_size(), 1, L.ptr(out), L.stream()))
     return out
 
 
@@ -146,8 +147,9 @@ def to_dense(feature: torch.Tensor, zIndices: torch.Tensor, zPtr: torch.Tensor, 
     if out.shape[0] * out.shape[1] * out.shape[2] != ncol or out.shape[3] != int(D):
         raise ValueError("out shape %s does not match z_ptr %s and D=%d"
                          % (tuple(out.shape), tuple(zPtr.shape), D))
-    L.check(L.lib().sph_to_dense(L.ptr(feature), L.ptr(zIndices), L.ptr(zPtr), feature.shape[0], ncol,
-                                 int(D), feature.shape[1] * feature.element_size(), L.ptr(out), L.stream()))
+    with L.on_device(feature.device):
+        L.check(L.lib().sph_to_dense(L.ptr(feature), L.ptr(zIndices), L.ptr(zPtr), feature.shape[0], ncol,
+                                     int(D), feature.shape[1] * feature.element_size(), L.ptr(out), L.stream()))
     return out
 
 
@@ -156,8 +158,9 @@ def to_dense_backward(d_featureOut: torch.Tensor, zIndices: torch.Tensor, zPtr: 
     d = d_featureOut.contiguous()
     n, c = zIndices.shape[0], d.shape[4]
     out = torch.zeros((n, c), dtype=d.dtype, device=d.device)
-    L.check(L.lib().sph_to_dense_backward(L.ptr(d), L.ptr(zIndices), L.ptr(zPtr), n, zPtr.numel(),
-                                          d.shape[3], c * d.element_size(), L.ptr(out), L.stream()))
+    with L.on_device(d.device):
+        L.check(L.lib().sph_to_dense_backward(L.ptr(d), L.ptr(zIndices), L.ptr(zPtr), n, zPtr.numel(),
+                                              d.shape[3], c * d.element_size(), L.ptr(out), L.stream()))
     return out
 
 

@@ -4,7 +4,6 @@ sphconv/utils/voxel_generator.py, sphconv/utils/coord_transform.py, include/poin
 ``points_to_voxel_v2`` keeps the reference's arguments and result dictionary
 (voxelize.py:126-214); the coordinate transform, the binning and the voxel numbering in
 order of first appearance run in one C call (``sph_points_to_voxel``)."""
-import contextlib
 import functools
 from typing import List, Optional
 
@@ -37,9 +36,6 @@ def _bins(coors_range, sphere_coors_range, coord_system: str, grid):
     f32 = np.float32
     rng = system_range(coors_range, sphere_coors_range, coord_system).astype(f32)
     return rng, [f32((rng[3 + i] - rng[i]) / f32(grid[i])) for i in range(3)]
-
-
-_SAME_DEVICE = contextlib.nullcontext()
 
 
 def points_to_voxel_v2(points, voxel_size, coors_range, sphere_coors_range, coor_to_voxelidx=None,
@@ -83,10 +79,9 @@ def points_to_voxel_v2(points, voxel_size, coors_range, sphere_coors_range, coor
     cell_out = torch.empty(n, dtype=torch.int64, device=dev) if return_cells else None
     if cells is not None:
         cells = cells.to(device=dev, dtype=torch.int64).contiguous()
-    # (entering a device context costs 3 us: only for points on another GPU)
-    with torch.cuda.device(dev) if dev.index != torch.cuda.current_device() else _SAME_DEVICE:
-        voxels, mask, coors, num, voxel_num = L.host().points_to_voxel(
-            pts, COORD_SYSTEMS[coord_system], [float(v) for v in rng[:3]], [float(v) for v in vs], grid, int(max_points), int(max_voxels), int(append_mode), cells, cell_out)
+    voxels, mask, coors, num, voxel_num = L.host().points_to_voxel(
+        pts, COORD_SYSTEMS[coord_system], [float(v) for v in rng[:3]], [float(v) for v in vs], grid, int(max_points),
+        int(max_voxels), int(append_mode), cells, cell_out)
     if pad_cols:
         voxels = torch.nn.functional.pad(voxels, (0, pad_cols))
     res = {"voxels": voxels, "coordinates": coors, "num_points_per_voxel": num,

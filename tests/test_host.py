@@ -98,3 +98,57 @@ def test_training_channel_limit_is_reported_before_forward():
     weight = torch.zeros((27, 192, 32), requires_grad=True)
     with pytest.raises(sphconv_amd.SphconvError, match="training takes 1..128 input channels"):
         ConvFunction.apply(feature, weight, None, None, [1, 1], 4)
+
+
+def _launching_entry_points():
+    """Entry points of the C ABI that take a stream."""
+    hdr = open(os.path.join(ROOT, "include", "sphconv_hip.h")).read()
+    names = re.findall(r"\b(sph_[a-z0-9_]+)\s*\([^;]*void \*stream\);", hdr)
+    assert len(names) > 20
+    return names
+
+
+def test_the_host_extension_launches_on_its_tensors_device():
+    """Every function of the host extension that launches has made its tensors' device current and takes the stream from
+    there: a launch on the current device's stream is not ordered with what torch ran on the tensors' device."""
+    src = open(os.path.join(ROOT, "sphconv_amd", "csrc", "host.cpp")).read()
+    assert src.count("getCurrentHIPStream") == 1
+    on_device = src[src.index("struct OnDevice"):]
+    assert "DeviceGuard guard" in on_device[:on_device.index("};")] and "getCurrentHIPStream(t.device().index())" in on_device[:on_device.index("};")]
+    launches = [m for m in re.finditer(r"\b(%s)\(" % "|".join(_launching_entry_points()), src)]
+    assert len(launches) >= 13
+    for m in launches:
+        opening = list(re.finditer(r"\n( {4})?\{\n", src[:m.start()]))[-1]     # of the function that holds the launch
+        head = src[max(src.rindex(end, 0, opening.start()) for end in ("}\n", ";\n")):opening.start()]
+        assert "const OnDevice here(" in src[opening.end():m.start()] or "const OnDevice &here" in head, m.group(1)
+
+
+def test_the_package_launches_on_its_tensors_device():
+    """The same for the calls of the C ABI that Python makes itself."""
+    import ast
+    names = set(_launching_entry_points())
+    seen = 0
+    for file in sorted(os.listdir(os.path.join(ROOT, "sphconv_amd"))):
+        if not file.endswith(".py"):
+            continue
+        tree = ast.parse(open(os.path.join(ROOT, "sphconv_amd", file)).read())
+        guarded = [n for w in ast.walk(tree) if isinstance(w, ast.With) for n in ast.walk(w)
+                   if any(isinstance(i.context_expr, ast.Call) and getattr(i.context_expr.func, "attr", "") == "on_device" for i in w.items)]
+        for call in ast.walk(tree):
+            if isinstance(call, ast.Call) and getattr(call.func, "attr", "") in names:
+                seen += 1
+                assert call in guarded, "%s:%d" % (file, call.lineno)
+    assert seen >= 10
+
+
+def test_stream_and_device_context_follow_the_tensors_device(monkeypatch):
+    entered = []
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 1000 + index, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "device", lambda d: entered.append(d) or L._IS_CURRENT)
+    assert L.stream() == 1000 and L.stream(torch.device("cuda")) == 1000
+    assert L.stream(torch.device("cuda", 1)) == 1001
+    for d in (torch.device("cuda", 1), torch.device("cuda", 0), torch.device("cuda"), torch.device("cpu")):
+        with L.on_device(d):
+            pass
+    assert entered == [torch.device("cuda", 1)]
