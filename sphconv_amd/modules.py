@@ -25,13 +25,23 @@ def is_sparse_conv(module) -> bool:
     return isinstance(module, SphModule) and module.is_convolution
 
 
+def _hooked(module) -> bool:
+    """Whether calling the module runs more than its forward (pruning computes its weight in such a hook)."""
+    return bool(module._forward_pre_hooks or module._forward_hooks)
+
+
 def _bn_affine(bn: nn.BatchNorm1d):
     """Evaluation-mode BatchNorm1d as y = x*scale + shift (fp32 [C]); computed once per state of
     the module's tensors (their version counters) and kept on the module."""
     # (straight from the module's tables: asking the module four times takes longer than the key)
     p, b = bn._parameters, bn._buffers
+    try:
+        tensors = (b["running_mean"], b["running_var"], p["weight"], p["bias"])
+    except KeyError:
+        # a tensor that is not in its table is computed, or a replica's: another one on each pass, nothing to keep
+        return _bn_affine_now(bn)
     key = [bn.eps]
-    for t in (b["running_mean"], b["running_var"], p["weight"], p["bias"]):
+    for t in tensors:
         if t is not None:
             key += (t.data_ptr(), t._version, t.dtype)
         else:
@@ -114,11 +124,11 @@ class Sequential(SphModule):
             return 0, None, False
         n, bn, relu = 0, None, False
         nxt = mods[i + 1] if i + 1 < len(mods) else None
-        if (type(nxt) is nn.BatchNorm1d and not nxt.training and nxt._buffers["running_mean"] is not None
-                and nxt.num_features == conv.out_channels):
+        if (type(nxt) is nn.BatchNorm1d and not nxt.training and nxt.running_mean is not None
+                and nxt.num_features == conv.out_channels and not _hooked(nxt)):
             bn, n = nxt, 1
             nxt = mods[i + 2] if i + 2 < len(mods) else None
-        if type(nxt) is nn.ReLU:
+        if type(nxt) is nn.ReLU and not _hooked(nxt):
             relu, n = True, n + 1
         return n, bn, relu
 

@@ -11,7 +11,7 @@ import torch
 import sphconv_amd
 from oracle import oracle as O
 from sphconv_amd import _lib as L
-from sphconv_amd import utils
+from sphconv_amd import modules, utils
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -152,3 +152,50 @@ def test_stream_and_device_context_follow_the_tensors_device(monkeypatch):
         with L.on_device(d):
             pass
     assert entered == [torch.device("cuda", 1)]
+
+
+def _affine_of(bn):
+    x = torch.linspace(-2, 2, 5 * bn.num_features).view(5, bn.num_features)
+    with torch.no_grad():
+        want = bn(x)
+        scale, shift = modules._bn_affine(bn)
+    torch.testing.assert_close(x * scale + shift, want, rtol=1e-5, atol=1e-5)     # a few fp32 roundings
+
+
+def test_batch_norm_whose_tensors_are_not_in_its_tables():
+    """Pruned, replicated and weight-normed modules hold a weight or a mean as a plain attribute."""
+    from torch.nn.utils import prune
+    for name in ("weight", "bias", "running_mean", "running_var"):
+        bn = torch.nn.BatchNorm1d(8).eval()
+        with torch.no_grad():
+            for t in (bn.weight, bn.bias, bn.running_mean, bn.running_var):
+                t.uniform_(0.5, 2.0)
+        _affine_of(bn)
+        if name in bn._parameters:
+            prune.random_unstructured(bn, name, 0.5)
+        else:
+            value = bn._buffers.pop(name)
+            setattr(bn, name, value)
+        for k in range(3):                      # its values change, at an address that may be an earlier one's
+            with torch.no_grad():
+                (bn._parameters.get(name + "_orig") if name + "_orig" in bn._parameters else getattr(bn, name)).mul_(1.5)
+            _affine_of(bn)
+        seq = sphconv_amd.Sequential(sphconv_amd.SubMConv3d(4, 8, 3), bn, torch.nn.ReLU()).eval()
+        with torch.no_grad():
+            n, found, relu = seq._fusable_tail(list(seq), 0)
+        assert (n, found, relu) == ((0, None, False) if name + "_orig" in bn._parameters else (2, bn, True))
+
+
+def test_modules_with_hooks_are_called_not_folded():
+    """A hook sees every call of its module: such a module is not folded into the convolution before it."""
+    seq = sphconv_amd.Sequential(sphconv_amd.SubMConv3d(4, 8, 3), torch.nn.BatchNorm1d(8), torch.nn.ReLU()).eval()
+    conv, bn, act = list(seq)
+    with torch.no_grad():
+        assert seq._fusable_tail([conv, bn, act], 0) == (2, bn, True)
+        h = act.register_forward_hook(lambda m, i, o: None)
+        assert seq._fusable_tail([conv, bn, act], 0) == (1, bn, False)
+        h.remove()
+        h = bn.register_forward_pre_hook(lambda m, i: None)
+        assert seq._fusable_tail([conv, bn, act], 0) == (0, None, False)
+        h.remove()
+        assert seq._fusable_tail([conv, bn, act], 0) == (2, bn, True)
