@@ -6,6 +6,8 @@ from collections import OrderedDict
 import torch
 from torch import nn
 
+from . import _lib as L
+
 
 _NO_RANGE = contextlib.nullcontext()
 
@@ -31,8 +33,9 @@ def _hooked(module) -> bool:
 
 
 def _bn_affine(bn: nn.BatchNorm1d):
-    """Evaluation-mode BatchNorm1d as y = x*scale + shift (fp32 [C]); computed once per state of
-    the module's tensors (their version counters) and kept on the module."""
+    """Evaluation-mode BatchNorm1d as y = x*scale + shift (fp32 [C]); computed once per state of the module's tensors and
+    kept on the module, for the stream it was computed on.  The state is the tensors themselves, which the entry holds (an
+    address alone is handed out again once its tensor is gone), with their storage and version counter."""
     # (straight from the module's tables: asking the module four times takes longer than the key)
     p, b = bn._parameters, bn._buffers
     try:
@@ -40,17 +43,19 @@ def _bn_affine(bn: nn.BatchNorm1d):
     except KeyError:
         # a tensor that is not in its table is computed, or a replica's: another one on each pass, nothing to keep
         return _bn_affine_now(bn)
-    key = [bn.eps]
+    state = [bn.eps]
     for t in tensors:
         if t is not None:
-            key += (t.data_ptr(), t._version, t.dtype)
-        else:
-            key.append(None)
-    cached = bn.__dict__.get("_sph_affine")
-    if cached is not None and cached[0] == key:
-        return cached[1], cached[2]
+            state += (t.data_ptr(), t._version, t.dtype)
+    kept = bn.__dict__.setdefault("_sph_affines", {})
+    stream = L.stream(tensors[0].device) if tensors[0].is_cuda else None
+    hit = kept.get(stream)
+    if hit is not None and hit[1] == state and all(a is b for a, b in zip(hit[0], tensors)):
+        return hit[2], hit[3]
     scale, shift = _bn_affine_now(bn)
-    bn._sph_affine = (key, scale, shift)
+    if len(kept) >= 16:
+        kept.clear()
+    kept[stream] = (tensors, state, scale, shift)
     return scale, shift
 
 

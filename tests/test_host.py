@@ -199,3 +199,38 @@ def test_modules_with_hooks_are_called_not_folded():
         assert seq._fusable_tail([conv, bn, act], 0) == (0, None, False)
         h.remove()
         assert seq._fusable_tail([conv, bn, act], 0) == (2, bn, True)
+
+
+def test_kept_affine_map_belongs_to_the_tensors_and_the_stream(monkeypatch):
+    """The affine map kept on a BatchNorm1d is not taken for another tensor that the allocator put at the same address, nor
+    on a stream that is not ordered behind its computation; a copy of the module has its own."""
+    import copy
+    import numpy as np
+    bn = torch.nn.BatchNorm1d(4).eval()
+    memory = np.ones(4, dtype=np.float32)
+    for value in (1.0, 2.0, 3.0):               # other values at one address, version 0 each time
+        memory[:] = value
+        bn.weight = torch.nn.Parameter(torch.from_numpy(memory))
+        with torch.no_grad():
+            torch.testing.assert_close(modules._bn_affine(bn)[0], torch.full((4,), value), rtol=1e-4, atol=0)
+    with torch.no_grad():
+        first = modules._bn_affine(bn)[0]
+        assert modules._bn_affine(bn)[0] is first
+        twin = copy.deepcopy(bn)
+        twin.running_var.mul_(4.0)
+        _affine_of(twin)
+        assert modules._bn_affine(bn)[0] is first
+
+    class OnGpu(torch.Tensor):                  # as far as the look-up can tell
+        is_cuda = True
+
+    stream = [7]
+    monkeypatch.setattr(modules.L, "stream", lambda device=None: stream[0])
+    bn._buffers["running_mean"] = bn.running_mean.as_subclass(OnGpu)
+    with torch.no_grad():
+        on7 = modules._bn_affine(bn)[0]
+        stream[0] = 8
+        on8 = modules._bn_affine(bn)[0]
+        assert on8 is not on7 and modules._bn_affine(bn)[0] is on8
+        stream[0] = 7
+        assert modules._bn_affine(bn)[0] is on7
