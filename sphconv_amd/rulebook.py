@@ -80,10 +80,12 @@ class _Geometry:
     by every book that has it (a network meets a few dozen)."""
 
     __slots__ = ("native", "batch", "in_shape", "out_shape", "kernel", "stride", "padding", "dilation", "kv", "in_cells",
-                 "out_cells", "steps", "odd_same", "z_shape", "cluster")
+                 "out_cells", "steps", "odd_same", "z_shape", "cluster", "key")
 
     def __init__(self, batch, in_shape, out_shape, kernel, stride, padding, dilation):
         self.batch = batch
+        # what two layers' geometries are compared by: the tables below start over now and then, and make another object
+        self.key = (batch, *in_shape, *out_shape, *kernel, *stride, *padding, *dilation)
         self.in_shape, self.out_shape, self.kernel = list(in_shape), list(out_shape), list(kernel)
         self.stride, self.padding, self.dilation = list(stride), list(padding), list(dilation)
         self.kv = kernel[0] * kernel[1] * kernel[2]
@@ -325,7 +327,7 @@ class RuleBook:
         """A strided layer's book: its output coordinates now, its pairs not built yet."""
         if ahead is None:
             ahead = cls._count(geometry, z_idx, z_ptr)
-        elif ahead.geometry is not geometry or ahead.z_idx.data_ptr() != z_idx.data_ptr() \
+        elif ahead.geometry.key != geometry.key or ahead.z_idx.data_ptr() != z_idx.data_ptr() \
                 or ahead.z_ptr.data_ptr() != z_ptr.data_ptr() or ahead.native.stream != L.stream(z_ptr.device):
             raise L.SphconvError("count_ahead() was called for another layer, tensor or stream")
         # the rows' columns are a by-product of the coordinates

@@ -234,3 +234,33 @@ def test_kept_affine_map_belongs_to_the_tensors_and_the_stream(monkeypatch):
         assert on8 is not on7 and modules._bn_affine(bn)[0] is on8
         stream[0] = 7
         assert modules._bn_affine(bn)[0] is on7
+
+
+def test_a_count_started_ahead_outlives_the_tables_of_geometries(monkeypatch):
+    """The tables of geometries start over after 4096 shapes: the layer whose count was started before is still that layer,
+    and another layer's count is still refused."""
+    from types import SimpleNamespace
+    from sphconv_amd import rulebook
+
+    def geometry(s0=16, stride=(2, 2, 2)):
+        return rulebook.layer_geometry(2, s0, 40, 16, (3, 3, 3), stride, (1, 1, 1), (1, 1, 1), False)[0]
+
+    z_idx, z_ptr = torch.zeros(5, dtype=torch.int32), torch.zeros((2, 16, 40), dtype=torch.int32)
+    out = torch.zeros(7, dtype=torch.int32)
+    monkeypatch.setattr(rulebook.L, "stream", lambda device=None: 3)
+
+    def count(g):
+        native = SimpleNamespace(stream=3, finish=lambda: (out, z_ptr, out))
+        return SimpleNamespace(geometry=g, z_idx=z_idx, z_ptr=z_ptr, native=native)
+
+    before = geometry()
+    assert geometry() is before
+    for s0 in range(17, 17 + 4096):
+        geometry(s0)
+    after = geometry()
+    assert after is not before
+    book = rulebook.RuleBook._strided(after, z_idx, z_ptr, count(before), None)
+    assert book.out_rows == 7 and book.in_rows == 5
+    for other in (geometry(18), geometry(16, (2, 2, 1))):
+        with pytest.raises(L.SphconvError, match="another layer"):
+            rulebook.RuleBook._strided(other, z_idx, z_ptr, count(before), None)
