@@ -3,6 +3,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
+from .utils import plain
 from .vfe import SimpleVoxel
 from .voxelize import VoxelGeneratorV3
 
@@ -29,7 +30,8 @@ def merge_batch_torch(batch_list):
     for name in names:
         parts = [example[name] for example in batch_list if name in example]
         if name == "coordinates" and len(parts) <= _MAX_PARTS and all(
-                c.is_cuda and c.dtype == torch.int32 and c.dim() == 2 and c.shape[1] == 3 and c.is_contiguous() for c in parts):
+                c.is_cuda and c.dtype == torch.int32 and c.dim() == 2 and c.shape[1] == 3 and c.is_contiguous()
+                and c.device == parts[0].device and plain(c) for c in parts):
             merged[name] = L.host().batch_coordinates(parts)                               # one kernel
             continue
         if name == "coordinates":

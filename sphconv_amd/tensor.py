@@ -6,6 +6,7 @@ import torch
 
 from . import sphconv_cuda as ext
 from .functional import InitTensorFunction, ToDenseFunction
+from .utils import plain
 
 
 class SparseTensorBase:
@@ -46,7 +47,7 @@ class SparseConvTensor(SparseTensorBase):
         assert raw_feature.device == indices.device
         super().__init__(batch_size, s0, s1, s2, raw_feature.shape[-1], raw_feature.device,
                          raw_feature.dtype, indices.dtype, None, None, None)
-        if torch.is_grad_enabled() and raw_feature.requires_grad:
+        if (torch.is_grad_enabled() and raw_feature.requires_grad) or not plain(raw_feature):
             self.feature, self.z_idx, self.z_ptr, self.row_cols = InitTensorFunction.apply(
                 raw_feature, indices, self.B, [self.D, self.W, self.H], True)
         else:

@@ -190,3 +190,19 @@ def test_layers_behind_a_strided_one_count_its_clusters(monkeypatch, kernel, str
     assert x.cluster > 1.0 if kernel[0] > stride[0] else x.cluster == 1.0
     G.assert_same_conv(out[0], out[1])
     G.assert_same_conv(out[0], out[2])
+
+
+def test_voxel_means_carry_tangents_and_transforms():
+    """The mean of a voxel's points as one kernel stands for torch's operations: with a tangent, under vmap and with counts
+    that lie on the host the result is still theirs."""
+    import torch.autograd.forward_ad as fwAD
+    voxels, num = torch.randn((50, 5, 6), device=G.DEV), torch.randint(1, 6, (50,), device=G.DEV, dtype=torch.int32)
+    tangent, vfe = torch.randn_like(voxels), SimpleVoxel(4)
+    want = lambda v: v[..., :4].sum(-2) / num.float()[:, None]
+    with fwAD.dual_level():
+        got = fwAD.unpack_dual(vfe(fwAD.make_dual(voxels, tangent), num, None))
+    torch.testing.assert_close(got.primal, want(voxels), rtol=1e-6, atol=1e-6)
+    torch.testing.assert_close(got.tangent, want(tangent), rtol=1e-6, atol=1e-6)
+    both = torch.stack([voxels, tangent])
+    torch.testing.assert_close(torch.func.vmap(lambda v: vfe(v, num, None))(both), want(both), rtol=1e-6, atol=1e-6)
+    torch.testing.assert_close(vfe(voxels, num.cpu(), None), want(voxels), rtol=1e-6, atol=1e-6)

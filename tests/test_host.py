@@ -264,3 +264,33 @@ def test_a_count_started_ahead_outlives_the_tables_of_geometries(monkeypatch):
     for other in (geometry(18), geometry(16, (2, 2, 1))):
         with pytest.raises(L.SphconvError, match="another layer"):
             rulebook.RuleBook._strided(other, z_idx, z_ptr, count(before), None)
+
+
+def test_what_is_more_than_values_does_not_go_past_torch(monkeypatch):
+    """Tangents, transforms, traces and tensor subclasses go the way of torch's own operations."""
+    import torch.autograd.forward_ad as fwAD
+    from sphconv_amd import tensor as tensor_mod
+    x = torch.randn(4, 3)
+    assert utils.plain(x) and utils.plain(torch.nn.Parameter(x)) and utils.plain(torch.zeros(4, dtype=torch.int32))
+    with fwAD.dual_level():
+        assert utils.plain(x) and not utils.plain(fwAD.make_dual(x, x))
+    seen = []
+    look = lambda t: seen.append(utils.plain(t)) or t * 1
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.jit.trace(look, (x,), check_trace=False)
+    assert seen == [False] * 3
+
+    class Own(torch.Tensor):
+        pass
+
+    assert not utils.plain(x.as_subclass(Own))
+
+    # a tensor made of rows with a tangent: refused by the autograd function, which has none, not dropped in silence
+    zeros = torch.zeros(4, dtype=torch.int32)
+    fake = lambda f, i, b, s: [f.detach().clone(), zeros, torch.zeros((1, 2, 2), dtype=torch.int32), zeros.clone(), zeros.clone()]
+    monkeypatch.setattr(tensor_mod.ext, "_init_tensor", fake)
+    indices = torch.zeros((4, 4), dtype=torch.int32)
+    assert sphconv_amd.SparseConvTensor(x, [2, 2, 2], 1, indices=indices).feature.shape == (4, 3)
+    with fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp"):
+        sphconv_amd.SparseConvTensor(fwAD.make_dual(x, x), [2, 2, 2], 1, indices=indices)
