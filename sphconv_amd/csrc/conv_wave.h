@@ -467,8 +467,20 @@ __device__ __forceinline__ void conv_run_store(const ConvArgs &a, int nwtot, con
 
 // Waves that share a tile's groups: the most of 4, 2 and 1 whose accumulator copies (acc_bytes each, beside `other` bytes
 // of LDS) leave room for all tiles at once on the chip's 256 CUs of 160 KB.
-inline int split_waves(int ntiles, size_t acc_bytes, size_t other)
+// Not where workgroups share a CU and the alternative is helper waves for the middle offset's run, for rows of 128 bytes
+// (8- or 16-bit): a group is then two full steps of fragments and rows, the CU's vector memory path is what its waves wait
+// for, and the helper waves are the ones that load less.  Shared : helper waves, grouped kernel / one launch, us, fp16 at
+// 3.1 pairs per row: 64 -> 64 at 247 tiles 9.1 : 11.2 / 13.7 : 15.6, at 275 12.9 : 11.3 / 17.5 : 16.0, at 459 14.0 : 12.3 /
+// 18.3 : 17.2; 64 -> 32 at 275 10.0 : 8.8 / 14.4 : 13.5, at 686 12.8 : 11.7 / 17.7 : 16.5; 64 -> 16 at 459 8.4 : 8.1 / 13.0 :
+// 12.9, at 686 11.2 : 9.8 / 15.6 : 14.7.  At 6.6 pairs per row, 467 tiles, 23.7 : 22.2 / 29.6 : 30.1, 17.3 : 17.3 / 23.3 : 24.7
+// and 14.1 : 14.7 / 20.2 : 22.6 (sixteen columns are therefore shared up to 512 tiles).  Shorter rows, fp32 and books without
+// the run are shared at every size: 32 -> 64 fp16 at 477 tiles 10.1 : 11.2 / 15.1 : 15.5, 48 -> 32 at 459 9.2 : 9.2 / 13.6 :
+// 14.2, 16 -> 64 fp32 at 477 18.1 : 19.3 / 22.6 : 23.7, strided 64 -> 64 at 309 11.2 : 11.3 / 15.4 : 15.7 (48 -> 32 at 686 loses
+// in the grouped kernel, 10.9 : 10.1 / 15.6 : 15.5, and gains at 6.6 pairs per row, 17.0 : 17.2 / 23.3 : 25.5 at 647).
+// helpers: that alternative is there (a book with the run, rows of up to 128 bytes); nwtot: column tiles of 16.
+inline int split_waves(sph_dtype dt, int row_bytes, int nwtot, bool helpers, int ntiles, size_t acc_bytes, size_t other)
 {
+    if (helpers && dt != SPH_F32 && row_bytes == 128 && ntiles > (nwtot > 1 ? 256 : 512)) return 1;
     for (int s = 4; s > 1; s /= 2) {
         const size_t wg = s * acc_bytes + other + 1024; // + static LDS and its rounding
         if (wg <= 160 * 1024 && ntiles <= 256 * (int)(160 * 1024 / wg)) return s;

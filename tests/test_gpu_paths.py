@@ -132,6 +132,30 @@ def test_waves_that_share_a_tile(dtype, oc, tiles):
     _close(fused, want, dtype)
 
 
+@pytest.mark.parametrize("ic,oc,tiles", [(64, 64, 256), (64, 64, 257), (64, 32, 256), (64, 32, 257), (64, 16, 512), (64, 16, 513),
+                                         (64, 16, 1025), (48, 32, 513)])
+@pytest.mark.parametrize("subm", [True, False])
+def test_long_rows_share_a_tile_or_have_helper_waves(ic, oc, tiles, subm):
+    """Rows of 128 bytes: waves that share a tile up to 256 or 512 tiles, helper waves for the middle offset's run beyond,
+    and sharing again where a book has no such run, the rows are shorter or the tiles so many that the helper waves do not
+    pay."""
+    rng = np.random.default_rng(tiles + oc)
+    n, shape = tiles * L.TILE_ROWS - 5, [16, 40 * tiles, 8]
+    case = G.build_case(_cells(rng, n, 1, shape), 1, shape, [3, 3, 3], [1, 1, 1], [1, 1, 1], True)
+    book = case["book"]
+    book.fwd.native.middle_run = int(subm)
+    feat = torch.tensor(rng.standard_normal((n, ic)), dtype=torch.float32).half()
+    w = torch.tensor(rng.standard_normal((27, ic, oc)) * 0.1, dtype=torch.float32).half()
+    want = O.rule_conv(feat.float().numpy(), w.float().numpy(), case["oracle"][2], case["oracle"][3], n)
+    _close(ext.rule_conv(feat.to(G.DEV), w.to(G.DEV), book, None, n), want, torch.float16)
+    if subm:
+        lazy = RuleBook.build_subm(book.z_idx, book.z_ptr, 1, shape, [3, 3, 3], row_cols=row_columns(book.z_ptr, n), lazy=True)
+        lazy.keep = False
+        fused = ext.rule_conv(feat.to(G.DEV), w.to(G.DEV), lazy, None, n)
+        assert lazy.built == (tiles > RuleBook.FUSED_MAX_TILES)
+        _close(fused, want, torch.float16)
+
+
 def test_one_column_stride_too_wide_for_the_tile_kernel():
     """Output coordinates of a layer whose columns lie 64 input columns apart, 500 bins deep: the bin masks of a tile's
     input columns would not fit LDS."""
