@@ -6,7 +6,8 @@
  * `sphconv.sphconv_cuda` (src/sphconv/all.cpp:14-38) calls instead of the CUDA
  * kernels.  Every pointer is a DEVICE pointer unless the comment says "host".
  * The library never allocates, frees or synchronises: the caller provides all
- * outputs and scratch, and every call only enqueues kernels on `stream`.
+ * outputs and scratch, and every call only enqueues kernels on `stream`, whose
+ * device must be the current one.
  *
  * Every function returns 0 on success or a negative sph_status; the message of
  * the last failure on the calling thread is returned by sph_last_error().

@@ -448,10 +448,12 @@ constexpr int kMaskWalk = 16;  // fiber entries fetched together when a mask is 
 // the whole workgroup of kThreads threads; returns behind a barrier.  s_masks: LDS for the mask join (used when
 // a.long_fibers; kMaskCols * K0 * K1 * 12 bytes, 8-byte aligned).
 // MASKS, LINES, COLUMNS: the joins the kernel holds (a.long_fibers and a.lines choose among them): a join that is left out
-// costs neither registers nor, the mask join, its 3 KB of static LDS.
+// costs neither registers nor, the mask join, its 3 KB of static LDS.  The join by lines checks the rows' columns as it goes,
+// the other two find them checked.
 template <bool TRANSPOSED, bool MASKS, bool LINES, bool COLUMNS, int NT>
 __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t *s_nbr, void *s_masks)
 {
+    static_assert(!(MASKS && LINES), "the mask join finds the rows' columns checked");
     __shared__ int s_col[R];
     __shared__ int s_first[2 * (NT / kWave)], s_flag[2];
 
@@ -546,7 +548,6 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
     // leaves the 64 bins sends the whole tile to the general join below.
     bool by_masks = false;
     if constexpr (MASKS) if (a.long_fibers) {
-        if constexpr (LINES) if (!checked && !check_hint()) continue;
         unsigned long long *s_cmask = (unsigned long long *)s_masks; // [K01][ncols], ncols <= kMaskCols
         int *s_cstart = (int *)(s_cmask + kMaskCols * K01);
         __shared__ int s_b[R], s_c0[R], s_c1[R], s_z[R];
@@ -661,7 +662,7 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
     // three entry loads per column: 5890 tiles of a submanifold layer 35.3 us either way, 920 tiles of a transposed book of
     // stride 2, where two lines of three at most can pair and mostly one column of theirs, 17.1 -> 12.2 us, ten tiles with
     // the convolution behind it 11.3 -> 10.8 us.
-    if constexpr (LINES) if (!by_masks && (!COLUMNS || a.lines)) {
+    if constexpr (LINES) if (!COLUMNS || a.lines) {
         const int C = a.lines, p_ncol = a.B * a.P.n0 * a.P.n1;
         const __amdgpu_buffer_rsrc_t r_ptr = __builtin_amdgcn_make_buffer_rsrc((void *)a.p_ptr, 0, p_ncol * 4, 0x00020000);
         const __amdgpu_buffer_rsrc_t r_idx = __builtin_amdgcn_make_buffer_rsrc((void *)a.p_idx, 0, a.p_rows * 4, 0x00020000);
