@@ -307,10 +307,11 @@ py::object rules_build_pack(const Tensor &z_idx, const Tensor &z_ptr, const Tens
 
 // Output coordinates of a strided layer.  start(): the count and its scan are enqueued, and behind them already the
 // kernel that writes the coordinates, into arrays of the most rows the layer can reach -- prod ceil(K / stride) per input
-// row -- so that the GPU has work while the host learns the row count and enqueues what needs it (the arrays handed out
-// are the leading part; beyond kAheadBytes the coordinates are written after the wait, into arrays of their size).
+// row -- so that the GPU has work while the host learns the row count and enqueues what needs it.  What is handed out is
+// then the leading part of arrays that may be several times its size and live as long as it does, so this is done where
+// the two arrays hold at most kAheadBytes; beyond, the coordinates are written after the wait, into arrays of their size.
 struct OutCoords {
-    static constexpr double kAheadBytes = 256e6;
+    static constexpr double kAheadBytes = 16 << 20;
     Tensor z_idx, z_ptr, oz_ptr, scratch, oz_idx, cols;
     const Geometry *geom;
     py::object geom_owner;

@@ -230,3 +230,31 @@ def test_voxel_means_carry_tangents_and_transforms():
     both = torch.stack([voxels, tangent])
     torch.testing.assert_close(torch.func.vmap(lambda v: vfe(v, num, None))(both), want(both), rtol=1e-6, atol=1e-6)
     torch.testing.assert_close(vfe(voxels, num.cpu(), None), want(voxels), rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("n", [30000, 400000])
+def test_output_coordinates_hold_no_more_than_they_may(n):
+    """Output coordinates written behind their count, into arrays of the most rows the layer can reach, and, where those
+    would hold more than 16 MiB, after the wait into arrays of their size."""
+    B, shape, out = 3, [64, 2048, 64], [32, 1024, 32]
+    idx = _cells(np.random.default_rng(n), n, B, shape)
+    order = np.lexsort(idx.T[::-1])
+    idx = idx[order]
+    counts = np.bincount((idx[:, 0] * shape[0] + idx[:, 1]) * shape[1] + idx[:, 2], minlength=B * shape[0] * shape[1])
+    z_ptr = np.cumsum(counts).astype(np.int32).reshape(B, *shape[:2])
+    book = RuleBook.build(G.t(idx[:, 3].copy()), G.t(z_ptr), B, shape, out, [3, 3, 3], [2, 2, 2], [1, 1, 1], lazy=True)
+    reached = np.zeros((B, *out), dtype=bool)
+    for k in np.ndindex(3, 3, 3):
+        at = idx[:, 1:] + 1 - np.array(k)
+        ok = (at % 2 == 0).all(1) & (at >= 0).all(1) & (at // 2 < np.array(out)).all(1)
+        o = at[ok] // 2
+        reached[idx[ok, 0], o[:, 0], o[:, 1], o[:, 2]] = True
+    want = np.argwhere(reached)
+    col = (want[:, 0] * out[0] + want[:, 1]) * out[1] + want[:, 2]
+    assert np.array_equal(book.oz_idx.cpu().numpy(), want[:, 3])
+    assert np.array_equal(book.out_row_cols.cpu().numpy(), col)
+    assert np.array_equal(book.oz_ptr.cpu().numpy().ravel(), np.cumsum(np.bincount(col, minlength=B * out[0] * out[1])))
+    for t in (book.oz_idx, book.out_row_cols):
+        assert t.untyped_storage().nbytes() <= max(4 * book.out_rows + 512, 8 << 20)
+    late = 8 * 8 * n > 16 << 20
+    assert (book.oz_idx.untyped_storage().nbytes() <= 4 * book.out_rows + 512) == late
