@@ -7,6 +7,7 @@ the HIP kernels consume (see ``include/sphconv_hip.h``) and materialises the
 padded tensors only when asked (:meth:`RuleBook.padded`).
 """
 import ctypes as C
+import threading
 from typing import List, Optional, Sequence
 
 import torch
@@ -504,20 +505,24 @@ class _CountAhead:
 
 
 # Scratch books of one-launch calls that keep no book (the kernel still wants one for tiles with more groups than
-# its LDS holds): one per device, stream and kernel volume, grown on demand.  Calls on one stream run one after the
-# other, so they can share it; calls on different streams get different ones.
-_SCRATCH_BOOKS = {}
+# its LDS holds): one per thread, device, stream and kernel volume, grown on demand.  Calls on one stream run one after
+# the other, so they can share its memory; calls on different streams get different ones.  Two threads may use one
+# stream, and a call writes its row count and its kind into the book before it launches: each thread has its own.
+_SCRATCH_BOOKS = threading.local()
 
 
 def _scratch_book(rows: int, kv: int, device) -> "_Buffers":
+    books = getattr(_SCRATCH_BOOKS, "books", None)
+    if books is None:
+        books = _SCRATCH_BOOKS.books = {}
     key = (device.index, L.stream(device), kv)
-    buf = _SCRATCH_BOOKS.get(key)
+    buf = books.get(key)
     if buf is None or buf.capacity < rows:
-        if len(_SCRATCH_BOOKS) >= 64:
-            _SCRATCH_BOOKS.clear()
+        if len(books) >= 64:
+            books.clear()
         buf = _Buffers(max(rows, 1 << 17), kv, device)
         buf.capacity = buf.rows
-        _SCRATCH_BOOKS[key] = buf
+        books[key] = buf
     buf.native.rows = rows
     return buf
 

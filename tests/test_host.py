@@ -294,3 +294,22 @@ def test_what_is_more_than_values_does_not_go_past_torch(monkeypatch):
     assert sphconv_amd.SparseConvTensor(x, [2, 2, 2], 1, indices=indices).feature.shape == (4, 3)
     with fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp"):
         sphconv_amd.SparseConvTensor(fwAD.make_dual(x, x), [2, 2, 2], 1, indices=indices)
+
+
+def test_threads_on_one_stream_have_scratch_books_of_their_own(monkeypatch):
+    """A one-launch call that keeps no book writes its row count and kind into a scratch book before it launches: a call of
+    another thread on the same stream must not get in between."""
+    import threading
+    from sphconv_amd import rulebook
+    monkeypatch.setattr(rulebook.L, "stream", lambda device=None: 5)
+    cpu = torch.device("cpu")
+    mine = rulebook._scratch_book(100, 27, cpu)
+    assert rulebook._scratch_book(300, 27, cpu) is mine and mine.native.rows == 300
+    theirs = []
+    t = threading.Thread(target=lambda: theirs.append(rulebook._scratch_book(200, 27, cpu)))
+    t.start()
+    t.join()
+    assert theirs[0].native.address != mine.native.address and theirs[0].struct().tile_ngrp != mine.struct().tile_ngrp
+    assert mine.native.rows == 300 and theirs[0].native.rows == 200
+    bigger = rulebook._scratch_book((1 << 17) + 1, 27, cpu)
+    assert bigger is not mine and rulebook._scratch_book(10, 27, cpu) is bigger
