@@ -9,6 +9,7 @@
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -62,13 +63,13 @@ template <typename T = void> T *ptr(const OptTensor &t) { return t ? ptr<T>(*t) 
 // kernel is launched on a stream that came from here and nowhere else: torch's own operations follow their tensors'
 // device, so a launch on the stream of whatever device happens to be current would not be ordered with what made its inputs.
 struct OnDevice {
-    c10::DeviceGuard guard;
+    c10::OptionalDeviceGuard guard; // (empty where the device is current anyway: leaving a guard sets the device again)
     hipStream_t stream;
-    explicit OnDevice(const Tensor &t) : guard(of(t)), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
-    static c10::Device of(const Tensor &t)
+    explicit OnDevice(const Tensor &t)
     {
         if (!t.is_cuda()) raise("expected a GPU tensor, got device " + t.device().str());
-        return t.device();
+        if (t.device().index() != c10::hip::current_device()) guard.reset_device(t.device());
+        stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
     }
 };
 
