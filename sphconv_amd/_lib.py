@@ -170,6 +170,11 @@ def stream(device=None):
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
+# Whether torch's current stream records a graph.  What is computed then exists only while the graph replays, in memory of
+# the graph's, and what the graph reads has to live as long as it does: nothing is kept from call to call.
+capturing = torch.cuda.is_current_stream_capturing
+
+
 _IS_CURRENT = contextlib.nullcontext()
 
 

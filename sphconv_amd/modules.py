@@ -32,30 +32,41 @@ def _hooked(module) -> bool:
     return bool(module._forward_pre_hooks or module._forward_hooks)
 
 
-def _bn_affine(bn: nn.BatchNorm1d):
+def _keeps_on(t: torch.Tensor):
+    """The stream that what is kept now belongs to (None for tensors on the host), or False where nothing may be kept: a
+    graph under capture computes everything itself."""
+    if not t.is_cuda:
+        return None
+    return False if L.capturing() else L.stream(t.device)
+
+
+def _bn_affine(bn: nn.BatchNorm1d, stream):
     """Evaluation-mode BatchNorm1d as y = x*scale + shift (fp32 [C]); computed once per state of the module's tensors and
-    kept on the module, for the stream it was computed on.  The state is the tensors themselves, which the entry holds (an
+    kept on the module, for the stream it was computed on (``_keeps_on``).  The state is the tensors themselves, which the entry holds (an
     address alone is handed out again once its tensor is gone), with their storage and version counter."""
     # (straight from the module's tables: asking the module four times takes longer than the key)
     p, b = bn._parameters, bn._buffers
+    if stream is False:
+        return _bn_affine_now(bn)
     try:
-        tensors = (b["running_mean"], b["running_var"], p["weight"], p["bias"])
+        mean, var, weight, bias = b["running_mean"], b["running_var"], p["weight"], p["bias"]
     except KeyError:
         # a tensor that is not in its table is computed, or a replica's: another one on each pass, nothing to keep
         return _bn_affine_now(bn)
     state = [bn.eps]
-    for t in tensors:
+    for t in (mean, var, weight, bias):
         if t is not None:
             state += (t.data_ptr(), t._version, t.dtype)
-    kept = bn.__dict__.setdefault("_sph_affines", {})
-    stream = L.stream(tensors[0].device) if tensors[0].is_cuda else None
+    kept = bn.__dict__.get("_sph_affines")
+    if kept is None:
+        kept = bn.__dict__["_sph_affines"] = {}
     hit = kept.get(stream)
-    if hit is not None and hit[1] == state and all(a is b for a, b in zip(hit[0], tensors)):
-        return hit[2], hit[3]
+    if hit is not None and hit[0] is mean and hit[1] is var and hit[2] is weight and hit[3] is bias and hit[4] == state:
+        return hit[5], hit[6]
     scale, shift = _bn_affine_now(bn)
     if len(kept) >= 16:
         kept.clear()
-    kept[stream] = (tensors, state, scale, shift)
+    kept[stream] = (mean, var, weight, bias, state, scale, shift)
     return scale, shift
 
 
@@ -129,7 +140,8 @@ class Sequential(SphModule):
             return 0, None, False
         n, bn, relu = 0, None, False
         nxt = mods[i + 1] if i + 1 < len(mods) else None
-        if (type(nxt) is nn.BatchNorm1d and not nxt.training and nxt.running_mean is not None
+        if (type(nxt) is nn.BatchNorm1d and not nxt.training
+                and (nxt._buffers.get("running_mean") is not None or nxt.running_mean is not None)
                 and nxt.num_features == conv.out_channels and not _hooked(nxt)):
             bn, n = nxt, 1
             nxt = mods[i + 2] if i + 2 < len(mods) else None
@@ -143,7 +155,7 @@ class Sequential(SphModule):
         only = [m for _, m in mods]
         conv = [is_sparse_conv(m) for m in only]
         profiling = torch.autograd._profiler_enabled()
-        skip = 0
+        skip, keeps_on = 0, None
         ahead = {}      # index of a strided convolution -> its count on the way
 
         def start_count(first):
@@ -174,7 +186,11 @@ class Sequential(SphModule):
                     skip, bn, relu = self._fusable_tail(only, i)
                     kw = {"ahead": ahead.pop(i)} if i in ahead else {}
                     if skip:
-                        scale, shift = _bn_affine(bn) if bn is not None else (None, None)
+                        scale = shift = None
+                        if bn is not None:
+                            if keeps_on is None:
+                                keeps_on = _keeps_on(input.feature)
+                            scale, shift = _bn_affine(bn, keeps_on)
                         input = module(input, epilogue=(scale, shift, relu), **kw)
                     else:
                         input = module(input, **kw)

@@ -512,6 +512,8 @@ _SCRATCH_BOOKS = threading.local()
 
 
 def _scratch_book(rows: int, kv: int, device) -> "_Buffers":
+    if L.capturing():                       # the graph's own, for as long as it needs it
+        return _Buffers(rows, kv, device)
     books = getattr(_SCRATCH_BOOKS, "books", None)
     if books is None:
         books = _SCRATCH_BOOKS.books = {}

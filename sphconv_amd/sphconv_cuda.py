@@ -54,12 +54,13 @@ def _packed_weight(weight: torch.Tensor, transpose: bool, reverse: bool = False,
     ``cache=True`` while no gradient is being recorded: then it is kept with the weight and reused until the
     weight's version counter, address, shape or type change.  Updates through ``weight.data`` do not move the
     version counter: call :func:`invalidate_packed` after them (modules: ``Convolution.invalidate_packed()``).
-    The kept copy belongs to the stream it was made on; other streams must order themselves behind it."""
+    The kept copy belongs to the stream it was made on; other streams must order themselves behind it.  While the stream
+    is captured nothing is kept, and no kept copy is used: the copy is made by the graph, on each replay."""
     w = weight.detach()
     if not w.is_contiguous():
         w = w.contiguous()
     cache_key = None
-    if cache and not torch.is_grad_enabled() and w.data_ptr() == weight.data_ptr():
+    if cache and not torch.is_grad_enabled() and w.data_ptr() == weight.data_ptr() and not L.capturing():
         base = weight._base if weight._base is not None else weight
         cache_key = (id(base), bool(transpose), bool(reverse), L.stream(w.device))
         state = (base._version, w.data_ptr(), tuple(w.shape), w.dtype)
@@ -76,7 +77,7 @@ def _kept_packed(weight: torch.Tensor) -> Optional[torch.Tensor]:
     """The kept fragment-ordered copy of ``weight`` (the parameter itself, of any shape) for the forward pass, if there
     is one and the weight has not changed since; None otherwise."""
     hit = _PACKED_CACHE.get((id(weight), False, False, L.stream(weight.device)))
-    if hit is None or hit[0]() is not weight:
+    if hit is None or hit[0]() is not weight or L.capturing():
         return None
     version, address, _, dtype = hit[1]
     return hit[2] if version == weight._version and address == weight.data_ptr() and dtype == weight.dtype else None

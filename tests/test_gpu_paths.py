@@ -258,3 +258,40 @@ def test_output_coordinates_hold_no_more_than_they_may(n):
         assert t.untyped_storage().nbytes() <= max(4 * book.out_rows + 512, 8 << 20)
     late = 8 * 8 * n > 16 << 20
     assert (book.oz_idx.untyped_storage().nbytes() <= 4 * book.out_rows + 512) == late
+
+
+@pytest.mark.parametrize("plain_layer", [True, False])
+@pytest.mark.parametrize("n", [3000, 150000])
+def test_a_captured_layer_follows_its_weight(plain_layer, n):
+    """A layer captured into a graph makes its own packed weight and affine map on each replay: it follows in-place updates,
+    and what eager passes keep, use or drop in between does not matter to it (one launch per layer, and two)."""
+    B, shape = 1, [32, 2048, 32]
+    rng = np.random.default_rng(n)
+    feat = torch.tensor(rng.standard_normal((n, 16)), dtype=torch.float32).half().to(G.DEV)
+    x = sphconv.SparseConvTensor(feat, shape, B, indices=G.t(_cells(rng, n, B, shape)))
+    conv = sphconv.SubMConv3d(16, 32, 3)
+    net = (conv if plain_layer else sphconv.Sequential(conv, torch.nn.BatchNorm1d(32), torch.nn.ReLU())).to(G.DEV).half().eval()
+    fresh = lambda: sphconv.SparseConvTensor(x.feature, shape, B, z_idx=x.z_idx, z_ptr=x.z_ptr, row_cols=x.row_cols)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad():
+        with torch.cuda.stream(side):
+            net(fresh())                                   # the stream now has kept copies
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            out = net(fresh()).feature
+        for i in range(4):
+            conv.weight.mul_(-1.5)                         # the kept copies are outdated
+            if not plain_layer:
+                net[1].running_mean.add_(0.25)
+            with torch.cuda.stream(side):
+                side.wait_stream(torch.cuda.default_stream())
+                net(fresh())                               # ... and replaced
+            want = net(fresh()).feature
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), i
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), i

@@ -158,7 +158,7 @@ def _affine_of(bn):
     x = torch.linspace(-2, 2, 5 * bn.num_features).view(5, bn.num_features)
     with torch.no_grad():
         want = bn(x)
-        scale, shift = modules._bn_affine(bn)
+        scale, shift = modules._bn_affine(bn, None)
     torch.testing.assert_close(x * scale + shift, want, rtol=1e-5, atol=1e-5)     # a few fp32 roundings
 
 
@@ -201,7 +201,7 @@ def test_modules_with_hooks_are_called_not_folded():
         assert seq._fusable_tail([conv, bn, act], 0) == (2, bn, True)
 
 
-def test_kept_affine_map_belongs_to_the_tensors_and_the_stream(monkeypatch):
+def test_kept_affine_map_belongs_to_the_tensors_and_the_stream():
     """The affine map kept on a BatchNorm1d is not taken for another tensor that the allocator put at the same address, nor
     on a stream that is not ordered behind its computation; a copy of the module has its own."""
     import copy
@@ -212,28 +212,18 @@ def test_kept_affine_map_belongs_to_the_tensors_and_the_stream(monkeypatch):
         memory[:] = value
         bn.weight = torch.nn.Parameter(torch.from_numpy(memory))
         with torch.no_grad():
-            torch.testing.assert_close(modules._bn_affine(bn)[0], torch.full((4,), value), rtol=1e-4, atol=0)
+            torch.testing.assert_close(modules._bn_affine(bn, None)[0], torch.full((4,), value), rtol=1e-4, atol=0)
     with torch.no_grad():
-        first = modules._bn_affine(bn)[0]
-        assert modules._bn_affine(bn)[0] is first
+        first = modules._bn_affine(bn, None)[0]
+        assert modules._bn_affine(bn, None)[0] is first
         twin = copy.deepcopy(bn)
         twin.running_var.mul_(4.0)
         _affine_of(twin)
-        assert modules._bn_affine(bn)[0] is first
+        assert modules._bn_affine(bn, None)[0] is first
 
-    class OnGpu(torch.Tensor):                  # as far as the look-up can tell
-        is_cuda = True
-
-    stream = [7]
-    monkeypatch.setattr(modules.L, "stream", lambda device=None: stream[0])
-    bn._buffers["running_mean"] = bn.running_mean.as_subclass(OnGpu)
-    with torch.no_grad():
-        on7 = modules._bn_affine(bn)[0]
-        stream[0] = 8
-        on8 = modules._bn_affine(bn)[0]
-        assert on8 is not on7 and modules._bn_affine(bn)[0] is on8
-        stream[0] = 7
-        assert modules._bn_affine(bn)[0] is on7
+        on7 = modules._bn_affine(bn, 7)[0]
+        on8 = modules._bn_affine(bn, 8)[0]
+        assert on8 is not on7 and modules._bn_affine(bn, 8)[0] is on8 and modules._bn_affine(bn, 7)[0] is on7
 
 
 def test_a_count_started_ahead_outlives_the_tables_of_geometries(monkeypatch):
@@ -302,6 +292,7 @@ def test_threads_on_one_stream_have_scratch_books_of_their_own(monkeypatch):
     import threading
     from sphconv_amd import rulebook
     monkeypatch.setattr(rulebook.L, "stream", lambda device=None: 5)
+    monkeypatch.setattr(rulebook.L, "capturing", lambda: False)
     cpu = torch.device("cpu")
     mine = rulebook._scratch_book(100, 27, cpu)
     assert rulebook._scratch_book(300, 27, cpu) is mine and mine.native.rows == 300
@@ -313,3 +304,53 @@ def test_threads_on_one_stream_have_scratch_books_of_their_own(monkeypatch):
     assert mine.native.rows == 300 and theirs[0].native.rows == 200
     bigger = rulebook._scratch_book((1 << 17) + 1, 27, cpu)
     assert bigger is not mine and rulebook._scratch_book(10, 27, cpu) is bigger
+
+
+def test_nothing_is_kept_or_reused_while_a_graph_is_captured(monkeypatch):
+    """Under capture nothing is computed yet, memory is the graph's, and what it reads must not be given back later: packed
+    weights, affine maps and scratch books are the graph's own."""
+    from sphconv_amd import rulebook, sphconv_cuda as ext
+    capturing = [False]
+    monkeypatch.setattr(L, "capturing", lambda: capturing[0])
+    monkeypatch.setattr(L, "stream", lambda device=None: 11)
+    made = []
+
+    class Host:
+        def pack_weight(self, *a):
+            made.append(torch.zeros(1))
+            return made[-1]
+
+    native = L.host()
+    weight = torch.nn.Parameter(torch.zeros((27, 4, 8)))
+    cpu = torch.device("cpu")
+    with monkeypatch.context() as m, torch.no_grad():
+        m.setattr(L, "host", lambda: Host())
+        ext.invalidate_packed(weight)
+        kept = ext._packed_weight(weight, False, cache=True)
+        assert ext._kept_packed(weight) is kept and ext._packed_weight(weight, False, cache=True) is kept
+        capturing[0] = True
+        assert ext._kept_packed(weight) is None
+        own = ext._packed_weight(weight, False, cache=True)
+        assert own is not kept and ext._packed_weight(weight, False, cache=True) is not own
+        capturing[0] = False
+        assert ext._kept_packed(weight) is kept
+        ext.invalidate_packed(weight)
+    assert L.host() is native
+    book = rulebook._scratch_book(50, 27, cpu)
+    capturing[0] = True
+    own = rulebook._scratch_book(50, 27, cpu)
+    assert own is not book and own.native.address != book.native.address and rulebook._scratch_book(50, 27, cpu) is not own
+    capturing[0] = False
+    assert rulebook._scratch_book(50, 27, cpu) is book
+
+    bn = torch.nn.BatchNorm1d(4).eval()
+    rows = torch.zeros(3, 4)
+    with torch.no_grad():
+        first = modules._bn_affine(bn, 11)[0]
+        on_gpu = type("OnGpu", (), {"is_cuda": True, "device": torch.device("cuda", 0)})
+        assert modules._keeps_on(on_gpu) == 11 and modules._keeps_on(rows) is None
+        capturing[0] = True
+        assert modules._keeps_on(on_gpu) is False
+        own = modules._bn_affine(bn, False)[0]
+        assert own is not first and modules._bn_affine(bn, False)[0] is not own
+        assert modules._bn_affine(bn, 11)[0] is first
