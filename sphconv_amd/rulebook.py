@@ -106,6 +106,9 @@ class _Geometry:
         self.native = L.host().Geometry(batch, self.in_shape, self.out_shape, self.kernel, self.stride, self.padding,
                                         self.dilation)
 
+    def __reduce__(self):
+        return _geometry, (self.batch, self.in_shape, self.out_shape, self.kernel, self.stride, self.padding, self.dilation)
+
 
 _GEOMETRIES = {}
 
@@ -200,12 +203,17 @@ class RuleBook:
     def fwd(self) -> _Buffers:
         """The forward book (stationary on output rows); a book made with ``lazy=True`` is built here."""
         if self._fwd is None:
-            self._fwd = self._build(False)
+            self._fwd = self._convert(False) if self._from_padded is not None else self._build(False)
         return self._fwd
 
     @fwd.setter
     def fwd(self, buf):
         self._fwd = buf
+
+    def __getstate__(self):
+        """What a copy or a saved module takes along: the coordinates, not the pairs, which it makes again when it needs
+        them."""
+        return dict(self.__dict__, _fwd=None, _bwd=None)
 
     @property
     def built(self) -> bool:

@@ -295,3 +295,27 @@ def test_a_captured_layer_follows_its_weight(plain_layer, n):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want), i
+
+
+@pytest.mark.parametrize("training,key", [(True, None), (False, None), (False, "k")])
+@pytest.mark.parametrize("stride", [1, 2])
+def test_a_layer_that_has_run_is_copied_and_saved(tmp_path, training, key, stride):
+    import copy
+    rng = np.random.default_rng(stride)
+    feat = torch.tensor(rng.standard_normal((900, 16)), dtype=torch.float32).to(G.DEV)
+    idx = G.t(_cells(rng, 900, 2, [12, 20, 16]))
+    conv = (sphconv.SubMConv3d(16, 32, 3, indice_key=key) if stride == 1 else
+            sphconv.SparseConv3d(16, 32, 3, stride=2, padding=1, indice_key=key)).to(G.DEV).train(training)
+    make = lambda: sphconv.SparseConvTensor(feat, [12, 20, 16], 2, indices=idx)
+    with torch.set_grad_enabled(training):
+        want = conv(make()).feature
+        twin = copy.deepcopy(conv)
+        torch.save(conv, tmp_path / "conv.pt")
+        saved = torch.load(tmp_path / "conv.pt", weights_only=False)
+        for c in (twin, saved):
+            assert torch.equal(c.rule_size, conv.rule_size)
+            assert torch.equal(c(make()).feature, want)
+    padded = RuleBook.from_padded(*conv.rule_book.padded((2, 2)), 900, want.shape[0])
+    again = copy.deepcopy(padded)
+    w = conv.weight.detach().view(27, 16, 32)
+    assert torch.equal(ext.rule_conv(feat, w, again, None, want.shape[0]), ext.rule_conv(feat, w, padded, None, want.shape[0]))

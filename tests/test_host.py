@@ -354,3 +354,17 @@ def test_nothing_is_kept_or_reused_while_a_graph_is_captured(monkeypatch):
         own = modules._bn_affine(bn, False)[0]
         assert own is not first and modules._bn_affine(bn, False)[0] is not own
         assert modules._bn_affine(bn, 11)[0] is first
+
+
+def test_rule_books_can_be_copied_and_saved():
+    """A module that has run holds its rule book, and is copied (for a moving average of its weights) and saved with it."""
+    import copy
+    import pickle
+    z_idx, z_ptr = torch.zeros(5, dtype=torch.int32), torch.full((1, 4, 4), 5, dtype=torch.int32)
+    book = sphconv_amd.RuleBook(z_idx, z_ptr, z_idx, z_ptr, 1, [4, 4, 8], [4, 4, 8], [3, 3, 3], [1, 1, 1], [1, 1, 1],
+                                [1, 1, 1], True)
+    conv = sphconv_amd.SubMConv3d(4, 8, 3)
+    conv.__dict__["rule_book"] = book
+    for twin in (copy.deepcopy(conv).rule_book, pickle.loads(pickle.dumps(book))):
+        assert twin is not book and twin.z_idx is twin.oz_idx and torch.equal(twin.z_ptr, z_ptr) and not twin.built
+        assert twin.kernel == [3, 3, 3] and twin.batch == 1 and twin.mirrored() and twin._geometry is book._geometry
