@@ -74,7 +74,7 @@ class ToDenseFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, feature, z_idx, z_ptr, shape: List[int]):
         ctx.save_for_backward(z_idx, z_ptr)
-        B, C, S0, S1, S2 = shape
+        B, C, S0, S1, S2 = (int(s) for s in shape)
         if feature.is_cuda and feature.element_size() <= 4:
             return ext.L.host().to_dense_channels_first(feature, z_idx, z_ptr, B, C, S0, S1, S2)
         res = torch.zeros((B, S0, S1, S2, C), device=feature.device, dtype=feature.dtype)

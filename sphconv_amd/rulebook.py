@@ -114,12 +114,13 @@ _GEOMETRIES = {}
 
 
 def _geometry(batch, in_shape, out_shape, kernel, stride, padding, dilation) -> _Geometry:
+    batch = int(batch)
     key = (batch, *in_shape, *out_shape, *kernel, *stride, *padding, *dilation)
     g = _GEOMETRIES.get(key)
     if g is None:
         if len(_GEOMETRIES) >= 4096:                     # a program with ever new shapes: start over
             _GEOMETRIES.clear()
-        g = _Geometry(int(batch), *(tuple(int(v) for v in x) for x in (in_shape, out_shape, kernel, stride, padding, dilation)))
+        g = _Geometry(batch, *(tuple(int(v) for v in x) for x in (in_shape, out_shape, kernel, stride, padding, dilation)))
         _GEOMETRIES[key] = g
     return g
 
@@ -130,6 +131,7 @@ _LAYERS = {}
 
 def layer_geometry(batch, D, W, H, kernel, stride, padding, dilation, subm):
     """-> (geometry, output shape) of a layer on a ``[batch, D, W, H]`` grid."""
+    batch = int(batch)
     key = (batch, D, W, H, kernel, stride, padding, dilation, subm)
     hit = _LAYERS.get(key)
     if hit is None:

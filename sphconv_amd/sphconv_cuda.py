@@ -119,10 +119,10 @@ def init_tensor(feature: torch.Tensor, indicesBZYX: torch.Tensor, batchSize: int
 
 def _init_tensor(feature, indices, batch, shape):
     """-> [outFeature, zIndices, zPtr, permutation, columns of the rows]"""
-    S0, S1, S2 = shape
-    out, z_idx, z_ptr, permutation, cols, outside, dup = L.host().init_tensor(feature, indices, batch, S0, S1, S2)
+    size = [int(batch), *(int(s) for s in shape)]
+    out, z_idx, z_ptr, permutation, cols, outside, dup = L.host().init_tensor(feature, indices, *size)
     if outside:
-        raise ValueError("voxel coordinate outside batch/spatial shape %s" % ([int(batch), int(S0), int(S1), int(S2)],))
+        raise ValueError("voxel coordinate outside batch/spatial shape %s" % size)
     if dup:
         raise ValueError("duplicate voxel coordinates")
     return [out, z_idx, z_ptr, permutation, cols]

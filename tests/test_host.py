@@ -368,3 +368,23 @@ def test_rule_books_can_be_copied_and_saved():
     for twin in (copy.deepcopy(conv).rule_book, pickle.loads(pickle.dumps(book))):
         assert twin is not book and twin.z_idx is twin.oz_idx and torch.equal(twin.z_ptr, z_ptr) and not twin.built
         assert twin.kernel == [3, 3, 3] and twin.batch == 1 and twin.mirrored() and twin._geometry is book._geometry
+
+
+@pytest.mark.parametrize("batch", [2, 2.0, torch.tensor(2), __import__("numpy").float32(2)])
+def test_batch_sizes_and_shapes_of_any_number_type(monkeypatch, batch):
+    """A batch size is often what a reduction over the coordinates returned."""
+    from sphconv_amd import rulebook, sphconv_cuda as ext
+    got = []
+
+    class Host:
+        def init_tensor(self, feature, indices, *size):
+            got.append(size)
+            return feature, None, None, None, None, 0, 0
+
+    with monkeypatch.context() as m:
+        m.setattr(L, "host", lambda: Host())
+        ext.init_tensor(torch.zeros(3, 4), torch.zeros((3, 4), dtype=torch.int32), batch, [4.0, 5, 6])
+    assert got == [(2, 4, 5, 6)] and all(type(v) is int for v in got[0])
+    layer = lambda: rulebook.layer_geometry(batch, 4, 5, 6, (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1), True)[0]
+    assert layer() is layer() is rulebook._geometry(2, [4, 5, 6], [4, 5, 6], (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1))
+    assert layer().z_shape == (2, 4, 5)
