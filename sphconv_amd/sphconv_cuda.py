@@ -242,6 +242,8 @@ def _conv_packed(feature, packed, kdim: int, ndim: int, book, outNNZ: int, scale
     """The convolution of ``rule_conv`` once its weight is in fragment order."""
     if book.out_rows != int(outNNZ):
         raise L.SphconvError("rules hold %d output rows, call says %d" % (book.out_rows, int(outNNZ)))
+    if feature.dim() != 2 or feature.shape[1] != kdim:
+        raise L.SphconvError("feature [N,iC] / weight [KV,iC,oC] mismatch: %s vs iC = %d" % (tuple(feature.shape), kdim))
     if not book.built and feature.is_cuda and feature.shape[0] == book.in_rows:
         out = book.fused_forward(feature, packed, kdim, ndim, scale, shift, relu)
         if out is not None:

@@ -388,3 +388,32 @@ def test_batch_sizes_and_shapes_of_any_number_type(monkeypatch, batch):
     layer = lambda: rulebook.layer_geometry(batch, 4, 5, 6, (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1), True)[0]
     assert layer() is layer() is rulebook._geometry(2, [4, 5, 6], [4, 5, 6], (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1))
     assert layer().z_shape == (2, 4, 5)
+
+
+def test_rows_of_another_width_do_not_reach_the_kernel(monkeypatch):
+    """A module that keeps its packed weight knows its channels from the tensor's C; what is convolved are its rows, which
+    somebody may have replaced."""
+    from types import SimpleNamespace
+    from sphconv_amd import sphconv_cuda as ext
+    z_idx, z_ptr = torch.zeros(3, dtype=torch.int32), torch.full((1, 2, 2), 3, dtype=torch.int32)
+    conv = sphconv_amd.SubMConv3d(8, 16, 3).eval()
+    launched = []
+    host = SimpleNamespace(rules_conv=lambda *a: launched.append(a), conv_apply=lambda *a: launched.append(a))
+    book = sphconv_amd.RuleBook(z_idx, z_ptr, z_idx, z_ptr, 1, [2, 2, 4], [2, 2, 4], [3, 3, 3], [1, 1, 1], [1, 1, 1], [1, 1, 1], True)
+    book.fwd = SimpleNamespace(groups=True, native=None)
+    monkeypatch.setattr(conv, "_rules", lambda *a, **k: (z_idx, z_ptr, book, None, [1, 1]))
+    monkeypatch.setattr(ext, "_kept_packed", lambda *a: torch.zeros(4))
+    x = sphconv_amd.SparseConvTensor(torch.zeros(3, 8), [2, 2, 4], 1, z_idx=z_idx, z_ptr=z_ptr)
+    conv._layer(x)
+    monkeypatch.setattr(L, "host", lambda: host)
+    monkeypatch.setattr(L, "stream", lambda *a: 0)
+    monkeypatch.setattr(L, "capturing", lambda: False)
+    for rows in (torch.zeros(3, 4), torch.zeros(3, 8, 1)):
+        x.feature = rows
+        with torch.no_grad(), pytest.raises(sphconv_amd.SphconvError, match="mismatch"):
+            conv(x)
+    assert not launched
+    x.feature = torch.zeros(3, 8)
+    host.conv_apply = lambda *a: torch.zeros(3, 16)
+    with torch.no_grad():
+        assert conv(x).feature.shape == (3, 16)
