@@ -110,15 +110,15 @@ def init_tensor(feature: torch.Tensor, indicesBZYX: torch.Tensor, batchSize: int
     fiber are ordered by ascending S2 (one legal order of the reference's output).
     Two counts the last kernel reports to the host check the coordinates (the reference checks nothing:
     coordinates outside the grid or duplicated ones corrupt its output)."""
-    if indicesBZYX.dtype != torch.int32 or indicesBZYX.dim() != 2 or indicesBZYX.shape[1] != 4:
-        raise ValueError("indices must be int32 [NNZ,4] (b,s0,s1,s2)")
-    if feature.dim() != 2 or feature.shape[0] != indicesBZYX.shape[0]:
-        raise ValueError("feature must be [NNZ,C]")
     return _init_tensor(feature, indicesBZYX, batchSize, spatialShape)[:4]
 
 
 def _init_tensor(feature, indices, batch, shape):
     """-> [outFeature, zIndices, zPtr, permutation, columns of the rows]"""
+    if indices.dtype != torch.int32 or indices.dim() != 2 or indices.shape[1] != 4:
+        raise ValueError("indices must be int32 [NNZ,4] (b,s0,s1,s2)")
+    if feature.dim() != 2 or feature.shape[0] != indices.shape[0]:
+        raise ValueError("feature must be [NNZ,C]")
     size = [int(batch), *(int(s) for s in shape)]
     out, z_idx, z_ptr, permutation, cols, outside, dup = L.host().init_tensor(feature, indices, *size)
     if outside:

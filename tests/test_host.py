@@ -417,3 +417,19 @@ def test_rows_of_another_width_do_not_reach_the_kernel(monkeypatch):
     host.conv_apply = lambda *a: torch.zeros(3, 16)
     with torch.no_grad():
         assert conv(x).feature.shape == (3, 16)
+
+
+@pytest.mark.parametrize("call", ["init_tensor", "function"])
+def test_coordinates_and_rows_are_checked_whoever_asks(monkeypatch, call):
+    """The autograd function of the public API is called by programs too: what the kernel reads is checked there as well."""
+    from types import SimpleNamespace
+    from sphconv_amd import sphconv_cuda as ext
+    from sphconv_amd.functional import InitTensorFunction
+    asked = []
+    monkeypatch.setattr(L, "host", lambda: SimpleNamespace(init_tensor=lambda *a: asked.append(a)))
+    make = ext.init_tensor if call == "init_tensor" else InitTensorFunction.apply
+    rows, indices = torch.zeros(5, 3), torch.zeros((5, 4), dtype=torch.int32)
+    for f, i in ((rows[:4], indices), (rows, indices.long()), (rows, indices[:, :3]), (rows, indices[0]), (rows[0], indices)):
+        with pytest.raises(ValueError, match="must be"):
+            make(f, i, 1, [2, 2, 2])
+    assert not asked
