@@ -408,6 +408,8 @@ Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf
     const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous(), d_out = d_out_.contiguous();
     const int ic = (int)feature.size(1), oc = (int)d_out.size(1);
+    // the kernel checks the rows that a book's groups gather, and takes those the book is stationary on as given
+    if ((transposed ? feature : d_out).size(0) < buf.book.rows) raise("fewer rows than the rule book holds");
     const int64_t n = (int64_t)sph_wgrad_partial_elems(buf.kv, ic, oc, buf.book.rows);
     const Tensor partial = at::empty({n > 0 ? n : 1}, feature.options().dtype(at::kFloat).requires_grad(false));
     const Tensor dw = at::empty({buf.kv, ic, oc}, feature.options().dtype(f32 ? at::kFloat : feature.scalar_type()).requires_grad(false));

@@ -307,7 +307,10 @@ def rule_conv_d_weight(feature: torch.Tensor, d_featureOut: torch.Tensor, rules,
         raise L.SphconvError("d_weight comes in the features' type or in float32, not %s" % out_dtype)
     # From the book with fewer tiles, if dgrad has made the transposed one: the same pairs lie in fewer, fuller groups
     # there (a strided layer on scattered voxels has more output than input rows, its forward groups five pairs of 16).
-    transposed = book.transposed_groups_built() and book.in_rows < book.out_rows
+    # (Its kernel takes the features for its stationary rows as they are; gathered rows are checked in the kernel.)
+    transposed = book.transposed_groups_built() and book.in_rows < book.out_rows and feature.shape[0] == book.in_rows
+    if d_out.shape[0] < book.out_rows:
+        raise L.SphconvError("rules hold %d output rows, their gradient %d" % (book.out_rows, d_out.shape[0]))
     return L.host().conv_wgrad(feature, d_out, book.grouped(transposed).native, transposed, out_dtype == torch.float32)
 
 

@@ -319,3 +319,21 @@ def test_a_layer_that_has_run_is_copied_and_saved(tmp_path, training, key, strid
     again = copy.deepcopy(padded)
     w = conv.weight.detach().view(27, 16, 32)
     assert torch.equal(ext.rule_conv(feat, w, again, None, want.shape[0]), ext.rule_conv(feat, w, padded, None, want.shape[0]))
+
+
+def test_weight_gradient_of_fewer_rows_than_the_book_holds():
+    """Features that end early: pairs beyond them count for nothing, whichever books exist; a gradient that does is refused."""
+    rng = np.random.default_rng(4)
+    case = G.build_case(_cells(rng, 300, 1, [12, 60, 40]), 1, [12, 60, 40], [3, 3, 3], [2, 2, 2], [1, 1, 1], False)
+    book = case["book"]
+    f, d = torch.randn((300, 16), device=G.DEV), torch.randn((book.out_rows, 24), device=G.DEV)
+    book.transposed()
+    assert book.in_rows < book.out_rows and book.transposed_groups_built()
+    padded = torch.cat([f[:170], torch.zeros_like(f[170:])])
+    torch.testing.assert_close(ext.rule_conv_d_weight(f[:170], d, book, None), ext.rule_conv_d_weight(padded, d, book, None),
+                               rtol=1e-5, atol=1e-4)
+    for transposed, a, b in ((True, f[:170], d), (False, f, d[:-1])):
+        with pytest.raises(L.SphconvError, match="fewer rows"):
+            L.host().conv_wgrad(a, b, book.grouped(transposed).native, transposed, False)
+    with pytest.raises(L.SphconvError, match="output rows"):
+        ext.rule_conv_d_weight(f, d[:-1], book, None)

@@ -433,3 +433,20 @@ def test_coordinates_and_rows_are_checked_whoever_asks(monkeypatch, call):
         with pytest.raises(ValueError, match="must be"):
             make(f, i, 1, [2, 2, 2])
     assert not asked
+
+
+def test_weight_gradients_take_the_book_their_rows_fit(monkeypatch):
+    """The gradient's kernel reads as many rows as its book is stationary on: fewer features than that keep to the forward
+    book, which gathers them and checks each, and fewer gradient rows are refused."""
+    from types import SimpleNamespace
+    from sphconv_amd import sphconv_cuda as ext
+    z_ptr = torch.full((1, 2, 2), 3, dtype=torch.int32)
+    book = sphconv_amd.RuleBook(torch.zeros(3, dtype=torch.int32), z_ptr, torch.zeros(6, dtype=torch.int32), z_ptr, 1, [2, 2, 4],
+                                [2, 2, 4], [3, 3, 3], [1, 1, 1], [1, 1, 1], [1, 1, 1], False)
+    book.fwd, book._bwd = (SimpleNamespace(groups=True, native=side) for side in ("forward", "transposed"))
+    monkeypatch.setattr(L, "host", lambda: SimpleNamespace(conv_wgrad=lambda f, d, native, transposed, f32: (native, transposed)))
+    d_out = torch.zeros(6, 4)
+    assert ext.rule_conv_d_weight(torch.zeros(3, 2), d_out, book, None) == ("transposed", True)
+    assert ext.rule_conv_d_weight(torch.zeros(2, 2), d_out, book, None) == ("forward", False)
+    with pytest.raises(sphconv_amd.SphconvError, match="output rows"):
+        ext.rule_conv_d_weight(torch.zeros(3, 2), d_out[:5], book, None)
