@@ -364,8 +364,11 @@ struct OutCoords {
 };
 
 // ---- convolution --------------------------------------------------------------------------------
-const sph_epilogue *epilogue(sph_epilogue &e, const OptTensor &scale, const OptTensor &shift, bool relu)
+const sph_epilogue *epilogue(sph_epilogue &e, const OptTensor &scale, const OptTensor &shift, bool relu, int ndim)
 {
+    for (const OptTensor *t : {&scale, &shift}) // the kernels read one float per output channel
+        if (*t && ((*t)->scalar_type() != at::kFloat || (*t)->numel() < ndim))
+            raise("scale and shift must be float32 with one value per output channel (" + std::to_string(ndim) + ")");
     e.scale = ptr<const float>(scale);
     e.shift = ptr<const float>(shift);
     e.relu = relu;
@@ -380,7 +383,7 @@ Tensor conv_apply(const Tensor &feature_, const Tensor &packed, int kdim, int nd
     const Tensor out = at::empty({buf.book.rows, ndim}, feature.options().requires_grad(false));
     sph_epilogue e;
     check(sph_conv_apply((sph_dtype)dtype_code(feature.scalar_type()), ptr(feature), (int)feature.size(0), kdim, packed.data_ptr(), ndim,
-                         &buf.book, epilogue(e, scale, shift, relu), out.data_ptr(), here.stream));
+                         &buf.book, epilogue(e, scale, shift, relu, ndim), out.data_ptr(), here.stream));
     return out;
 }
 
@@ -397,7 +400,7 @@ py::object rules_conv(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz
     const int rc = sph_rules_conv((const int32_t *)z_idx.data_ptr(), (const int32_t *)z_ptr.data_ptr(), (int)z_idx.size(0),
                                   (const int32_t *)oz_idx.data_ptr(), (const int32_t *)oz_ptr.data_ptr(), out_rows, &geom.g, &buf.book,
                                   flags, row_table(row_cols, out_rows), (sph_dtype)dtype_code(feature.scalar_type()), ptr(feature), kdim,
-                                  packed.data_ptr(), ndim, epilogue(e, scale, shift, relu), out.data_ptr(), here.stream);
+                                  packed.data_ptr(), ndim, epilogue(e, scale, shift, relu, ndim), out.data_ptr(), here.stream);
     if (rc == SPH_ERR_UNSUPPORTED) return py::none();
     check(rc);
     return py::cast(out);
@@ -451,6 +454,8 @@ Tensor to_dense_channels_first(const Tensor &feature_, const Tensor &z_idx, cons
     const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous();
     if (feature.size(1) != C || z_ptr.numel() != (int64_t)B * S0 * S1) raise("rows and pointers do not match the dense shape");
+    if (z_idx.scalar_type() != at::kInt || z_ptr.scalar_type() != at::kInt || z_idx.numel() < feature.size(0))
+        raise("z_idx and z_ptr must be int32, with an entry of z_idx per row");
     const Tensor out = at::empty({B, C, S0, S1, S2}, feature.options().requires_grad(false));
     check(sph_to_dense_channels_first(ptr(feature), ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), (int)feature.size(0), B * S0 * S1, S0 * S1,
                                       S2, C, (int)feature.element_size(), out.data_ptr(), here.stream));

@@ -19,7 +19,7 @@ class SimpleVoxel(nn.Module):
         if (features.is_cuda and features.dtype == torch.float32 and num_voxels.dtype == torch.int32 and features.dim() == 3
                 and num_voxels.shape == features.shape[:1] and not features.requires_grad and features.is_contiguous()
                 and num_voxels.is_contiguous() and num_voxels.device == features.device
-                and 0 < self.num_input_features <= features.shape[2] and plain(features) and plain(num_voxels)):
+                and 0 < self.num_input_features <= features.shape[2] and features.shape[1] > 0 and plain(features) and plain(num_voxels)):
             return L.host().voxel_mean(features, num_voxels, self.num_input_features)      # one kernel
         # features [voxels, max_points, >=num_input_features], unused slots are zero
         points_mean = features[:, :, :self.num_input_features].sum(dim=1, keepdim=False) \

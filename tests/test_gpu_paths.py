@@ -337,3 +337,23 @@ def test_weight_gradient_of_fewer_rows_than_the_book_holds():
             L.host().conv_wgrad(a, b, book.grouped(transposed).native, transposed, False)
     with pytest.raises(L.SphconvError, match="output rows"):
         ext.rule_conv_d_weight(f, d[:-1], book, None)
+
+
+def test_small_arrays_are_checked_before_the_launch():
+    """What the kernels read beside the rows: one float per output channel of scale and shift, an index per row."""
+    rng = np.random.default_rng(0)
+    idx = G.t(_cells(rng, 200, 1, [6, 8, 10]))
+    x = sphconv.SparseConvTensor(torch.randn((200, 16), device=G.DEV), [6, 8, 10], 1, indices=idx)
+    book = RuleBook.build_subm(x.z_idx, x.z_ptr, 1, [6, 8, 10], [3, 3, 3])
+    w = torch.randn((27, 16, 32), device=G.DEV)
+    good = torch.rand(32, device=G.DEV)
+    assert ext.rule_conv(x.feature, w, book, None, 200, scale=good, shift=good).shape == (200, 32)
+    for bad in (good[:31].contiguous(), good.half(), good.double()):
+        for kw in ({"scale": bad}, {"scale": good, "shift": bad}):
+            with pytest.raises(L.SphconvError, match="one value per output channel"):
+                ext.rule_conv(x.feature, w, book, None, 200, **kw)
+    for z_idx, z_ptr in ((x.z_idx[:199], x.z_ptr), (x.z_idx.long(), x.z_ptr), (x.z_idx, x.z_ptr.long())):
+        with pytest.raises(L.SphconvError, match="int32"):
+            sphconv.SparseConvTensor(x.feature, [6, 8, 10], 1, z_idx=z_idx, z_ptr=z_ptr).dense()
+    empty = SimpleVoxel(4)(torch.zeros((7, 0, 4), device=G.DEV), torch.ones(7, device=G.DEV, dtype=torch.int32), None)
+    assert torch.equal(empty, torch.zeros((7, 4), device=G.DEV))
