@@ -167,12 +167,13 @@ __device__ __forceinline__ void acc_add4(uint32_t *p, typename Traits<DT>::acc4 
 // = book order.  Indices run two blocks ahead; gathers and weight fragments are
 // requested three to four groups before their use, their address arithmetic is
 // interleaved with the MFMAs.
-// What bounds the loop, 64->64 bf16 on 5890 tiles of 34 groups (93.6 us with inputs in cache), timed without a part at a
-// time: without the fragment loads 70.0 us, without the row loads 81.5, sums in registers instead of LDS 91.4, vector
-// additions instead of the MFMAs 96.8, one row stored per tile 86.0; without fragment loads and LDS 59.5, MFMAs alone 47.2.
-// All fragments from offset 0, the same loads served by the nearest cache, are 90.8: it is the CU's vector memory return
-// path (8 KiB of weight fragments + 2 KiB of rows per group), not a miss behind it; the LDS read-MFMA-write chain lies
-// under it and shows once the loads are gone.
+// What bounds the loop, 64->64 bf16 on 5890 tiles of 34 groups, inputs from HBM (124 us; from cache 94): timed without one
+// part at a time, without the fragment loads 88 us, with all of them from offset 0 (the same loads, served by the nearest
+// cache) 113, without the row loads 112, one row stored per tile 105, sums in registers instead of LDS 124.5, vector
+// additions instead of the MFMAs 125; without fragment and row loads 83, without fragments and LDS 81, MFMAs alone 62.
+// So it is the CU's vector memory return path (8 KiB of weight fragments + 2 KiB of rows per group), two thirds of its
+// share whatever cache serves it, then the store; neither the LDS chain nor the matrix cores.  int8 (2376 tiles, of which
+// the chip holds 1024 at once, 34.9 us) has no such part: fragments 31.8, LDS 31.1, store 30.5, MFMAs alone 20.7.
 // ---------------------------------------------------------------------------
 constexpr int kBlk = 4; // groups per pipeline block (4 x 16 index entries = one 64-lane load)
 constexpr int kRsrcFlags = 0x00020000; // raw buffer descriptor, 32-bit data format
