@@ -111,7 +111,7 @@ PinnedWords &pinned()
 
 // A word set to -1 that a kernel on `st` will overwrite.  wait() returns as soon as the store arrives, without an
 // event (recording one costs 4.6 us) and without waiting for what was enqueued behind that kernel; should the store
-// not arrive within a few milliseconds the stream is waited for instead, which also reports an error it holds.
+// not arrive within 20 ms the stream is waited for instead, which also reports an error it holds.
 class HostWord {
     int64_t *w;
     hipStream_t st;
