@@ -172,7 +172,7 @@ def stream(device=None):
 
 # Whether torch's current stream records a graph.  What is computed then exists only while the graph replays, in memory of
 # the graph's, and what the graph reads has to live as long as it does: nothing is kept from call to call.
-capturing = torch.cuda.is_current_stream_capturing
+capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
 
 
 _IS_CURRENT = contextlib.nullcontext()

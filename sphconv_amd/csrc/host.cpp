@@ -30,9 +30,9 @@ namespace {
 
 PyObject *g_error = nullptr; // the package's SphconvError
 
-[[noreturn]] void raise(const std::string &msg)
+[[noreturn]] void raise(const std::string &msg, PyObject *type = nullptr)
 {
-    PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, msg.c_str());
+    PyErr_SetString(type ? type : g_error ? g_error : PyExc_RuntimeError, msg.c_str());
     throw py::error_already_set();
 }
 void check(int rc)
@@ -375,9 +375,18 @@ const sph_epilogue *epilogue(sph_epilogue &e, const OptTensor &scale, const OptT
     return &e;
 }
 
+// the kernels take the rows to be as wide as the weight says
+void check_rows(const Tensor &feature, int kdim)
+{
+    if (feature.dim() != 2 || feature.size(1) != kdim)
+        raise("feature [N,iC] / weight [KV,iC,oC] mismatch: iC = " + std::to_string(kdim) + ", rows of " +
+              std::to_string(feature.dim() ? feature.size(-1) : 0));
+}
+
 Tensor conv_apply(const Tensor &feature_, const Tensor &packed, int kdim, int ndim, BookBuffers &buf, const OptTensor &scale,
                   const OptTensor &shift, bool relu)
 {
+    check_rows(feature_, kdim);
     const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous();
     const Tensor out = at::empty({buf.book.rows, ndim}, feature.options().requires_grad(false));
@@ -392,8 +401,10 @@ py::object rules_conv(const Tensor &z_idx, const Tensor &z_ptr, const Tensor &oz
                       BookBuffers &buf, int flags, const OptTensor &row_cols, const Tensor &feature_, const Tensor &packed, int kdim,
                       int ndim, const OptTensor &scale, const OptTensor &shift, bool relu)
 {
+    check_rows(feature_, kdim);
     const OnDevice here(feature_);
     const Tensor feature = feature_.contiguous();
+    if (feature.size(0) != z_idx.size(0)) raise("the rows and their coordinates differ in number");
     const int out_rows = (int)oz_idx.size(0);
     const Tensor out = at::empty({out_rows, ndim}, feature.options().requires_grad(false));
     sph_epilogue e;
@@ -430,6 +441,9 @@ Tensor conv_wgrad(const Tensor &feature_, const Tensor &d_out_, BookBuffers &buf
 // -> out feature, z_idx, z_ptr, permutation, row_cols, coordinates outside the grid, duplicated coordinates
 py::tuple init_tensor(const Tensor &feature_, const Tensor &indices_, int B, int S0, int S1, int S2)
 {
+    if (indices_.scalar_type() != at::kInt || indices_.dim() != 2 || indices_.size(1) != 4)
+        raise("indices must be int32 [NNZ,4] (b,s0,s1,s2)", PyExc_ValueError);
+    if (feature_.dim() != 2 || feature_.size(0) != indices_.size(0)) raise("feature must be [NNZ,C]", PyExc_ValueError);
     const OnDevice here(indices_);
     const Tensor indices = indices_.contiguous(), feature = feature_.contiguous();
     const int n = (int)indices.size(0);

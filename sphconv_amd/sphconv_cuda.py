@@ -115,14 +115,10 @@ def init_tensor(feature: torch.Tensor, indicesBZYX: torch.Tensor, batchSize: int
 
 def _init_tensor(feature, indices, batch, shape):
     """-> [outFeature, zIndices, zPtr, permutation, columns of the rows]"""
-    if indices.dtype != torch.int32 or indices.dim() != 2 or indices.shape[1] != 4:
-        raise ValueError("indices must be int32 [NNZ,4] (b,s0,s1,s2)")
-    if feature.dim() != 2 or feature.shape[0] != indices.shape[0]:
-        raise ValueError("feature must be [NNZ,C]")
-    size = [int(batch), *(int(s) for s in shape)]
-    out, z_idx, z_ptr, permutation, cols, outside, dup = L.host().init_tensor(feature, indices, *size)
+    S0, S1, S2 = shape
+    out, z_idx, z_ptr, permutation, cols, outside, dup = L.host().init_tensor(feature, indices, int(batch), int(S0), int(S1), int(S2))
     if outside:
-        raise ValueError("voxel coordinate outside batch/spatial shape %s" % size)
+        raise ValueError("voxel coordinate outside batch/spatial shape %s" % ([int(batch), int(S0), int(S1), int(S2)],))
     if dup:
         raise ValueError("duplicate voxel coordinates")
     return [out, z_idx, z_ptr, permutation, cols]
@@ -242,8 +238,6 @@ def _conv_packed(feature, packed, kdim: int, ndim: int, book, outNNZ: int, scale
     """The convolution of ``rule_conv`` once its weight is in fragment order."""
     if book.out_rows != int(outNNZ):
         raise L.SphconvError("rules hold %d output rows, call says %d" % (book.out_rows, int(outNNZ)))
-    if feature.dim() != 2 or feature.shape[1] != kdim:
-        raise L.SphconvError("feature [N,iC] / weight [KV,iC,oC] mismatch: %s vs iC = %d" % (tuple(feature.shape), kdim))
     if not book.built and feature.is_cuda and feature.shape[0] == book.in_rows:
         out = book.fused_forward(feature, packed, kdim, ndim, scale, shift, relu)
         if out is not None:

@@ -5,6 +5,7 @@ from itertools import repeat
 from typing import Iterable, List, Sequence
 
 import torch
+from torch.autograd import forward_ad
 
 
 def out_spatial(in_spatial: Sequence[int], kernel_size: Sequence[int], stride: Sequence[int],
@@ -35,12 +36,16 @@ def _calculate_fan_in_and_fan_out(tensor: torch.Tensor):
     return tensor.size(-1) * receptive, tensor.size(-2) * receptive
 
 
+# (looked up once: a voxeliser's pass asks four times)
+_transforms_active, _is_tracing = torch._C._are_functorch_transforms_active, torch._C._is_tracing
+
+
 def plain(t: torch.Tensor) -> bool:
     """Whether an operation that is made of torch's operations (or is an autograd function) may call a kernel on ``t``
     directly instead: nobody asks for more than the values.  Not while forward-mode derivatives are carried along, a
     function transform (``vmap``, ``grad``) or a trace runs, or ``t`` is of a class with operations of its own."""
-    return (type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and not torch._C._are_functorch_transforms_active() \
-        and not torch.jit.is_tracing() and torch.autograd.forward_ad.unpack_dual(t).tangent is None
+    return (type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and not _transforms_active() and not _is_tracing() \
+        and (forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None)
 
 
 def kaiming_uniform_(tensor: torch.Tensor, a: float = 0, mode: str = "fan_in",

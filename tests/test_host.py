@@ -395,44 +395,32 @@ def test_rows_of_another_width_do_not_reach_the_kernel(monkeypatch):
     somebody may have replaced."""
     from types import SimpleNamespace
     from sphconv_amd import sphconv_cuda as ext
+    from sphconv_amd.rulebook import _Buffers
     z_idx, z_ptr = torch.zeros(3, dtype=torch.int32), torch.full((1, 2, 2), 3, dtype=torch.int32)
     conv = sphconv_amd.SubMConv3d(8, 16, 3).eval()
-    launched = []
-    host = SimpleNamespace(rules_conv=lambda *a: launched.append(a), conv_apply=lambda *a: launched.append(a))
     book = sphconv_amd.RuleBook(z_idx, z_ptr, z_idx, z_ptr, 1, [2, 2, 4], [2, 2, 4], [3, 3, 3], [1, 1, 1], [1, 1, 1], [1, 1, 1], True)
-    book.fwd = SimpleNamespace(groups=True, native=None)
+    book.fwd = _Buffers(3, 27, torch.device("cpu"))
     monkeypatch.setattr(conv, "_rules", lambda *a, **k: (z_idx, z_ptr, book, None, [1, 1]))
     monkeypatch.setattr(ext, "_kept_packed", lambda *a: torch.zeros(4))
     x = sphconv_amd.SparseConvTensor(torch.zeros(3, 8), [2, 2, 4], 1, z_idx=z_idx, z_ptr=z_ptr)
-    conv._layer(x)
-    monkeypatch.setattr(L, "host", lambda: host)
-    monkeypatch.setattr(L, "stream", lambda *a: 0)
-    monkeypatch.setattr(L, "capturing", lambda: False)
-    for rows in (torch.zeros(3, 4), torch.zeros(3, 8, 1)):
+    for rows, message in ((torch.zeros(3, 4), "mismatch"), (torch.zeros(3, 8, 1), "mismatch"), (torch.zeros(3, 8), "GPU tensor")):
         x.feature = rows
-        with torch.no_grad(), pytest.raises(sphconv_amd.SphconvError, match="mismatch"):
+        with torch.no_grad(), pytest.raises(sphconv_amd.SphconvError, match=message):
             conv(x)
-    assert not launched
-    x.feature = torch.zeros(3, 8)
-    host.conv_apply = lambda *a: torch.zeros(3, 16)
-    with torch.no_grad():
-        assert conv(x).feature.shape == (3, 16)
 
 
 @pytest.mark.parametrize("call", ["init_tensor", "function"])
-def test_coordinates_and_rows_are_checked_whoever_asks(monkeypatch, call):
+def test_coordinates_and_rows_are_checked_whoever_asks(call):
     """The autograd function of the public API is called by programs too: what the kernel reads is checked there as well."""
-    from types import SimpleNamespace
     from sphconv_amd import sphconv_cuda as ext
     from sphconv_amd.functional import InitTensorFunction
-    asked = []
-    monkeypatch.setattr(L, "host", lambda: SimpleNamespace(init_tensor=lambda *a: asked.append(a)))
     make = ext.init_tensor if call == "init_tensor" else InitTensorFunction.apply
     rows, indices = torch.zeros(5, 3), torch.zeros((5, 4), dtype=torch.int32)
     for f, i in ((rows[:4], indices), (rows, indices.long()), (rows, indices[:, :3]), (rows, indices[0]), (rows[0], indices)):
         with pytest.raises(ValueError, match="must be"):
             make(f, i, 1, [2, 2, 2])
-    assert not asked
+    with pytest.raises(sphconv_amd.SphconvError, match="GPU tensor"):
+        make(rows, indices, 1, [2, 2, 2])
 
 
 def test_weight_gradients_take_the_book_their_rows_fit(monkeypatch):
