@@ -50,10 +50,14 @@ def _bn_affine(bn: nn.BatchNorm1d, stream):
         return _bn_affine_now(bn)
     try:
         mean, var, weight, bias = b["running_mean"], b["running_var"], p["weight"], p["bias"]
+        # a pass in training mode changes the running statistics behind their version counters' back, and counts itself here
+        passes = b["num_batches_tracked"]
     except KeyError:
         # a tensor that is not in its table is computed, or a replica's: another one on each pass, nothing to keep
         return _bn_affine_now(bn)
-    state = [bn.eps]
+    if passes is None:
+        return _bn_affine_now(bn)
+    state = [bn.eps, passes.data_ptr(), passes._version]
     for t in (mean, var, weight, bias):
         if t is not None:
             state += (t.data_ptr(), t._version, t.dtype)
@@ -61,12 +65,13 @@ def _bn_affine(bn: nn.BatchNorm1d, stream):
     if kept is None:
         kept = bn.__dict__["_sph_affines"] = {}
     hit = kept.get(stream)
-    if hit is not None and hit[0] is mean and hit[1] is var and hit[2] is weight and hit[3] is bias and hit[4] == state:
-        return hit[5], hit[6]
+    if hit is not None and hit[0] is mean and hit[1] is var and hit[2] is weight and hit[3] is bias and hit[4] is passes \
+            and hit[5] == state:
+        return hit[6], hit[7]
     scale, shift = _bn_affine_now(bn)
     if len(kept) >= 16:
         kept.clear()
-    kept[stream] = (mean, var, weight, bias, state, scale, shift)
+    kept[stream] = (mean, var, weight, bias, passes, state, scale, shift)
     return scale, shift
 
 

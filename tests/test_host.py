@@ -438,3 +438,22 @@ def test_weight_gradients_take_the_book_their_rows_fit(monkeypatch):
     assert ext.rule_conv_d_weight(torch.zeros(2, 2), d_out, book, None) == ("forward", False)
     with pytest.raises(sphconv_amd.SphconvError, match="output rows"):
         ext.rule_conv_d_weight(torch.zeros(3, 2), d_out[:5], book, None)
+
+
+@pytest.mark.parametrize("momentum,affine", [(0.1, True), (0.1, False), (None, True)])
+def test_kept_affine_map_follows_passes_in_training_mode(momentum, affine):
+    """A training pass updates the running statistics without moving their version counters, also where no optimizer step
+    follows (frozen or absent weights, statistics being gathered anew)."""
+    bn = torch.nn.BatchNorm1d(4, momentum=momentum, affine=affine)
+    for k in range(3):
+        bn.train()
+        bn(torch.randn(16, 4) * (k + 1) + 3)
+        bn.eval()
+        _affine_of(bn)
+    bn.reset_running_stats()
+    _affine_of(bn)
+    bn.num_batches_tracked = None
+    with torch.no_grad():
+        _affine_of(bn)
+        torch.nn.functional.batch_norm(torch.randn(16, 4), bn.running_mean, bn.running_var, training=True)
+        _affine_of(bn)
