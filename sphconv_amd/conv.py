@@ -58,8 +58,15 @@ class Convolution(SphModule):
     def invalidate_packed(self):
         """Forgets the fragment-ordered copy of the weight that forward passes in eval mode keep under
         ``torch.no_grad()``.  In-place updates that bump the weight's version counter (optimizer steps,
-        ``load_state_dict``, ``weight.mul_()``) are followed without this; updates through ``weight.data`` are not."""
+        ``load_state_dict``, ``weight.mul_()``) are followed without this; updates through ``weight.data`` only where a
+        pass in training mode or with gradients, or a call of ``train()`` or ``eval()``, lies between."""
+        self.__dict__["_keeps_packed"] = False
         ext.invalidate_packed(self.weight)
+
+    def train(self, mode: bool = True):
+        if self.__dict__.get("_keeps_packed"):
+            self.invalidate_packed()
+        return super().train(mode)
 
     @property
     def rule_size(self):
@@ -153,13 +160,20 @@ class Conv3d(Convolution):
         if epilogue is not None and training:
             raise RuntimeError("a fused epilogue has no backward: call under torch.no_grad()")
         rows = oz_idx.shape[0]
+        if (grad or self.training) and self.__dict__.get("_keeps_packed"):
+            # the program is changing weights, some do it through .data (an optimizer of its own, copies of fp32 masters)
+            self.invalidate_packed()
         if training:
             out_feature = ConvFunction.apply(feature, weight.view(-1, self.in_channels, self.out_channels), book,
                                              rule_size, tile_grid_shape, rows)
         else:
             scale, shift, relu = epilogue if epilogue is not None else (None, None, False)
             keep = not self.training and not grad and weight.dtype == feature.dtype
-            packed = ext._kept_packed(weight) if keep and native else None
+            packed = None
+            if keep:
+                self.__dict__["_keeps_packed"] = True
+                if native:
+                    packed = ext._kept_packed(weight)
             if packed is not None:
                 out_feature = ext._conv_packed(feature, packed, self.in_channels, self.out_channels, book, rows, scale,
                                                shift, bool(relu))

@@ -202,6 +202,7 @@ class Sequential(SphModule):
                     if conv[i] and not module.subm:
                         start_count(i + 1)      # new coordinates: the next strided layer can start counting
             elif isinstance(input, SparseConvTensor):
+                module.__dict__.pop("_sph_affines", None)       # run on its own, as while it is trained
                 input.feature = module(input.feature)
             else:
                 input = module(input)

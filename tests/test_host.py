@@ -457,3 +457,66 @@ def test_kept_affine_map_follows_passes_in_training_mode(momentum, affine):
         _affine_of(bn)
         torch.nn.functional.batch_norm(torch.randn(16, 4), bn.running_mean, bn.running_var, training=True)
         _affine_of(bn)
+
+
+def test_kept_packed_weight_is_dropped_when_the_program_trains(monkeypatch):
+    """Optimizers and mixed-precision wrappers that write through ``weight.data`` leave no trace on the weight: a pass with
+    gradients or in training mode, and a change of mode, drop the copy that evaluation keeps."""
+    from types import SimpleNamespace
+    from sphconv_amd import sphconv_cuda as ext
+    z_idx, z_ptr = torch.zeros(3, dtype=torch.int32), torch.full((1, 2, 2), 3, dtype=torch.int32)
+    conv = sphconv_amd.SubMConv3d(8, 16, 3).eval()
+    book = sphconv_amd.RuleBook(z_idx, z_ptr, z_idx, z_ptr, 1, [2, 2, 4], [2, 2, 4], [3, 3, 3], [1, 1, 1], [1, 1, 1], [1, 1, 1], True)
+    book.fwd = SimpleNamespace(groups=True, native=None)
+    monkeypatch.setattr(conv, "_rules", lambda *a, **k: (z_idx, z_ptr, book, None, [1, 1]))
+    x = sphconv_amd.SparseConvTensor(torch.zeros(3, 8), [2, 2, 4], 1, z_idx=z_idx, z_ptr=z_ptr)
+    conv._layer(x)
+    used, made = [], []
+    host = SimpleNamespace(conv_apply=lambda f, packed, *a: used.append(packed) or torch.zeros(3, 16),
+                           pack_weight=lambda w, *a: made.append(w.sum().item()) or made[-1])
+    monkeypatch.setattr(L, "host", lambda: host)
+    monkeypatch.setattr(L, "stream", lambda *a: 0)
+    monkeypatch.setattr(L, "capturing", lambda: False)
+
+    def evaluate():
+        with torch.no_grad():
+            conv(x)
+        return used[-1]
+
+    now = lambda: conv.weight.sum().item()
+    assert evaluate() == now() and evaluate() == now() and len(made) == 1        # kept
+
+    def step():
+        conv.weight.data.add_(1.0)
+
+    conv.train()
+    step()
+    conv.eval()
+    assert evaluate() == now() and len(made) == 2
+    conv.train()
+    with torch.no_grad():
+        conv(x)                                                                  # keeps nothing
+    step()
+    conv.training = False                                                        # without a call of eval()
+    assert evaluate() == now()
+    monkeypatch.setattr(sphconv_amd.conv.ConvFunction, "apply", lambda *a: torch.zeros(3, 16))
+    conv(x)                                                                      # gradients in evaluation mode (fine-tuning)
+    step()
+    assert evaluate() == now()
+    kept = len(made)
+    assert evaluate() == now() and len(made) == kept
+    step()
+    conv.invalidate_packed()
+    assert evaluate() == now()
+
+
+def test_affine_map_is_dropped_where_the_module_runs_on_its_own(monkeypatch):
+    bn = torch.nn.BatchNorm1d(4).eval()
+    z_idx, z_ptr = torch.zeros(3, dtype=torch.int32), torch.full((1, 2, 2), 3, dtype=torch.int32)
+    seq = sphconv_amd.Sequential(bn)
+    with torch.no_grad():
+        modules._bn_affine(bn, None)
+    assert bn.__dict__["_sph_affines"]
+    seq(sphconv_amd.SparseConvTensor(torch.zeros(3, 4), [2, 2, 4], 1, z_idx=z_idx, z_ptr=z_ptr))
+    bn.weight.data.mul_(2.0)
+    _affine_of(bn)
