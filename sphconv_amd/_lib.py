@@ -171,17 +171,20 @@ def stream(device=None):
 
 
 # Whether torch's current stream records a graph.  What is computed then exists only while the graph replays, in memory of
-# the graph's, and what the graph reads has to live as long as it does: nothing is kept from call to call.
+# the graph's, and what the graph reads has to live as long as it does: nothing is kept from call to call.  (The default
+# stream, handle 0, cannot be captured: who has the handle asks only for another.)
 capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
 
 
 _IS_CURRENT = contextlib.nullcontext()
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)     # (there is a tensor on a GPU already)
 
 
 def on_device(device):
     """Context for calls of the C ABI on tensors of ``device``: kernels are launched on the current device, and on that
     device's stream.  (Entering a device context costs 3 us: only where the device is not the current one.)"""
-    if device.type != "cuda" or device.index is None or device.index == torch.cuda.current_device():
+    index = device.index
+    if index is None or device.type != "cuda" or index == _current_device():
         return _IS_CURRENT
     return torch.cuda.device(device)
 

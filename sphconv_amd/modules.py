@@ -27,17 +27,13 @@ def is_sparse_conv(module) -> bool:
     return isinstance(module, SphModule) and module.is_convolution
 
 
-def _hooked(module) -> bool:
-    """Whether calling the module runs more than its forward (pruning computes its weight in such a hook)."""
-    return bool(module._forward_pre_hooks or module._forward_hooks)
-
-
 def _keeps_on(t: torch.Tensor):
     """The stream that what is kept now belongs to (None for tensors on the host), or False where nothing may be kept: a
     graph under capture computes everything itself."""
     if not t.is_cuda:
         return None
-    return False if L.capturing() else L.stream(t.device)
+    stream = L.stream(t.device)
+    return False if stream and L.capturing() else stream
 
 
 def _bn_affine(bn: nn.BatchNorm1d, stream):
@@ -57,10 +53,11 @@ def _bn_affine(bn: nn.BatchNorm1d, stream):
         return _bn_affine_now(bn)
     if passes is None:
         return _bn_affine_now(bn)
-    state = [bn.eps, passes.data_ptr(), passes._version]
-    for t in (mean, var, weight, bias):
-        if t is not None:
-            state += (t.data_ptr(), t._version, t.dtype)
+    state = [bn.eps, passes._version, mean.data_ptr(), mean._version, mean.dtype, var.data_ptr(), var._version, var.dtype]
+    if weight is not None:
+        state += (weight.data_ptr(), weight._version, weight.dtype)
+    if bias is not None:
+        state += (bias.data_ptr(), bias._version, bias.dtype)
     kept = bn.__dict__.get("_sph_affines")
     if kept is None:
         kept = bn.__dict__["_sph_affines"] = {}
@@ -136,7 +133,8 @@ class Sequential(SphModule):
         self.add_module(name, module)
 
     def _fusable_tail(self, mods, i):
-        """(number of modules after mods[i] that fold into its store, BatchNorm1d or None, relu)."""
+        """(number of modules after mods[i] that fold into its store, BatchNorm1d or None, relu).  A module with hooks
+        does not: a hook sees every call (pruning computes its weight in one)."""
         conv = mods[i]
         if not (self.fuse_eval and is_sparse_conv(conv)) or torch.is_grad_enabled():
             return 0, None, False
@@ -147,10 +145,10 @@ class Sequential(SphModule):
         nxt = mods[i + 1] if i + 1 < len(mods) else None
         if (type(nxt) is nn.BatchNorm1d and not nxt.training
                 and (nxt._buffers.get("running_mean") is not None or nxt.running_mean is not None)
-                and nxt.num_features == conv.out_channels and not _hooked(nxt)):
+                and nxt.num_features == conv.out_channels and not nxt._forward_pre_hooks and not nxt._forward_hooks):
             bn, n = nxt, 1
             nxt = mods[i + 2] if i + 2 < len(mods) else None
-        if type(nxt) is nn.ReLU and not _hooked(nxt):
+        if type(nxt) is nn.ReLU and not nxt._forward_pre_hooks and not nxt._forward_hooks:
             relu, n = True, n + 1
         return n, bn, relu
 

@@ -522,12 +522,13 @@ _SCRATCH_BOOKS = threading.local()
 
 
 def _scratch_book(rows: int, kv: int, device) -> "_Buffers":
-    if L.capturing():                       # the graph's own, for as long as it needs it
+    stream = L.stream(device)
+    if stream and L.capturing():            # the graph's own, for as long as it needs it
         return _Buffers(rows, kv, device)
     books = getattr(_SCRATCH_BOOKS, "books", None)
     if books is None:
         books = _SCRATCH_BOOKS.books = {}
-    key = (device.index, L.stream(device), kv)
+    key = (device.index, stream, kv)
     buf = books.get(key)
     if buf is None or buf.capacity < rows:
         if len(books) >= 64:

@@ -60,9 +60,10 @@ def _packed_weight(weight: torch.Tensor, transpose: bool, reverse: bool = False,
     if not w.is_contiguous():
         w = w.contiguous()
     cache_key = None
-    if cache and not torch.is_grad_enabled() and w.data_ptr() == weight.data_ptr() and not L.capturing():
+    stream = L.stream(w.device) if cache else 0
+    if cache and not torch.is_grad_enabled() and w.data_ptr() == weight.data_ptr() and not (stream and L.capturing()):
         base = weight._base if weight._base is not None else weight
-        cache_key = (id(base), bool(transpose), bool(reverse), L.stream(w.device))
+        cache_key = (id(base), bool(transpose), bool(reverse), stream)
         state = (base._version, w.data_ptr(), tuple(w.shape), w.dtype)
         hit = _PACKED_CACHE.get(cache_key)
         if hit is not None and hit[0]() is base and hit[1] == state:
@@ -76,8 +77,9 @@ def _packed_weight(weight: torch.Tensor, transpose: bool, reverse: bool = False,
 def _kept_packed(weight: torch.Tensor) -> Optional[torch.Tensor]:
     """The kept fragment-ordered copy of ``weight`` (the parameter itself, of any shape) for the forward pass, if there
     is one and the weight has not changed since; None otherwise."""
-    hit = _PACKED_CACHE.get((id(weight), False, False, L.stream(weight.device)))
-    if hit is None or hit[0]() is not weight or L.capturing():
+    stream = L.stream(weight.device)
+    hit = _PACKED_CACHE.get((id(weight), False, False, stream))
+    if hit is None or hit[0]() is not weight or (stream and L.capturing()):
         return None
     version, address, _, dtype = hit[1]
     return hit[2] if version == weight._version and address == weight.data_ptr() and dtype == weight.dtype else None

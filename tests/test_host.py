@@ -145,6 +145,7 @@ def test_stream_and_device_context_follow_the_tensors_device(monkeypatch):
     entered = []
     monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 1000 + index, raising=False)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(L, "_current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "device", lambda d: entered.append(d) or L._IS_CURRENT)
     assert L.stream() == 1000 and L.stream(torch.device("cuda")) == 1000
     assert L.stream(torch.device("cuda", 1)) == 1001
