@@ -6,7 +6,8 @@
 // into MFMA operand registers (16 B per lane), multiplies by the pre-packed weight
 // fragments of that offset and adds the result into its private LDS accumulator
 // tile; the tile is written to HBM once, with the epilogue fused.  No barriers, no
-// atomics, summation order fixed by the book.  conv_apply_kernel is the general
+// atomics, summation order fixed by the book.  Long grids go to relay.hip, which keeps the
+// weight in registers.  conv_apply_kernel is the general
 // fallback for unaligned or very long rows.  When the book also keeps its pairs by
 // stationary row (dense neighbourhoods), conv_rows_kernel_* walks (offset, block of 16
 // rows) steps with the accumulators in registers instead; with rows of up to 64 bytes and
@@ -22,6 +23,7 @@
 #include "common.h"
 #include "pack.h"
 #include "conv_wave.h"
+#include "relay.h"
 
 #include <cstdlib>
 
@@ -1346,6 +1348,7 @@ int launch_conv(const ConvArgs &a, int ntiles, hipStream_t st)
     // made by a 24-bit multiply
     const bool small = (double)a.feat_rows * a.row_bytes < 2147483648.0 && a.feat_rows < (1 << 24);
     if (a.aligned_in && a.feat_rows > 0 && small) {
+        if (sph_relay_ok(DT, a, NW, ntiles)) return sph_relay_launch(DT, a, NW, ntiles, st);
         switch (a.nsteps) {
         case 1: return launch_conv_wave_ct<DT, 1>(a, NW, ntiles, st);
         case 2: return launch_conv_wave_ct<DT, 2>(a, NW, ntiles, st);

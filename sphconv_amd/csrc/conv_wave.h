@@ -6,9 +6,21 @@
 #include "pack.h"
 #include "tile_consts.h"
 
+// One call of sph_conv_apply, as its kernels take it.
+struct ConvArgs {
+    const char *feat;
+    int feat_rows, kdim, row_bytes;
+    const char *wp;
+    int nsteps, ndim;
+    sph_book book;
+    int cap;
+    const float *scale, *shift;
+    int relu;
+    char *out;
+    int aligned_in, aligned_out;
+};
+
 namespace {
-
-
 
 typedef int int4v __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
@@ -68,19 +80,6 @@ __device__ __forceinline__ int4v mfma_step<SPH_I8>(int4v a, int4v b, int4v d)
 {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, d, 0, 0, 0);
 }
-
-struct ConvArgs {
-    const char *feat;
-    int feat_rows, kdim, row_bytes;
-    const char *wp;
-    int nsteps, ndim;
-    sph_book book;
-    int cap;
-    const float *scale, *shift;
-    int relu;
-    char *out;
-    int aligned_in, aligned_out;
-};
 
 // can sph_conv_apply walk this call by stationary row?
 inline bool rows_path_ok(const ConvArgs &a)

@@ -1,0 +1,136 @@
+"""The grouped convolution with its weight in registers (csrc/relay.hip), which large books take: against the sum over the
+book's pairs in float64, on books just above the sizes it starts at, with a last tile that is not full."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_helpers as G
+from sphconv_amd import _lib as L
+from sphconv_amd import rulebook
+from sphconv_amd import sphconv_cuda as ext
+from sphconv_amd.rulebook import RuleBook
+
+pytestmark = pytest.mark.gpu
+TYPES = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16, "i8": torch.int8}
+
+
+def _scene(rows, shape, per_column, seed):
+    """z_idx, z_ptr of at least one scene's worth of `rows` voxels, `per_column` of them in an occupied column on average."""
+    rng = np.random.default_rng(seed)
+    S0, S1, S2 = shape
+    counts = np.minimum(rng.poisson(per_column, S0 * S1), S2)
+    bins = np.argsort(rng.random((S0 * S1, S2)), axis=1)
+    keep = np.arange(S2)[None, :] < counts[:, None]
+    cells = np.sort((np.arange(S0 * S1)[:, None] * S2 + bins)[keep])[:rows]
+    assert cells.size == rows, "the grid holds %d voxels" % cells.size
+    z_ptr = np.cumsum(np.bincount(cells // S2, minlength=S0 * S1)).astype(np.int32).reshape(1, S0, S1)
+    return G.t((cells % S2).astype(np.int32)), G.t(z_ptr)
+
+
+def _pairs(buf):
+    """(offset, gathered row, owner row) of every pair of a book, on the GPU."""
+    nt, cap, kv = buf.ntiles, buf.cap, buf.kv
+    koff = buf.tile_koff[:nt].int()
+    group = torch.arange(cap, device=koff.device)
+    k = (group[None, :, None] >= koff[:, None, 1:]).sum(2)                    # offset of each group; kv behind the last
+    gat, own = buf.grp_gather.view(-1, cap, L.GROUP)[:nt], buf.grp_owner.view(-1, cap, L.GROUP)[:nt]
+    live = (own >= 0) & (k < kv)[:, :, None]
+    return k[:, :, None].expand_as(own)[live].long(), gat[live].long(), own[live].long()
+
+
+def _check(book, dtype, ic, oc, seed, hint=None, epilogue=False, inf=False):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    buf, n, m, kv = book.fwd, book.in_rows, book.out_rows, book.kv
+    k, gat, own = _pairs(buf)
+    int8 = dtype == torch.int8
+    if int8:
+        feat = torch.randint(-128, 128, (n, ic), generator=g, device="cuda", dtype=torch.int8)
+        w = torch.randint(-128, 128, (kv, ic, oc), generator=g, device="cuda", dtype=torch.int8)
+    else:
+        feat = torch.randn((n, ic), generator=g, device="cuda").to(dtype)
+        w = (torch.randn((kv, ic, oc), generator=g, device="cuda") / (kv * ic) ** 0.5).to(dtype)
+    if inf:
+        w[kv // 2, 0, 0] = float("inf")
+        feat[n // 2, 0] = 0.0
+    scale = torch.rand(oc, generator=g, device="cuda") + 0.5 if epilogue or int8 else None
+    if int8:
+        scale = scale / 3000.0
+    shift = torch.randn(oc, generator=g, device="cuda") if epilogue else None
+    want, size = torch.zeros((2, m, oc), device="cuda", dtype=torch.float64)
+    for i in range(kv):
+        at = k == i
+        x, y = feat[gat[at]].double(), w[i].double()
+        want.index_add_(0, own[at], x @ y)
+        size.index_add_(0, own[at], x.abs() @ y.abs())
+    packed = ext._packed_weight(w, False)
+    st = buf.struct()
+    was = st.middle_run
+    if hint is not None:
+        st.middle_run = hint
+    epi = L.Epilogue(L.ptr(scale), L.ptr(shift), int(epilogue))
+    outs = []
+    for _ in range(2):
+        out = torch.full((m + 1, oc), 3, device="cuda").to(dtype)          # a row behind the last that nobody may touch
+        L.check(L.lib().sph_conv_apply(L.dtype_code(dtype), L.ptr(feat), n, ic, L.ptr(packed), oc, C.byref(st), C.byref(epi),
+                                       L.ptr(out), L.stream()))
+        outs.append(out)
+    st.middle_run = was
+    assert torch.equal(outs[0].view(torch.int8), outs[1].view(torch.int8)) and (outs[0][m] == 3).all()
+    out = outs[0][:m]
+    if int8:
+        exact = torch.round(want.float() * scale).clamp(-128, 127)         # integer sums below 2**24: exact in float32
+        assert torch.equal(out.float(), exact)
+        return
+    if epilogue:
+        want, size = torch.relu(want * scale + shift), size * scale + shift.abs()
+    # fp32 sums of at most kv * ic products (of the few a row has), then one rounding to the storage type
+    unit = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    bound = 1e-6 * size + unit * want.abs() + (2.0 ** -24 if dtype == torch.float16 else 0.0)
+    if inf:
+        fine = torch.isfinite(want)
+        assert not fine.all() and torch.equal(torch.isfinite(out), fine)
+        out, want, bound = out[fine], want[fine], bound[fine]
+    assert ((out.double() - want).abs() <= bound).all(), float(((out.double() - want).abs() / bound).max())
+
+
+@pytest.fixture(autouse=True)
+def _by_groups(monkeypatch):
+    monkeypatch.setattr(rulebook, "BY_ROW_MIN_PAIRS", float("inf"))
+
+
+@pytest.mark.parametrize("dtype,ic,oc,tiles", [
+    ("f16", 64, 64, 1025), ("bf16", 64, 64, 1032), ("f16", 32, 64, 1025), ("bf16", 24, 40, 1027), ("f16", 64, 32, 1025),
+    ("bf16", 40, 24, 1025), ("f32", 16, 64, 1025), ("f32", 32, 32, 1026), ("f32", 4, 16, 2049), ("f16", 16, 16, 2049),
+    ("bf16", 64, 8, 2050), ("f16", 16, 32, 2049), ("i8", 64, 64, 1025), ("i8", 32, 16, 2049), ("i8", 128, 48, 1025)])
+@pytest.mark.parametrize("per_column", [0.9, 4.0])          # one group per offset and tile; two and more (several passes)
+def test_submanifold(dtype, ic, oc, tiles, per_column):
+    rows = tiles * L.TILE_ROWS - 77
+    S1 = int(rows / per_column / 64 * 1.1) + 8
+    z_idx, z_ptr = _scene(rows, (64, S1, 32), per_column, ic + oc)
+    book = RuleBook.build_subm(z_idx, z_ptr, 1, [64, S1, 32], [3, 3, 3])
+    _check(book, TYPES[dtype], ic, oc, 7, epilogue=dtype in ("bf16", "f32"))
+
+
+@pytest.mark.parametrize("kernel,stride", [((3, 3, 3), (2, 2, 2)), ((2, 3, 3), (1, 2, 2)), ((5, 5, 1), (2, 2, 1)),
+                                           ((2, 2, 3), (2, 1, 1)), ((5, 1, 2), (1, 1, 1))])
+@pytest.mark.parametrize("dtype,ic,oc", [("f16", 32, 64), ("f32", 32, 32), ("bf16", 64, 64)])
+def test_other_kernels(kernel, stride, dtype, ic, oc):
+    """Kernel volumes of 10 to 27 offsets, which the gathering waves share unevenly, without the middle offset's run; and with
+    a run claimed that is not there (its pairs are strewn over the tile's rows)."""
+    z_idx, z_ptr = _scene(140000, (64, 1600, 32), 1.6, 11)
+    book = RuleBook.build(z_idx, z_ptr, 1, [64, 1600, 32],
+                          [(s + 2 * (k // 2) - k) // t + 1 for s, k, t in zip((64, 1600, 32), kernel, stride)],
+                          list(kernel), list(stride), [k // 2 for k in kernel])
+    assert book.fwd.ntiles > 1024
+    _check(book, TYPES[dtype], ic, oc, 3)
+    _check(book, TYPES[dtype], ic, oc, 3, hint=1)
+
+
+@pytest.mark.parametrize("hint", [0, 1])
+def test_a_weight_that_is_not_finite_reaches_its_pairs_only(hint):
+    """An infinite weight at the middle offset: rows without that pair, padding slots and rows behind the last stay finite."""
+    z_idx, z_ptr = _scene(140000, (64, 1600, 32), 1.6, 12)
+    book = RuleBook.build(z_idx, z_ptr, 1, [64, 1600, 32], [64, 1600, 32], [3, 3, 3], [1, 1, 1], [1, 1, 1])
+    _check(book, torch.float16, 32, 64, 5, hint=hint, inf=True)
