@@ -99,6 +99,40 @@ __device__ int block_upper_bound(const int32_t *a, int n, int target, int max_sp
     return lo;
 }
 
+// Columns of rows r0 .. r1 - 1 (those of a tile) to s_col, -1 for a row that no column holds, by the whole workgroup: rounds of
+// probes to the neighbourhood of the first, then a walk.  The walk tolerates starting early (columns before the tile hold none
+// of its rows), so the search stops once the window is below one walk step: a single round of probes for grids of up to 131072
+// columns.  s_first: 2 * NT / kWave ints, s_flag: 2.  meanwhile() as in block_upper_bound.  Ends behind a barrier.
+template <int NT, class F>
+__device__ __forceinline__ void search_columns(const int32_t *q_ptr, int q_ncol, int q_rows, int r0, int r1, int *s_col, int *s_first,
+                                               int *s_flag, F &&meanwhile)
+{
+    constexpr int kWalk = 2 * NT; // columns per walk step, two consecutive ones per thread
+    const int tid = threadIdx.x;
+    const int c_first = block_upper_bound<NT>(q_ptr, q_ncol, r0, kWalk, s_first, [&]() {
+        meanwhile();
+        for (int i = tid; i < R; i += NT) s_col[i] = -1;
+    });
+    bool done = (c_first >= q_ncol);
+    for (int cb = c_first, step = 0; !done; cb += kWalk, step ^= 1) { // the steps alternate between two flags: one barrier each
+        const int last = min(cb + kWalk - 1, q_ncol - 1);
+        const int c = cb + 2 * tid;
+        if (c <= last) {
+            // q_ptr[c-1], q_ptr[c], q_ptr[c+1] bound the fibers of columns c and c+1
+            int p0 = c ? clampi(q_ptr[c - 1], 0, q_rows) : 0;
+            int p1 = clampi(q_ptr[c], 0, q_rows);
+            int p2 = (c + 1 <= last) ? clampi(q_ptr[c + 1], 0, q_rows) : p1;
+            if (p1 < p0) p1 = p0;
+            if (p2 < p1) p2 = p1;
+            for (int r = max(p0, r0); r < min(p1, r1); r++) s_col[r - r0] = c;
+            for (int r = max(p1, r0); r < min(p2, r1); r++) s_col[r - r0] = c + 1;
+            if (c == last || c + 1 == last) s_flag[step] = (p2 >= r1) || (last == q_ncol - 1);
+        }
+        lds_barrier();
+        done = s_flag[step] != 0;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Shared tail of the book builders: the block holds, in LDS, a table
 // nbr[row_local * KV + k] = gathered row or -1 for the R rows of tile `tile`
@@ -471,9 +505,7 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
     const int my_rl = tid & (R - 1);
     const int my_zz = (my_rl < nrows) ? a.q_idx[r0 + my_rl] : 0;
 
-    // 1. rows -> columns.  The walk below tolerates starting early (columns before the
-    // tile hold none of its rows), so the search stops once the window is below one
-    // walk step: a single round of probes for grids of up to 131072 columns.
+    // 1. rows -> columns.
     // With a table of the rows' columns the search is one coalesced load; every entry is checked against the two
     // pointers that bound its column (for a submanifold layer the join below asks for the same two), and one entry
     // that fails sends the whole tile to the search.
@@ -507,30 +539,10 @@ __device__ __forceinline__ void tile_table(const BuildArgs &a, int tile, int32_t
     };
     if constexpr (!LINES) if (!search) check_hint(); // (nothing to overlap it with)
     for (;;) { // once, or twice where the table of the rows' columns was wrong
-    constexpr int kWalk = 2 * NT; // columns per walk step, two consecutive ones per thread
     if (search) {
-        const int c_first = block_upper_bound<NT>(a.q_ptr, q_ncol, r0, kWalk, s_first, [&]() {
+        search_columns<NT>(a.q_ptr, q_ncol, a.q_rows, r0, r1, s_col, s_first, s_flag, [&]() {
             for (int i = tid; i < R * KV / 4; i += NT) ((int4 *)s_nbr)[i] = make_int4(-1, -1, -1, -1); // R * KV is a multiple of 4
-            for (int i = tid; i < R; i += NT) s_col[i] = -1;
         });
-        bool done = (c_first >= q_ncol);
-    for (int cb = c_first, step = 0; !done; cb += kWalk, step ^= 1) { // the steps alternate between two flags: one barrier each
-        const int last = min(cb + kWalk - 1, q_ncol - 1);
-        const int c = cb + 2 * tid;
-        if (c <= last) {
-            // q_ptr[c-1], q_ptr[c], q_ptr[c+1] bound the fibers of columns c and c+1
-            int p0 = c ? clampi(a.q_ptr[c - 1], 0, a.q_rows) : 0;
-            int p1 = clampi(a.q_ptr[c], 0, a.q_rows);
-            int p2 = (c + 1 <= last) ? clampi(a.q_ptr[c + 1], 0, a.q_rows) : p1;
-            if (p1 < p0) p1 = p0;
-            if (p2 < p1) p2 = p1;
-            for (int r = max(p0, r0); r < min(p1, r1); r++) s_col[r - r0] = c;
-            for (int r = max(p1, r0); r < min(p2, r1); r++) s_col[r - r0] = c + 1;
-            if (c == last || c + 1 == last) s_flag[step] = (p2 >= r1) || (last == q_ncol - 1);
-        }
-        lds_barrier();
-        done = s_flag[step] != 0;
-    }
         my_c = my_rl < nrows ? s_col[my_rl] : -1;
         checked = true;
         search = false;

@@ -1,0 +1,141 @@
+"""The rule kernel with a thread per stationary row (csrc/rules_rows.h), which grids of more than 512 tiles take: every pair
+against a look-up in a dense grid of row numbers, and the order of the groups."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_helpers as G
+from sphconv_amd import _lib as L
+from sphconv_amd import rulebook
+from sphconv_amd.rulebook import RuleBook
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _by_groups(monkeypatch):
+    monkeypatch.setattr(rulebook, "BY_ROW_MIN_PAIRS", float("inf"))
+
+
+def _scene(shape, batch, per_column, seed, shuffle=False):
+    """z_idx, z_ptr and the column of every row; 0 to S2 voxels a column, `per_column` on average."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    S0, S1, S2 = shape
+    occ = torch.rand((batch * S0 * S1, S2), generator=g, device="cuda") < torch.rand((batch * S0 * S1, 1), generator=g, device="cuda") * 2 * per_column / S2
+    col, z = occ.nonzero(as_tuple=True)
+    if shuffle:                                        # the order inside a column is the caller's
+        order = torch.argsort(col * 4096 + torch.randint(0, 4096, col.shape, generator=g, device="cuda"), stable=True)
+        col, z = col[order], z[order]
+    z_ptr = occ.sum(1).cumsum(0).int().view(batch, S0, S1)
+    return z.int().contiguous(), z_ptr.contiguous(), col.int().contiguous()
+
+
+def _expected(q, p, shape_p, kernel, stride, pad, transposed):
+    """(offset, gathered row, owner row) of all pairs, by offset and owner; q, p: (z_idx, column, shape) of the two sides."""
+    (qz, qc, qs), (pz, pc, ps) = q, p
+    per = ps[0] * ps[1]
+    n_cells = (int(pc.max()) // per + 1) * per * ps[2] if pc.numel() else 0
+    cells = torch.full((max(n_cells, 1),), -1, dtype=torch.long, device="cuda")
+    cells.scatter_reduce_(0, pc.long() * ps[2] + pz.long(), torch.arange(pz.numel(), device="cuda"), "amax")
+    b, c0, c1, z = qc.long() // (qs[0] * qs[1]), qc.long() // qs[1] % qs[0], qc.long() % qs[1], qz.long()
+    out = []
+    for k in range(kernel[0] * kernel[1] * kernel[2]):
+        ks = (k // (kernel[1] * kernel[2]), k // kernel[2] % kernel[1], k % kernel[2])
+        at, ok = [], torch.ones_like(z, dtype=torch.bool)
+        for x, kd, s, pd, n in zip((c0, c1, z), ks, stride, pad, ps):
+            if transposed:
+                t = x + pd - kd
+                ok &= (t >= 0) & (t % s == 0)
+                y = torch.div(t, s, rounding_mode="floor")
+            else:
+                y = x * s - pd + kd
+            ok &= (y >= 0) & (y < n)
+            at.append(y.clamp(0, n - 1))
+        cell = ((b * ps[0] + at[0]) * ps[1] + at[1]) * ps[2] + at[2]
+        ok &= cell < cells.numel()
+        row = torch.where(ok, cells[cell.clamp(max=cells.numel() - 1)], -1)
+        own = (row >= 0).nonzero()[:, 0]
+        out.append(torch.stack([torch.full_like(own, k), row[own], own]))
+    return torch.cat(out, 1)
+
+
+def _check(buf, want):
+    nt, cap, kv = buf.ntiles, buf.cap, buf.kv
+    koff, ngrp = buf.tile_koff[:nt].int(), buf.tile_ngrp[:nt]
+    group = torch.arange(cap, device=koff.device)
+    k = (group[None, :, None] >= koff[:, None, 1:]).sum(2)
+    used = k < kv
+    assert torch.equal(used.sum(1).int(), ngrp) and (koff[:, 0] == 0).all()
+    assert torch.equal(buf.grp_k.view(-1, cap)[:nt][used], k[used].int())
+    gat, own = buf.grp_gather.view(-1, cap, 16)[:nt], buf.grp_owner.view(-1, cap, 16)[:nt]
+    live = (own >= 0) & used[:, :, None]
+    assert torch.equal(live[used], (gat >= 0)[used])
+    # groups are filled from the front, and only an offset's last one is not full
+    assert (live[:, :, 1:] <= live[:, :, :-1]).all()
+    full = live.all(2)
+    same = (k[:, 1:] == k[:, :-1]) & used[:, 1:]
+    assert full[:, :-1][same].all() and live[:, :, 0][used].all()
+    tile = torch.arange(nt, device=own.device)[:, None, None].expand_as(own)
+    assert torch.equal(own[live] // L.TILE_ROWS, tile[live].int())
+    got = torch.stack([k[:, :, None].expand_as(own)[live].long(), gat[live].long(), own[live].long()])
+    # in the book: tile by tile, offsets ascending, owners ascending
+    order = torch.argsort((want[2] // L.TILE_ROWS) * 64 + want[0], stable=True)
+    assert torch.equal(got, want[:, order])
+
+
+def _columns(z_ptr, rows):
+    return torch.searchsorted(z_ptr.view(-1).long(), torch.arange(rows, device="cuda"), right=True).int()
+
+
+def _build(z_idx, z_ptr, oz_idx, oz_ptr, book, transposed, cols):
+    buf = rulebook._Buffers(book.in_rows if transposed else book.out_rows, book.kv, z_idx.device)
+    L.check(L.lib().sph_rules_build(L.ptr(z_idx), L.ptr(z_ptr), book.in_rows, L.ptr(oz_idx), L.ptr(oz_ptr), book.out_rows,
+                                    C.byref(book.geom()), int(transposed), C.byref(buf.struct()), L.ptr(cols), L.stream()))
+    return buf
+
+
+SUBM = [((3, 3, 3), 1.5), ((3, 3, 3), 3.3), ((3, 3, 1), 1.5), ((1, 3, 3), 2.0), ((3, 1, 1), 1.5), ((3, 3, 3), 0.4)]
+
+
+@pytest.mark.parametrize("columns", ["given", "none", "shifted", "random", "one wrong", "outside"])
+@pytest.mark.parametrize("kernel,per_column", SUBM)
+def test_submanifold(kernel, per_column, columns):
+    batch, shape = 3, (31, int(27000 / per_column / 31) + 9, 40)
+    z_idx, z_ptr, col = _scene(shape, batch, per_column, 3, shuffle=per_column == 2.0)
+    book = RuleBook.build_subm(z_idx, z_ptr, batch, list(shape), list(kernel))
+    assert book.fwd.ntiles > 512
+    cols = col.clone()
+    if columns == "none":
+        cols = None
+    elif columns == "shifted":
+        cols = cols.roll(1)
+    elif columns == "random":
+        cols = torch.randint_like(cols, 0, batch * shape[0] * shape[1])
+    elif columns == "one wrong":
+        cols[::777] += 1
+    elif columns == "outside":
+        cols[5::333] = -7
+        cols[9::555] = 2 ** 31 - 1
+    want = _expected((z_idx, col, shape), (z_idx, col, shape), shape, kernel, (1, 1, 1), [k // 2 for k in kernel], False)
+    _check(_build(z_idx, z_ptr, z_idx, z_ptr, book, False, cols), want)
+
+
+@pytest.mark.parametrize("kernel,stride,pad", [((3, 3, 3), (2, 2, 2), (1, 1, 1)), ((3, 3, 3), (1, 2, 2), (1, 1, 1)),
+                                               ((3, 3, 3), (3, 3, 2), (0, 1, 1)), ((2, 2, 1), (2, 2, 1), (0, 0, 0)),
+                                               ((3, 2, 4), (2, 1, 2), (1, 0, 1)), ((2, 3, 3), (1, 1, 3), (0, 1, 1)),
+                                               ((3, 3, 1), (2, 1, 1), (1, 1, 0))])
+@pytest.mark.parametrize("hint", [True, False])
+def test_strided(kernel, stride, pad, hint):
+    batch, shape = 2, (62, 1500, 24)
+    z_idx, z_ptr, col = _scene(shape, batch, 1.2, 5)
+    oshape = [(s + 2 * p - k) // t + 1 for s, k, t, p in zip(shape, kernel, stride, pad)]
+    book = RuleBook.build(z_idx, z_ptr, batch, list(shape), oshape, list(kernel), list(stride), list(pad))
+    ocol = _columns(book.oz_ptr, book.out_rows)
+    sides = (z_idx, col, shape), (book.oz_idx, ocol, oshape)
+    assert book.in_rows > 1024 * L.TILE_ROWS and book.out_rows > 512 * L.TILE_ROWS
+    _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, False, ocol if hint else None),
+           _expected(sides[1], sides[0], shape, kernel, stride, pad, False))
+    _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, True, col if hint else None),
+           _expected(sides[0], sides[1], oshape, kernel, stride, pad, True))
