@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "rules_tile.h"
+#include "rules_masks.h"
 #include "rules_rows.h"
 
 namespace {
@@ -501,6 +502,17 @@ static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_p
     a.lines = join_lines(a, transposed != 0);
     hipStream_t st = (hipStream_t)stream;
     const bool by_lines = a.lines && !a.long_fibers;
+    if (masks_build_ok(a, transposed != 0, KV)) {
+        const bool k27 = a.cv.K0 * a.cv.K1 == 9 && a.cv.K2 == 3;
+        void (*masks)(BuildArgs) = k27 ? (a.q_rowcol ? build_nbr_kernel<true, 9, 3> : build_nbr_kernel<false, 9, 3>)
+                                       : (a.q_rowcol ? build_nbr_kernel<true, 0, 0> : build_nbr_kernel<false, 0, 0>);
+        const int pack_masks = pack ? sph_div_up(sph_pack_total(pack->job), kNbrThreads) : 0;
+        const size_t lds_nbr = masks_lds(a.cv.K0 * a.cv.K1);
+        const int rc = allow_lds(masks, lds_nbr, who);
+        if (rc) return rc;
+        hipLaunchKernelGGL(masks, dim3(a.tile_blocks + pack_masks), dim3(kNbrThreads), lds_nbr, st, a);
+        return sph_check_launch(who);
+    }
     if (rows_build_ok(a, transposed != 0, KV, nt)) {
         const bool c3 = a.lines == 3, nl3 = (transposed ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0) == 3;
 #define SPH_ROWS(T, C, NL, KVT) (a.q_rowcol ? build_rows_kernel<T, C, NL, KVT, true> : build_rows_kernel<T, C, NL, KVT, false>)
