@@ -11,7 +11,7 @@
 // fallback for unaligned or very long rows.  When the book also keeps its pairs by
 // stationary row (dense neighbourhoods), conv_rows_kernel_* walks (offset, block of 16
 // rows) steps with the accumulators in registers instead; with rows of up to 64 bytes and
-// up to 32 output columns conv_rows_win_kernel does so from a copy of the gathered rows
+// up to 64 output columns conv_rows_win_kernel does so from a copy of the gathered rows
 // in LDS.
 //
 // wgrad (sph_conv_wgrad): work items are (kernel offset, chunk of 64 tiles, slice of 64
@@ -435,51 +435,56 @@ __global__ __launch_bounds__(512) void conv_rows_kernel_split(ConvArgs a, int nw
 
 
 // ---------------------------------------------------------------------------
-// By stationary row, gathered rows staged in LDS: rows of up to 64 bytes (one MFMA K step), up to 32
-// output columns, one wave per tile.
+// By stationary row, gathered rows staged in LDS: rows of up to 64 bytes (one MFMA K step), up to 64
+// output columns, two waves per tile.
 //
 // With one K step a (offset, block) step is one or two MFMAs behind a gather of 16 rows; the plain by-row
 // kernel then waits for its gathers (every one a miss of the vector L1: a tile's 27 offsets ask for each
 // neighbouring row about ten times, with the other waves' traffic in between).  The rows a tile's offsets
 // gather lie close together in the feature array: for 9 consecutive offsets (one value of k0 in a 3x3x3
 // kernel) they are the tile's own range of rows of one line of the grid, a column more on either side.
-// So the offsets are taken in phases of 9: the wave finds the range [lo, hi] of rows the phase gathers,
-// brings it to LDS as it lies (direct global -> LDS loads, all in flight at once), rewrites the phase's
-// table as one byte per (offset, row) (place in the window; slots without a pair point at a row of zeros
-// behind it), and every step's gather is then one 16-byte LDS read per lane, with nothing to select
-// afterwards.  A phase whose rows do not fit the window (a tile that straddles two lines of the grid,
+// So the offsets are taken in phases of 9: the tile's two waves, with 64 rows each, find the range [lo, hi]
+// of rows the phase gathers, bring it to LDS as it lies (direct global -> LDS loads, all in flight at once),
+// rewrite the phase's table as one byte per (offset, row) (place in the window; slots without a pair point at
+// a row of zeros behind it), and every step's gather is then one 16-byte LDS read per lane, with nothing to
+// select afterwards.  A phase whose rows do not fit the window (a tile that straddles two lines of the grid,
 // strided layers with wide footprints) gathers from the feature array instead.  The order of summation
-// per row is the plain kernel's (offsets ascending), so results are bit-identical.  Bounds: the LDS
-// (about 10 cycles per 16-row read and CU, against 8 for the step's two MFMAs) and, per phase, one round
-// trip for the window; the registers (accumulators, three offsets of weights, the next table) allow two
-// waves per SIMD, and with 64 output columns they do not suffice (the compiler spills and the kernel
-// halves its speed), so those layers stay with the plain kernel.
-// Measured, fp16, grid 4x32x1024x32 at 40 % occupancy (1.68 M rows, 10.9 pairs per row): 32->32 178 us
-// against 250 us with gathers from the feature array, 16->32 156 against 210.
+// per row is the plain kernel's (offsets ascending), so results are bit-identical.
+// What bounds it: the round trips of the windows.  On 12 744 tiles, 32 -> 32, waves wait for memory 58 % of their
+// time, the vector memory path is 64 % busy (two fifths of it weight fragments), the LDS 37 %, the matrix cores 27 %.
+// With one wave per tile (256 registers: two waves per SIMD) there was less to fill the waits with; two halve a
+// wave's accumulators and table, so three waves share a SIMD, with one window for two of them, at the price of
+// twice the weight loads.  us, one wave a tile -> two, fp16: 32 -> 32 on 12 744 tiles (10.9 pairs a row)
+// 154.6 -> 146.7, 16 -> 32 149.0 -> 140.1; on 4056 tiles (24.8 pairs) 74.3 -> 61.2; on 1248 tiles 23.3 -> 18.2.  With
+// the registers of one wave there was no room for 64 columns either: 32 -> 64 on 4056 tiles, gathers from the feature array
+// against the window, 96.5 : 85.6.  Held to four waves per SIMD (128 registers) it spills and takes 245 us.
 // ---------------------------------------------------------------------------
 constexpr int kWinPhase = 9;           // offsets per window
 constexpr int kWinBytes = 16 * 1024;   // bytes of feature rows a window holds (up to 255 rows)
 constexpr int kWinTab = kWinPhase * R; // one byte per (offset, row)
 constexpr int kWinMaxRows = 255;       // most rows of a window: a byte names any of them or the row of zeros
+constexpr int kWinWaves = 2;           // waves of a tile: 64 rows each, one window
+constexpr int kWinRows = R / kWinWaves;
 
 template <sph_dtype DT, int CT, bool MASKED>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void conv_rows_win_kernel(ConvArgs a, int nwtot)
+__global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_eu(CT == 4 ? 2 : 3))) void conv_rows_win_kernel(ConvArgs a, int nwtot)
 {
     typedef typename Traits<DT>::elem elem;
     typedef typename Traits<DT>::acc4 acc4;
-    typedef int int2v __attribute__((ext_vector_type(2)));
-    constexpr int NB = R / SPH_GROUP;        // 8 blocks of 16 rows
-    constexpr int HB = 4;                    // blocks per stage
+    constexpr int NB = kWinRows / SPH_GROUP; // 4 blocks of 16 rows
+    constexpr int HB = CT == 4 ? 2 : 4;      // blocks per stage
     constexpr int SPO = NB / HB;             // stages per offset
-    constexpr int TL = kWinPhase * R / 2 / kWave; // int2 table entries per lane and phase
+    static_assert(kWinRows == kWave, "a lane brings its row's entry of every offset");
     constexpr int WR = 3;                    // sets of weight fragments: requested three offsets ahead
     static_assert(kWinPhase % WR == 0, "the ring must divide a phase");
     extern __shared__ __attribute__((aligned(16))) char s_mem[];
-    uint8_t *s_tab = (uint8_t *)s_mem;       // [kWinPhase][SPO][16 rows][HB blocks]
-    char *s_win = s_mem + kWinTab;           // the window's rows, as they lie in the feature array
-    int32_t *s_tab32 = (int32_t *)s_win;     // a phase without a window: [kWinPhase][R] rows of the feature array
-
+    __shared__ int2 s_range[2][kWinWaves];   // rows a wave's part of the phase gathers, by the phase's parity
     const int lane = threadIdx.x & (kWave - 1);
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    uint8_t *s_tab = (uint8_t *)s_mem + part * (kWinPhase * kWinRows); // [kWinPhase][SPO][16 rows][HB blocks], a wave's own
+    char *s_win = s_mem + kWinTab;           // the window's rows, as they lie in the feature array
+    int32_t *s_tab32 = (int32_t *)s_win + part * (kWinPhase * kWinRows); // a phase without a window: [kWinPhase][64] rows of the feature array
+
     const int tile = sph_xcd_tile(blockIdx.x, (a.book.rows + R - 1) / R);
     const int r0 = tile * R;
     if (r0 >= a.book.rows) return;
@@ -499,16 +504,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void co
 #pragma unroll
         for (int c = 0; c < CT; c++) acc[j][c] = acc4{0, 0, 0, 0};
 
-    int2v tn[TL]; // the next phase's table, on its way while this phase is worked through
+    int tn[kWinPhase]; // the next phase's table, on its way while this phase is worked through
     auto load_tab = [&](int ph) {
-        const int phc = min(ph, nph - 1);
-        const int2v *src = (const int2v *)(a.book.tile_nbr + ((long)tile * KV + phc * kWinPhase) * R);
-        const int n2 = min(kWinPhase, KV - phc * kWinPhase) * R / 2;
+        const int k0 = min(ph, nph - 1) * kWinPhase;
+        const int32_t *src = a.book.tile_nbr + ((long)tile * KV + k0) * R + part * kWinRows + lane;
 #pragma unroll
-        for (int i = 0; i < TL; i++) {
-            const int e = lane + kWave * i;
-            tn[i] = src[e < n2 ? e : 0];
-        }
+        for (int i = 0; i < kWinPhase; i++) tn[i] = src[min(i, KV - 1 - k0) * R];
     };
     auto load_w = [&](int k, int4v (&w)[CT]) {
         const char *wk = wlane + (long)min(k, KV - 1) * wstep;
@@ -524,28 +525,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void co
         const int k0 = ph * kWinPhase;
         const int nk = min(kWinPhase, KV - k0);
         // this phase's table: validate, find the range of rows it gathers
-        int2v t[TL];
-        int lo = 0x7fffffff, hi = -1;
+        int t[kWinPhase], lo = 0x7fffffff, hi = -1;
 #pragma unroll
-        for (int i = 0; i < TL; i++) {
-            const int e = lane + kWave * i;
-            int2v v = tn[i];
-            const bool in = e < nk * R / 2;
-            v.x = (in && (unsigned)v.x < (unsigned)a.feat_rows) ? v.x : -1;
-            v.y = (in && (unsigned)v.y < (unsigned)a.feat_rows) ? v.y : -1;
-            if (v.x >= 0) { lo = min(lo, v.x); hi = max(hi, v.x); }
-            if (v.y >= 0) { lo = min(lo, v.y); hi = max(hi, v.y); }
-            t[i] = v;
+        for (int i = 0; i < kWinPhase; i++) {
+            t[i] = (i < nk && (unsigned)tn[i] < (unsigned)a.feat_rows) ? tn[i] : -1;
+            lo = (int)min((unsigned)lo, (unsigned)t[i]); // (-1 is the largest unsigned number)
+            hi = max(hi, t[i]);
         }
-        load_tab(ph + 1);
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            lo = min(lo, __shfl_xor(lo, o, kWave));
-            hi = max(hi, __shfl_xor(hi, o, kWave));
-        }
+        lo = ~wave_max_last(~lo); // lowest: 0x7fffffff, a lane without a pair, is the least of the complements
+        hi = wave_max_last(hi);
+        // direct loads write LDS behind the back of the LDS unit's own queue: the last phase's reads must
+        // have returned before the window is overwritten
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (lane == kWave - 1) s_range[ph & 1][part] = make_int2(lo, hi);
+        lds_barrier();
+        lo = min(s_range[ph & 1][0].x, s_range[ph & 1][1].x);
+        hi = max(s_range[ph & 1][0].y, s_range[ph & 1][1].y);
         lo = __builtin_amdgcn_readfirstlane(lo);
         hi = __builtin_amdgcn_readfirstlane(hi);
         if (hi < 0) { // no pair at these offsets
+            load_tab(ph + 1);
 #pragma unroll
             for (int i = 0; i < WR; i++) load_w(k0 + kWinPhase + i, wr[i]);
             continue;
@@ -553,35 +552,29 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void co
         // a window holds rows lo..hi and, behind them, one row of zeros that slots without a pair read
         const int nrow = hi - lo + 1;
         const bool win = nrow <= kWinMaxRows && nrow * rb <= kWinBytes;
-        // direct loads write LDS behind the back of the LDS unit's own queue: the last phase's reads must
-        // have returned before the window is overwritten
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (win) {
 #pragma unroll
-            for (int i = 0; i < TL; i++) {
-                // entries 2e and 2e + 1 of the phase: offset e / 64, row 2e % 128 and the next one (same block)
-                const int e = lane + kWave * i;
-                const int row = (2 * e) & (R - 1), blk = row >> 4, n = row & 15;
-                uint8_t *dst = s_tab + (e >> 6) * R + (blk / HB) * (SPH_GROUP * HB) + n * HB + blk % HB;
-                dst[0] = (uint8_t)(t[i].x >= 0 ? t[i].x - lo : nrow);
-                dst[HB] = (uint8_t)(t[i].y >= 0 ? t[i].y - lo : nrow);
-            }
+            for (int i = 0; i < kWinPhase; i++)
+                s_tab[i * kWinRows + (lane >> 4) / HB * (SPH_GROUP * HB) + (lane & 15) * HB + (lane >> 4) % HB] =
+                    (uint8_t)(t[i] >= 0 ? t[i] - lo : nrow);
             // lane l of load i fills the 16 bytes at i * 1024 + l * 16 of the window
             const int nbytes = nrow * rb;
             const int nld = (nbytes + kWave * 16 - 1) / (kWave * 16);
             const char *src = a.feat + (long)lo * rb;
-            for (int i = 0; i < nld; i++) {
+            for (int i = part; i < nld; i += kWinWaves) {
                 const char *g = src + min((i * kWave + lane) * 16, nbytes - 16);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
                                                  (__attribute__((address_space(3))) void *)(s_win + i * (kWave * 16)), 16, 0, 0);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            lds_barrier();
+            load_tab(ph + 1);
             if (lane * 16 < rb) *(int4v *)(s_win + nbytes + lane * 16) = int4v{0, 0, 0, 0}; // behind the loads: their last kilobyte may reach here
             // stages (offset, HB blocks): table entries two stages ahead, rows one stage ahead
             constexpr int ns = kWinPhase * SPO;
             auto tab = [&](int st, int (&id)[HB]) {
                 const int sc = min(st, ns - 1);
-                const uint8_t *p = s_tab + (sc / SPO) * R + (sc % SPO) * (SPH_GROUP * HB) + (lane & 15) * HB;
+                const uint8_t *p = s_tab + (sc / SPO) * kWinRows + (sc % SPO) * (SPH_GROUP * HB) + (lane & 15) * HB;
                 const uint32_t pk = HB == 4 ? *(const uint32_t *)p : *(const uint16_t *)p;
 #pragma unroll
                 for (int j = 0; j < HB; j++) id[j] = (pk >> (8 * j)) & 255;
@@ -625,7 +618,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void co
         } else {
             // the rows lie too far apart: gathers from the feature array, one offset at a time
 #pragma unroll
-            for (int i = 0; i < TL; i++) ((int2v *)s_tab32)[lane + kWave * i] = t[i];
+            for (int i = 0; i < kWinPhase; i++) s_tab32[i * kWinRows + lane] = t[i];
+            load_tab(ph + 1);
 #pragma unroll 1
             for (int k9 = 0; k9 < nk; k9++) {
                 int4v w[CT];
@@ -636,7 +630,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void co
                     int4v x[HB];
 #pragma unroll
                     for (int j = 0; j < HB; j++) {
-                        id[j] = s_tab32[k9 * R + (h * HB + j) * SPH_GROUP + (lane & 15)];
+                        id[j] = s_tab32[k9 * kWinRows + (h * HB + j) * SPH_GROUP + (lane & 15)];
                         x[j] = *(const int4v *)(a.feat + (long)max(id[j], 0) * rb + choff);
                     }
 #pragma unroll
@@ -670,7 +664,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void co
     elem *out = (elem *)a.out + (long)r0 * a.ndim;
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const int row = b * SPH_GROUP + (lane & 15);
+        const int row = part * kWinRows + b * SPH_GROUP + (lane & 15);
         if (row >= nrows) continue;
 #pragma unroll
         for (int c = 0; c < CT; c++) {
@@ -1304,11 +1298,11 @@ int launch_conv_rows_m(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
     // the table, and for 128-byte rows a wave's exchange buffer (up to 4 chunk sets of 16 rows x 80 bytes)
     const size_t lds = (size_t)a.book.KV * R * sizeof(int32_t) + (NS >= 2 ? (size_t)waves * ws * 4 * SPH_GROUP * 80 : 0);
     const dim3 grid(sph_xcd_grid(ntiles)), block(waves * ws * kWave);
-    if constexpr (NS == 1 && CT <= 2) {
-        // one K step, up to 32 columns: the gathered rows go through an LDS window (with 64 columns the
-        // accumulators leave no registers for that kernel's pipeline)
-        if (ws == 1 && waves == 1) {
-            hipLaunchKernelGGL((conv_rows_win_kernel<DT, CT, MASKED>), grid, dim3(kWave), kWinTab + kWinBytes + 64, st, a, nwtot);
+    if constexpr (NS == 1) {
+        // one K step, up to 64 columns: the gathered rows go through an LDS window.  Short grids are faster with four waves per
+        // tile: 312 tiles 17.2 : 19.2 us with 32 columns, but 23.3 : 20.9 with 64.
+        if (waves == 1 && (CT == 4 ? ntiles > 256 : ws == 1)) {
+            hipLaunchKernelGGL((conv_rows_win_kernel<DT, CT, MASKED>), grid, dim3(kWinWaves * kWave), kWinTab + kWinBytes + 64, st, a, nwtot);
             return sph_check_launch("sph_conv_apply");
         }
     }
