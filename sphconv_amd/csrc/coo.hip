@@ -10,13 +10,14 @@
 //   2. coo_mark_kernel   every row sets its cell's bit in its column's bitmap (one 64-bit atomic without a result:
 //                        nothing waits for it)
 //   3. sum-scan (scan.h) of the columns' bit counts, made from the bitmap as they are read -> z_ptr
-//   4. coo_place_kernel  rank = set bits of the column below s2 (popcounts of up to S2/64 words); writes z_idx, the
-//                        permutation, the row's column, moves the feature row and reports the status.  Rows that
+//   4. coo_place_kernel  rank = set bits of the column below s2 (popcounts of up to S2/64 words); writes the
+//                        permutation, moves the feature row and reports the status; z_idx and
+//                        the rows' columns come from the row or from the bitmap.  Rows that
 //                        share a cell set one bit between them: their number is what the bits are short of the rows.
 // (the reference keeps four bytes per cell for the same purpose, tensor.cu:21-36.)
 // What bounds it: the random accesses, one atomic and one feature row per input row.  623 k rows in random order on a
 // 4x64x2048x64 grid, 16 fp16 channels: 118 us in eight launches with per-column counters, slots, a scatter into segments
-// and a walk of each row's segment; four launches now.
+// and a walk of each row's segment; 66 us in four launches now.
 // A bitmap of more than 1 GiB (8.6e9 cells) falls back to that walk, which needs memory by rows only:
 //   coo_count_kernel    slot = atomicAdd(count[column]) per row (arrival order, only used to park the row inside its
 //                       column's segment); sum-scan -> z_ptr
@@ -162,10 +163,32 @@ struct CooRows {
     int32_t *status, *host_status;           // host_status (may be null): the same two words where the host reads them
 };
 
-// gpr threads per row, one 16-byte (G) granule of its features each; gpr = 1 without features
-template <typename G>
-__global__ __launch_bounds__(256) void coo_place_kernel(const int32_t *idx, int n, CooGrid g, CooRows r, int gpr)
+// Whether the columns write what their bits say of their rows.  us of the place kernel, by rows : by columns: 623 k rows in random
+// order, 524 k words 48.7 : 28.7; 94 k rows, 131 k words 6.5 : 5.4; 24 k rows, 262 k words (eight to a column) 4.1 : 5.8.
+inline bool coo_by_columns(int n, int ncol, int words) { return 4 * (double)n >= (double)ncol * words; }
+
+// What a column's bits say of its rows, a thread per column: their S2 coordinates and their column.
+__device__ __forceinline__ void coo_columns(int col, int n, const CooGrid &g, const CooRows &r)
 {
+    if (col >= g.B * g.S0 * g.S1) return;
+    int pos = col ? r.z_ptr[col - 1] : 0;
+    for (int w = 0; w < g.words; w++)
+        for (unsigned long long m = r.bits[(size_t)col * g.words + w]; m && pos < n; m &= m - 1, pos++) {
+            r.z_idx[pos] = w * 64 + __ffsll((long long)m) - 1;
+            if (r.row_cols) r.row_cols[pos] = col;
+        }
+}
+
+// gpr threads per row, one 16-byte (G) granule of its features each; gpr = 1 without features.  z_idx and row_cols are written by
+// rows, two 4-byte writes to lines of their own for each where the rows come in no order, or, where the bitmap has few words
+// more than there are rows (coo_by_columns), by workgroups of the columns behind those of the rows (row_blocks).
+template <typename G>
+__global__ __launch_bounds__(256) void coo_place_kernel(const int32_t *idx, int n, CooGrid g, CooRows r, int gpr, int row_blocks)
+{
+    if ((int)blockIdx.x >= row_blocks) {
+        coo_columns((blockIdx.x - row_blocks) * 256 + threadIdx.x, n, g, r);
+        return;
+    }
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
     if (t == 0) {
         const int outside = r.status[0], ncol = g.B * g.S0 * g.S1;
@@ -189,9 +212,11 @@ __global__ __launch_bounds__(256) void coo_place_kernel(const int32_t *idx, int 
     const int pos = (col ? r.z_ptr[col - 1] : 0) + rank;
     if ((unsigned)pos >= (unsigned)n) return;
     if (q == 0) {
-        r.z_idx[pos] = c.w;
         r.permutation[i] = pos;
-        if (r.row_cols) r.row_cols[pos] = col;
+        if ((int)gridDim.x == row_blocks) { // no workgroups for the columns
+            r.z_idx[pos] = c.w;
+            if (r.row_cols) r.row_cols[pos] = col;
+        }
     }
     if (r.feature) ((G *)r.out)[(long)pos * gpr + q] = ((const G *)r.feature)[(long)i * gpr + q];
 }
@@ -357,12 +382,13 @@ SPH_EXPORT int sph_init_tensor_rows(const int32_t *indices, int n, int B, int S0
         r.out = (char *)out_feature;
         gpr = row_bytes / gran;
     }
-    const dim3 grid((unsigned)(((long)n * gpr + 255) / 256 + (n == 0)));
+    const int row_blocks = (int)(((long)n * gpr + 255) / 256 + (n == 0));
+    const dim3 grid((unsigned)row_blocks + (unsigned)(coo_by_columns(n, ncol, l.words) ? sph_div_up(ncol, 256) : 0));
     switch (here ? gran : 16) {
-    case 16: hipLaunchKernelGGL(coo_place_kernel<uint4>, grid, block, 0, st, indices, n, g, r, gpr); break;
-    case 4: hipLaunchKernelGGL(coo_place_kernel<uint32_t>, grid, block, 0, st, indices, n, g, r, gpr); break;
-    case 2: hipLaunchKernelGGL(coo_place_kernel<uint16_t>, grid, block, 0, st, indices, n, g, r, gpr); break;
-    default: hipLaunchKernelGGL(coo_place_kernel<uint8_t>, grid, block, 0, st, indices, n, g, r, gpr); break;
+    case 16: hipLaunchKernelGGL(coo_place_kernel<uint4>, grid, block, 0, st, indices, n, g, r, gpr, row_blocks); break;
+    case 4: hipLaunchKernelGGL(coo_place_kernel<uint32_t>, grid, block, 0, st, indices, n, g, r, gpr, row_blocks); break;
+    case 2: hipLaunchKernelGGL(coo_place_kernel<uint16_t>, grid, block, 0, st, indices, n, g, r, gpr, row_blocks); break;
+    default: hipLaunchKernelGGL(coo_place_kernel<uint8_t>, grid, block, 0, st, indices, n, g, r, gpr, row_blocks); break;
     }
     rc = sph_check_launch(who);
     if (rc) return rc;
