@@ -17,6 +17,9 @@ namespace {
 // 13.2 (19.3 -> 15.8), stride 2 on 12 744 tiles 62.6 -> 45.0 (76.5 -> 56.5), 6355 tiles 33.3 -> 24.8 (40.3 -> 30.8).  A single
 // scan's 926 tiles last as long either way (9.1 : 9.0), but three scans in flight 19.5 us a scan against 21.7; at 300 tiles the
 // tile's chain counts (8.4 : 7.9), and 914 tiles of a transposed book are 11.4 : 10.9 (there 1024 is the line).
+// Long fibers (four entries on average) are the masks' of rules_tile.h, but a row of a transposed book meets at most two columns
+// of three on each line, and walks them in less time than masks take up to 16 entries a column: 1336 tiles of a ragged scene 28.6 ->
+// 21.9, 1230 tiles, 16 entries 14.5 -> 12.1, 3277 tiles, 16 entries 26.8 -> 23.2, but 4101 tiles, 32 entries 34.0 : 36.9.
 // On the way: with the checks of the rows' columns before the pointers are asked for, entries past a column's second one by one,
 // the table read an offset at a time, and masks kept from the counting for the placing (54 scalar registers, spilled), no faster
 // than the general kernel (32 and 72 us).
@@ -26,7 +29,8 @@ constexpr int kRowTag = 24; // a pair in the slot array: gathered row, and the o
 inline bool rows_build_ok(const BuildArgs &a, bool transposed, int KV, int ntiles)
 {
     const int nlines = transposed ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0;
-    return !a.long_fibers && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
+    const bool short_enough = !a.long_fibers || (transposed && (double)a.p_rows <= 16.0 * a.B * a.P.n0 * a.P.n1);
+    return short_enough && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
            a.p_rows < (1 << kRowTag) && (double)a.B * a.Q.n0 * a.Q.n1 < (1 << 24) && (double)a.B * a.P.n0 * a.P.n1 < (1 << 24) &&
            ntiles > (transposed ? 1024 : 512);
 }

@@ -139,3 +139,17 @@ def test_strided(kernel, stride, pad, hint):
            _expected(sides[1], sides[0], shape, kernel, stride, pad, False))
     _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, True, col if hint else None),
            _expected(sides[0], sides[1], oshape, kernel, stride, pad, True))
+
+
+@pytest.mark.parametrize("depth,per_column", [(24, 8.0), (32, 15.0), (12, 2.5)])
+@pytest.mark.parametrize("hint", [True, False])
+def test_transposed_long_columns(depth, per_column, hint):
+    """Four to sixteen rows a column of the gathered side."""
+    batch, shape, kernel, stride, pad = 2, (62, int(2300 / per_column), depth), (3, 3, 3), (2, 2, 2), (1, 1, 1)
+    z_idx, z_ptr, col = _scene(shape, batch, per_column, 6)
+    oshape = [(s + 2 * p - k) // t + 1 for s, k, t, p in zip(shape, kernel, stride, pad)]
+    book = RuleBook.build(z_idx, z_ptr, batch, list(shape), oshape, list(kernel), list(stride), list(pad))
+    assert 4 * book.oz_ptr.numel() <= book.out_rows <= 16 * book.oz_ptr.numel() and book.in_rows > 1024 * L.TILE_ROWS
+    sides = (z_idx, col, shape), (book.oz_idx, _columns(book.oz_ptr, book.out_rows), oshape)
+    _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, True, col if hint else None),
+           _expected(sides[0], sides[1], oshape, kernel, stride, pad, True))
