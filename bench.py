@@ -374,7 +374,7 @@ def kernel_sources_digest():
     taken on): the recorded traffic is only reported while these files are what it was measured on."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("conv.hip", "rules.hip", "fused.hip", "conv_wave.h", "rules_tile.h", "tile_consts.h", "common.h", "pack.h"):
+    for name in ("conv.hip", "rules.hip", "fused.hip", "conv_wave.h", "rules_tile.h", "rules_rows.h", "tile_consts.h", "common.h", "pack.h"):
         with open(os.path.join(ROOT, "sphconv_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()
@@ -436,7 +436,9 @@ def record_traffic(fetch_csv, write_csv, seed, voxels):
         blocks = ((n + 127) // 128 + 7) // 8 * 8        # tiles, rounded up to whole rounds over the 8 XCDs
         tiles = (n + 127) // 128
         wanted = {"conv": ("conv_wave_run_kernel", lambda g: g == blocks * 192),   # wave 0 + two helper waves per tile
-                  "rules": ("build_book_kernel<false, true>", lambda g: g == blocks * 256),
+                  # a workgroup of 128 threads per tile on grids of more than 512
+                  "rules": ("build_rows_kernel<false", lambda g: g == blocks * 128) if tiles > 512 else
+                           ("build_book_kernel<false, true>", lambda g: g == blocks * 256),
                   # one launch: workgroups of 256 threads up to 768 tiles, of 128 beyond
                   "rules_conv": ("rules_conv_kernel", lambda g: g == blocks * (256 if tiles <= 768 else 128))}
         for key, (pat, grid_ok) in wanted.items():
@@ -644,7 +646,8 @@ class Workload:
     def rooflines(self, kern, seed):
         """(the step's dominant kernel, the rule kernel, the convolution kernel): algorithmic bytes per launch over
         the kernel's average duration, against the HBM peak."""
-        rules = self._roofline("build_book_kernel<false,true>", "rules", self.rule_bytes, kern["rulegen_ms"], seed)
+        name = "build_rows_kernel<false,3,3,27,true>" if self.ntiles > 512 else "build_book_kernel<false,true>"
+        rules = self._roofline(name, "rules", self.rule_bytes, kern["rulegen_ms"], seed)
         conv = self._roofline("conv_wave_run_kernel<f16,2,4,false>", "conv", self.conv_bytes, kern["conv_forward_ms"], seed)
         if self.one_launch and getattr(self, "step_launches", 1) == 1:
             name = "rules_conv_kernel<f16,2,4,false,%d>" % (256 if self.ntiles <= 768 else 128)

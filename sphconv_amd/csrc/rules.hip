@@ -19,7 +19,7 @@
 namespace {
 
 // Book builder: one workgroup per tile of R stationary rows (tile_table, then emit_groups); workgroups behind
-// the tiles' pack a weight.
+// the tiles' pack a weight.  Long grids take the kernel of rules_rows.h, dense books by row that of rules_masks.h.
 // LINES: the kernel for joins by lines alone; else the one for masks and columns (long fibers, wide kernels).
 template <bool TRANSPOSED, bool LINES>
 __global__ __launch_bounds__(kThreads) void build_book_kernel(BuildArgs a)

@@ -148,9 +148,10 @@ def layer_geometry(batch, D, W, H, kernel, stride, padding, dilation, subm):
 BY_ROW_MIN_PAIRS = 10.0
 # A book built for a forward pass that is known to go by rows, with no gradient being recorded, leaves
 # its groups out (a fifth of the bytes the rule kernel writes), which moves the break-even down:
-# measured on a 4x32x1024x32 grid, rules + convolution, by rows against by groups: 153/155 us at an
-# estimate of 5.4 pairs per row, 177/205 at 6.75, 215/285 at 8.1 (32->32 fp16); 358/325, 432/460,
-# 502/598 (64->64).  The threshold of such books is this fraction of the one above.
+# measured on a 4x32x1024x32 grid, rules + convolution, by rows against by groups: 99/115 us at an
+# estimate of 5.4 pairs per row, 113/149 at 6.75, 141/194 at 8.1 (32->32 fp16); 273/215, 347/314,
+# 412/413 (64->64): one line between the two.  The threshold of such books is this fraction of the one
+# above (where a book with groups and the table breaks even at 10.8: 298/297 and 653/670).
 BY_ROW_FORWARD_ONLY = 0.65
 
 
