@@ -17,7 +17,7 @@ constexpr int kNbrCols = 64; // distinct columns of a tile that masks are made f
 
 inline bool masks_build_ok(const BuildArgs &a, bool transposed, int KV)
 {
-    return !transposed && a.long_fibers && KV <= 32 && a.book.tile_nbr && !a.book.grp_gather && a.P.n2 + a.cv.p2 <= 64 &&
+    return !transposed && a.long_fibers && KV <= 32 && a.book.tile_nbr && !a.book.grp_gather && a.cv.p2 <= 64 - a.P.n2 &&
            (double)a.Q.n2 * a.cv.s2 < (1 << 22) && a.p_rows < (1 << 28);
 }
 
