@@ -287,7 +287,8 @@ __device__ __forceinline__ void relay_ends(const ConvArgs &a, char *s_acc, int h
     }
 
     int4v fa[NB][NS];              // rows of the run, in their rows' places, of the tile that begins next
-    int gi[RH / kWave], ow[RH / kWave]; // indices of the tile after it
+    int gi[RH / kWave], ow[RH / kWave]; // indices of the tile after it,
+    bool in_run[RH / kWave];            // and whether the run is that long (what is read behind its end are zeros, not "no row")
     unsigned short x_lo, x_hi;     // groups of the run, the tile after that
     unsigned long long stray[RH / kWave] = {}; // its rows that the run has no pair for in their places, a bit for each
     auto load_ko = [&](int t) {
@@ -299,7 +300,8 @@ __device__ __forceinline__ void relay_ends(const ConvArgs &a, char *s_acc, int h
 #pragma unroll
         for (int h = 0; h < RH / kWave; h++) {
             const int at = x_lo * SPH_GROUP + half * RH + h * kWave + lane;
-            const int off = at < x_hi * SPH_GROUP ? (min(t, tile_last) * a.cap * SPH_GROUP + at) * 4 : kOut;
+            in_run[h] = at < x_hi * SPH_GROUP;
+            const int off = in_run[h] ? (min(t, tile_last) * a.cap * SPH_GROUP + at) * 4 : kOut;
             gi[h] = __builtin_amdgcn_raw_buffer_load_b32(r_gat, off, 0, 0);
             ow[h] = __builtin_amdgcn_raw_buffer_load_b32(r_own, off, 0, 0);
         }
@@ -311,7 +313,7 @@ __device__ __forceinline__ void relay_ends(const ConvArgs &a, char *s_acc, int h
 #pragma unroll
         for (int h = 0; h < RH / kWave; h++) {
             const int row = half * RH + h * kWave + lane;
-            const bool here = row < nrows && ow[h] == r0 + row && (unsigned)gi[h] < (unsigned)a.feat_rows;
+            const bool here = row < nrows && in_run[h] && ow[h] == r0 + row && (unsigned)gi[h] < (unsigned)a.feat_rows;
             stray[h] = __builtin_amdgcn_ballot_w64(row < nrows && !here);
             quarters(here ? (int)__umul24((unsigned)gi[h], (unsigned)a.row_bytes) : kOut, off[h]);
         }

@@ -134,3 +134,28 @@ def test_a_weight_that_is_not_finite_reaches_its_pairs_only(hint):
     z_idx, z_ptr = _scene(140000, (64, 1600, 32), 1.6, 12)
     book = RuleBook.build(z_idx, z_ptr, 1, [64, 1600, 32], [64, 1600, 32], [3, 3, 3], [1, 1, 1], [1, 1, 1])
     _check(book, torch.float16, 32, 64, 5, hint=hint, inf=True)
+
+
+@pytest.mark.parametrize("kernel,stride,pad", [((2, 3, 3), (1, 1, 1), (1, 1, 1)), ((3, 2, 3), (1, 1, 1), (1, 1, 1)),
+                                               ((3, 3, 3), (1, 1, 1), (0, 0, 0)), ((3, 3, 3), (2, 2, 2), (1, 1, 1))])
+@pytest.mark.parametrize("dtype,ic,oc", [("f32", 32, 32), ("f16", 64, 64), ("bf16", 16, 16), ("i8", 64, 64)])
+def test_no_pair_at_the_middle_offset_of_the_first_tile(kernel, stride, pad, dtype, ic, oc):
+    """A run claimed at a middle offset that pairs no row with itself (even kernels, padding other than K // 2, a stride),
+    and of which the first tile holds nothing at all: its rows begin with zero, row 0 too."""
+    rng = np.random.default_rng(23)
+    shape, subm = (64, 3200, 32), stride == (1, 1, 1)
+    occ = rng.random((64 * 3200, 32)) < 1.7 / 32
+    odd = int(not subm)                                       # the middle offset's pairs lie an odd number of bins apart
+    occ[:6400, 1 - odd::2] = False                            # (stride 2: at the even ones)
+    col, z = np.nonzero(occ)
+    z_ptr = G.t(np.cumsum(occ.sum(1)).astype(np.int32).reshape(1, 64, 3200))
+    z_idx = G.t(z.astype(np.int32))
+    if subm:
+        book = RuleBook.build_subm(z_idx, z_ptr, 1, list(shape), list(kernel), list(pad))
+    else:
+        book = RuleBook.build(z_idx, z_ptr, 1, list(shape), [(s + 2 * p - k) // t + 1 for s, k, t, p in zip(shape, kernel, stride, pad)],
+                              list(kernel), list(stride), list(pad))
+    mid, koff = book.kv // 2, book.fwd.tile_koff[:book.fwd.ntiles].int()
+    assert book.fwd.ntiles > 2048 and koff[0, mid] == koff[0, mid + 1] and (koff[:, mid] < koff[:, mid + 1]).any()
+    for hint in (0, 1):
+        _check(book, TYPES[dtype], ic, oc, 31, hint=hint)
