@@ -30,7 +30,12 @@ inline bool rows_build_ok(const BuildArgs &a, bool transposed, int KV, int ntile
 {
     const int nlines = transposed ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0;
     const bool short_enough = !a.long_fibers || (transposed && (double)a.p_rows <= 16.0 * a.B * a.P.n0 * a.P.n1);
-    return short_enough && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
+    // the coordinates' products are signed 24-bit ones: an axis, stride or padding of up to 2^22 (a coordinate and a padding
+    // add up) keeps every factor below 2^23; columns are divided by unsigned ones
+    const int most = 1 << 22;
+    const bool small = a.Q.n0 <= most && a.Q.n1 <= most && a.Q.n2 <= most && (double)a.B * a.P.n0 <= most && a.P.n1 <= most &&
+                       a.cv.s0 <= most && a.cv.s1 <= most && a.cv.s2 <= most && a.cv.p0 <= most && a.cv.p1 <= most;
+    return small && short_enough && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
            a.p_rows < (1 << kRowTag) && (double)a.B * a.Q.n0 * a.Q.n1 < (1 << 24) && (double)a.B * a.P.n0 * a.P.n1 < (1 << 24) &&
            ntiles > (transposed ? 1024 : 512);
 }

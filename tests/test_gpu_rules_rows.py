@@ -153,3 +153,22 @@ def test_transposed_long_columns(depth, per_column, hint):
     sides = (z_idx, col, shape), (book.oz_idx, _columns(book.oz_ptr, book.out_rows), oshape)
     _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, True, col if hint else None),
            _expected(sides[0], sides[1], oshape, kernel, stride, pad, True))
+
+
+@pytest.mark.parametrize("shape", [(2 ** 23 + 300, 1, 4), (1, 2 ** 23 + 300, 4)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_an_axis_of_more_columns_than_24_bit_products_take(shape, transposed):
+    """Columns on either side of 2 ** 23 on one axis: a coordinate with that bit set is negative to a signed 24-bit product."""
+    axis, rows = shape.index(max(shape)), 150000
+    g = torch.Generator(device="cuda").manual_seed(9)
+    span = 90000                                       # the last columns of the axis
+    occ = torch.rand((span, shape[2]), generator=g, device="cuda") < 1.8 / shape[2]
+    col, z = occ.nonzero(as_tuple=True)
+    assert rows < col.numel()
+    col, z = (col + shape[axis] - span).int(), z.int().contiguous()
+    z_ptr = torch.bincount(col.long(), minlength=shape[axis]).cumsum(0).int().view(1, *shape[:2])
+    kernel, pad = (3, 3, 3), (1, 1, 1)
+    book = RuleBook.build_subm(z, z_ptr, 1, list(shape), list(kernel), lazy=True)
+    assert book.out_rows > 1024 * L.TILE_ROWS
+    side = z, col, shape
+    _check(_build(z, z_ptr, z, z_ptr, book, transposed, col), _expected(side, side, shape, kernel, (1, 1, 1), pad, transposed))
