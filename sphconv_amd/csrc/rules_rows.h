@@ -35,7 +35,9 @@ inline bool rows_build_ok(const BuildArgs &a, bool transposed, int KV, int ntile
     const int most = 1 << 22;
     const bool small = a.Q.n0 <= most && a.Q.n1 <= most && a.Q.n2 <= most && (double)a.B * a.P.n0 <= most && a.P.n1 <= most &&
                        a.cv.s0 <= most && a.cv.s1 <= most && a.cv.s2 <= most && a.cv.p0 <= most && a.cv.p1 <= most;
-    return small && short_enough && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
+    // groups are stored sixteen bytes at a time; the caller's arrays need not be aligned to that
+    const bool aligned = (((uintptr_t)a.book.grp_gather | (uintptr_t)a.book.grp_owner) & 15) == 0;
+    return small && aligned && short_enough && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
            a.p_rows < (1 << kRowTag) && (double)a.B * a.Q.n0 * a.Q.n1 < (1 << 24) && (double)a.B * a.P.n0 * a.P.n1 < (1 << 24) &&
            ntiles > (transposed ? 1024 : 512);
 }

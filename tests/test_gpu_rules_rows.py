@@ -172,3 +172,29 @@ def test_an_axis_of_more_columns_than_24_bit_products_take(shape, transposed):
     assert book.out_rows > 1024 * L.TILE_ROWS
     side = z, col, shape
     _check(_build(z, z_ptr, z, z_ptr, book, transposed, col), _expected(side, side, shape, kernel, (1, 1, 1), pad, transposed))
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_arrays_of_a_caller_that_lie_anywhere(transposed):
+    """A book whose arrays are aligned to their elements only: the same book as with arrays of the extension's."""
+    batch, shape, kernel = 3, (31, 3800, 40), (3, 3, 3)
+    z_idx, z_ptr, col = _scene(shape, batch, 0.4, 3)
+    book = RuleBook.build_subm(z_idx, z_ptr, batch, list(shape), list(kernel), lazy=True)
+    buf = _build(z_idx, z_ptr, z_idx, z_ptr, book, transposed, col)
+    assert buf.ntiles > 1024
+    fields = ("tile_ngrp", "tile_koff", "grp_k", "grp_gather", "grp_owner")
+    for shift in (1, 2, 3):
+        own, st = {}, L.Book()
+        for name in fields:
+            own[name] = torch.full((getattr(buf, name).numel() + 8,), -7, dtype=getattr(buf, name).dtype, device="cuda")
+            setattr(st, name, own[name][shift:].data_ptr())
+        st.rows, st.KV = buf.rows, buf.kv
+        L.check(L.lib().sph_rules_build(L.ptr(z_idx), L.ptr(z_ptr), book.in_rows, L.ptr(z_idx), L.ptr(z_ptr), book.out_rows,
+                                        C.byref(book.geom()), int(transposed), C.byref(st), L.ptr(col), L.stream()))
+        used = torch.arange(buf.cap, device="cuda")[None] < buf.tile_ngrp[:buf.ntiles, None]
+        for name in fields:
+            want, got = getattr(buf, name).view(-1), own[name][shift:shift + getattr(buf, name).numel()]
+            assert (own[name][:shift] == -7).all() and (own[name][shift + want.numel():] == -7).all()
+            if name.startswith("grp_"):
+                want, got = (x.view(buf.ntiles, buf.cap, -1)[used] for x in (want, got))
+            assert torch.equal(got, want), name
