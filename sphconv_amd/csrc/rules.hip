@@ -514,12 +514,8 @@ static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_p
         return sph_check_launch(who);
     }
     if (rows_build_ok(a, transposed != 0, KV, nt)) {
-        const bool c3 = a.lines == 3, nl3 = (transposed ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0) == 3;
-#define SPH_ROWS(T, C, NL, KVT) (a.q_rowcol ? build_rows_kernel<T, C, NL, KVT, true> : build_rows_kernel<T, C, NL, KVT, false>)
-        void (*rows)(BuildArgs);
-        if (transposed) rows = KV == 27 && !c3 && !nl3 ? SPH_ROWS(true, 2, 2, 27) : (c3 ? SPH_ROWS(true, 3, 3, 32) : SPH_ROWS(true, 2, 3, 32));
-        else rows = KV == 27 && c3 && nl3 ? SPH_ROWS(false, 3, 3, 27) : (c3 ? SPH_ROWS(false, 3, 3, 32) : SPH_ROWS(false, 2, 3, 32));
-#undef SPH_ROWS
+        void (*rows)(BuildArgs) = transposed ? (a.q_rowcol ? rows_kernel<true, true>(a, KV) : rows_kernel<true, false>(a, KV))
+                                             : (a.q_rowcol ? rows_kernel<false, true>(a, KV) : rows_kernel<false, false>(a, KV));
         const int pack_rows = pack ? sph_div_up(sph_pack_total(pack->job), kRowThreads) : 0;
         lds = (size_t)R * KV * sizeof(int32_t) + kRowScratch;
         const int rc = allow_lds(rows, lds, who);

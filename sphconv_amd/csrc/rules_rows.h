@@ -1,35 +1,59 @@
 // Rule generation with a thread per stationary row, for long grids (included by rules.hip).
 #pragma once
+#include <climits>
+#include <type_traits>
+
 #include "rules_tile.h"
 
 namespace {
 
 // The kernel of rules_tile.h is made for the length of one tile's chain: 256 threads, two or more items of work each, and on
 // large grids a vector ALU that is 90 % busy with 2460 instructions a tile.  This one is made for few of them (1310): a thread
-// has one row and takes the entries of its up to NL x C columns column by column, keeps the offsets it found a pair at as bits
+// has one row and takes the entries of its NL x C columns column by column, keeps the offsets it found a pair at as bits
 // of one register, and writes only the pairs it found (the table needs no clearing and is read where a bit is set).  A wave
 // takes its own 64 rows through all offsets: a ballot per offset, counts in the lanes of one register, one exchange of counts
 // between the tile's two waves.  The pairs go to their slots tagged with their owner's row, and out sixteen bytes at a time.
 // Books with up to 32 offsets and rows below 2^24.  The rows' columns come from the caller's table or from a search by the
 // workgroup (in a tile with a table entry that turns out wrong every thread searches for its row's own).
 // What bounds it: the vector ALU, 72 % busy over the kernel (5890 tiles), between the ends of nine workgroups' rounds.
-// us, before -> now, with the rows' columns (without): submanifold 5890 tiles 31.8 -> 21.5 (37.8 -> 26.9), 2376 tiles 16.4 ->
-// 13.2 (19.3 -> 15.8), stride 2 on 12 744 tiles 62.6 -> 45.0 (76.5 -> 56.5), 6355 tiles 33.3 -> 24.8 (40.3 -> 30.8).  A single
-// scan's 926 tiles last as long either way (9.1 : 9.0), but three scans in flight 19.5 us a scan against 21.7; at 300 tiles the
-// tile's chain counts (8.4 : 7.9), and 914 tiles of a transposed book are 11.4 : 10.9 (there 1024 is the line).
-// Long fibers (four entries on average) are the masks' of rules_tile.h, but a row of a transposed book meets at most two columns
-// of three on each line, and walks them in less time than masks take up to 16 entries a column: 1336 tiles of a ragged scene 28.6 ->
-// 21.9, 1230 tiles, 16 entries 14.5 -> 12.1, 3277 tiles, 16 entries 26.8 -> 23.2, but 4101 tiles, 32 entries 34.0 : 36.9.
+// us, the kernel of rules_tile.h -> this one, with the rows' columns (without), columns of one to three entries as a scan has
+// them: submanifold 3x3x3 530 tiles 7.8 -> 6.9 (8.7 -> 8.0), 930 tiles 8.6 -> 7.2 (9.5 -> 8.4), 2400 tiles 15.9 -> 12.8 (18.4 ->
+// 15.2), 5890 tiles 31.8 -> 21.5 (37.8 -> 26.9); 3x3x1 530 tiles 6.5 -> 6.1 (7.5 -> 7.1), 1x3x3 6.0 -> 5.1 (7.0 -> 5.9); stride 2
+// transposed 1100 tiles 19.0 -> 12.9, 2400 tiles 32.1 -> 21.3.  A call among others gains more: three scans of 926 tiles in
+// flight 21.7 -> 19.5 us a scan.
+// Asking for as many lines and columns as the call has, instead of three by three, is what keeps small kernels
+// here: 1x3x3 as three lines 530 tiles 6.7, 4800 tiles 16.8, as one 5.1 and 10.9; 3x1x1 with stride 2 transposed 1100 tiles 9.0, now 6.1.
 // On the way: with the checks of the rows' columns before the pointers are asked for, entries past a column's second one by one,
 // the table read an offset at a time, and masks kept from the counting for the placing (54 scalar registers, spilled), no faster
-// than the general kernel (32 and 72 us).
+// than the general kernel (32 and 72 us); a test of every column before its third entry 10 % slower.
 constexpr int kRowThreads = R;
 constexpr int kRowTag = 24; // a pair in the slot array: gathered row, and the owner's row in the tile from this bit on
 
+// Lines of the gathered grid a row can pair with.
+inline int rows_lines(const BuildArgs &a, bool transposed) { return transposed ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0; }
+
 inline bool rows_build_ok(const BuildArgs &a, bool transposed, int KV, int ntiles)
 {
-    const int nlines = transposed ? (a.cv.K0 + a.cv.s0 - 1) / a.cv.s0 : a.cv.K0;
-    const bool short_enough = !a.long_fibers || (transposed && (double)a.p_rows <= 16.0 * a.B * a.P.n0 * a.P.n1);
+    const int nlines = rows_lines(a, transposed);
+    // Entries a column of the gathered side holds on average.  A round takes as long as the wave's longest column needs, so what
+    // has many or uneven ones stays with the kernels of rules_tile.h until there are tiles enough.  us, theirs : this one's,
+    // submanifold 3x3x3:
+    //   1 to 3 entries in 60 % of the columns   530 tiles  7.8 :  6.9   930 tiles  8.6 :  7.2   2400 tiles 15.9 : 12.8
+    //   Poisson, 1.2 a column                   530 tiles  7.7 :  8.0   930 tiles  8.6 :  8.7   2400 tiles 15.9 : 14.5
+    //   Poisson, 3.9 a column                   600 tiles  9.8 : 10.5  1300 tiles 13.0 : 12.6   3000 tiles 22.9 : 20.7
+    //   3.9, in a third of the columns          600 tiles 12.2 : 15.5  1300 tiles 16.4 : 17.5   3000 tiles 28.8 : 28.7
+    //   512 bins, 8.0 in a third                600 tiles 15.7 : 21.2  1300 tiles 18.9 : 22.9   3000 tiles 32.5 : 39.5
+    // A row of a transposed book meets at most two columns of three on each line; what it replaces there is, up to 64 bins and
+    // from four entries on, the join by masks.  Stride 2 transposed:
+    //   64 bins, 12.5 entries a column   1100 tiles 19.0 : 12.9   2400 tiles 32.1 : 21.3  (32 entries 4101 tiles 34.0 : 36.9)
+    //   256 bins, 13                     1100 tiles 14.2 : 15.0   1700 tiles 19.5 : 16.9   3000 tiles 27.7 : 26.1
+    //   256 bins, 25                     1100 tiles 17.5 : 18.4   1700 tiles 24.3 : 21.6   3000 tiles 34.9 : 32.6
+    //   256 bins, 48                     1100 tiles 22.9 : 24.6   3000 tiles, in a fifth of the columns 61.0 : 63.5
+    // (at 914 tiles 10.9 : 11.4).
+    const double each = a.p_rows / ((double)a.B * a.P.n0 * a.P.n1);
+    int line;
+    if (transposed) line = each < 4.0 || (a.long_fibers && each <= 16.0) ? 1024 : (!a.long_fibers && each <= 32.0 ? 1536 : INT_MAX);
+    else line = a.long_fibers || each > 4.0 ? INT_MAX : (each <= 1.5 ? 512 : 2048);
     // the coordinates' products are signed 24-bit ones: an axis, stride or padding of up to 2^22 (a coordinate and a padding
     // add up) keeps every factor below 2^23; columns are divided by unsigned ones
     const int most = 1 << 22;
@@ -37,9 +61,8 @@ inline bool rows_build_ok(const BuildArgs &a, bool transposed, int KV, int ntile
                        a.cv.s0 <= most && a.cv.s1 <= most && a.cv.s2 <= most && a.cv.p0 <= most && a.cv.p1 <= most;
     // groups are stored sixteen bytes at a time; the caller's arrays need not be aligned to that
     const bool aligned = (((uintptr_t)a.book.grp_gather | (uintptr_t)a.book.grp_owner) & 15) == 0;
-    return small && aligned && short_enough && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
-           a.p_rows < (1 << kRowTag) && (double)a.B * a.Q.n0 * a.Q.n1 < (1 << 24) && (double)a.B * a.P.n0 * a.P.n1 < (1 << 24) &&
-           ntiles > (transposed ? 1024 : 512);
+    return small && aligned && ntiles > line && a.lines >= 1 && nlines <= 3 && KV <= 32 && a.book.grp_gather && !a.book.tile_nbr &&
+           a.p_rows < (1 << kRowTag) && (double)a.B * a.Q.n0 * a.Q.n1 < (1 << 24) && (double)a.B * a.P.n0 * a.P.n1 < (1 << 24);
 }
 
 // Groups whose slots are in LDS at a time (a tile has 33 to 36 at the densities of a scan): with the table 16.7 KB at 27
@@ -164,8 +187,9 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
     c = min(c, q_ncol - 1);
     }
 
-    // entries t = 0 and 1 of every column, all on their way together, then 2 and 3 where a lane has them, then any more
-    int at[NL][C], n[NL][C], v[NL][C][2]; // at: byte offset of the column's first entry
+    // entries t = 0 and 1 of every column, all on their way together, then 2 and 3 (or to 5) where a lane has them, then four at a
+    // time of the columns that have any left for one of the wave's rows
+    int at[NL][C], n[NL][C]; // at: byte offset of the column's first entry
 #pragma unroll
     for (int j = 0; j < NL; j++) {
 #pragma unroll
@@ -176,24 +200,30 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
             n[j][i] = col_ok[i] && line_ok[j] ? p[j][i + 1] - p[j][i] : 0;
         }
     }
-    auto request = [&](int t) {
-#pragma unroll
-        for (int j = 0; j < NL; j++)
-#pragma unroll
-            for (int i = 0; i < C; i++)
-#pragma unroll
-                for (int q = 0; q < 2; q++) v[j][i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, at[j][i] + 4 * t + 4 * q, 0, 0);
-    };
     unsigned found = 0; // bit k: a pair at offset k
     const int tag = tid << kRowTag;
     int32_t *mine = s_nbr + __mul24(tid, KV);
-    auto pairs = [&](int t) {
+    auto entries = [&](int t, auto number, auto uneven) { // entries t, t + 1, .. of all columns, or (uneven) of those that have one
+        constexpr int N = decltype(number)::value;
+        int v[NL][C][N];
+        bool go[NL][C];
 #pragma unroll
         for (int j = 0; j < NL; j++)
 #pragma unroll
-            for (int i = 0; i < C; i++)
+            for (int i = 0; i < C; i++) {
+                go[j][i] = !decltype(uneven)::value || __any(n[j][i] > t);
+                if (go[j][i]) {
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
+                    for (int q = 0; q < N; q++) v[j][i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, at[j][i] + 4 * t + 4 * q, 0, 0);
+                }
+            }
+#pragma unroll
+        for (int j = 0; j < NL; j++)
+#pragma unroll
+            for (int i = 0; i < C; i++) {
+                if (!go[j][i]) continue;
+#pragma unroll
+                for (int q = 0; q < N; q++) {
                     int z = v[j][i][q];
                     asm volatile("" : "+v"(z)); // (the load stays where it was asked for, and does not move behind the condition)
                     const int k2 = TRANSPOSED ? off_z - __mul24(z, a.cv.s2) : off_z + z;
@@ -203,26 +233,35 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
                         mine[k] = p[j][i] + (tag + t + q);
                     }
                 }
+            }
     };
     int most = 0;
 #pragma unroll
     for (int j = 0; j < NL; j++)
 #pragma unroll
         for (int i = 0; i < C; i++) most = max(most, n[j][i]);
-    request(0);
-    pairs(0);
-    for (int t = 2; __any(most > t); t += 2) {
-        request(t);
-        pairs(t);
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    entries(0, two, std::false_type());
+    if (__any(most > 4)) {
+        entries(2, four, std::false_type());
+        for (int t = 6; __any(most > t); t += 4) entries(t, four, std::true_type());
+    } else if (__any(most > 2)) {
+        entries(2, two, std::false_type());
     }
 
+    constexpr int kBatch = 9; // offsets taken together: table entries read at once, and tests against the number of offsets
     // pairs of every offset in the wave's rows: lane k of `count`
     int count = 0;
 #pragma unroll
-    for (int k = 0; k < KVT; k++)
-        if (KVT < 32 || k < KV) {
-            const int pop = __popcll(__builtin_amdgcn_ballot_w64((found & (1u << k)) != 0));
-            asm("v_writelane_b32 %0, %1, %2" : "+v"(count) : "s"(pop), "n"(k));
+    for (int kb = 0; kb < KVT; kb += kBatch)
+        if (KVT < 32 || kb < KV) {
+#pragma unroll
+            for (int k = kb; k < kb + kBatch && k < KVT; k++)
+                if (KVT < 32 || k < KV) {
+                    const int pop = __popcll(__builtin_amdgcn_ballot_w64((found & (1u << k)) != 0));
+                    asm("v_writelane_b32 %0, %1, %2" : "+v"(count) : "s"(pop), "n"(k));
+                }
         }
     if (lane < 32) s_cnt[wave * 32 + lane] = count;
     lds_barrier();
@@ -241,9 +280,9 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
     const int begin = first * SPH_GROUP + (wave ? cnt0 : 0); // slot of the wave's first pair of offset `lane`
     // the pairs of groups w0 .. w0 + kRowGroups - 1 to their slots
     auto to_slots = [&](int w0, bool all) {
-        constexpr int kBatch = 9; // table entries read together
 #pragma unroll
         for (int kb = 0; kb < KVT; kb += kBatch) {
+            if (KVT == 32 && kb >= KV) continue;
             int e[kBatch];
 #pragma unroll
             for (int i = 0; i < kBatch; i++) e[i] = mine[min(kb + i, KV - 1)];
@@ -293,6 +332,20 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
         lds_barrier();
         store(w0, min(ngrp - w0, kRowGroups));
     }
+}
+
+// The kernel for the call's number of lines and of columns on a line (one to three each), and for 27 offsets where that is 3x3x3.
+template <bool TRANSPOSED, bool HINT>
+inline void (*rows_kernel(const BuildArgs &a, int KV))(BuildArgs)
+{
+    constexpr int cube = TRANSPOSED ? 2 : 3;
+    const int nl = rows_lines(a, TRANSPOSED), c = a.lines;
+    if (KV == 27 && c == cube && nl == cube) return build_rows_kernel<TRANSPOSED, cube, cube, 27, HINT>;
+    if (KV == 27 && c == 2 && nl == 3) return build_rows_kernel<TRANSPOSED, 2, 3, 27, HINT>;
+#define SPH_ROWS(C, NL) if (c == C && nl == NL) return build_rows_kernel<TRANSPOSED, C, NL, 32, HINT>;
+    SPH_ROWS(1, 1) SPH_ROWS(1, 2) SPH_ROWS(1, 3) SPH_ROWS(2, 1) SPH_ROWS(2, 2) SPH_ROWS(2, 3) SPH_ROWS(3, 1) SPH_ROWS(3, 2)
+#undef SPH_ROWS
+    return build_rows_kernel<TRANSPOSED, 3, 3, 32, HINT>;
 }
 
 } // namespace

@@ -198,3 +198,45 @@ def test_arrays_of_a_caller_that_lie_anywhere(transposed):
             if name.startswith("grp_"):
                 want, got = (x.view(buf.ntiles, buf.cap, -1)[used] for x in (want, got))
             assert torch.equal(got, want), name
+
+
+LINES = [((k0, k1, 3), t) for k0 in (1, 2, 3) for k1 in (1, 2, 3) for t in (False, True)] + \
+        [((3, 3, 1), True), ((3, 3, 2), False), ((1, 1, 32), False), ((2, 1, 13), True), ((3, 3, 3), False), ((2, 3, 5), False)]
+
+
+@pytest.mark.parametrize("hint", [True, False])
+@pytest.mark.parametrize("kernel,transposed", LINES)
+def test_lines_and_columns(kernel, transposed, hint):
+    """One to three lines of one to three columns, kernels of one offset to thirty-two, columns of up to eight entries."""
+    batch, shape, pad = 2, (37, 1700, 40), [k // 2 for k in kernel]
+    z_idx, z_ptr, col = _scene(shape, batch, 1.3, 7)
+    book = RuleBook.build_subm(z_idx, z_ptr, batch, list(shape), list(kernel), lazy=True)
+    assert book.out_rows > 1024 * L.TILE_ROWS and int(torch.diff(z_ptr.view(-1)).max()) > 6
+    side = z_idx, col, shape
+    _check(_build(z_idx, z_ptr, z_idx, z_ptr, book, transposed, col if hint else None),
+           _expected(side, side, shape, kernel, (1, 1, 1), pad, transposed))
+
+
+@pytest.mark.parametrize("shape,per_column,share", [((64, 1500, 40), 1.6, 1.0), ((64, 1250, 64), 3.7, 0.3), ((64, 4100, 512), 1.3, 0.1),
+                                                    ((64, 1300, 512), 3.9, 0.3), ((64, 600, 512), 8.0, 0.5)])
+@pytest.mark.parametrize("kernel,stride,transposed", [((3, 3, 3), (1, 1, 1), False), ((3, 3, 3), (2, 2, 2), False),
+                                                      ((3, 3, 3), (2, 2, 2), True), ((1, 3, 3), (1, 2, 2), True)])
+def test_uneven_columns(shape, per_column, share, kernel, stride, transposed):
+    """Books of either side of every line on the entries of a column, with rows in a share of the columns only."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    ncol, pad = shape[0] * shape[1], [k // 2 for k in kernel]
+    occ = torch.rand((ncol, shape[2]), generator=g, device="cuda") < per_column / share / shape[2]
+    occ &= torch.rand((ncol, 1), generator=g, device="cuda") < share
+    col, z = occ.nonzero(as_tuple=True)
+    z_idx, col = z.int().contiguous(), col.int().contiguous()
+    z_ptr = occ.sum(1).cumsum(0).int().view(1, *shape[:2]).contiguous()
+    if stride == (1, 1, 1):
+        book, oshape = RuleBook.build_subm(z_idx, z_ptr, 1, list(shape), list(kernel), lazy=True), shape
+    else:
+        oshape = [(s + 2 * p - k) // t + 1 for s, k, t, p in zip(shape, kernel, stride, pad)]
+        book = RuleBook.build(z_idx, z_ptr, 1, list(shape), oshape, list(kernel), list(stride), pad, lazy=True)
+    ocol = _columns(book.oz_ptr, book.out_rows)
+    ins, outs = (z_idx, col, shape), (book.oz_idx, ocol, oshape)
+    q, p = (ins, outs) if transposed else (outs, ins)
+    _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, transposed, q[1]),
+           _expected(q, p, p[2], kernel, stride, pad, transposed))
