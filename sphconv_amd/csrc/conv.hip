@@ -436,14 +436,14 @@ __global__ __launch_bounds__(512) void conv_rows_kernel_split(ConvArgs a, int nw
 
 // ---------------------------------------------------------------------------
 // By stationary row, gathered rows staged in LDS: rows of up to 64 bytes (one MFMA K step), up to 64
-// output columns, two waves per tile.
+// output columns, one or two waves per tile.
 //
 // With one K step a (offset, block) step is one or two MFMAs behind a gather of 16 rows; the plain by-row
 // kernel then waits for its gathers (every one a miss of the vector L1: a tile's 27 offsets ask for each
 // neighbouring row about ten times, with the other waves' traffic in between).  The rows a tile's offsets
 // gather lie close together in the feature array: for 9 consecutive offsets (one value of k0 in a 3x3x3
 // kernel) they are the tile's own range of rows of one line of the grid, a column more on either side.
-// So the offsets are taken in phases of 9: the tile's two waves, with 64 rows each, find the range [lo, hi]
+// So the offsets are taken in phases of 9: the tile's waves, with 128 or 64 rows each, find the range [lo, hi]
 // of rows the phase gathers, bring it to LDS as it lies (direct global -> LDS loads, all in flight at once),
 // rewrite the phase's table as one byte per (offset, row) (place in the window; slots without a pair point at
 // a row of zeros behind it), and every step's gather is then one 16-byte LDS read per lane, with nothing to
@@ -455,35 +455,35 @@ __global__ __launch_bounds__(512) void conv_rows_kernel_split(ConvArgs a, int nw
 // With one wave per tile (256 registers: two waves per SIMD) there was less to fill the waits with; two halve a
 // wave's accumulators and table, so three waves share a SIMD, with one window for two of them, at the price of
 // twice the weight loads.  us, one wave a tile -> two, fp16: 32 -> 32 on 12 744 tiles (10.9 pairs a row)
-// 154.6 -> 146.7, 16 -> 32 149.0 -> 140.1; on 4056 tiles (24.8 pairs) 74.3 -> 61.2; on 1248 tiles 23.3 -> 18.2.  With
-// the registers of one wave there was no room for 64 columns either: 32 -> 64 on 4056 tiles, gathers from the feature array
-// against the window, 96.5 : 85.6.  Held to four waves per SIMD (128 registers) it spills and takes 245 us.
+// 154.6 -> 146.7, 16 -> 32 149.0 -> 140.1; on 4056 tiles (24.8 pairs) 74.3 -> 61.2; on 1248 tiles 23.3 -> 18.2 (where one
+// wave is the better one: win_one_wave).  With the registers of one wave there was no room for 64 columns either; with two it
+// depends (win_ok).  Held to four waves per SIMD (128 registers) it spills and takes 245 us.
 // ---------------------------------------------------------------------------
 constexpr int kWinPhase = 9;           // offsets per window
 constexpr int kWinBytes = 16 * 1024;   // bytes of feature rows a window holds (up to 255 rows)
 constexpr int kWinTab = kWinPhase * R; // one byte per (offset, row)
 constexpr int kWinMaxRows = 255;       // most rows of a window: a byte names any of them or the row of zeros
-constexpr int kWinWaves = 2;           // waves of a tile: 64 rows each, one window
-constexpr int kWinRows = R / kWinWaves;
 
-template <sph_dtype DT, int CT, bool MASKED>
-__global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_eu(CT == 4 ? 2 : 3))) void conv_rows_win_kernel(ConvArgs a, int nwtot)
+// W: waves of a tile, R / W rows each, with one window.
+template <sph_dtype DT, int CT, bool MASKED, int W>
+__global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(CT == 4 || W == 1 ? 2 : 3))) void conv_rows_win_kernel(ConvArgs a, int nwtot)
 {
     typedef typename Traits<DT>::elem elem;
     typedef typename Traits<DT>::acc4 acc4;
-    constexpr int NB = kWinRows / SPH_GROUP; // 4 blocks of 16 rows
+    constexpr int RW = R / W;                // rows of a wave
+    constexpr int RL = RW / kWave;           // of which a lane brings the table's entries
+    constexpr int NB = RW / SPH_GROUP;       // blocks of 16 rows
     constexpr int HB = CT == 4 ? 2 : 4;      // blocks per stage
     constexpr int SPO = NB / HB;             // stages per offset
-    static_assert(kWinRows == kWave, "a lane brings its row's entry of every offset");
     constexpr int WR = 3;                    // sets of weight fragments: requested three offsets ahead
     static_assert(kWinPhase % WR == 0, "the ring must divide a phase");
     extern __shared__ __attribute__((aligned(16))) char s_mem[];
-    __shared__ int2 s_range[2][kWinWaves];   // rows a wave's part of the phase gathers, by the phase's parity
+    __shared__ int2 s_range[2][W];   // rows a wave's part of the phase gathers, by the phase's parity
     const int lane = threadIdx.x & (kWave - 1);
     const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    uint8_t *s_tab = (uint8_t *)s_mem + part * (kWinPhase * kWinRows); // [kWinPhase][SPO][16 rows][HB blocks], a wave's own
+    uint8_t *s_tab = (uint8_t *)s_mem + part * (kWinPhase * RW); // [kWinPhase][SPO][16 rows][HB blocks], a wave's own
     char *s_win = s_mem + kWinTab;           // the window's rows, as they lie in the feature array
-    int32_t *s_tab32 = (int32_t *)s_win + part * (kWinPhase * kWinRows); // a phase without a window: [kWinPhase][64] rows of the feature array
+    int32_t *s_tab32 = (int32_t *)s_win + part * (kWinPhase * RW); // a phase without a window: [kWinPhase][RW] rows of the feature array
 
     const int tile = sph_xcd_tile(blockIdx.x, (a.book.rows + R - 1) / R);
     const int r0 = tile * R;
@@ -504,12 +504,14 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int c = 0; c < CT; c++) acc[j][c] = acc4{0, 0, 0, 0};
 
-    int tn[kWinPhase]; // the next phase's table, on its way while this phase is worked through
+    int tn[kWinPhase][RL]; // the next phase's table, on its way while this phase is worked through
     auto load_tab = [&](int ph) {
         const int k0 = min(ph, nph - 1) * kWinPhase;
-        const int32_t *src = a.book.tile_nbr + ((long)tile * KV + k0) * R + part * kWinRows + lane;
+        const int32_t *src = a.book.tile_nbr + ((long)tile * KV + k0) * R + part * RW + lane;
 #pragma unroll
-        for (int i = 0; i < kWinPhase; i++) tn[i] = src[min(i, KV - 1 - k0) * R];
+        for (int i = 0; i < kWinPhase; i++)
+#pragma unroll
+            for (int r = 0; r < RL; r++) tn[i][r] = src[min(i, KV - 1 - k0) * R + r * kWave];
     };
     auto load_w = [&](int k, int4v (&w)[CT]) {
         const char *wk = wlane + (long)min(k, KV - 1) * wstep;
@@ -525,13 +527,15 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
         const int k0 = ph * kWinPhase;
         const int nk = min(kWinPhase, KV - k0);
         // this phase's table: validate, find the range of rows it gathers
-        int t[kWinPhase], lo = 0x7fffffff, hi = -1;
+        int t[kWinPhase][RL], lo = 0x7fffffff, hi = -1;
 #pragma unroll
-        for (int i = 0; i < kWinPhase; i++) {
-            t[i] = (i < nk && (unsigned)tn[i] < (unsigned)a.feat_rows) ? tn[i] : -1;
-            lo = (int)min((unsigned)lo, (unsigned)t[i]); // (-1 is the largest unsigned number)
-            hi = max(hi, t[i]);
-        }
+        for (int i = 0; i < kWinPhase; i++)
+#pragma unroll
+            for (int r = 0; r < RL; r++) {
+                t[i][r] = (i < nk && (unsigned)tn[i][r] < (unsigned)a.feat_rows) ? tn[i][r] : -1;
+                lo = (int)min((unsigned)lo, (unsigned)t[i][r]); // (-1 is the largest unsigned number)
+                hi = max(hi, t[i][r]);
+            }
         lo = ~wave_max_last(~lo); // lowest: 0x7fffffff, a lane without a pair, is the least of the complements
         hi = wave_max_last(hi);
         // direct loads write LDS behind the back of the LDS unit's own queue: the last phase's reads must
@@ -539,8 +543,8 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (lane == kWave - 1) s_range[ph & 1][part] = make_int2(lo, hi);
         lds_barrier();
-        lo = min(s_range[ph & 1][0].x, s_range[ph & 1][1].x);
-        hi = max(s_range[ph & 1][0].y, s_range[ph & 1][1].y);
+        lo = min(s_range[ph & 1][0].x, s_range[ph & 1][W - 1].x);
+        hi = max(s_range[ph & 1][0].y, s_range[ph & 1][W - 1].y);
         lo = __builtin_amdgcn_readfirstlane(lo);
         hi = __builtin_amdgcn_readfirstlane(hi);
         if (hi < 0) { // no pair at these offsets
@@ -555,13 +559,17 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
         if (win) {
 #pragma unroll
             for (int i = 0; i < kWinPhase; i++)
-                s_tab[i * kWinRows + (lane >> 4) / HB * (SPH_GROUP * HB) + (lane & 15) * HB + (lane >> 4) % HB] =
-                    (uint8_t)(t[i] >= 0 ? t[i] - lo : nrow);
+#pragma unroll
+                for (int r = 0; r < RL; r++) {
+                    const int blk = r * (kWave / SPH_GROUP) + (lane >> 4);
+                    s_tab[i * RW + blk / HB * (SPH_GROUP * HB) + (lane & 15) * HB + blk % HB] =
+                        (uint8_t)(t[i][r] >= 0 ? t[i][r] - lo : nrow);
+                }
             // lane l of load i fills the 16 bytes at i * 1024 + l * 16 of the window
             const int nbytes = nrow * rb;
             const int nld = (nbytes + kWave * 16 - 1) / (kWave * 16);
             const char *src = a.feat + (long)lo * rb;
-            for (int i = part; i < nld; i += kWinWaves) {
+            for (int i = part; i < nld; i += W) {
                 const char *g = src + min((i * kWave + lane) * 16, nbytes - 16);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
                                                  (__attribute__((address_space(3))) void *)(s_win + i * (kWave * 16)), 16, 0, 0);
@@ -574,7 +582,7 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
             constexpr int ns = kWinPhase * SPO;
             auto tab = [&](int st, int (&id)[HB]) {
                 const int sc = min(st, ns - 1);
-                const uint8_t *p = s_tab + (sc / SPO) * kWinRows + (sc % SPO) * (SPH_GROUP * HB) + (lane & 15) * HB;
+                const uint8_t *p = s_tab + (sc / SPO) * RW + (sc % SPO) * (SPH_GROUP * HB) + (lane & 15) * HB;
                 const uint32_t pk = HB == 4 ? *(const uint32_t *)p : *(const uint16_t *)p;
 #pragma unroll
                 for (int j = 0; j < HB; j++) id[j] = (pk >> (8 * j)) & 255;
@@ -618,7 +626,9 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
         } else {
             // the rows lie too far apart: gathers from the feature array, one offset at a time
 #pragma unroll
-            for (int i = 0; i < kWinPhase; i++) s_tab32[i * kWinRows + lane] = t[i];
+            for (int i = 0; i < kWinPhase; i++)
+#pragma unroll
+                for (int r = 0; r < RL; r++) s_tab32[i * RW + r * kWave + lane] = t[i][r];
             load_tab(ph + 1);
 #pragma unroll 1
             for (int k9 = 0; k9 < nk; k9++) {
@@ -630,7 +640,7 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
                     int4v x[HB];
 #pragma unroll
                     for (int j = 0; j < HB; j++) {
-                        id[j] = s_tab32[k9 * kWinRows + (h * HB + j) * SPH_GROUP + (lane & 15)];
+                        id[j] = s_tab32[k9 * RW + (h * HB + j) * SPH_GROUP + (lane & 15)];
                         x[j] = *(const int4v *)(a.feat + (long)max(id[j], 0) * rb + choff);
                     }
 #pragma unroll
@@ -664,7 +674,7 @@ __global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_
     elem *out = (elem *)a.out + (long)r0 * a.ndim;
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const int row = part * kWinRows + b * SPH_GROUP + (lane & 15);
+        const int row = part * RW + b * SPH_GROUP + (lane & 15);
         if (row >= nrows) continue;
 #pragma unroll
         for (int c = 0; c < CT; c++) {
@@ -1290,6 +1300,35 @@ int launch_conv_wave_ct(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st
     }
 }
 
+// Whether a layer of one K step goes through the window.  With up to 32 columns always, on grids of more than 1024 tiles (shorter
+// ones are faster with four waves per tile: 312 tiles, 32 -> 32 fp16, 17.2 : 19.2 us).  With 64 columns two waves of a tile have
+// only two waves of a SIMD beside them, and it depends.  Times with the window over times without, 3x3x3, 0.4 of the bins:
+//   tiles             260   400   600   800  1000  1100  1250  1500  1800  2000  3000  4000
+//   fp16 32 -> 64    0.92  0.91  0.74  0.62  0.64  0.96  0.95  0.96  0.84  0.95  0.80  0.84
+//   int8 64 -> 64    0.93  0.93  0.73  0.61  0.62  0.86  0.85  0.89  0.80  0.83  0.72  0.82
+//   fp32 16 -> 64    1.44  1.43  0.99  0.87  0.88  0.82  0.94  1.06  1.04  1.12  1.03  1.06   (5x3x3: 0.90 0.93 0.83 0.88 at the end)
+//   fp16, 3x3x1      1.09  1.16  0.94  0.78  0.81  1.43  1.43  1.42  1.24  1.35  1.26  1.35   (one phase: nothing overlaps its window)
+//   fp16, 2x2x2      1.29  1.30  1.15  0.92  0.93  1.49  1.52  1.56  1.40  1.43  1.37  1.54   (a phase costs nine offsets; 3x2x2 alike)
+//   fp16, stride 2   1.36  1.32  1.13        0.95        1.33        1.11  1.22  0.99  1.02   (3.2 gathered rows to a row: windows too small;
+//   stride 1,2,2     0.94  1.02  0.83        0.72        1.05        0.91  0.98  0.88  0.92    1.6 to a row: they fit)
+template <sph_dtype DT, int CT>
+bool win_ok(const ConvArgs &a, int ntiles)
+{
+    if (CT < 4) return ntiles > 1024;
+    if (a.book.KV % kWinPhase != 0 || a.feat_rows > 2.0 * a.book.rows) return false;
+    if (a.book.KV == kWinPhase) return ntiles > 768 && ntiles <= 1024;
+    if (DT == SPH_F32) return ntiles > 768 && (ntiles <= 1280 || a.book.KV > 4 * kWinPhase);
+    // (without it 2048 tiles are on the chip at once: 2037 tiles, 6.9 pairs a row, fp16 32 -> 64 1.09, 16 -> 64 1.16; int8 1.04)
+    if (DT != SPH_I8 && ntiles > 1920 && ntiles <= 2048) return false;
+    return ntiles > 256;
+}
+
+// One wave per tile instead of two (32 columns): with two 1536 tiles are on the chip at once, with one 2048.  us, one : two:
+// fp16 32 -> 32 1500 tiles 23.9 : 19.7, 1800 tiles 24.9 : 27.7, 2300 tiles 39.5 : 31.3, 4000 tiles 52.0 : 51.1; fp32 16 -> 32 1250
+// tiles 66.2 : 52.6, 2000 tiles 71.4 : 86.5, 3300 tiles 135.2 : 130.5, 4000 tiles 138.8 : 146.0 (its matrix cores leave fewer waits to fill).
+template <sph_dtype DT>
+bool win_one_wave(int ntiles) { return (ntiles > 1536 && ntiles <= 2048) || (DT == SPH_F32 && ntiles > 3584); }
+
 template <sph_dtype DT, int NS, int CT, bool MASKED>
 int launch_conv_rows_m(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
 {
@@ -1300,10 +1339,16 @@ int launch_conv_rows_m(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
     const size_t lds = (size_t)a.book.KV * R * sizeof(int32_t) + (NS >= 2 ? (size_t)waves * ws * 4 * SPH_GROUP * 80 : 0);
     const dim3 grid(sph_xcd_grid(ntiles)), block(waves * ws * kWave);
     if constexpr (NS == 1) {
-        // one K step, up to 64 columns: the gathered rows go through an LDS window.  Short grids are faster with four waves per
-        // tile: 312 tiles 17.2 : 19.2 us with 32 columns, but 23.3 : 20.9 with 64.
-        if (waves == 1 && (CT == 4 ? ntiles > 256 : ws == 1)) {
-            hipLaunchKernelGGL((conv_rows_win_kernel<DT, CT, MASKED>), grid, dim3(kWinWaves * kWave), kWinTab + kWinBytes + 64, st, a, nwtot);
+        // one K step, up to 64 columns: the gathered rows go through an LDS window
+        if (waves == 1 && win_ok<DT, CT>(a, ntiles)) {
+            const size_t lds_win = kWinTab + kWinBytes + 64;
+            if constexpr (CT == 2) {
+                if (win_one_wave<DT>(ntiles)) {
+                    hipLaunchKernelGGL((conv_rows_win_kernel<DT, CT, MASKED, 1>), grid, dim3(kWave), lds_win, st, a, nwtot);
+                    return sph_check_launch("sph_conv_apply");
+                }
+            }
+            hipLaunchKernelGGL((conv_rows_win_kernel<DT, CT, MASKED, 2>), grid, dim3(2 * kWave), lds_win, st, a, nwtot);
             return sph_check_launch("sph_conv_apply");
         }
     }

@@ -39,14 +39,29 @@ def _table(nt, kv, rows, gen):
 @pytest.mark.parametrize("ic,oc,dtype", [(32, 32, torch.float16), (32, 64, torch.bfloat16), (24, 40, torch.float16), (8, 16, torch.float16),
                                          (16, 16, torch.bfloat16), (16, 64, torch.float32), (64, 64, torch.int8), (32, 16, torch.int8)])
 def test_window(monkeypatch, kernel, ic, oc, dtype):
+    _check(monkeypatch, kernel, ic, oc, dtype, 1030)
+
+
+@pytest.mark.parametrize("kernel,ic,oc,dtype,tiles", [
+    ([3, 3, 3], 32, 32, torch.float16, 1537), ([3, 3, 1], 24, 24, torch.bfloat16, 2048), ([3, 3, 3], 32, 32, torch.int8, 1600),
+    ([2, 2, 3], 16, 32, torch.float32, 1700), ([3, 3, 3], 8, 24, torch.float32, 3585), ([3, 3, 2], 32, 24, torch.float16, 2049),
+    ([3, 3, 3], 32, 64, torch.float16, 257), ([3, 3, 3], 64, 48, torch.int8, 256), ([3, 3, 1], 16, 64, torch.bfloat16, 769),
+    ([3, 3, 1], 32, 64, torch.float16, 1024), ([3, 3, 2], 32, 48, torch.bfloat16, 300), ([3, 3, 5], 16, 64, torch.float32, 1281),
+    ([3, 3, 3], 16, 64, torch.bfloat16, 1921), ([3, 3, 3], 16, 48, torch.float32, 1280), ([2, 2, 2], 32, 64, torch.float16, 1300)])
+def test_either_side_of_the_lines(monkeypatch, kernel, ic, oc, dtype, tiles):
+    """One wave per tile and two, 64 columns with the window and without, at the sizes where one takes over from the other."""
+    _check(monkeypatch, kernel, ic, oc, dtype, tiles)
+
+
+def _check(monkeypatch, kernel, ic, oc, dtype, tiles):
     monkeypatch.setattr(rulebook, "BY_ROW_MIN_PAIRS", 0.0)
     gen = torch.Generator(device="cuda").manual_seed(ic + oc)
-    rows = 1029 * 128 + 57
+    rows = (tiles - 1) * 128 + 57
     z_ptr = torch.arange(1, rows + 1, device="cuda").int().view(1, 1, rows)
     book = RuleBook.build_subm(torch.zeros(rows, dtype=torch.int32, device="cuda"), z_ptr, 1, [1, rows, 1], kernel,
                                padding=[k // 2 for k in kernel])
     buf = book.fwd
-    assert buf.tile_nbr is not None and buf.ntiles == 1030
+    assert buf.tile_nbr is not None and buf.ntiles == tiles
     buf.tile_nbr.copy_(_table(buf.ntiles, buf.kv, rows, gen))
     nbr = buf.tile_nbr.permute(0, 2, 1).reshape(-1, buf.kv)[:rows].long()
     if dtype == torch.int8:
