@@ -2,7 +2,7 @@
 //
 // The kernels of conv.hip give a tile of 128 rows to a workgroup, which loads the weight fragments of a group with the
 // group: 8 of the 10 KiB that a group of 16 pairs takes through the compute unit's vector memory path at 64 -> 64 in 16 bit.
-// All 27 offsets' fragments are 221 KiB, which no LDS holds but a compute unit's registers do (512 KiB).  So here a workgroup is
+// All 27 offsets' fragments are 216 KiB, which no LDS holds but a compute unit's registers do (512 KiB).  So here a workgroup is
 // as large as a compute unit and stays for many tiles; three stages of waves keep the fragments of a third of the offsets each,
 // and the tiles pass from stage to stage, one barrier a tile, with their accumulators in LDS (four tiles in flight):
 //   stage 3 gives a tile its first sums (the middle offset's run, or zeros),
@@ -507,24 +507,37 @@ int relay_launch_m(const ConvArgs &a, int ntiles, hipStream_t st)
 
 } // namespace
 
-// Where the relay kernel is the faster one, us against the kernels of conv.hip (a tile takes five steps, so a short grid is all
-// start and end):
-//   64 -> 64 fp16   893 tiles 20.1 : 22.5   1485 tiles 24.2 : 34.3   2376 tiles 32.0 : 47.1
-//   32 -> 64 fp16   893 tiles 17.4 : 16.9   1485 tiles 20.6 : 25.2   2376 tiles 26.4 : 33.7
-//   32 -> 32 fp32   893 tiles 26.1 : 21.2   1485 tiles 33.9 : 42.6   2376 tiles 42.8 : 52.0
-//   32 -> 32 fp16  1485 tiles 16.1 : 15.6   2376 tiles 18.8 : 23.9   4871 tiles 25.6 : 33.6
-//   64 -> 16 bf16  1485 tiles 17.9 : 19.3   2420 tiles 21.5 : 24.5   4871 tiles 31.3 : 41.9
-//   16 -> 16 fp16  1485 tiles 12.9 : 12.7   2420 tiles 14.8 : 15.1   4871 tiles 19.3 : 23.7
-// (inputs mostly from the caches; the weight's copy in fragment order is in all of them.)  Kernels of up to
-// nine offsets stay with conv.hip: their weight is a third and a tile's groups meet three stages unevenly (3x3x1 64 -> 64 of
+// Tiles above which the relay is the faster one (a tile takes five steps, so a short grid is all start and end), in a call on its
+// own and with three scans in flight, where the kernels of conv.hip fill one another's ends and the relay, which takes whole
+// compute units, keeps the others out.  us of rules + convolution, conv.hip : relay, alone and in flight, scans of 1.5 to 2 pairs a row:
+//   64 -> 64 fp16   1065 tiles 38.1 : 33.1, 23.1 : 24.0   1207 tiles 42.0 : 33.8, 26.7 : 26.4   2003 tiles 57.2 : 45.0, 47.5 : 38.3
+//   32 -> 64 fp16   1065 tiles 29.4 : 27.1, 14.7 : 17.9   1804 tiles 37.2 : 36.1, 28.5 : 27.9   2205 tiles 44.8 : 40.5, 34.4 : 32.8
+//   64 -> 64 int8   1065 tiles 30.7 : 28.9, 16.1 : 19.1   1804 tiles 39.0 : 36.3, 28.0 : 28.7   2205 tiles 47.1 : 40.9, 35.2 : 33.6
+//   32 -> 32 fp32   1207 tiles 37.8 : 41.1, 27.0 : 31.8   1355 tiles 50.7 : 44.7, 29.6 : 34.3   2205 tiles 64.0 : 54.8, 47.7 : 47.2
+//   32 -> 64 fp32   1065 tiles 63.8 : 51.8, 39.4 : 39.4   1207 tiles 76.2 : 52.7, 44.0 : 42.5   2205 tiles 106  : 76.9, 80.0 : 67.4
+//   32 -> 32 fp16   2205 tiles 35.1 : 29.8, 25.7 : 24.0
+//   16 -> 32 fp32   2205 tiles 44.4 : 39.9, 31.8 : 33.3   2609 tiles 50.0 : 45.5, 37.5 : 37.9   3212 tiles 59.8 : 51.9, 47.3 : 45.1
+//   16 -> 16 fp16   2205 tiles 23.6 : 24.9, 15.1 : 16.4   3212 tiles 32.8 : 32.2, 25.3 : 24.2   4215 tiles 42.7 : 38.5, 33.9 : 30.5
+//    4 -> 16 fp32   3212 tiles 36.4 : 39.3, 27.2 : 29.8   4215 tiles 47.0 : 46.5, 36.5 : 37.1   6013 tiles 64.8 : 60.8, 54.6 : 50.5
+// Kernels of up to nine offsets stay with conv.hip: their weight is a third and a tile's groups meet three stages unevenly (3x3x1 64 -> 64 of
 // stride 2 on 5029 tiles 62.4 : 51.4, submanifold on 4871 tiles 49.5 : 58.3).
+static int relay_line(sph_dtype dt, int nsteps, int nwtot, bool in_flight)
+{
+    const int fragments = nsteps * nwtot; // of one offset: what the relay keeps in registers and the others load with every group
+    if (fragments == 1) return 3584;
+    if (fragments == 2) return in_flight ? 2560 : 2048;
+    if (!in_flight) return dt == SPH_F32 && nwtot == 2 ? 1280 : 1024;
+    if (dt == SPH_F32 && nwtot == 4) return 1152;
+    return fragments == 8 ? 1280 : 1920;
+}
+
 bool sph_relay_ok(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles)
 {
     const int KV = a.book.KV;
     if (!a.aligned_in || !a.aligned_out || a.nsteps > 2 || nwtot > 4) return false;
     if (KV <= kRelayPart || KV > (kRelayStages - 1) * kRelayPart) return false;
     if ((double)ntiles * a.cap * SPH_GROUP * 4 >= 2147483648.0) return false; // 32-bit offsets into the book
-    return ntiles > (a.nsteps * nwtot >= 4 ? 1024 : 2048);
+    return ntiles > relay_line(dt, a.nsteps, nwtot, a.book.middle_run == SPH_RUN_IN_FLIGHT);
 }
 
 int sph_relay_launch(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)

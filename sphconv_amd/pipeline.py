@@ -58,7 +58,8 @@ class ScanPipeline:
         # kernels overlap better from 768 tiles on (measured at 937 tiles on three streams: 24.7 against 25.9 us per scan)
         self._fused_max_tiles = 768 if len(self._streams) >= 3 else RuleBook.FUSED_MAX_TILES
         for book in self._books:
-            book.struct().middle_run = 1              # submanifold: every row pairs with itself at the middle offset
+            # submanifold: every row pairs with itself at the middle offset
+            book.struct().middle_run = L.RUN_IN_FLIGHT if len(self._streams) >= 3 else L.RUN
         self._packed = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         self._packed_ready = torch.cuda.Event()
         self.fused = bool(fused)

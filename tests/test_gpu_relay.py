@@ -10,6 +10,7 @@ import gpu_helpers as G
 from sphconv_amd import _lib as L
 from sphconv_amd import rulebook
 from sphconv_amd import sphconv_cuda as ext
+from sphconv_amd.pipeline import ScanPipeline
 from sphconv_amd.rulebook import RuleBook
 
 pytestmark = pytest.mark.gpu
@@ -80,7 +81,8 @@ def _check(book, dtype, ic, oc, seed, hint=None, epilogue=False, inf=False):
     assert torch.equal(outs[0].view(torch.int8), outs[1].view(torch.int8)) and (outs[0][m] == 3).all()
     out = outs[0][:m]
     if int8:
-        exact = torch.round(want.float() * scale).clamp(-128, 127)         # integer sums below 2**24: exact in float32
+        assert want.abs().max() < 2 ** 24                                  # integer sums below 2**24: exact in float32
+        exact = torch.round(want.float() * scale).clamp(-128, 127)
         assert torch.equal(out.float(), exact)
         return
     if epilogue:
@@ -102,8 +104,9 @@ def _by_groups(monkeypatch):
 
 @pytest.mark.parametrize("dtype,ic,oc,tiles", [
     ("f16", 64, 64, 1025), ("bf16", 64, 64, 1032), ("f16", 32, 64, 1025), ("bf16", 24, 40, 1027), ("f16", 64, 32, 1025),
-    ("bf16", 40, 24, 1025), ("f32", 16, 64, 1025), ("f32", 32, 32, 1026), ("f32", 4, 16, 2049), ("f16", 16, 16, 2049),
-    ("bf16", 64, 8, 2050), ("f16", 16, 32, 2049), ("i8", 64, 64, 1025), ("i8", 32, 16, 2049), ("i8", 128, 48, 1025)])
+    ("bf16", 40, 24, 1025), ("f32", 16, 64, 1025), ("f32", 32, 32, 1026), ("f32", 32, 32, 1282), ("f32", 4, 16, 2049), ("f32", 4, 16, 3585), ("f16", 16, 16, 2049),
+    ("f16", 16, 16, 3586),
+    ("bf16", 64, 8, 2050), ("f16", 16, 32, 2049), ("i8", 64, 64, 1025), ("i8", 32, 16, 2049), ("i8", 32, 16, 3585), ("i8", 128, 48, 1025)])
 @pytest.mark.parametrize("per_column", [0.9, 4.0])          # one group per offset and tile; two and more (several passes)
 def test_submanifold(dtype, ic, oc, tiles, per_column):
     rows = tiles * L.TILE_ROWS - 77
@@ -119,11 +122,11 @@ def test_submanifold(dtype, ic, oc, tiles, per_column):
 def test_other_kernels(kernel, stride, dtype, ic, oc):
     """Kernel volumes of 10 to 27 offsets, which the gathering waves share unevenly, without the middle offset's run; and with
     a run claimed that is not there (its pairs are strewn over the tile's rows)."""
-    z_idx, z_ptr = _scene(140000, (64, 1600, 32), 1.6, 11)
-    book = RuleBook.build(z_idx, z_ptr, 1, [64, 1600, 32],
-                          [(s + 2 * (k // 2) - k) // t + 1 for s, k, t in zip((64, 1600, 32), kernel, stride)],
+    z_idx, z_ptr = _scene(170000, (64, 1800, 32), 1.6, 11)
+    book = RuleBook.build(z_idx, z_ptr, 1, [64, 1800, 32],
+                          [(s + 2 * (k // 2) - k) // t + 1 for s, k, t in zip((64, 1800, 32), kernel, stride)],
                           list(kernel), list(stride), [k // 2 for k in kernel])
-    assert book.fwd.ntiles > 1024
+    assert book.fwd.ntiles > 1280
     _check(book, TYPES[dtype], ic, oc, 3)
     _check(book, TYPES[dtype], ic, oc, 3, hint=1)
 
@@ -143,12 +146,12 @@ def test_no_pair_at_the_middle_offset_of_the_first_tile(kernel, stride, pad, dty
     """A run claimed at a middle offset that pairs no row with itself (even kernels, padding other than K // 2, a stride),
     and of which the first tile holds nothing at all: its rows begin with zero, row 0 too."""
     rng = np.random.default_rng(23)
-    shape, subm = (64, 3200, 32), stride == (1, 1, 1)
-    occ = rng.random((64 * 3200, 32)) < 1.7 / 32
+    shape, subm = (64, 4400, 32), stride == (1, 1, 1)
+    occ = rng.random((64 * 4400, 32)) < 1.7 / 32
     odd = int(not subm)                                       # the middle offset's pairs lie an odd number of bins apart
     occ[:6400, 1 - odd::2] = False                            # (stride 2: at the even ones)
     col, z = np.nonzero(occ)
-    z_ptr = G.t(np.cumsum(occ.sum(1)).astype(np.int32).reshape(1, 64, 3200))
+    z_ptr = G.t(np.cumsum(occ.sum(1)).astype(np.int32).reshape(1, 64, 4400))
     z_idx = G.t(z.astype(np.int32))
     if subm:
         book = RuleBook.build_subm(z_idx, z_ptr, 1, list(shape), list(kernel), list(pad))
@@ -156,6 +159,58 @@ def test_no_pair_at_the_middle_offset_of_the_first_tile(kernel, stride, pad, dty
         book = RuleBook.build(z_idx, z_ptr, 1, list(shape), [(s + 2 * p - k) // t + 1 for s, k, t, p in zip(shape, kernel, stride, pad)],
                               list(kernel), list(stride), list(pad))
     mid, koff = book.kv // 2, book.fwd.tile_koff[:book.fwd.ntiles].int()
-    assert book.fwd.ntiles > 2048 and koff[0, mid] == koff[0, mid + 1] and (koff[:, mid] < koff[:, mid + 1]).any()
+    assert book.fwd.ntiles > 3584 and koff[0, mid] == koff[0, mid + 1] and (koff[:, mid] < koff[:, mid + 1]).any()
     for hint in (0, 1):
         _check(book, TYPES[dtype], ic, oc, 31, hint=hint)
+
+
+@pytest.mark.parametrize("tiles", [1026, 1282])             # up to 1280 tiles scans in flight take the kernels of conv.hip
+def test_scans_on_three_streams(tiles):
+    """Scans in flight beside one another: each output is that of the call on its own."""
+    rows = tiles * L.TILE_ROWS - 40
+    S1 = int(rows / 64 / 1.5 * 1.1)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = (torch.randn((27, 64, 64), generator=g, device="cuda") / 40).half()
+    pipe = ScanPipeline(w, 1, [64, S1, 32], max_voxels=rows, streams=3)
+    scans = []
+    for seed in range(5):
+        z_idx, z_ptr = _scene(rows - 900 * seed % 1300, (64, S1, 32), 1.5, seed)
+        feat = torch.randn((z_idx.numel(), 64), generator=g, device="cuda").half()
+        book = RuleBook.build_subm(z_idx, z_ptr, 1, [64, S1, 32], [3, 3, 3])
+        scans.append((feat, z_idx, z_ptr, ext.rule_conv(feat, w, book, None, z_idx.numel())))
+    torch.cuda.synchronize()
+    for _ in range(3):
+        held = []
+        for feat, z_idx, z_ptr, want in scans:
+            out, slot = pipe.submit(feat, z_idx, z_ptr)
+            held.append((out, slot, want))
+            if len(held) == 3:
+                for out, slot, want in held:
+                    pipe.wait(slot)
+                    G.assert_same_conv(out, want)
+                held = []
+        for out, slot, want in held:
+            pipe.wait(slot)
+            G.assert_same_conv(out, want)
+
+
+@pytest.mark.parametrize("dtype,ic,oc,tiles", [("f16", 64, 64, 1025), ("f32", 32, 32, 1281)])
+def test_in_a_graph(dtype, ic, oc, tiles):
+    """Captured once, replayed on new features with other work and synchronisations in between: the eager results."""
+    rows = tiles * L.TILE_ROWS - 5
+    S1 = int(rows / 64 / 1.5 * 1.1)
+    z_idx, z_ptr = _scene(rows, (64, S1, 32), 1.5, 4)
+    book = RuleBook.build_subm(z_idx, z_ptr, 1, [64, S1, 32], [3, 3, 3])
+    g = torch.Generator(device="cuda").manual_seed(5)
+    feat = torch.randn((rows, ic), generator=g, device="cuda").to(TYPES[dtype])
+    w = (torch.randn((27, ic, oc), generator=g, device="cuda") / 40).to(TYPES[dtype])
+    ext.rule_conv(feat, w, book, None, rows)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ext.rule_conv(feat, w, book, None, rows)
+    for seed in range(4):
+        feat.copy_(torch.randn((rows, ic), generator=g, device="cuda"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ext.rule_conv(feat, w, book, None, rows))
