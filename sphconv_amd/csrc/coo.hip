@@ -113,11 +113,22 @@ __device__ __forceinline__ bool coo_inside(const int4 &c, const CooGrid &g)
            (unsigned)c.w < (unsigned)g.S2;
 }
 
-__global__ __launch_bounds__(256) void coo_mark_kernel(const int32_t *idx, int n, CooGrid g, unsigned long long *bits, int32_t *status)
+// Whether a wave's rows lie strewn over the grid: more than a quarter of them are not among the next columns of the row before.
+__device__ __forceinline__ bool coo_strewn(const int4 &c, const CooGrid &g)
+{
+    const unsigned col = ((unsigned)c.x * g.S0 + (unsigned)c.y) * g.S1 + (unsigned)c.z;
+    const unsigned before = (unsigned)__shfl_up((int)col, 1, 64);
+    return __popcll(__ballot((threadIdx.x & 63) != 0 && col - before > 32u)) > 16;
+}
+
+// *strewn (zero before, may be null): set where one of the sampled waves finds its rows so
+__global__ __launch_bounds__(256) void coo_mark_kernel(const int32_t *idx, int n, CooGrid g, unsigned long long *bits, int32_t *status,
+                                                       int32_t *strewn)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int4 c = ((const int4 *)idx)[i]; // (b, s0, s1, s2)
+    if (strewn && blockIdx.x % 8 == 0 && coo_strewn(c, g) && threadIdx.x % 64 == 0) *strewn = 1;
     if (!coo_inside(c, g)) {
         atomicAdd(&status[0], 1);
         return;
@@ -161,11 +172,21 @@ struct CooRows {
     const char *feature;                     // null: no rows to move
     char *out;
     int32_t *status, *host_status;           // host_status (may be null): the same two words where the host reads them
+    const int32_t *strewn;                   // null: the rows write z_idx and row_cols; else the columns do where *strewn is not 0
 };
 
-// Whether the columns write what their bits say of their rows.  us of the place kernel, by rows : by columns: 623 k rows in random
-// order, 524 k words 48.7 : 28.7; 94 k rows, 131 k words 6.5 : 5.4; 24 k rows, 262 k words (eight to a column) 4.1 : 5.8.
-inline bool coo_by_columns(int n, int ncol, int words) { return 4 * (double)n >= (double)ncol * words; }
+// Whether the columns may write what their bits say of their rows, a thread each: where the bitmap has few words more than there are
+// rows, and the columns are neither deep nor full (a thread goes through its words and rows one by one).  us of the call, 32-byte
+// features, by rows : by columns, rows in random order:
+//   623 k rows, 524 k columns of 64 bins 78.5 : 65.8      140 k, 524 k columns 31.2 : 30.1    94 k, 131 k columns 19.2 : 18.3
+//   35 k, 131 k columns 14.4 : 14.9     4000, 4096 columns 10.9 : 11.2   (what the mark kernel found is read in front of all else)
+//   20 k, 1024 columns 12.3 : 15.7      200 k, 4096 columns of 128 bins 24.9 : 34.4     200 k, 1024 columns of 4096 bins 55.7 : 120
+// Rows that come in the columns' order write next to one another, and the columns would cost more than they save (623 k rows 38.3 :
+// 40.8): the mark kernel looks at the order of an eighth of the rows, and the place kernel goes by what it found (39.2).
+inline bool coo_by_columns(int n, int ncol, int words)
+{
+    return n >= 65536 && words <= 4 && 4 * (double)n >= (double)ncol * words && n <= 8 * (double)ncol;
+}
 
 // What a column's bits say of its rows, a thread per column: their S2 coordinates and their column.
 __device__ __forceinline__ void coo_columns(int col, int n, const CooGrid &g, const CooRows &r)
@@ -180,13 +201,14 @@ __device__ __forceinline__ void coo_columns(int col, int n, const CooGrid &g, co
 }
 
 // gpr threads per row, one 16-byte (G) granule of its features each; gpr = 1 without features.  z_idx and row_cols are written by
-// rows, two 4-byte writes to lines of their own for each where the rows come in no order, or, where the bitmap has few words
-// more than there are rows (coo_by_columns), by workgroups of the columns behind those of the rows (row_blocks).
+// rows, two 4-byte writes to lines of their own for each where the rows come in no order, or there (coo_by_columns) by
+// workgroups of the columns behind those of the rows (row_blocks).
 template <typename G>
 __global__ __launch_bounds__(256) void coo_place_kernel(const int32_t *idx, int n, CooGrid g, CooRows r, int gpr, int row_blocks)
 {
+    const bool by_columns = r.strewn && *r.strewn != 0;
     if ((int)blockIdx.x >= row_blocks) {
-        coo_columns((blockIdx.x - row_blocks) * 256 + threadIdx.x, n, g, r);
+        if (by_columns) coo_columns((blockIdx.x - row_blocks) * 256 + threadIdx.x, n, g, r);
         return;
     }
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
@@ -213,7 +235,7 @@ __global__ __launch_bounds__(256) void coo_place_kernel(const int32_t *idx, int 
     if ((unsigned)pos >= (unsigned)n) return;
     if (q == 0) {
         r.permutation[i] = pos;
-        if ((int)gridDim.x == row_blocks) { // no workgroups for the columns
+        if (!by_columns) {
             r.z_idx[pos] = c.w;
             if (r.row_cols) r.row_cols[pos] = col;
         }
@@ -354,13 +376,17 @@ SPH_EXPORT int sph_init_tensor_rows(const int32_t *indices, int n, int B, int S0
     SPH_REQUIRE(workspace_bytes >= l.total, SPH_ERR_ARG, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, l.total);
     char *ws = (char *)workspace;
     CooGrid g{B, S0, S1, S2, l.words};
-    CooRows r{z_ptr, (const unsigned long long *)(ws + l.bits), z_idx, permutation, row_cols, nullptr, nullptr, status, host_status};
+    CooRows r{z_ptr, (const unsigned long long *)(ws + l.bits), z_idx, permutation, row_cols, nullptr, nullptr, status, host_status, nullptr};
+    // (the second word of the scan's state is nobody's, and cleared with it)
+    int32_t *strewn = coo_by_columns(n, ncol, l.words) ? (int32_t *)(ws + l.temp) + 1 : nullptr;
+    r.strewn = strewn;
     const long n16 = (long)(l.total / 16);
     hipLaunchKernelGGL(coo_clear_kernel, dim3((unsigned)(n16 < 256L * 2048 ? (n16 + 255) / 256 : 2048)), dim3(256), 0, st,
                        (uint4 *)workspace, n16, status);
     const dim3 block(256);
     if (n > 0)
-        hipLaunchKernelGGL(coo_mark_kernel, dim3(sph_div_up(n, 256)), block, 0, st, indices, n, g, (unsigned long long *)(ws + l.bits), status);
+        hipLaunchKernelGGL(coo_mark_kernel, dim3(sph_div_up(n, 256)), block, 0, st, indices, n, g, (unsigned long long *)(ws + l.bits), status,
+                           strewn);
     hipError_t e;
     switch (l.words) {
     case 1: e = scan_columns<1>(r.bits, 1, z_ptr, ncol, ws + l.temp, st); break;
@@ -383,7 +409,7 @@ SPH_EXPORT int sph_init_tensor_rows(const int32_t *indices, int n, int B, int S0
         gpr = row_bytes / gran;
     }
     const int row_blocks = (int)(((long)n * gpr + 255) / 256 + (n == 0));
-    const dim3 grid((unsigned)row_blocks + (unsigned)(coo_by_columns(n, ncol, l.words) ? sph_div_up(ncol, 256) : 0));
+    const dim3 grid((unsigned)row_blocks + (unsigned)(strewn ? sph_div_up(ncol, 256) : 0));
     switch (here ? gran : 16) {
     case 16: hipLaunchKernelGGL(coo_place_kernel<uint4>, grid, block, 0, st, indices, n, g, r, gpr, row_blocks); break;
     case 4: hipLaunchKernelGGL(coo_place_kernel<uint32_t>, grid, block, 0, st, indices, n, g, r, gpr, row_blocks); break;
