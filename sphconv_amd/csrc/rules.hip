@@ -502,7 +502,7 @@ static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_p
     a.lines = join_lines(a, transposed != 0);
     hipStream_t st = (hipStream_t)stream;
     const bool by_lines = a.lines && !a.long_fibers;
-    if (masks_build_ok(a, transposed != 0, KV)) {
+    if (masks_build_ok(a, transposed != 0, KV, nt)) {
         const bool k27 = a.cv.K0 * a.cv.K1 == 9 && a.cv.K2 == 3;
         void (*masks)(BuildArgs) = k27 ? (a.q_rowcol ? build_nbr_kernel<true, 9, 3> : build_nbr_kernel<false, 9, 3>)
                                        : (a.q_rowcol ? build_nbr_kernel<true, 0, 0> : build_nbr_kernel<false, 0, 0>);

@@ -10,15 +10,22 @@ namespace {
 // offsets of a fiber share it.
 // What bounds it: the table's bytes (13.8 KB a tile, written at 4.0 TB/s with 12 744 tiles), on small grids four dependent
 // loads.  us, the mask join with the table in LDS -> now: 12 744 tiles 78.0 -> 44.1, 4056 tiles 30.3 -> 17.9, 1248 tiles 16.1 ->
-// 11.6, 512 tiles 10.5 -> 7.8, 64 tiles 9.6 -> 8.5: no size keeps the other one.
-// Left to it: transposed books, books with groups, kernels of more than 32 offsets (their masks outgrow the LDS).
+// 11.6, 512 tiles 10.5 -> 7.8, 64 tiles 9.6 -> 8.5.
+// That is for columns alike.  Where sparse columns lie beside full ones, a tile of more than 64 columns walks: one entry at a
+// time that took up to twice the mask join's time (5.9 entries a column on average, 865 tiles 14.8 : 26.0), the first two of nine fibers
+// and then eight of three at once 16.1 (307 tiles 10.9 : 13.3, 2588 tiles 27.1 : 20.6).  Two passes of masks over such a
+// tile were slower (22.1), and so was a walk from 32 columns on, for columns of four entries (1003 tiles 7.3 : 6.3 -> 7.8).
+// Left to it: transposed books, books with groups, kernels of more than 32 offsets (their masks outgrow the LDS), short grids with
+// few rows to a column (masks_build_ok).
 constexpr int kNbrThreads = R;
 constexpr int kNbrCols = 64; // distinct columns of a tile that masks are made for
 
-inline bool masks_build_ok(const BuildArgs &a, bool transposed, int KV)
+// On short grids the tile's chain counts, and with few rows to a column a tile has many columns, their fibers more than a thread each:
+// stride 2 on a full grid of four bins, two rows to a column, 125 tiles 7.5 : 8.6 us, 375 tiles 9.0 : 9.5, 750 tiles 11.6 : 10.3.
+inline bool masks_build_ok(const BuildArgs &a, bool transposed, int KV, int ntiles)
 {
     return !transposed && a.long_fibers && KV <= 32 && a.book.tile_nbr && !a.book.grp_gather && a.cv.p2 <= 64 - a.P.n2 &&
-           (double)a.Q.n2 * a.cv.s2 < (1 << 22) && a.p_rows < (1 << 28);
+           (double)a.Q.n2 * a.cv.s2 < (1 << 22) && a.p_rows < (1 << 28) && (ntiles > 512 || a.q_rows >= 4.0 * a.B * a.Q.n0 * a.Q.n1);
 }
 
 inline size_t masks_lds(int K01) { return (size_t)kNbrCols * K01 * (sizeof(unsigned long long) + sizeof(int)) + kNbrCols * sizeof(int4); }
@@ -174,23 +181,55 @@ __global__ __launch_bounds__(kNbrThreads) void build_nbr_kernel(BuildArgs a)
         }
         return;
     }
-    // Fibers that do not ascend or leave the bins, or a tile of many short ones: every row walks its own.
+    // Fibers that do not ascend or leave the bins, or a tile of many short ones: every row walks its own, several at a time.
     for (int k = 0; k < KV; k++) dst[k * R] = -1;
-    if (!live) return;
-    for (int k01 = 0; k01 < K01; k01++) {
-        const int k0 = (int)(((unsigned)k01 * inv_k1) >> 16), k1 = k01 - k0 * a.cv.K1;
-        const int y0 = y0b + k0, y1 = y1b + k1;
-        if ((unsigned)y0 >= (unsigned)a.P.n0 || (unsigned)y1 >= (unsigned)a.P.n1) continue;
-        int st, e;
-        fiber_range(a.p_ptr, (colb + y0) * a.P.n1 + y1, a.p_rows, st, e);
-        for (int t = st; t < e; t += 4) {
-            int v[4];
+    constexpr int kWalk = 9; // fibers at a time
+    for (int base = 0; base < K01; base += kWalk) {
+        int st[kWalk], n[kWalk];
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = a.p_idx[min(t + q, e - 1)];
+        for (int i = 0; i < kWalk; i++) {
+            st[i] = n[i] = 0;
+            const int k01 = base + i;
+            if (k01 >= K01) continue;
+            const int k0 = (int)(((unsigned)k01 * inv_k1) >> 16), k1 = k01 - k0 * a.cv.K1;
+            const int y0 = y0b + k0, y1 = y1b + k1;
+            const bool ok = live && (unsigned)y0 < (unsigned)a.P.n0 && (unsigned)y1 < (unsigned)a.P.n1;
+            const int pc = ok ? (colb + y0) * a.P.n1 + y1 : 0;
+            const int from = a.p_ptr[max(pc - 1, 0)], to = a.p_ptr[pc];
+            st[i] = pc > 0 ? from : 0;
+            n[i] = ok ? to : 0;
+        }
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int k2 = v[q] - (zz * a.cv.s2 - a.cv.p2);
-                if (t + q < e && (unsigned)k2 < (unsigned)K2) dst[(k01 * K2 + k2) * R] = t + q;
+        for (int i = 0; i < kWalk; i++) {
+            st[i] = clampi(st[i], 0, a.p_rows);
+            n[i] = clampi(n[i], 0, a.p_rows) - st[i];
+        }
+        auto pair = [&](int i, int t, int z) {
+            const int k2 = z - (zz * a.cv.s2 - a.cv.p2);
+            if (t < n[i] && (unsigned)k2 < (unsigned)K2) dst[((base + i) * K2 + k2) * R] = st[i] + t;
+        };
+        int v[kWalk][2]; // the first two entries of every fiber, then eight at a time of three fibers (a line of the grid, mostly)
+#pragma unroll
+        for (int i = 0; i < kWalk; i++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) v[i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, (st[i] + q) * 4, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kWalk; i++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) pair(i, q, v[i][q]);
+#pragma unroll
+        for (int i0 = 0; i0 < kWalk; i0 += 3) {
+            const int most = max(n[i0], max(n[i0 + 1], n[i0 + 2]));
+            for (int t = 2; __any(most > t); t += 8) {
+                int u[3][8];
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+#pragma unroll
+                    for (int q = 0; q < 8; q++) u[i][q] = __builtin_amdgcn_raw_buffer_load_b32(r_idx, (st[i0 + i] + t + q) * 4, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+#pragma unroll
+                    for (int q = 0; q < 8; q++) pair(i0 + i, t + q, u[i][q]);
             }
         }
     }

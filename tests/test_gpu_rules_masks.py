@@ -80,3 +80,27 @@ def test_many_columns_in_a_tile():
     c, z = occ.view(-1, shape[2]).nonzero(as_tuple=True)
     z_ptr = occ.sum(2).view(-1).cumsum(0).int().view(1, shape[0], shape[1])
     _check(z.int(), z_ptr, c.int(), shape, 1, (3, 3, 3), (1, 1, 1), [1, 1, 1])
+
+
+@pytest.mark.parametrize("cols", ["given", "outside"])
+@pytest.mark.parametrize("kernel", [(3, 3, 3), (2, 2, 2), (5, 3, 2), (4, 5, 1), (1, 1, 4)])
+@pytest.mark.parametrize("depth,low,high,share,block", [(16, 0.06, 0.6, 0.5, 256), (32, 0.02, 0.9, 0.3, 100), (40, 0.03, 0.5, 0.4, 7)])
+def test_sparse_columns_beside_full_ones(depth, low, high, share, block, kernel, cols):
+    """Tiles of up to 128 columns whose rows walk their fibers, of one entry to forty."""
+    shape, g = (24, 1600, depth), torch.Generator(device="cuda").manual_seed(2)
+    ncol = shape[0] * shape[1]
+    dense = (torch.rand(ncol // block + 1, generator=g, device="cuda") < share).repeat_interleave(block)[:ncol, None]
+    occ = torch.rand((ncol, depth), generator=g, device="cuda") < torch.where(dense, high, low)
+    c, z = occ.nonzero(as_tuple=True)
+    z_ptr = occ.sum(1).cumsum(0).int().view(1, shape[0], shape[1])
+    _check(z.int().contiguous(), z_ptr, c.int().contiguous(), shape, 1, kernel, (1, 1, 1), [k // 2 for k in kernel], cols)
+
+
+@pytest.mark.parametrize("rows", [510, 2000])
+def test_two_rows_to_a_column_of_the_outputs(rows):
+    """Outputs of a shallow full grid, 64 columns a tile: the general kernel's up to 512 tiles."""
+    shape = (2 * 32, 2 * rows, 4)
+    z_idx = torch.arange(4, dtype=torch.int32, device="cuda").repeat(shape[0] * shape[1])
+    z_ptr = (torch.arange(shape[0] * shape[1], device="cuda").int() * 4 + 4).view(1, *shape[:2])
+    col = torch.arange(shape[0] * shape[1], device="cuda").int().repeat_interleave(4)
+    _check(z_idx, z_ptr, col, shape, 1, (3, 3, 3), (2, 2, 2), (1, 1, 1))
