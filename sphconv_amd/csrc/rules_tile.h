@@ -101,8 +101,9 @@ __device__ int block_upper_bound(const int32_t *a, int n, int target, int max_sp
 
 // Columns of rows r0 .. r1 - 1 (those of a tile) to s_col, -1 for a row that no column holds, by the whole workgroup: rounds of
 // probes to the neighbourhood of the first, then a walk.  The walk tolerates starting early (columns before the tile hold none
-// of its rows), so the search stops once the window is below one walk step: a single round of probes for grids of up to 131072
-// columns.  s_first: 2 * NT / kWave ints, s_flag: 2.  meanwhile() as in block_upper_bound.  Ends behind a barrier.
+// of its rows), so the search stops once the window is below one walk step: a single round of probes for grids of up to 2 * NT * NT
+// columns (131072 with 256 threads, 32768 with 128).  s_first: 2 * NT / kWave ints, s_flag: 2.  meanwhile() as in block_upper_bound.
+// Ends behind a barrier.
 template <int NT, class F>
 __device__ __forceinline__ void search_columns(const int32_t *q_ptr, int q_ncol, int q_rows, int r0, int r1, int *s_col, int *s_first,
                                                int *s_flag, F &&meanwhile)

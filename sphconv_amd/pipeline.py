@@ -55,7 +55,8 @@ class ScanPipeline:
         self._streams = [torch.cuda.Stream(device=dev) for _ in range(int(streams))]
         self._books = [_Buffers(self.max_voxels, self.kv, dev) for _ in self._streams]
         # One launch per scan while a scan's tiles are resident at once; with three or more scans in flight the two
-        # kernels overlap better from 768 tiles on (measured at 937 tiles on three streams: 24.7 against 25.9 us per scan)
+        # kernels overlap better from 768 tiles on (64 -> 64 fp16 on three streams, us per scan, one launch : two: 600 tiles
+        # 13.2 : 13.5, 760 tiles 16.3 : 15.5, 930 tiles 20.3 : 18.7)
         self._fused_max_tiles = 768 if len(self._streams) >= 3 else RuleBook.FUSED_MAX_TILES
         for book in self._books:
             # submanifold: every row pairs with itself at the middle offset
