@@ -21,11 +21,12 @@ constexpr int kNbrThreads = R;
 constexpr int kNbrCols = 64; // distinct columns of a tile that masks are made for
 
 // On short grids the tile's chain counts, and with few rows to a column a tile has many columns, their fibers more than a thread each:
-// stride 2 on a full grid of four bins, two rows to a column, 125 tiles 7.5 : 8.6 us, 375 tiles 9.0 : 9.5, 750 tiles 11.6 : 10.3.
+// stride 2 on a full grid of four bins, two rows to a column, 125 tiles 7.5 : 8.6 us, 375 tiles 9.0 : 9.5, 750 tiles 11.6 : 10.3;
+// with three 75 tiles 7.2 : 8.1, with nearly four 63 tiles 9.1 : 7.3.
 inline bool masks_build_ok(const BuildArgs &a, bool transposed, int KV, int ntiles)
 {
     return !transposed && a.long_fibers && KV <= 32 && a.book.tile_nbr && !a.book.grp_gather && a.cv.p2 <= 64 - a.P.n2 &&
-           (double)a.Q.n2 * a.cv.s2 < (1 << 22) && a.p_rows < (1 << 28) && (ntiles > 512 || a.q_rows >= 4.0 * a.B * a.Q.n0 * a.Q.n1);
+           (double)a.Q.n2 * a.cv.s2 < (1 << 22) && a.p_rows < (1 << 28) && (ntiles > 512 || a.q_rows >= 3.5 * a.B * a.Q.n0 * a.Q.n1);
 }
 
 inline size_t masks_lds(int K01) { return (size_t)kNbrCols * K01 * (sizeof(unsigned long long) + sizeof(int)) + kNbrCols * sizeof(int4); }

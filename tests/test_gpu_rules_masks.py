@@ -96,11 +96,12 @@ def test_sparse_columns_beside_full_ones(depth, low, high, share, block, kernel,
     _check(z.int().contiguous(), z_ptr, c.int().contiguous(), shape, 1, kernel, (1, 1, 1), [k // 2 for k in kernel], cols)
 
 
-@pytest.mark.parametrize("rows", [510, 2000])
-def test_two_rows_to_a_column_of_the_outputs(rows):
-    """Outputs of a shallow full grid, 64 columns a tile: the general kernel's up to 512 tiles."""
-    shape = (2 * 32, 2 * rows, 4)
-    z_idx = torch.arange(4, dtype=torch.int32, device="cuda").repeat(shape[0] * shape[1])
-    z_ptr = (torch.arange(shape[0] * shape[1], device="cuda").int() * 4 + 4).view(1, *shape[:2])
-    col = torch.arange(shape[0] * shape[1], device="cuda").int().repeat_interleave(4)
+@pytest.mark.parametrize("rows,depth", [(510, 4), (2000, 4), (510, 6), (510, 8)])
+def test_few_rows_to_a_column_of_the_outputs(rows, depth):
+    """Outputs of a shallow full grid, two to four rows a column: the general kernel's up to 512 tiles where there are fewer than four."""
+    shape = (2 * 32, 2 * rows, depth)
+    ncol = shape[0] * shape[1]
+    z_idx = torch.arange(depth, dtype=torch.int32, device="cuda").repeat(ncol)
+    z_ptr = (torch.arange(ncol, device="cuda").int() * depth + depth).view(1, *shape[:2])
+    col = torch.arange(ncol, device="cuda").int().repeat_interleave(depth)
     _check(z_idx, z_ptr, col, shape, 1, (3, 3, 3), (2, 2, 2), (1, 1, 1))
