@@ -371,10 +371,12 @@ def configs_ms(torch, seed, iters):
 
 def kernel_sources_digest():
     """sha256 over the sources of the kernels whose HBM traffic is on record (what a counter run was
-    taken on): the recorded traffic is only reported while these files are what it was measured on."""
+    taken on), and over those that decide whether it is these kernels that run: the recorded traffic is only reported while
+    the files are what it was measured on."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("conv.hip", "rules.hip", "fused.hip", "conv_wave.h", "rules_tile.h", "rules_rows.h", "tile_consts.h", "common.h", "pack.h"):
+    for name in ("conv.hip", "relay.hip", "relay.h", "rules.hip", "fused.hip", "conv_wave.h", "rules_tile.h", "rules_rows.h",
+                 "rules_masks.h", "tile_consts.h", "common.h", "pack.h"):
         with open(os.path.join(ROOT, "sphconv_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()
