@@ -334,7 +334,8 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
     }
 }
 
-// The kernel for the call's number of lines and of columns on a line (one to three each), and for 27 offsets where that is 3x3x3.
+// The kernel for the call's number of lines and of columns on a line (one to three each); with the loops' lengths fixed for 27
+// offsets of stride 1, of stride 2 transposed, and of two columns by three lines.
 template <bool TRANSPOSED, bool HINT>
 inline void (*rows_kernel(const BuildArgs &a, int KV))(BuildArgs)
 {
