@@ -648,7 +648,7 @@ class Workload:
     def rooflines(self, kern, seed):
         """(the step's dominant kernel, the rule kernel, the convolution kernel): algorithmic bytes per launch over
         the kernel's average duration, against the HBM peak."""
-        name = "build_rows_kernel<false,3,3,27,true>" if self.ntiles > 512 else "build_book_kernel<false,true>"
+        name = "build_rows_kernel<false,3,3,27,true,4>" if self.ntiles > 512 else "build_book_kernel<false,true>"
         rules = self._roofline(name, "rules", self.rule_bytes, kern["rulegen_ms"], seed)
         conv = self._roofline("conv_wave_run_kernel<f16,2,4,false>", "conv", self.conv_bytes, kern["conv_forward_ms"], seed)
         if self.one_launch and getattr(self, "step_launches", 1) == 1:

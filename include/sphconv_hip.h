@@ -98,12 +98,12 @@ typedef struct sph_book {
      * it can walk by rows (rows of 16-byte multiples up to 128 bytes) and refuses the others,
      * sph_conv_wgrad and sph_rules_to_padded_count refuse the book. */
     int32_t *tile_nbr;
-    /* Set by the caller, read by sph_conv_apply and sph_rules_conv: not 0 = the middle offset KV/2 holds a run of full groups in
-     * most tiles, as in a submanifold layer, where it pairs every row with itself (and in that layer's transposed book).
-     * The kernels by groups then load that run's weight fragments once: helper waves take it on short grids, the wave that
-     * begins a tile on long ones.  0 (also what a zero-initialised struct says): no assumption; results are the same either
-     * way, up to the order of summation.  SPH_RUN_IN_FLIGHT says besides that the caller keeps three calls or more in flight
-     * on streams of their own: kernels that share the chip better are then taken up to larger grids. */
+    /* Set by the caller, read by sph_conv_apply, sph_rules_conv and sph_rules_build*: not 0 = the middle offset KV/2 holds a run
+     * of full groups in most tiles, as in a submanifold layer, where it pairs every row with itself (and in that layer's
+     * transposed book).  The kernels by groups then load that run's weight fragments once: helper waves take it on short
+     * grids, the wave that begins a tile on long ones.  0 (also what a zero-initialised struct says): no assumption; results
+     * are the same either way, up to the order of summation.  SPH_RUN_IN_FLIGHT says besides that the caller keeps three calls
+     * or more in flight on streams of their own: kernels that share the chip better are then taken up to larger grids. */
     int32_t middle_run;
 } sph_book;
 

@@ -514,8 +514,8 @@ static int rules_build(const char *who, const int32_t *z_idx, const int32_t *z_p
         return sph_check_launch(who);
     }
     if (rows_build_ok(a, transposed != 0, KV, nt)) {
-        void (*rows)(BuildArgs) = transposed ? (a.q_rowcol ? rows_kernel<true, true>(a, KV) : rows_kernel<true, false>(a, KV))
-                                             : (a.q_rowcol ? rows_kernel<false, true>(a, KV) : rows_kernel<false, false>(a, KV));
+        void (*rows)(BuildArgs) = transposed ? (a.q_rowcol ? rows_kernel<true, true>(a, KV, nt) : rows_kernel<true, false>(a, KV, nt))
+                                             : (a.q_rowcol ? rows_kernel<false, true>(a, KV, nt) : rows_kernel<false, false>(a, KV, nt));
         const int pack_rows = pack ? sph_div_up(sph_pack_total(pack->job), kRowThreads) : 0;
         lds = (size_t)R * KV * sizeof(int32_t) + kRowScratch;
         const int rc = allow_lds(rows, lds, who);

@@ -72,7 +72,8 @@ constexpr int kRowGroups = 40;
 constexpr size_t kRowScratch = (size_t)kRowGroups * SPH_GROUP * 4 + 2 * 32 * 4 + 2 * 4;
 
 // KVT: the kernel volume, or 32 for any up to that.  HINT: the rows' columns are given (and checked), else searched for.
-template <bool TRANSPOSED, int C, int NL, int KVT, bool HINT>
+// LATER: entries a column's later rounds take at most (4, or 2 where registers count: rows_kernel).
+template <bool TRANSPOSED, int C, int NL, int KVT, bool HINT, int LATER = 4>
 __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) int32_t s_nbr[];
@@ -243,7 +244,9 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
     const std::integral_constant<int, 2> two;
     const std::integral_constant<int, 4> four;
     entries(0, two, std::false_type());
-    if (__any(most > 4)) {
+    if constexpr (LATER == 2) {
+        for (int t = 2; __any(most > t); t += 2) entries(t, two, std::false_type());
+    } else if (__any(most > 4)) {
         entries(2, four, std::false_type());
         for (int t = 6; __any(most > t); t += 4) entries(t, four, std::true_type());
     } else if (__any(most > 2)) {
@@ -336,12 +339,22 @@ __global__ __launch_bounds__(kRowThreads) void build_rows_kernel(BuildArgs a)
 
 // The kernel for the call's number of lines and of columns on a line (one to three each); with the loops' lengths fixed for 27
 // offsets of stride 1, of stride 2 transposed, and of two columns by three lines.
+// The rounds of four entries take 84 registers there where rounds of two take 56, and leave less room for the convolution of the
+// scan before.  Up to the line where the relay has the compute units to itself, rounds of two are the better ones for scans in flight:
+// us a scan, 64 -> 64 fp16 on three streams, four : two, 1 to 3 entries in 60 % of the columns 930 tiles 17.5 : 17.2, 1100 tiles
+// 20.7 : 20.4, 1900 tiles 31.0 : 31.1, 4000 tiles 58.5 : 58.7 (Poisson columns 18.0 : 18.1, 21.0 : 21.2, 32.4 : 33.0, 60.9 : 62.3);
+// a call on its own 1300 tiles 8.4 : 8.7, 5890 tiles 22.5 : 23.4.
+constexpr int kRowFlightTiles = 1280;
 template <bool TRANSPOSED, bool HINT>
-inline void (*rows_kernel(const BuildArgs &a, int KV))(BuildArgs)
+inline void (*rows_kernel(const BuildArgs &a, int KV, int ntiles))(BuildArgs)
 {
     constexpr int cube = TRANSPOSED ? 2 : 3;
     const int nl = rows_lines(a, TRANSPOSED), c = a.lines;
-    if (KV == 27 && c == cube && nl == cube) return build_rows_kernel<TRANSPOSED, cube, cube, 27, HINT>;
+    if (KV == 27 && c == cube && nl == cube) {
+        if (!TRANSPOSED && a.book.middle_run == SPH_RUN_IN_FLIGHT && ntiles <= kRowFlightTiles)
+            return build_rows_kernel<false, 3, 3, 27, HINT, 2>;
+        return build_rows_kernel<TRANSPOSED, cube, cube, 27, HINT>;
+    }
     if (KV == 27 && c == 2 && nl == 3) return build_rows_kernel<TRANSPOSED, 2, 3, 27, HINT>;
 #define SPH_ROWS(C, NL) if (c == C && nl == NL) return build_rows_kernel<TRANSPOSED, C, NL, 32, HINT>;
     SPH_ROWS(1, 1) SPH_ROWS(1, 2) SPH_ROWS(1, 3) SPH_ROWS(2, 1) SPH_ROWS(2, 2) SPH_ROWS(2, 3) SPH_ROWS(3, 1) SPH_ROWS(3, 2)

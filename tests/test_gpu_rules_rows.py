@@ -89,8 +89,9 @@ def _columns(z_ptr, rows):
     return torch.searchsorted(z_ptr.view(-1).long(), torch.arange(rows, device="cuda"), right=True).int()
 
 
-def _build(z_idx, z_ptr, oz_idx, oz_ptr, book, transposed, cols):
+def _build(z_idx, z_ptr, oz_idx, oz_ptr, book, transposed, cols, run=0):
     buf = rulebook._Buffers(book.in_rows if transposed else book.out_rows, book.kv, z_idx.device)
+    buf.struct().middle_run = run
     L.check(L.lib().sph_rules_build(L.ptr(z_idx), L.ptr(z_ptr), book.in_rows, L.ptr(oz_idx), L.ptr(oz_ptr), book.out_rows,
                                     C.byref(book.geom()), int(transposed), C.byref(buf.struct()), L.ptr(cols), L.stream()))
     return buf
@@ -240,3 +241,24 @@ def test_uneven_columns(shape, per_column, share, kernel, stride, transposed):
     q, p = (ins, outs) if transposed else (outs, ins)
     _check(_build(z_idx, z_ptr, book.oz_idx, book.oz_ptr, book, transposed, q[1]),
            _expected(q, p, p[2], kernel, stride, pad, transposed))
+
+
+@pytest.mark.parametrize("cols", ["given", "none", "one wrong"])
+@pytest.mark.parametrize("tiles,per_column,share", [(560, 1.2, 1.0), (1279, 0.4, 0.2), (1290, 1.4, 0.5), (1000, 1.3, 0.05)])
+def test_scans_in_flight(tiles, per_column, share, cols):
+    """Rounds of two entries up to 1280 tiles, of four beyond; columns of up to forty entries."""
+    shape = (64, int(tiles * 128 / per_column / 64), 48)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    ncol = shape[0] * shape[1]
+    occ = torch.rand((ncol, shape[2]), generator=g, device="cuda") < per_column / share / shape[2]
+    occ &= torch.rand((ncol, 1), generator=g, device="cuda") < share
+    col, z = occ.nonzero(as_tuple=True)
+    z_idx, col = z.int().contiguous(), col.int().contiguous()
+    z_ptr = occ.sum(1).cumsum(0).int().view(1, *shape[:2]).contiguous()
+    book = RuleBook.build_subm(z_idx, z_ptr, 1, list(shape), [3, 3, 3], lazy=True)
+    given = col.clone()
+    if cols == "one wrong":
+        given[::777] += 1
+    side = z_idx, col, shape
+    _check(_build(z_idx, z_ptr, z_idx, z_ptr, book, False, None if cols == "none" else given, L.RUN_IN_FLIGHT),
+           _expected(side, side, shape, (3, 3, 3), (1, 1, 1), [1, 1, 1], False))
