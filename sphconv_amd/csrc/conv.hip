@@ -13,13 +13,6 @@
 // rows) steps with the accumulators in registers instead; with rows of up to 64 bytes and
 // up to 64 output columns conv_rows_win_kernel does so from a copy of the gathered rows
 // in LDS.
-//
-// wgrad (sph_conv_wgrad): work items are (kernel offset, chunk of 64 tiles, slice of 64
-// groups); a wave gathers 32 pairs' rows with 16-byte loads into its own LDS area and
-// reads MFMA operands with the pair index as the K dimension through transposing LDS
-// reads; the [64,64] block stays in registers, one fp32 partial per workgroup, summed
-// in a fixed order by a second kernel.  wgrad_kernel is the general fallback for rows
-// that are not whole 16-byte chunks.
 #include "common.h"
 #include "pack.h"
 #include "conv_wave.h"
@@ -685,532 +678,10 @@ __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(CT ==
     }
 }
 
-// ---------------------------------------------------------------------------
-// wgrad
-// ---------------------------------------------------------------------------
-struct WgradArgs {
-    const char *feat;
-    int in_rows, iC;
-    const char *dout;
-    int out_rows, oC;
-    sph_book book;
-    const int32_t *list_in, *list_out; // the book's two lists: input rows and output rows of the groups
-    int cap, ntiles, nchunk;
-    float *partial;
-    int *flags;      // wave kernel: one per partial slot, 1 = the slot was written
-    int nslice;      // wave kernel: workgroups per chunk at the centre offset (slices h, h + nslice, ... each)
-    int all_slices;  // wave kernel: every offset has its later slices' workgroups (small grids), not only the centre
-    int nslots;
-};
-
-constexpr int kWgThreads = 256;
-constexpr int kWgWaves = kWgThreads / kWave;
-constexpr int kMaxTilesPerWave = 16; // (128/16)^2 / 4 waves
-
-template <sph_dtype DT>
-__global__ __launch_bounds__(kWgThreads) void wgrad_kernel(WgradArgs a)
-{
-    typedef typename Traits<DT>::elem elem;
-    constexpr int KW = Traits<DT>::KW;
-    constexpr int PB = 4 * KW;            // pairs per batch = K of one super step
-    constexpr int LDP = PB + 16 / (int)sizeof(elem); // padded pair stride, keeps 16-byte alignment
-    extern __shared__ char s_raw[];
-    const int iCp = (a.iC + 15) & ~15, oCp = (a.oC + 15) & ~15;
-    elem *At = (elem *)s_raw;               // [iCp][LDP]
-    elem *Gt = At + (long)iCp * LDP;        // [oCp][LDP]
-    __shared__ int s_in[PB], s_out[PB];
-
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int KV = a.book.KV;
-    const int k = blockIdx.x / a.nchunk, chunk = blockIdx.x - k * a.nchunk;
-    const int tpc = (a.ntiles + a.nchunk - 1) / a.nchunk;
-    const int t0 = chunk * tpc, t1 = min(t0 + tpc, a.ntiles);
-    const int MI = iCp / 16, NI = oCp / 16, MT = MI * NI;
-
-    float4v acc[kMaxTilesPerWave];
-#pragma unroll
-    for (int j = 0; j < kMaxTilesPerWave; j++) acc[j] = float4v{0, 0, 0, 0};
-
-    for (int t = t0; t < t1; t++) {
-        const int g0 = a.book.tile_koff[(long)t * (KV + 1) + k];
-        const int g1 = a.book.tile_koff[(long)t * (KV + 1) + k + 1];
-        for (int gb = g0; gb < g1; gb += PB / SPH_GROUP) {
-            __syncthreads(); // previous batch fully consumed
-            if (tid < PB) {
-                int g = gb + tid / SPH_GROUP;
-                int vi = -1, vo = -1;
-                if (g < g1) {
-                    long slot = ((long)t * a.cap + g) * SPH_GROUP + (tid & (SPH_GROUP - 1));
-                    vi = a.list_in[slot];
-                    vo = a.list_out[slot];
-                }
-                if ((unsigned)vi >= (unsigned)a.in_rows || (unsigned)vo >= (unsigned)a.out_rows) vi = vo = -1;
-                s_in[tid] = vi;
-                s_out[tid] = vo;
-            }
-            __syncthreads();
-            for (int e = tid; e < PB * iCp; e += kWgThreads) {
-                int p = e / iCp, c = e - p * iCp;
-                int row = s_in[p];
-                elem v = (elem)0;
-                if (row >= 0 && c < a.iC) v = ((const elem *)a.feat)[(long)row * a.iC + c];
-                At[c * LDP + p] = v;
-            }
-            for (int e = tid; e < PB * oCp; e += kWgThreads) {
-                int p = e / oCp, c = e - p * oCp;
-                int row = s_out[p];
-                elem v = (elem)0;
-                if (row >= 0 && c < a.oC) v = ((const elem *)a.dout)[(long)row * a.oC + c];
-                Gt[c * LDP + p] = v;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < kMaxTilesPerWave; j++) {
-                int ti = wave + j * kWgWaves;
-                if (ti < MT) {
-                    int mi = ti / NI, ni = ti - mi * NI;
-                    int4v fa = *(const int4v *)(At + (mi * 16 + (lane & 15)) * LDP + (lane >> 4) * KW);
-                    int4v fb = *(const int4v *)(Gt + (ni * 16 + (lane & 15)) * LDP + (lane >> 4) * KW);
-                    acc[j] = mfma_step<DT>(fa, fb, acc[j]);
-                }
-            }
-        }
-    }
-    float *part = a.partial + ((long)k * a.nchunk + chunk) * a.iC * a.oC;
-#pragma unroll
-    for (int j = 0; j < kMaxTilesPerWave; j++) {
-        int ti = wave + j * kWgWaves;
-        if (ti < MT) {
-            int mi = ti / NI, ni = ti - mi * NI;
-            int co = ni * 16 + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                int ci = mi * 16 + (lane >> 4) * 4 + r;
-                if (ci < a.iC && co < a.oC) part[(long)ci * a.oC + co] = acc[j][r];
-            }
-        }
-    }
-}
-
-template <typename OUT>
-__global__ void wgrad_reduce_kernel(const float *partial, int KV, int nchunk, int per_k, OUT *dw)
-{
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)KV * per_k) return;
-    int k = (int)(i / per_k), e = (int)(i - (long)k * per_k);
-    const float *p = partial + (long)k * nchunk * per_k + e;
-    float s = 0.f;
-    for (int c = 0; c < nchunk; c++) s += p[(long)c * per_k];
-    dw[i] = (OUT)s;
-}
-
-// ---------------------------------------------------------------------------
-// wgrad, fast path (rows are whole 16-byte chunks).
-//
-// Work item = (offset k, chunk of 64 tiles, slice of 64 groups of that chunk's groups at
-// k, 64x64 block of [iC,oC]).  A chunk holds at most 64*8 groups per offset; four
-// workgroups are launched per (offset, chunk), workgroup h takes slices h and h+4, and
-// those whose first slice lies beyond the chunk's real group count exit at once (a
-// submanifold book has 8 groups per tile at the centre offset and about one elsewhere:
-// slicing by groups, not tiles, is what balances the grid).
-// The four waves of the workgroup take the slice's batches (32 pairs; 16 for fp32) round
-// robin and never synchronise until the end: a wave gathers the batch's feature rows and
-// d_out rows with 16-byte loads into its own LDS area in natural [pair][channel] order,
-// and reads MFMA operands with the pair index as the K dimension through transposing
-// LDS reads (16-bit types) or strided 4-byte reads (fp32).  The block lives in registers;
-// the workgroup's four blocks are summed through LDS into one fp32 partial, and
-// wgrad_slot_reduce_kernel adds the written slots in a fixed order.
-// The book is the layer's forward one or its transposed one (list_in, list_out): a strided layer on scattered voxels has
-// its pairs in 3.1 times fewer tiles stationary on the input rows, with groups more than twice as full (64->64 fp32 on
-// eight 64x512x512 scans, stride 2: 117 us from the forward book, 59 us from the transposed one with the empty fours left out;
-// 24->40 bf16: 52 -> 38 us).  Chunks of 32 or 16 tiles, for more workgroups, were slower (62 and 65 us).
-// What bounds it (64->64 fp16, 8 waves per CU): LDS traffic (8 KiB staged and 8 KiB read
-// back per batch and wave) and the MFMAs, about equally.
-// ---------------------------------------------------------------------------
-constexpr int kWsTiles = 64;   // tiles per chunk (one lane each)
-constexpr int kWsSlice = 64;   // groups per slice
-constexpr int kWsSlices = 8;   // most workgroups per chunk at the centre offset (workgroup h takes slices h, h + nslice, ...);
-                               // WgradArgs::nslice = 8 on small books, 4 on large ones; one workgroup elsewhere
-constexpr int kWsBlock = 64;   // channels per block side
-
-typedef short short4v __attribute__((ext_vector_type(4)));
-
-// MFMA operand of 16 channels x one batch of pairs from a staging area laid out
-// [pair][channel], row stride rs bytes.  16-bit types: lane (m = lane%16, q = lane/16)
-// receives pairs 8q..8q+7 of channel m through two transposing reads (element j of lane
-// 4a+b = the b-th element at the address given by lane a+4j of the same 16 lanes).
-// fp32: component j of lane (m, q) = pair 4j+q of channel m.
-template <sph_dtype DT>
-__device__ __forceinline__ int wgrad_frag_offset(int rs, int lane)
-{
-    if constexpr (sizeof(typename Traits<DT>::elem) == 2) {
-        const int s = lane & 15, q = lane >> 4;
-        return (8 * q + (s >> 2)) * rs + 4 * (s & 3) * 2;
-    } else {
-        return (lane >> 4) * rs + (lane & 15) * 4;
-    }
-}
-template <sph_dtype DT>
-__device__ __forceinline__ int4v wgrad_frag(const char *p, int rs)
-{
-    if constexpr (sizeof(typename Traits<DT>::elem) == 2) {
-        typedef __attribute__((address_space(3))) short4v lds_s4;
-        short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p);
-        short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(p + 4 * rs));
-        union { struct { short4v l, h; } s; int4v v; } u;
-        u.s.l = lo; u.s.h = hi;
-        return u.v;
-    } else {
-        union { float f[4]; int4v v; } u;
-#pragma unroll
-        for (int j = 0; j < 4; j++) u.f[j] = *(const float *)(p + 4 * j * rs);
-        return u.v;
-    }
-}
-
-template <sph_dtype DT, int MI, int NI>
-__global__ __launch_bounds__(256, 2) void wgrad_wave_kernel(WgradArgs a)
-{
-    typedef typename Traits<DT>::elem elem;
-    constexpr int E = (int)sizeof(elem);
-    constexpr int GPB = E == 2 ? 2 : 1;                // groups per batch: one MFMA super step of 32 or 16 pairs
-    constexpr int PB = GPB * SPH_GROUP;                // pairs per batch
-    // MI, NI: 16-channel tiles of the block's two sides (1, 2 or 4; narrower blocks are zero padded).
-    // A batch of rows of MI tiles is MI 16-byte loads per lane.
-    extern __shared__ __attribute__((aligned(16))) char s_raw[];
-
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int KV = a.book.KV;
-    // Work items u = chunk*KV + k are dealt to the XCDs in contiguous runs (workgroups go to
-    // the XCDs round robin): the offsets of one chunk gather the same ~2 MiB of rows, which
-    // then stay in that XCD's L2.  The slice index is slowest, so that the first slices --
-    // often the only ones with work -- spread over all XCDs and start first.
-    const int items = KV * a.nchunk, items_grid = (items + SPH_NUM_XCD - 1) / SPH_NUM_XCD * SPH_NUM_XCD;
-    int h, chunk, k;
-    if ((int)blockIdx.x < items_grid) {
-        h = 0;
-        const int u = sph_xcd_tile(blockIdx.x, items);
-        if (u >= items) return;
-        chunk = u / KV;
-        k = u - chunk * KV;
-    } else {
-        // Later slices: a submanifold book has 8 groups per tile at the centre offset and about one elsewhere, and
-        // a workgroup without work still costs its dispatch (three quarters of the grid found none when every offset
-        // had four).  So only the centre offset has them, numbered first, and at the other offsets the first
-        // workgroup takes every slice -- unless the grid is small (all_slices): then a dense book's offsets need
-        // their four workgroups each to fill the chip, and they follow the centre's.
-        const int kc = KV / 2, v = (int)blockIdx.x - items_grid, nc = (a.nslice - 1) * a.nchunk;
-        if (v < nc) {
-            h = 1 + v / a.nchunk;
-            chunk = v % a.nchunk;
-            k = kc;
-        } else {
-            const int r = v - nc, per = a.nchunk * (KV - 1);
-            if (!a.all_slices || KV == 1 || r >= (a.nslice - 1) * per) return;
-            h = 1 + r / per;
-            const int q = r % per, kk = q % (KV - 1);
-            chunk = q / (KV - 1);
-            k = kk + (kk >= kc ? 1 : 0);
-        }
-    }
-    const int slice_step = (a.all_slices || k == KV / 2) ? a.nslice : 1;
-    const int sbn = (a.oC + kWsBlock - 1) / kWsBlock;
-    const int ci0 = (blockIdx.y / sbn) * kWsBlock, co0 = (blockIdx.y % sbn) * kWsBlock;
-    const int cA = min(kWsBlock, a.iC - ci0), cG = min(kWsBlock, a.oC - co0);
-    const int slot = (k * a.nchunk + chunk) * a.nslice + h;
-
-    // groups of this offset in the chunk's tiles: lane = tile, prefix sums over the wave
-    const int t0 = chunk * kWsTiles;
-    int g0 = 0, n = 0;
-    if (t0 + lane < a.ntiles) {
-        const unsigned short *ko = a.book.tile_koff + (long)(t0 + lane) * (KV + 1) + k;
-        g0 = min((int)ko[0], a.cap);
-        n = min(max((int)ko[1] - g0, 0), min(a.cap - g0, R / SPH_GROUP));
-    }
-    const int incl = wave_inclusive_sum(n); // lane shifts of the vector ALU, no LDS round trip per step
-    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
-    if (slice_step == 1 && tid < a.nslice - 1 && blockIdx.y == 0) a.flags[slot + 1 + tid] = 0; // slots nobody fills
-    if (h * kWsSlice >= total) {
-        if (tid == 0 && blockIdx.y == 0) a.flags[slot] = 0;
-        return;
-    }
-
-    // wave-private staging: feature rows then d_out rows, [pair][channels + 16 bytes]
-    constexpr int rsA = MI * 16 * E + 16, rsG = NI * 16 * E + 16;
-    const int cprA = cA * E / 16, cprG = cG * E / 16;      // real 16-byte chunks per row
-    char *xa = s_raw + (size_t)wave * PB * (rsA + rsG);
-    char *xg = xa + PB * rsA;
-    for (int i = lane; i < PB * (rsA + rsG) / 16; i += kWave) ((int4v *)xa)[i] = int4v{0, 0, 0, 0};
-
-    float4v acc[MI][NI];
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NI; j++) acc[i][j] = float4v{0, 0, 0, 0};
-
-    // Per-lane constants of the row copies: which pair and 16-byte chunk each of the lane's
-    // loads moves, its offset in the source row and in the staging area (-1: none).
-    int pairA[MI], srcA[MI], dstA[MI], pairG[NI], srcG[NI], dstG[NI];
-    // (rows of 32, 64 or 128 bytes are 2, 4 or 8 chunks: a shift instead of the forty instructions of a division)
-    const bool p2A = (cprA & (cprA - 1)) == 0, p2G = (cprG & (cprG - 1)) == 0;
-    const int shA = __ffs(cprA) - 1, shG = __ffs(cprG) - 1;
-#pragma unroll
-    for (int it = 0; it < MI; it++) {
-        const int i = it * kWave + lane;
-        const int pa = p2A ? i >> shA : i / cprA, ca = i - pa * cprA;
-        pairA[it] = min(pa, PB - 1); srcA[it] = ci0 * E + ca * 16; dstA[it] = pa < PB ? pa * rsA + ca * 16 : -1;
-    }
-#pragma unroll
-    for (int it = 0; it < NI; it++) {
-        const int i = it * kWave + lane;
-        const int pg = p2G ? i >> shG : i / cprG, cg = i - pg * cprG;
-        pairG[it] = min(pg, PB - 1); srcG[it] = co0 * E + cg * 16; dstG[it] = pg < PB ? pg * rsG + cg * 16 : -1;
-    }
-    const unsigned strideA = a.iC * E, strideG = a.oC * E;   // arrays are below 4 GiB (checked by the launcher)
-
-    // Book slot of every group of a slice: lane l looks up flattened group s0+l (the tile
-    // whose prefix range holds it, by binary search over the tile lanes) once per slice.
-    const long slot_max = (long)a.ntiles * a.cap * SPH_GROUP - 1;
-    auto slot_bases = [&](int s0) -> int {
-        const int f = s0 + lane;
-        int lo = 0;
-#pragma unroll
-        for (int step = kWave / 2; step >= 1; step >>= 1) {
-            const int v = __shfl(incl, lo + step - 1, kWave);
-            if (v <= f) lo += step;
-        }
-        lo = min(lo, kWave - 1);
-        const int g = __shfl(g0, lo, kWave) + f - (__shfl(incl, lo, kWave) - __shfl(n, lo, kWave));
-        const long sl = ((long)(t0 + lo) * a.cap + g) * SPH_GROUP;
-        return (int)min(max(sl, 0L), slot_max - (SPH_GROUP - 1));   // ntiles*cap*16 fits 31 bits (checked by the launcher)
-    };
-    // Book entries of batch b of the slice: lane l < 32 loads the gathered (input) row of pair
-    // l%PB, lane 32+l its owner (output) row.  The load is unconditional; the value is only
-    // looked at once all of the wave's index loads are on their way.
-    auto load_idx = [&](int bases, int s0, int s1, int b, bool &valid) -> int {
-        const int pr = lane & (PB - 1);
-        const int fl = GPB * b + (pr >> 4);                 // group within the slice
-        valid = s0 + fl < s1;
-        const int base = __shfl(bases, fl & (kWave - 1), kWave);
-        return (lane < 32 ? a.list_in : a.list_out)[base + (pr & 15)];
-    };
-    // Row loads are unconditional (clamped to row 0; in_rows and out_rows are positive here)
-    // so that several batches stay in flight; slots without a pair are zeroed when the rows
-    // are staged.  Returns the mask of pairs that exist.
-    auto gather = [&](int idx, int4v (&ra)[MI], int4v (&rg)[NI]) -> unsigned {
-        // all lane exchanges first, then all loads: one wait on the LDS queue instead of one per row
-        const int other = __shfl_xor(idx, 32, kWave);
-        int rowA[MI], rowG[NI];
-#pragma unroll
-        for (int it = 0; it < MI; it++) rowA[it] = __shfl(idx, pairA[it], kWave);
-#pragma unroll
-        for (int it = 0; it < NI; it++) rowG[it] = __shfl(idx, 32 + pairG[it], kWave);
-        __builtin_amdgcn_sched_barrier(0);
-        const unsigned ok = (unsigned)__ballot(idx >= 0 && other >= 0);
-#pragma unroll
-        for (int it = 0; it < MI; it++)
-            ra[it] = *(const int4v *)(a.feat + ((unsigned)max(rowA[it], 0) * strideA + (unsigned)srcA[it]));
-#pragma unroll
-        for (int it = 0; it < NI; it++)
-            rg[it] = *(const int4v *)(a.dout + ((unsigned)max(rowG[it], 0) * strideG + (unsigned)srcG[it]));
-        return ok;
-    };
-    auto stage = [&](unsigned ok, const int4v (&ra)[MI], const int4v (&rg)[NI]) {
-#pragma unroll
-        for (int it = 0; it < MI; it++)
-            if (dstA[it] >= 0) *(int4v *)(xa + dstA[it]) = ((ok >> pairA[it]) & 1) ? ra[it] : int4v{0, 0, 0, 0};
-#pragma unroll
-        for (int it = 0; it < NI; it++)
-            if (dstG[it] >= 0) *(int4v *)(xg + dstG[it]) = ((ok >> pairG[it]) & 1) ? rg[it] : int4v{0, 0, 0, 0};
-    };
-    const char *fragA = xa + wgrad_frag_offset<DT>(rsA, lane), *fragG = xg + wgrad_frag_offset<DT>(rsG, lane);
-    // `ok`: pairs of the staged batch that exist.  fp32 takes the pairs four at a time and leaves out the fours behind the
-    // last of them (a group's pairs come first, its padding behind): at 32 cycles an MFMA the padding was most of what
-    // the kernel did on a strided layer's books, whose groups hold five pairs of sixteen.
-    auto multiply = [&](unsigned ok) {
-        int4v fa[MI], fb[NI];
-#pragma unroll
-        for (int i = 0; i < MI; i++) fa[i] = wgrad_frag<DT>(fragA + i * 16 * E, rsA);
-#pragma unroll
-        for (int i = 0; i < NI; i++) fb[i] = wgrad_frag<DT>(fragG + i * 16 * E, rsG);
-        if constexpr (E == 4) {
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                if (!(ok >> (4 * s))) break; // wave-uniform
-#pragma unroll
-                for (int i = 0; i < MI; i++)
-#pragma unroll
-                    for (int j = 0; j < NI; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float4v, fa[i])[s],
-                                                                         __builtin_bit_cast(float4v, fb[j])[s], acc[i][j], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < MI; i++)
-#pragma unroll
-                for (int j = 0; j < NI; j++) acc[i][j] = mfma_step<DT>(fa[i], fb[j], acc[i][j]);
-        }
-    };
-
-    // Per slice, this wave owns batches wave, wave+4, ... (at most NB).  All their index
-    // entries are requested at once; then the rows run DEPTH-1 batches ahead of their
-    // staging through DEPTH register sets, and staging runs one batch ahead of the MFMAs.
-    // The single staging area is safe because LDS operations of a wave execute in order.
-    constexpr int NB = kWsSlice / GPB / 4;
-    constexpr int DEPTH = 3;
-    for (int s0 = h * kWsSlice; s0 < total; s0 += slice_step * kWsSlice) {
-        const int s1 = min(total, s0 + kWsSlice);
-        const int nbatch = (s1 - s0 + GPB - 1) / GPB;
-        const int bases = slot_bases(s0);
-        int idx[NB];
-        bool valid[NB];
-#pragma unroll
-        for (int j = 0; j < NB; j++) idx[j] = load_idx(bases, s0, s1, wave + 4 * j, valid[j]);
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-            idx[j] = (valid[j] && (unsigned)idx[j] < (unsigned)(lane < 32 ? a.in_rows : a.out_rows)) ? idx[j] : -1;
-        int4v ra[DEPTH][MI], rg[DEPTH][NI];
-        unsigned ok[DEPTH], staged = 0;
-#pragma unroll
-        for (int j = 0; j < DEPTH - 1; j++)
-            if (j < NB) ok[j] = gather(idx[j], ra[j], rg[j]);
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            if (wave + 4 * j < nbatch) {     // wave-uniform
-                if (j + DEPTH - 1 < NB)
-                    ok[(j + DEPTH - 1) % DEPTH] = gather(idx[j + DEPTH - 1], ra[(j + DEPTH - 1) % DEPTH], rg[(j + DEPTH - 1) % DEPTH]);
-                if (j > 0) multiply(staged);      // batch j-1, from LDS
-                asm volatile("" ::: "memory");    // keep the staging writes behind the transposing reads
-                stage(ok[j % DEPTH], ra[j % DEPTH], rg[j % DEPTH]);
-                staged = ok[j % DEPTH] & (unsigned)((1ull << PB) - 1);
-                asm volatile("" ::: "memory");
-            }
-        }
-        if (wave < nbatch) multiply(staged);      // the last staged batch
-    }
-
-    // Sum the four waves' blocks through LDS (over the staging areas), pairwise: (0+2, 1+3),
-    // then (0+1).  The partial is stored in accumulator order -- tile (i,j), lane, 4 values:
-    // element [16i + 4(lane/16) + r][16j + lane%16] -- as 16-byte stores; the reduction kernel
-    // puts it back in [iC,oC] order.
-    float4v *red = (float4v *)s_raw;
-    constexpr int BLK = MI * NI * kWave;   // float4 per block
-    __syncthreads();
-    if (wave >= 2) {
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NI; j++) red[(wave - 2) * BLK + (i * NI + j) * kWave + lane] = acc[i][j];
-    }
-    __syncthreads();
-    if (wave < 2) {
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NI; j++) acc[i][j] += red[wave * BLK + (i * NI + j) * kWave + lane];
-    }
-    __syncthreads();
-    if (wave == 1) {
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NI; j++) red[(i * NI + j) * kWave + lane] = acc[i][j];
-    }
-    __syncthreads();
-    if (wave == 0) {
-        float4v *part = (float4v *)(a.partial + ((long)slot * gridDim.y + blockIdx.y) * (kWsBlock * kWsBlock));
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NI; j++) part[(i * NI + j) * kWave + lane] = acc[i][j] + red[(i * NI + j) * kWave + lane];
-        if (lane == 0 && blockIdx.y == 0) a.flags[slot] = 1;
-    }
-}
-
-// dw[k][ci][co] = sum of the written slots of offset k, in slot order.  A slot holds one
-// 64x64 block per (iC,oC) block pair, each in accumulator order of MI x NI tiles (see
-// wgrad_wave_kernel).  A thread owns one 16-byte item of a block (four ci of one co), so the
-// slots are read as they were written; a workgroup covers 32 consecutive items, its 8 groups of
-// 32 threads each add every 8th slot (up to sixteen loads in flight), and the 8 sub-sums are added in a
-// fixed order.
-template <typename OUT>
-__global__ __launch_bounds__(256) void wgrad_slot_reduce_kernel(const float *partial, const int *flags, int slots_per_k,
-                                                                int iC, int oC, int mi_tiles, int ni_tiles, OUT *dw)
-{
-    __shared__ float4v s_sum[8][32];
-    __shared__ unsigned long long s_flags[16];
-    const int k = blockIdx.z, b = blockIdx.y, t = threadIdx.x & 31, j = threadIdx.x >> 5;
-    const int q = blockIdx.x * 32 + t;       // 16-byte item of the block, in accumulator order
-    const int sbn = (oC + kWsBlock - 1) / kWsBlock, nblk = ((iC + kWsBlock - 1) / kWsBlock) * sbn;
-    const int tile = q >> 6, lane = q & 63;
-    const bool live = tile < mi_tiles * ni_tiles;
-    const long blk = (long)kWsBlock * kWsBlock, step = (long)nblk * blk;
-    const float *p = partial + ((long)k * slots_per_k * nblk + b) * blk + q * 4;
-    const int *f = flags + (long)k * slots_per_k;
-    float4v s = {0.f, 0.f, 0.f, 0.f};
-    // The flags of 1024 slots at a time become 16 ballot words in LDS, so that a thread's data loads do not
-    // wait for flag loads: per round a thread takes its 16 candidates of two words (slots j, j+8, ... of each),
-    // the loads of the written ones in flight together, and adds them in slot order.
-    for (int base = 0; base < slots_per_k; base += 1024) {
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const int c = base + w * 256 + (int)threadIdx.x;
-            const unsigned long long m = __ballot(c < slots_per_k && f[c] != 0);
-            if ((threadIdx.x & (kWave - 1)) == 0) s_flags[w * 4 + (threadIdx.x >> 6)] = m;
-        }
-        __syncthreads();
-        if (!live) continue;
-        const int nwords = min(16, (slots_per_k - base + 63) >> 6);
-        for (int w0 = 0; w0 < nwords; w0 += 2) {
-            const unsigned long long m0 = s_flags[w0] >> j, m1 = w0 + 1 < nwords ? s_flags[w0 + 1] >> j : 0ull;
-            float4v v[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) {
-                const unsigned long long m = u < 8 ? m0 : m1;
-                const int cc = base + (w0 + (u >> 3)) * 64 + j + 8 * (u & 7);
-                v[u] = float4v{0.f, 0.f, 0.f, 0.f};
-                if ((m >> (8 * (u & 7))) & 1ull) v[u] = *(const float4v *)(p + cc * step);
-            }
-#pragma unroll
-            for (int u = 0; u < 16; u++) s += v[u];
-        }
-    }
-    s_sum[j][t] = s;
-    __syncthreads();
-    if (j == 0 && live) {
-        float4v r = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int g = 0; g < 8; g++) r += s_sum[g][t];
-        // accumulator order inside the block: tile (li/16, lj/16), lane = 16*((li%16)/4) + lj%16, value li%4
-        const int ci = (b / sbn) * kWsBlock + (tile / ni_tiles) * 16 + (lane >> 4) * 4;
-        const int co = (b % sbn) * kWsBlock + (tile % ni_tiles) * 16 + (lane & 15);
-        if (co < oC) {
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                if (ci + v < iC) dw[((long)k * iC + ci + v) * oC + co] = (OUT)r[v];
-        }
-    }
-}
-
 inline int elem_size(sph_dtype dt) { return sph_elem_size(dt); }
 inline int frag_elems(sph_dtype dt) { return sph_frag_elems(dt); }
 inline int pad_waves(int ndim) { return sph_pad_waves(ndim); }
 inline int num_steps(sph_dtype dt, int kdim) { return sph_num_steps(dt, kdim); }
-inline int wgrad_chunks(int ntiles) { return ntiles < 32 ? (ntiles < 1 ? 1 : ntiles) : 32; }
-
-template <typename K>
-inline int set_lds(K kernel, size_t bytes)
-{
-    if (bytes > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-        if (e != hipSuccess) {
-            sph_set_error("hipFuncSetAttribute(%zu bytes of LDS): %s", bytes, hipGetErrorString(e));
-            return SPH_ERR_LAUNCH;
-        }
-    }
-    return SPH_OK;
-}
 
 template <sph_dtype DT, int NW, int NSTEP>
 int launch_conv_ns(const ConvArgs &a, int ntiles, hipStream_t st)
@@ -1404,99 +875,6 @@ int launch_conv_nw(const ConvArgs &a, int nw, int ntiles, hipStream_t st)
     }
 }
 
-// 16-channel tiles of one side of the widest block: 1, 2 or 4
-inline int wgrad_tiles(int channels)
-{
-    const int t = sph_div_up(channels < kWsBlock ? channels : kWsBlock, 16);
-    return t <= 1 ? 1 : (t <= 2 ? 2 : 4);
-}
-inline size_t wgrad_wave_lds(int e, int mi, int ni)
-{
-    const int pb = (e == 2 ? 2 : 1) * SPH_GROUP;
-    const size_t stage = (size_t)4 * pb * ((mi * 16 * e + 16) + (ni * 16 * e + 16));
-    const size_t red = (size_t)2 * mi * ni * kWave * 4 * sizeof(float); // two waves' blocks at once
-    return stage > red ? stage : red;
-}
-inline int wgrad_wave_chunks(int ntiles) { return ntiles < 1 ? 1 : sph_div_up(ntiles, kWsTiles); }
-inline bool wgrad_wave_ok(sph_dtype dt, int iC, int oC)
-{
-    const int e = elem_size(dt);
-    return (iC * e) % 16 == 0 && (oC * e) % 16 == 0;
-}
-
-template <sph_dtype DT>
-int launch_wgrad(const WgradArgs &a0, void *dw, bool f32_out, hipStream_t st)
-{
-    typedef typename Traits<DT>::elem elem;
-    const int KV = a0.book.KV;
-    const int per_k = a0.iC * a0.oC;
-    const long total = (long)KV * per_k;
-    const bool aligned = ((uintptr_t)a0.feat % 16 == 0) && ((uintptr_t)a0.dout % 16 == 0);
-    const bool small = (double)a0.in_rows * a0.iC * sizeof(elem) < 4294967296.0 &&
-                       (double)a0.out_rows * a0.oC * sizeof(elem) < 4294967296.0 &&
-                       (double)a0.ntiles * a0.cap * SPH_GROUP < 2147483648.0;
-    if (wgrad_wave_ok(DT, a0.iC, a0.oC) && aligned && small && a0.in_rows > 0 && a0.out_rows > 0) {
-        WgradArgs a = a0;
-        const int sb = sph_div_up(a.iC, kWsBlock) * sph_div_up(a.oC, kWsBlock);
-        a.nchunk = wgrad_wave_chunks(a.ntiles);
-        // the centre offset's chain is what a small book's kernel lasts: eight workgroups share it there; on large
-        // books four, which halves the partial blocks to write and add (measured: headline scan 29 -> 23.5 us with
-        // eight, 8 scans 109 -> 115 us)
-        a.nslice = a.nchunk <= 16 ? kWsSlices : kWsSlices / 2;
-        a.nslots = KV * a.nchunk * a.nslice;
-        a.flags = (int *)(a.partial + (size_t)a.nslots * sb * kWsBlock * kWsBlock);
-        // later slices for every offset only where the whole grid stays small (measured: a full 4x4x128x4 grid, one
-        // chunk, 15 us with them and 33 us without; 8 chunks 32 against 35 us; from 12 chunks on the shorter grid wins)
-        a.all_slices = KV * a.nchunk * 4 <= 1024;
-        const dim3 grid(sph_xcd_grid(KV * a.nchunk) + (a.nslice - 1) * a.nchunk * (a.all_slices ? KV : 1), sb);
-        const int mi = wgrad_tiles(a.iC), ni = wgrad_tiles(a.oC);
-        int rc;
-#define SPH_WGRAD_CASE(M, N)                                                                      \
-    if (mi == M && ni == N) {                                                                     \
-        const size_t lds = wgrad_wave_lds((int)sizeof(elem), M, N);                               \
-        rc = set_lds(wgrad_wave_kernel<DT, M, N>, lds);                                           \
-        if (rc) return rc;                                                                        \
-        hipLaunchKernelGGL((wgrad_wave_kernel<DT, M, N>), grid, dim3(256), lds, st, a);           \
-    }
-        SPH_WGRAD_CASE(1, 1) SPH_WGRAD_CASE(1, 2) SPH_WGRAD_CASE(1, 4)
-        SPH_WGRAD_CASE(2, 1) SPH_WGRAD_CASE(2, 2) SPH_WGRAD_CASE(2, 4)
-        SPH_WGRAD_CASE(4, 1) SPH_WGRAD_CASE(4, 2) SPH_WGRAD_CASE(4, 4)
-#undef SPH_WGRAD_CASE
-        rc = sph_check_launch("sph_conv_wgrad");
-        if (rc) return rc;
-        if (f32_out)
-            hipLaunchKernelGGL(wgrad_slot_reduce_kernel<float>, dim3((unsigned)(mi * ni * 2), sb, KV), dim3(256), 0, st,
-                               a.partial, a.flags, a.nchunk * a.nslice, a.iC, a.oC, mi, ni, (float *)dw);
-        else
-            hipLaunchKernelGGL(wgrad_slot_reduce_kernel<elem>, dim3((unsigned)(mi * ni * 2), sb, KV), dim3(256), 0, st,
-                               a.partial, a.flags, a.nchunk * a.nslice, a.iC, a.oC, mi, ni, (elem *)dw);
-        return sph_check_launch("sph_conv_wgrad(reduce)");
-    }
-    const WgradArgs &a = a0;
-    constexpr int LDP = 4 * Traits<DT>::KW + 16 / (int)sizeof(elem);
-    const int iCp = (a.iC + 15) & ~15, oCp = (a.oC + 15) & ~15;
-    size_t lds = (size_t)(iCp + oCp) * LDP * sizeof(elem);
-    hipLaunchKernelGGL(wgrad_kernel<DT>, dim3(KV * a.nchunk), dim3(kWgThreads), lds, st, a);
-    int rc = sph_check_launch("sph_conv_wgrad");
-    if (rc) return rc;
-    if (f32_out)
-        hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                           a.partial, KV, a.nchunk, per_k, (float *)dw);
-    else
-        hipLaunchKernelGGL(wgrad_reduce_kernel<elem>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                           a.partial, KV, a.nchunk, per_k, (elem *)dw);
-    return sph_check_launch("sph_conv_wgrad(reduce)");
-}
-
-inline int book_has_groups(const sph_book *b) { return b->grp_k && b->grp_gather && b->grp_owner; }
-
-// the groups may be missing (all three arrays null) in a book that keeps its pairs by row
-inline int book_ok(const sph_book *b)
-{
-    return b && b->tile_ngrp && b->tile_koff && b->rows >= 0 && b->KV > 0 && b->KV <= SPH_MAX_KV &&
-           (book_has_groups(b) || (b->tile_nbr && !b->grp_k && !b->grp_gather && !b->grp_owner));
-}
-
 } // namespace
 
 SPH_EXPORT size_t sph_weight_packed_bytes(sph_dtype dt, int KV, int kdim, int ndim)
@@ -1571,66 +949,4 @@ SPH_EXPORT int sph_conv_apply(sph_dtype dt, const void *feature, int feature_row
     case SPH_BF16: return launch_conv_nw<SPH_BF16>(a, nw, nt, st);
     default: return launch_conv_nw<SPH_I8>(a, nw, nt, st);
     }
-}
-
-SPH_EXPORT size_t sph_wgrad_partial_elems(int KV, int iC, int oC, int out_rows)
-{
-    if (KV <= 0 || iC <= 0 || oC <= 0) return 0;
-    const int ntiles = sph_book_tiles(out_rows);
-    const size_t general = (size_t)KV * wgrad_chunks(ntiles) * iC * oC;
-    const size_t slots = (size_t)KV * wgrad_wave_chunks(ntiles) * kWsSlices;
-    const size_t blocks = (size_t)sph_div_up(iC, kWsBlock) * sph_div_up(oC, kWsBlock);
-    const size_t fast = slots * blocks * kWsBlock * kWsBlock + slots; // 64x64 blocks + one flag word per slot
-    return general > fast ? general : fast;
-}
-
-// `book`: stationary on the output rows, or on the input rows (`transposed`); other_rows: the rows its groups gather
-static int conv_wgrad(sph_dtype dt, const void *feature, int iC, const void *d_out, int oC, const sph_book *book, int other_rows,
-                      bool transposed, float *partial, void *d_weight, int d_weight_f32, void *stream)
-{
-    SPH_REQUIRE(book_ok(book) && book_has_groups(book), SPH_ERR_ARG, "sph_conv_wgrad: bad book (it must hold its groups)");
-    SPH_REQUIRE(partial && d_weight, SPH_ERR_ARG, "sph_conv_wgrad: null pointer");
-    SPH_REQUIRE(dt == SPH_F32 || dt == SPH_F16 || dt == SPH_BF16, SPH_ERR_UNSUPPORTED,
-                "sph_conv_wgrad: dtype %d has no weight gradient", (int)dt);
-    SPH_REQUIRE(iC > 0 && iC <= 128 && oC > 0 && oC <= 128, SPH_ERR_UNSUPPORTED,
-                "sph_conv_wgrad: channels %d->%d not in 1..128", iC, oC);
-    const int in_rows = transposed ? book->rows : other_rows, out_rows = transposed ? other_rows : book->rows;
-    SPH_REQUIRE((in_rows == 0 || feature) && (out_rows == 0 || d_out), SPH_ERR_ARG, "sph_conv_wgrad: null pointer");
-    WgradArgs a;
-    a.feat = (const char *)feature;
-    a.in_rows = in_rows;
-    a.iC = iC;
-    a.dout = (const char *)d_out;
-    a.out_rows = out_rows;
-    a.oC = oC;
-    a.book = *book;
-    a.list_in = transposed ? book->grp_owner : book->grp_gather;
-    a.list_out = transposed ? book->grp_gather : book->grp_owner;
-    a.cap = sph_book_cap(book->KV);
-    a.ntiles = sph_book_tiles(book->rows);
-    a.nchunk = wgrad_chunks(a.ntiles);
-    a.partial = partial;
-    a.nslots = 0;
-    a.flags = nullptr;
-    a.all_slices = 0;
-    a.nslice = kWsSlices;
-    hipStream_t st = (hipStream_t)stream;
-    switch (dt) {
-    case SPH_F32: return launch_wgrad<SPH_F32>(a, d_weight, true, st);
-    case SPH_F16: return launch_wgrad<SPH_F16>(a, d_weight, d_weight_f32 != 0, st);
-    default: return launch_wgrad<SPH_BF16>(a, d_weight, d_weight_f32 != 0, st);
-    }
-}
-
-SPH_EXPORT int sph_conv_wgrad(sph_dtype dt, const void *feature, int in_rows, int iC, const void *d_out,
-                              int oC, const sph_book *fwd_book, float *partial, void *d_weight, int d_weight_f32,
-                              void *stream)
-{
-    return conv_wgrad(dt, feature, iC, d_out, oC, fwd_book, in_rows, false, partial, d_weight, d_weight_f32, stream);
-}
-
-SPH_EXPORT int sph_conv_wgrad_transposed(sph_dtype dt, const void *feature, int iC, const void *d_out, int out_rows, int oC,
-                                         const sph_book *t_book, float *partial, void *d_weight, int d_weight_f32, void *stream)
-{
-    return conv_wgrad(dt, feature, iC, d_out, oC, t_book, out_rows, true, partial, d_weight, d_weight_f32, stream);
 }

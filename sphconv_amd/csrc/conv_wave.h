@@ -81,6 +81,28 @@ __device__ __forceinline__ int4v mfma_step<SPH_I8>(int4v a, int4v b, int4v d)
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, d, 0, 0, 0);
 }
 
+inline int book_has_groups(const sph_book *b) { return b->grp_k && b->grp_gather && b->grp_owner; }
+
+// the groups may be missing (all three arrays null) in a book that keeps its pairs by row
+inline int book_ok(const sph_book *b)
+{
+    return b && b->tile_ngrp && b->tile_koff && b->rows >= 0 && b->KV > 0 && b->KV <= SPH_MAX_KV &&
+           (book_has_groups(b) || (b->tile_nbr && !b->grp_k && !b->grp_gather && !b->grp_owner));
+}
+
+template <typename K>
+inline int set_lds(K kernel, size_t bytes)
+{
+    if (bytes > 48 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (e != hipSuccess) {
+            sph_set_error("hipFuncSetAttribute(%zu bytes of LDS): %s", bytes, hipGetErrorString(e));
+            return SPH_ERR_LAUNCH;
+        }
+    }
+    return SPH_OK;
+}
+
 // can sph_conv_apply walk this call by stationary row?
 inline bool rows_path_ok(const ConvArgs &a)
 {

@@ -456,13 +456,7 @@ int launch_split(const ConvArgs &a, int nwtot, hipStream_t st, int lds)
     constexpr int least = tab + 4 * (NB / 2) * CT * 1024; // the exchange of the waves' sums
     lds = lds < least ? least : lds;
     const int cap_rows = (lds - tab) / (NS * 64);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void *)conv_rows_split_kernel<DT, NS, CT, MASKED, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) {
-            sph_set_error("hipFuncSetAttribute(%d bytes of LDS): %s", lds, hipGetErrorString(e));
-            return SPH_ERR_LAUNCH;
-        }
-    }
+    if (int rc = set_lds(conv_rows_split_kernel<DT, NS, CT, MASKED, NB>, lds)) return rc;
     const int units = sph_div_up(a.book.rows, NB * SPH_GROUP);
     hipLaunchKernelGGL((conv_rows_split_kernel<DT, NS, CT, MASKED, NB>), dim3(sph_xcd_grid(units), sph_div_up(nwtot, CT)),
                        dim3(4 * kWave), lds, st, a, nwtot, cap_rows);
