@@ -18,6 +18,7 @@
 #include "conv_wave.h"
 #include "relay.h"
 #include "rows_split.h"
+#include "rows_hold.h"
 
 #include <cstdlib>
 
@@ -225,7 +226,8 @@ __global__ __launch_bounds__(kWave * S) __attribute__((amdgpu_waves_per_eu(1))) 
 // 16x16x32 MFMAs issue every 16 cycles): a stage's selects, LDS exchange and waits are in
 // series with its MFMAs, and two waves per SIMD do not cover them.
 // ---------------------------------------------------------------------------
-// (Short grids, and long ones of 128-byte rows whose rows lie close together, share a row's offsets between waves: rows_split.hip.)
+// (Short grids, and long ones of 128-byte rows whose rows lie close together, share a row's offsets between waves: rows_split.hip; long
+// grids into 17 to 32 columns keep the weight in LDS: rows_hold.hip.)
 template <sph_dtype DT, int NS, int CT, bool MASKED>
 __device__ __forceinline__ void conv_rows_body(const ConvArgs &a, int nwtot)
 {
@@ -845,6 +847,7 @@ int launch_conv(const ConvArgs &a, int ntiles, hipStream_t st)
 {
     // by stationary row, when the book keeps that form (rows of up to 128 bytes; its table must fit LDS)
     if (rows_path_ok(a)) {
+        if (sph_rows_hold_ok(DT, a, NW, ntiles)) return sph_rows_hold_launch(DT, a, st);
         if (!win_first<DT>(a, NW, ntiles) && sph_rows_split_ok(DT, a, NW, ntiles)) return sph_rows_split_launch(DT, a, NW, ntiles, st);
         if (a.nsteps == 1) return launch_conv_rows_ct<DT, 1>(a, NW, ntiles, st);
         return launch_conv_rows_ct<DT, 2>(a, NW, ntiles, st);
