@@ -18,9 +18,11 @@
 #include <memory>
 #include <mutex>
 #include <optional>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/sphconv_hip.h"
+#include "outcoords.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -159,6 +161,46 @@ public:
         return both ? __atomic_load_n(w, __ATOMIC_ACQUIRE) : (int64_t) __atomic_load_n((int32_t *)w, __ATOMIC_ACQUIRE);
     }
 };
+
+// ---- cells on the GPU that a count adds to --------------------------------------------------------
+// Zeros before and after a count, so a count in flight has cells of its own and the next one needs no launch that clears them.
+// Pages of 64 counts' cells (139 KB) for each device, as many as there were counts in flight at once; like the pinned words they
+// live as long as the process, and cells whose count nobody has seen end are not handed out again.
+class CountCells {
+    std::mutex m;
+    std::vector<Tensor> pages;
+    std::unordered_map<int, std::vector<uint64_t *>> free_;
+
+public:
+    uint64_t *take(const OnDevice &here, const Tensor &like)
+    {
+        const int device = like.device().index();
+        std::lock_guard<std::mutex> lock(m);
+        std::vector<uint64_t *> &f = free_[device];
+        if (f.empty()) {
+            const int words = sph_outcoords2_cell_words();
+            Tensor page = at::zeros({64, words}, like.options().dtype(at::kLong).requires_grad(false));
+            // another stream's count may be the first to use them
+            const hipError_t e = hipStreamSynchronize(here.stream);
+            if (e != hipSuccess) raise(std::string("clearing the cells of a count: ") + hipGetErrorString(e));
+            pages.push_back(page);
+            for (int i = 63; i >= 0; i--) f.push_back((uint64_t *)page.data_ptr<int64_t>() + (int64_t)i * words);
+        }
+        uint64_t *c = f.back();
+        f.pop_back();
+        return c;
+    }
+    void give(int device, uint64_t *c)
+    {
+        std::lock_guard<std::mutex> lock(m);
+        free_[device].push_back(c);
+    }
+};
+CountCells &count_cells()
+{
+    static CountCells *p = new CountCells; // never destroyed, as the pinned words
+    return *p;
+}
 
 // ---- geometry and books -------------------------------------------------------------------------
 struct Geometry {
@@ -306,33 +348,46 @@ py::object rules_build_pack(const Tensor &z_idx, const Tensor &z_ptr, const Tens
     return py::cast(p[0]);
 }
 
-// Output coordinates of a strided layer.  start(): the count and its scan are enqueued, and behind them already the
+// Output coordinates of a strided layer.  start(): the count is enqueued, and behind it already the
 // kernel that writes the coordinates, into arrays of the most rows the layer can reach -- prod ceil(K / stride) per input
 // row -- so that the GPU has work while the host learns the row count and enqueues what needs it.  What is handed out is
 // then the leading part of arrays that may be several times its size and live as long as it does, so this is done where
 // the two arrays hold at most kAheadBytes; beyond, the coordinates are written after the wait, into arrays of their size.
+// Two launches, or three (a scan between them) for deep or very large grids and where a stream is being recorded.
 struct OutCoords {
     static constexpr double kAheadBytes = 16 << 20;
     Tensor z_idx, z_ptr, oz_ptr, scratch, oz_idx, cols;
     const Geometry *geom;
     py::object geom_owner;
     HostWord total;
+    uint64_t *cells = nullptr; // of a count in two launches
     long bound;
-    bool filled = false;
+    bool filled = false, returned = false;
     OutCoords(const OnDevice &here, Tensor zi, Tensor zp, py::object g)
         : z_idx(std::move(zi)), z_ptr(std::move(zp)), geom(g.cast<const Geometry *>()), geom_owner(g), total(here)
     {
         const sph_geom &q = geom->g;
-        const int n = sph_outcoords_scratch_ints(&q);
+        int n = sph_outcoords2_scratch_ints(&q);
         if (n < 0) check(n);
+        hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+        if (n > 0 && (hipStreamIsCapturing(here.stream, &recording) != hipSuccess || recording != hipStreamCaptureStatusNone)) n = 0;
+        const bool two = n > 0;
+        if (!two) {
+            n = sph_outcoords_scratch_ints(&q);
+            if (n < 0) check(n);
+        }
         oz_ptr = at::empty({q.B, q.O[0], q.O[1]}, z_ptr.options());
         scratch = ints(n + (n & 1) + 2, z_ptr);
         const int rows = (int)z_idx.size(0);
         double most = rows;
         for (int d = 0; d < 3; d++) most *= (q.K[d] + q.stride[d] - 1) / q.stride[d];
         most = std::min(most, (double)q.B * q.O[0] * q.O[1] * q.O[2]);
-        check(sph_outcoords_count(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), rows, &q, ptr<int32_t>(oz_ptr), ptr<int32_t>(scratch),
-                                  total.address(), total.on()));
+        if (two) {
+            cells = count_cells().take(here, z_ptr);
+            check(sph_outcoords2_count(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), rows, &q, ptr<int32_t>(scratch), cells, total.address(), total.on()));
+        } else
+            check(sph_outcoords_count(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), rows, &q, ptr<int32_t>(oz_ptr), ptr<int32_t>(scratch),
+                                      total.address(), total.on()));
         if (most * 8 <= kAheadBytes) {
             bound = (long)most;
             fill(here, bound);
@@ -343,8 +398,12 @@ struct OutCoords {
     {
         oz_idx = ints(rows, z_ptr);
         cols = ints(rows, z_ptr);
-        check(sph_outcoords_fill(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), (int)z_idx.size(0), &geom->g, ptr<int32_t>(scratch),
-                                 ptr<int32_t>(oz_ptr), ptr<int32_t>(oz_idx), (int)rows, ptr<int32_t>(cols), total.on()));
+        if (cells)
+            check(sph_outcoords2_fill(&geom->g, ptr<int32_t>(scratch), ptr<int32_t>(oz_ptr), ptr<int32_t>(oz_idx), (int)rows, ptr<int32_t>(cols),
+                                      total.on()));
+        else
+            check(sph_outcoords_fill(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), (int)z_idx.size(0), &geom->g, ptr<int32_t>(scratch),
+                                     ptr<int32_t>(oz_ptr), ptr<int32_t>(oz_idx), (int)rows, ptr<int32_t>(cols), total.on()));
         filled = true;
     }
     uintptr_t on() const { return (uintptr_t)total.on(); }
@@ -352,6 +411,10 @@ struct OutCoords {
     std::tuple<Tensor, Tensor, Tensor> finish()
     {
         const long rows = (long)total.wait(false);
+        if (cells && !returned) { // all zeros again
+            count_cells().give(z_ptr.device().index(), cells);
+            returned = true;
+        }
         if (rows < 0 || (filled && rows > bound)) raise("the output coordinates of a strided layer are inconsistent");
         if (!filled) fill(OnDevice(z_ptr), rows);
         else if (rows < bound) {

@@ -8,6 +8,7 @@
 #include "common.h"
 #include "pack.h"
 #include "scan.h"
+#include "outcoords.h"
 
 #include <cstring>
 #include <mutex>
@@ -182,20 +183,42 @@ __global__ __launch_bounds__(kCountThreads) void outcoords_count_kernel(OutArgs 
     if (part == 0) counts[oc] = cnt;
 }
 
+// The sum of all n workgroups' v to *total (pinned host memory), by the last of them: each adds itself and its value to one of sixteen
+// cells, the last of a cell adds that cell's to the seventeenth.  Adding to one address queues at about 20 ns an addition, so 1024
+// workgroups on one cell took 20 us; a cell is 128 bytes from the next.  The cells are zeros before and, by the time the total is seen, after.
+constexpr int kCells = 16, kCellWords = 16;
+__device__ __forceinline__ void sum_of_all(int v, int i, int n, unsigned long long *cells, int32_t *total)
+{
+    auto add = [](unsigned long long *cell, int value, int of) -> int { // the cell's sum, if this was the last of its `of` additions, or -1
+        const unsigned long long old = __hip_atomic_fetch_add(cell, 1ull << 32 | (unsigned)value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((int)(old >> 32) != of - 1) return -1;
+        __hip_atomic_store(cell, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the store has arrived
+        return (int)(unsigned)old + value;
+    };
+    const int c = i % kCells, sum = add(cells + c * kCellWords, v, (n - c + kCells - 1) / kCells);
+    if (sum < 0) return;
+    const int all = add(cells + kCells * kCellWords, sum, min(n, kCells));
+    if (all >= 0) __hip_atomic_store(total, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The usual kernel: a workgroup takes `tc` neighbouring output columns of
 // one (b, o0) line, turns each of the K0 x ((tc - 1) * s1 + K1) input columns that reach them into the bins it covers on
 // the output side, once, and every output column ORs K0 * K1 of those words.  With 16 lanes per output column walking
 // the fibers themselves every fiber was walked by each of the two to nine columns it reaches, by lanes of which seven of
 // sixteen had none, and a bin was found by trying every k2: 19.3 us at the 131 072 output columns of four scans (64x2048x64,
 // 3x3x3, stride 2), instruction bound; this way 8.3 us, half of it the chain of dependent loads of the longest fibers.
-// NCH: words of 64 bins per column (O2 <= 64 * NCH).
-template <int NCH>
+// NCH: words of 64 bins per column (O2 <= 64 * NCH).  SUM: no counts are written but every workgroup's sum of them, to counts[blockIdx.x],
+// and the sum of all to *total.
+template <int NCH, bool SUM>
 __global__ __launch_bounds__(kThreads) void outcoords_count_tile_kernel(OutArgs a, int32_t *counts, unsigned long long *masks,
-                                                                        int *scan_state, int scan_state_n, int tc, int tiles1)
+                                                                        int *scan_state, int scan_state_n, int tc, int tiles1,
+                                                                        unsigned long long *cells, int32_t *total)
 {
     extern __shared__ unsigned long long s_words[]; // [NCH][K0 * W]
+    __shared__ int s_sum[kThreads / kWave];
     const int tid = threadIdx.x;
-    if (blockIdx.x == 0)
+    if (!SUM && blockIdx.x == 0)
         for (int i = tid; i < scan_state_n; i += kThreads) scan_state[i] = 0;
     const int nchunk = mask_chunks(a.O.n2);
     const int t1 = blockIdx.x % tiles1, line = blockIdx.x / tiles1;
@@ -243,6 +266,7 @@ __global__ __launch_bounds__(kThreads) void outcoords_count_tile_kernel(OutArgs 
         for (int c = 0; c < NCH; c++) s_words[c * n_in + it] = m[c];
     }
     lds_barrier();
+    int sum = 0;
     for (int j = tid; j < n1; j += kThreads) {
         const long oc = (long)line * a.O.n1 + o1_0 + j;
         int cnt = 0;
@@ -255,7 +279,20 @@ __global__ __launch_bounds__(kThreads) void outcoords_count_tile_kernel(OutArgs 
             cnt += __popcll(m);
             if (masks) masks[oc * nchunk + c] = m;
         }
-        counts[oc] = cnt;
+        if (SUM) sum += cnt;
+        else counts[oc] = cnt;
+    }
+    if (SUM) {
+        sum = wave_inclusive_sum(sum);
+        if ((tid & (kWave - 1)) == kWave - 1) s_sum[tid / kWave] = sum;
+        lds_barrier();
+        if (tid == 0) {
+            int s = 0;
+#pragma unroll
+            for (int w = 0; w < kThreads / kWave; w++) s += s_sum[w];
+            counts[blockIdx.x] = s;
+            sum_of_all(s, (int)blockIdx.x, (int)gridDim.x, cells, total);
+        }
     }
 }
 
@@ -288,6 +325,66 @@ __global__ __launch_bounds__(kThreads) void outcoords_fill_tile_kernel(int ncol,
         for (int i = tid; i < n; i += kThreads) {
             oz_idx[w + i] = s_z[i];
             if (row_cols) row_cols[w + i] = c0 + s_c[i];
+        }
+        lds_barrier();
+    }
+}
+
+// The same behind a count that left its workgroups' sums: a workgroup takes whole tiles of the count's (256 columns at most), adds up
+// the sums of those before them and scans its own columns' counts, which the masks say; it writes oz_ptr too.  One launch less on the
+// way to the coordinates than with the scan of all counts in between: 131 072 output columns, 1024 workgroups of the count, 8.4 + 4.6 + 8.0 us
+// in three launches with a gap of 4 us beside the scan, 9.8 + 8.8 in two.
+__global__ __launch_bounds__(kThreads) void outcoords_place_kernel(int O1, int tc, int tiles1, int tiles, int nchunk, const int32_t *sums,
+                                                                   const unsigned long long *masks, int32_t *oz_ptr, int32_t *oz_idx,
+                                                                   int out_rows, int32_t *row_cols)
+{
+    __shared__ uint16_t s_z[kFillWindow];
+    __shared__ unsigned char s_c[kFillWindow];
+    __shared__ int s_col[kThreads], s_part[2][kThreads / kWave];
+    const int tid = threadIdx.x, wave = tid / kWave;
+    const int t0 = blockIdx.x * (kThreads / tc), t = t0 + tid / tc;
+    const int line = t / tiles1, o1 = (t - line * tiles1) * tc + tid % tc;
+    const bool live = t < tiles && o1 < O1;
+    const long c = live ? (long)line * O1 + o1 : 0;
+    int count = 0, before = 0;
+    if (live)
+        for (int ch = 0; ch < nchunk; ch++) count += __popcll(masks[c * nchunk + ch]);
+    for (int i = tid * 4; i < t0; i += kThreads * 4) { // (the array goes on to a multiple of four)
+        const int4 v = *(const int4 *)(sums + i);
+        before += v.x + (i + 1 < t0 ? v.y : 0) + (i + 2 < t0 ? v.z : 0) + (i + 3 < t0 ? v.w : 0);
+    }
+    const int incl = wave_inclusive_sum(count);
+    before = wave_inclusive_sum(before);
+    s_col[tid] = (int)c;
+    if ((tid & (kWave - 1)) == kWave - 1) {
+        s_part[0][wave] = incl;
+        s_part[1][wave] = before;
+    }
+    lds_barrier();
+    int first = 0, all = 0, mine = incl;
+#pragma unroll
+    for (int w = 0; w < kThreads / kWave; w++) {
+        first += s_part[1][w];
+        all += s_part[0][w];
+        mine += w < wave ? s_part[0][w] : 0;
+    }
+    if (live) oz_ptr[c] = first + mine;
+    const int last = clampi(first + all, 0, out_rows), start = first + mine - count;
+    for (int w = clampi(first, 0, out_rows); w < last; w += kFillWindow) {
+        if (count) {
+            int at = start - w;
+            for (int ch = 0; ch < nchunk; ch++)
+                for (unsigned long long m = masks[c * nchunk + ch]; m; m &= m - 1, at++)
+                    if ((unsigned)at < (unsigned)kFillWindow) {
+                        s_z[at] = (uint16_t)(ch * 64 + __ffsll((long long)m) - 1);
+                        s_c[at] = (unsigned char)tid;
+                    }
+        }
+        lds_barrier();
+        const int n = min(kFillWindow, last - w);
+        for (int i = tid; i < n; i += kThreads) {
+            oz_idx[w + i] = s_z[i];
+            if (row_cols) row_cols[w + i] = s_col[s_c[i]];
         }
         lds_barrier();
     }
@@ -610,6 +707,34 @@ static OutArgs out_args(const int32_t *z_idx, const int32_t *z_ptr, int in_rows,
     return a;
 }
 
+// Tiles of outcoords_count_tile_kernel: as many output columns as leave the chip two workgroups per CU (fewer fibers are then read
+// twice), and fit 32 KB of words.  nch = 0: another kernel's grid.
+struct CountTiles { int nch, tc, tiles1; long tiles; size_t lds; };
+static CountTiles count_tiles(const sph_geom *g)
+{
+    const int nchunk = mask_chunks(g->O[2]), nch = nchunk <= 1 ? 1 : (nchunk <= 2 ? 2 : (nchunk <= 4 ? 4 : kMaskChunks));
+    const long lines = (long)g->B * g->O[0];
+    auto words = [&](int tc) { return (size_t)nch * g->K[0] * ((size_t)(tc - 1) * g->stride[1] + g->K[1]) * 8; };
+    int tc = 128;
+    while (tc > 16 && (lines * sph_div_up(g->O[1], tc) < 512 || words(tc) > 32 * 1024)) tc /= 2;
+    const long tiles = lines * sph_div_up(g->O[1], tc);
+    const bool ok = nchunk <= kMaskChunks && words(tc) <= 32 * 1024 && tiles < 2147483647L;
+    return CountTiles{ok ? nch : 0, tc, sph_div_up(g->O[1], tc), tiles, words(tc)};
+}
+
+template <bool SUM>
+static void launch_count_tiles(const CountTiles &t, const OutArgs &a, int32_t *counts, unsigned long long *masks, int *state, int nstate,
+                               unsigned long long *cells, int32_t *total, hipStream_t st)
+{
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)t.tiles), dim3(kThreads), t.lds, st, a, counts, masks, state, nstate, t.tc, t.tiles1, cells, total);
+    };
+    if (t.nch == 1) go(outcoords_count_tile_kernel<1, SUM>);
+    else if (t.nch == 2) go(outcoords_count_tile_kernel<2, SUM>);
+    else if (t.nch == 4) go(outcoords_count_tile_kernel<4, SUM>);
+    else go(outcoords_count_tile_kernel<kMaskChunks, SUM>);
+}
+
 static int outcoords_count(const char *who, const int32_t *z_idx, const int32_t *z_ptr, int in_rows, const sph_geom *g,
                            int32_t *oz_ptr, int32_t *scratch, int32_t *total, void *stream)
 {
@@ -617,26 +742,10 @@ static int outcoords_count(const char *who, const int32_t *z_idx, const int32_t 
     SPH_REQUIRE(z_ptr && oz_ptr && scratch && in_rows >= 0 && (in_rows == 0 || z_idx), SPH_ERR_ARG, "%s: null argument", who);
     SPH_REQUIRE((uintptr_t)scratch % 8 == 0, SPH_ERR_ARG, "%s: scratch must be 8-byte aligned", who);
     const long ncol = (long)g->B * g->O[0] * g->O[1];
-    // Output columns per workgroup: as many as leave the chip two workgroups per CU (fewer fibers are then read twice), and
-    // fit 32 KB of words.
-    const int nchunk = mask_chunks(g->O[2]), nch = nchunk <= 1 ? 1 : (nchunk <= 2 ? 2 : (nchunk <= 4 ? 4 : kMaskChunks));
-    const long lines = (long)g->B * g->O[0];
-    auto words = [&](int tc) { return (size_t)nch * g->K[0] * ((size_t)(tc - 1) * g->stride[1] + g->K[1]) * 8; };
-    int tc = 128;
-    while (tc > 16 && (lines * sph_div_up(g->O[1], tc) < 512 || words(tc) > 32 * 1024)) tc /= 2;
-    const long tiles = lines * sph_div_up(g->O[1], tc);
-    if (nchunk <= kMaskChunks && words(tc) <= 32 * 1024 && tiles < 2147483647L) {
-        const OutArgs oa = out_args(z_idx, z_ptr, in_rows, g);
-        unsigned long long *masks = outcoords_masks(g, scratch);
-        const int tiles1 = sph_div_up(g->O[1], tc), ns = sph_scan::state_ints(ncol);
-#define SPH_COUNT(N)                                                                                                      \
-    hipLaunchKernelGGL(outcoords_count_tile_kernel<N>, dim3((unsigned)tiles), dim3(kThreads), words(tc), (hipStream_t)stream, oa, \
-                       oz_ptr, masks, (int *)scratch, ns, tc, tiles1)
-        if (nch == 1) SPH_COUNT(1);
-        else if (nch == 2) SPH_COUNT(2);
-        else if (nch == 4) SPH_COUNT(4);
-        else SPH_COUNT(kMaskChunks);
-#undef SPH_COUNT
+    const CountTiles tiles = count_tiles(g);
+    if (tiles.nch) {
+        launch_count_tiles<false>(tiles, out_args(z_idx, z_ptr, in_rows, g), oz_ptr, outcoords_masks(g, scratch), (int *)scratch,
+                                  sph_scan::state_ints(ncol), nullptr, nullptr, (hipStream_t)stream);
     } else
         hipLaunchKernelGGL(outcoords_count_kernel, dim3((unsigned)((ncol + kCountCols - 1) / kCountCols)), dim3(kCountThreads), 0, (hipStream_t)stream,
                        out_args(z_idx, z_ptr, in_rows, g), oz_ptr, outcoords_masks(g, scratch), (int *)scratch,
@@ -649,6 +758,53 @@ static int outcoords_count(const char *who, const int32_t *z_idx, const int32_t 
         sph_set_error("%s: scan: %s", who, hipGetErrorString(e));
         return SPH_ERR_LAUNCH;
     }
+    return sph_check_launch(who);
+}
+
+// ---------------------------------------------------------------------------
+// The same in two launches (outcoords.h): the count leaves its workgroups' sums and the row count, the second one adds those up.
+// Every workgroup of the second reads the sums before its own, so there are at most kMostSums of them (4 loads a thread); where
+// there are more, or no masks are kept, the scan of the counts is the better way.
+// ---------------------------------------------------------------------------
+constexpr long kMostSums = 4096;
+static long two_launch_sums(const sph_geom *g)
+{
+    const CountTiles t = count_tiles(g);
+    return t.nch && keeps_masks(g) && t.tiles <= kMostSums ? (t.tiles + 3) / 4 * 4 : 0;
+}
+static unsigned long long *two_launch_masks(const sph_geom *g, int32_t *scratch) { return (unsigned long long *)(scratch + two_launch_sums(g)); }
+
+SPH_EXPORT int sph_outcoords2_cell_words() { return (kCells + 1) * kCellWords; }
+
+SPH_EXPORT int sph_outcoords2_scratch_ints(const sph_geom *g)
+{
+    SPH_REQUIRE(sph_geom_ok(g), SPH_ERR_ARG, "sph_outcoords2_scratch_ints: bad geometry");
+    const long sums = two_launch_sums(g), n = sums + 2L * g->B * g->O[0] * g->O[1] * mask_chunks(g->O[2]);
+    return sums && n < 2147483647L ? (int)n : 0;
+}
+
+SPH_EXPORT int sph_outcoords2_count(const int32_t *z_idx, const int32_t *z_ptr, int in_rows, const sph_geom *g, int32_t *scratch,
+                                    uint64_t *cells, int32_t *total, void *stream)
+{
+    const char *who = "sph_outcoords2_count";
+    SPH_REQUIRE(sph_geom_ok(g) && two_launch_sums(g), SPH_ERR_ARG, "%s: not a geometry for it", who);
+    SPH_REQUIRE(z_ptr && scratch && cells && total && in_rows >= 0 && (in_rows == 0 || z_idx), SPH_ERR_ARG, "%s: null argument", who);
+    SPH_REQUIRE((uintptr_t)scratch % 16 == 0, SPH_ERR_ARG, "%s: scratch must be 16-byte aligned", who);
+    launch_count_tiles<true>(count_tiles(g), out_args(z_idx, z_ptr, in_rows, g), scratch, two_launch_masks(g, scratch), nullptr, 0,
+                             (unsigned long long *)cells, total, (hipStream_t)stream);
+    return sph_check_launch(who);
+}
+
+SPH_EXPORT int sph_outcoords2_fill(const sph_geom *g, const int32_t *scratch, int32_t *oz_ptr, int32_t *oz_idx, int out_rows,
+                                   int32_t *row_cols, void *stream)
+{
+    const char *who = "sph_outcoords2_fill";
+    SPH_REQUIRE(sph_geom_ok(g) && two_launch_sums(g), SPH_ERR_ARG, "%s: not a geometry for it", who);
+    SPH_REQUIRE(scratch && oz_ptr && out_rows >= 0 && (out_rows == 0 || oz_idx), SPH_ERR_ARG, "%s: null argument", who);
+    const CountTiles t = count_tiles(g);
+    hipLaunchKernelGGL(outcoords_place_kernel, dim3((unsigned)sph_div_up((int)t.tiles, kThreads / t.tc)), dim3(kThreads), 0, (hipStream_t)stream,
+                       g->O[1], t.tc, t.tiles1, (int)t.tiles, mask_chunks(g->O[2]), scratch, two_launch_masks(g, (int32_t *)scratch), oz_ptr,
+                       oz_idx, out_rows, row_cols);
     return sph_check_launch(who);
 }
 
