@@ -138,6 +138,178 @@ __global__ __launch_bounds__(128) void conv_wave_kernel(ConvArgs a, int nwtot)
     conv_wave_store<DT, CT>(a, nwtot, s_acc, col0, r0, nrows, lane, kWave);
 }
 
+// Two tiles at a time, for fp32 rows of 132 to 256 bytes into 33 to 64 columns, where a group of 16 pairs takes 64 matrix instructions of
+// 32 cycles, empty slots or not.  At LiDAR sparsity a tile has about one group at an offset and five pairs in it: the last groups
+// of two neighbouring tiles at an offset are merged where their pairs fit one.  Two waves take 32 columns each of 256
+// accumulator rows, as much LDS for a wave as one that takes 64 columns of one tile.  A row's sum is in conv_wave_kernel's order.
+// Where merging would save less than a quarter of the groups, or the list has no room, each wave takes one tile as conv_wave_kernel does
+// (full grids: 64 -> 64 on 922 tiles of 24 pairs a row 241 : 234 us, 1021 tiles of 12 151 : 144).
+// What bounds it: in conv_wave_kernel the matrix cores, 69 % of the time with two slots of three empty; here the rows and fragments,
+// 12 KB for a group and wave (a quarter more than half of what one wave with all columns loads), and two round trips more to make the list.
+// us, 64 -> 64: strided layer of eight 64x512x512 scans, 2848 tiles, 117.7 -> 96.4; submanifold, 1.6 pairs a row beside its own, 4048
+// tiles 185 -> 168, 1207 tiles 84.6 -> 74.8.  Rows and fragments requested as far ahead as conv_wave_groups does, two groups of 1024 cycles:
+// no gain (124); five 104 to 112, six 102 to 108 (behind 62 loads a wave cannot have more counted).
+constexpr int kPairRoom = 104;   // merged groups that fit the LDS beside the accumulators of two workgroups per compute unit
+constexpr int kPairRows = 2 * R;
+constexpr int kPairLists = kPairRoom * (SPH_GROUP * 5 + 4 + 4 + 1); // gat, desc, count of the first, own, gk
+// The merged groups into 32 columns of the two tiles' rows.  A group is 32 matrix instructions here, half as long as in conv_wave_groups, so rows
+// and fragments are requested kPairAhead groups ahead (a wave has its SIMD to itself: 512 registers).
+constexpr int kPairAhead = 6;
+template <int NS, bool MASKED>
+__device__ __forceinline__ void pair_groups(const ConvArgs &a, int nwtot, const int32_t *gat, const unsigned char *own, const unsigned char *gk,
+                                            int total, uint32_t *s_acc, int col0, int lane)
+{
+    constexpr int CT = 2, D = kPairAhead;
+    const int LDW = nwtot * 16 + 4, wstep = nwtot * (kWave * 16);
+    const __amdgpu_buffer_rsrc_t r_feat = __builtin_amdgcn_make_buffer_rsrc((void *)a.feat, 0, a.feat_rows * a.row_bytes, kRsrcFlags);
+    const __amdgpu_buffer_rsrc_t r_w = __builtin_amdgcn_make_buffer_rsrc((void *)a.wp, 0, a.book.KV * NS * wstep, kRsrcFlags);
+    const int w_lane = (col0 / 16) * (kWave * 16) + lane * 16, chunk = (lane >> 4) * 16, acc_lane = (col0 + (lane >> 4) * 4) * 4;
+    int4v x[D][NS], w[D][NS][CT];
+    struct Entry { int gi, k; };
+    auto entry = [&](int j) -> Entry { // (behind the last group: that one again)
+        const int g = min(j, total - 1);
+        return Entry{gat[g * SPH_GROUP + (lane & 15)], gk[g]};
+    };
+    auto acc_row = [&](int j) -> uint32_t * {
+        const int g = min(j, total - 1), at = g * SPH_GROUP + (lane & 15);
+        const int row = j < total && gat[at] >= 0 ? own[at] : kPairRows;
+        return (uint32_t *)((char *)s_acc + (int)__umul24(row, LDW * 4) + acc_lane);
+    };
+    auto load = [&](const Entry &e, int4v (&xs)[NS], int4v (&ws)[NS][CT], int st) {
+        const int off = (int)__umul24((unsigned)max(e.gi, 0), (unsigned)a.row_bytes) + chunk, k = __builtin_amdgcn_readfirstlane(e.k);
+        xs[st] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(r_feat, off + st * 64, 0, 0));
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+            ws[st][c] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(r_w, w_lane + st * wstep + c * (kWave * 16), k * (NS * wstep), 0));
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        const Entry e = entry(d);
+#pragma unroll
+        for (int st = 0; st < NS; st++) load(e, x[d], w[d], st);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    conv_wave_clear<CT, kPairRows>(s_acc, LDW, col0, lane);
+    Entry next = entry(D);
+    uint32_t *p = acc_row(0);
+    for (int j0 = 0; j0 < total; j0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int j = j0 + d;
+            float4v acc[CT];
+#pragma unroll
+            for (int c = 0; c < CT; c++) acc[c] = *(const float4v *)(p + c * 16);
+            const Entry e = next;
+            next = entry(j + D + 1);
+            uint32_t *p_next = acc_row(j + 1);
+#pragma unroll
+            for (int st = 0; st < NS; st++) {
+                int4v v = x[d][st];
+                if constexpr (MASKED) {
+                    const bool live = st * 64 + chunk < a.row_bytes;
+                    v = live ? v : int4v{0, 0, 0, 0};
+                }
+#pragma unroll
+                for (int c = 0; c < CT; c++) acc[c] = mfma_step<SPH_F32>(w[d][st][c], v, acc[c]);
+                load(e, x[d], w[d], st);
+            }
+#pragma unroll
+            for (int c = 0; c < CT; c++) *(float4v *)(p + c * 16) = acc[c];
+            p = p_next;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+template <int NS, bool MASKED>
+__global__ __launch_bounds__(2 * kWave) __attribute__((amdgpu_waves_per_eu(1))) void conv_wave_pair_kernel(ConvArgs a, int nwtot)
+{
+    extern __shared__ __attribute__((aligned(16))) uint32_t s_acc[]; // [kPairRows + 1][LDW], then the merged groups
+    const int LDW = nwtot * 16 + 4;
+    int32_t *s_gat = (int32_t *)(s_acc + (kPairRows + 1) * LDW), *s_desc = s_gat + kPairRoom * SPH_GROUP, *s_first = s_desc + kPairRoom;
+    unsigned char *s_own = (unsigned char *)(s_first + kPairRoom), *s_gk = s_own + kPairRoom * SPH_GROUP;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const int ntiles = (a.book.rows + R - 1) / R, npairs = (ntiles + 1) / 2;
+    const int pair = sph_xcd_tile(blockIdx.x, npairs);
+    if (pair >= npairs) return; // whole workgroups leave
+    const int r0 = pair * kPairRows, nrows = min(kPairRows, a.book.rows - r0), KV = a.book.KV;
+    const int col0 = wave * 32;
+    const int tile[2] = {2 * pair, min(2 * pair + 1, ntiles - 1)};
+    const bool two = 2 * pair + 1 < ntiles;
+
+    // (each offset can save one group, so with more than four of them to an offset merging is out of the question)
+    int ng[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) ng[t] = t == 0 || two ? min(max(a.book.tile_ngrp[tile[t]], 0), a.cap) : 0;
+    const bool few = ng[0] + ng[1] <= 4 * KV;
+    // lane k: the tiles' groups at offset k, and how many slots of the last ones are taken (both waves find the same)
+    int g0[2] = {}, n[2] = {}, taken[2] = {};
+    if (few) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const unsigned short *ko = a.book.tile_koff + (long)tile[t] * (KV + 1) + min(lane, KV - 1);
+            g0[t] = min((int)ko[0], a.cap);
+            n[t] = lane < KV && (t == 0 || two) ? min(max((int)ko[1] - g0[t], 0), a.cap - g0[t]) : 0;
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int g = min(g0[t] + max(n[t] - 1, 0), a.cap - 1);
+            const int4v *e = (const int4v *)(a.book.grp_gather + ((long)tile[t] * a.cap + g) * SPH_GROUP);
+            int last = 0;
+#pragma unroll
+            for (int i = 0; i < SPH_GROUP / 4; i++) {
+                const int4v v = e[i];
+#pragma unroll
+                for (int j = 0; j < 4; j++) last = v[j] >= 0 ? i * 4 + j + 1 : last;
+            }
+            taken[t] = last;
+        }
+    }
+    const bool merge = n[0] > 0 && n[1] > 0 && taken[0] + taken[1] <= SPH_GROUP;
+    const int mine = n[0] + n[1] - (merge ? 1 : 0);
+    const int incl = wave_inclusive_sum(mine);
+    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+    const int apart = __builtin_amdgcn_readlane(wave_inclusive_sum(n[0] + n[1]), kWave - 1);
+    if (few && total <= kPairRoom && total * 4 <= apart * 3) {
+        // where group j of the list comes from: the group of the first tile in the low half, of the second in the high one (0xffff: none)
+        if (wave == 0)
+            for (int i = 0, j = incl - mine; i < mine; i++, j++) {
+                const bool both = merge && i == n[0] - 1;
+                const bool first = i < n[0];
+                const int ib = merge ? i - n[0] + 1 : i - n[0]; // the second tile's: its last one first, where it is merged
+                const int gb = merge ? (ib == 0 ? n[1] - 1 : ib - 1) : ib;
+                s_desc[j] = (first ? g0[0] + i : 0xffff) | (!first || both ? g0[1] + gb : 0xffff) << 16;
+                s_first[j] = first ? (both ? taken[0] : SPH_GROUP) : 0;
+                s_gk[j] = (unsigned char)lane;
+            }
+        lds_barrier();
+        for (int i = tid; i < total * SPH_GROUP; i += 2 * kWave) {
+            const int j = i / SPH_GROUP, s = i % SPH_GROUP, d = s_desc[j], nf = s_first[j];
+            const bool first = s < nf;
+            const unsigned g = first ? d & 0xffff : (unsigned)d >> 16;
+            const long slot = ((long)(first ? tile[0] : tile[1]) * a.cap + min(g, (unsigned)a.cap - 1)) * SPH_GROUP + (first ? s : s - nf);
+            const int gi = a.book.grp_gather[slot], ow = a.book.grp_owner[slot] - r0;
+            const bool ok = g != 0xffff && (unsigned)gi < (unsigned)a.feat_rows && (unsigned)ow < (unsigned)nrows;
+            s_gat[i] = ok ? gi : -1;
+            s_own[i] = (unsigned char)ow;
+        }
+        lds_barrier();
+        pair_groups<NS, MASKED>(a, nwtot, s_gat, s_own, s_gk, total, s_acc, col0, lane);
+        conv_wave_store<SPH_F32, 2>(a, nwtot, s_acc, col0, r0, nrows, lane, kWave);
+    } else {
+        // too full for the list, or for merging to pay: a wave takes all columns of one tile
+        const int first = wave * R;
+        if (first < nrows) {
+            const int mine = wave ? ng[1] : ng[0];
+            const BookMeta meta(a.book, a.cap, 2 * pair + wave, mine, r0, nrows, a.feat_rows);
+            conv_wave_clear<4, R - 1>(s_acc + first * LDW, LDW, 0, lane); // (the row for slots without a pair is both waves', and nobody's result)
+            conv_wave_groups<SPH_F32, NS, 4, MASKED, kPairRows>(a, nwtot, meta, mine, s_acc, 0, lane, false);
+            conv_wave_store<SPH_F32, 4>(a, nwtot, s_acc + first * LDW, 0, r0 + first, min(R, nrows - first), lane, kWave);
+        }
+    }
+}
+inline size_t pair_lds(int nwtot) { return (size_t)(kPairRows + 1) * (nwtot * 16 + 4) * 4 + kPairLists; }
+
 // The same with two helper waves per tile (up to 64 output columns, rows of up to 128 bytes).  A submanifold book
 // has a run of up to eight full groups at the middle offset (every row's pair with itself), which all use one set
 // of weight fragments: the helper waves load those fragments once, take the run's groups between them, multiply
@@ -704,6 +876,15 @@ int launch_conv_split(const ConvArgs &a, int nwtot, int ntiles, size_t lds, hipS
     return sph_check_launch("sph_conv_apply");
 }
 
+// Not below 513 tiles, where conv_wave_split_kernel shares a tile's groups between waves (64 -> 64, two tiles : those, 304 tiles 31.2 : 30.2,
+// 475 tiles 69 : 42), not for small kernels (9 offsets, 608 tiles 27.7 : 24.3, 2412 tiles 79 : 72: nothing to merge beside the middle's
+// full groups) and not where more rows are gathered than made (a strided layer's transposed book, 11 pairs to a group: 177 : 164).
+inline bool pair_ok(const ConvArgs &a, int nwtot, int ntiles)
+{
+    return nwtot == 4 && a.book.KV >= 18 && a.book.KV <= kWave && a.feat_rows <= a.book.rows && a.book.tile_koff &&
+           (uintptr_t)a.book.grp_gather % 16 == 0 && ntiles > 512;
+}
+
 template <sph_dtype DT, int NS, int CT, bool MASKED>
 int launch_conv_wave(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
 {
@@ -715,6 +896,15 @@ int launch_conv_wave(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
     // and the helper waves' barriers cost a full chip more than the run saves: 16 -> 16 on 4912 tiles 22.6 / 25.8 us)
     constexpr bool kRunKernel = NS <= 2 && !(DT == SPH_F32 && NS == 2 && CT == 4);
     const bool helpers = kRunKernel && waves == 1 && a.book.tile_koff && a.book.middle_run && (NS * CT >= 4 || ntiles <= 1024);
+    if constexpr (DT == SPH_F32 && NS == 4 && CT == 4) {
+        if (pair_ok(a, nwtot, ntiles)) {
+            const size_t lds2 = pair_lds(nwtot);
+            int rc = set_lds(conv_wave_pair_kernel<NS, MASKED>, lds2);
+            if (rc) return rc;
+            hipLaunchKernelGGL((conv_wave_pair_kernel<NS, MASKED>), dim3(sph_xcd_grid((ntiles + 1) / 2)), dim3(2 * kWave), lds2, st, a, nwtot);
+            return sph_check_launch("sph_conv_apply");
+        }
+    }
     if (waves == 1) {
         const int s = split_waves(DT, a.row_bytes, nwtot, helpers, ntiles, lds, 0);
         if (s == 4) return launch_conv_split<DT, NS, CT, MASKED, 4>(a, nwtot, ntiles, 4 * lds, st);

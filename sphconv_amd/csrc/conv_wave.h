@@ -279,14 +279,14 @@ struct LdsMeta {
 };
 
 // Clears the wave's CT*16 columns of the accumulator tile (and of the scratch row behind it).
-template <int CT>
+template <int CT, int ROWS = R>
 __device__ __forceinline__ void conv_wave_clear(uint32_t *s_acc, int LDW, int col0, int lane)
 {
-    for (int i = lane; i < (R + 1) * CT * 4; i += kWave)
+    for (int i = lane; i < (ROWS + 1) * CT * 4; i += kWave)
         *(int4v *)&s_acc[(i / (CT * 4)) * LDW + col0 + (i % (CT * 4)) * 4] = int4v{0, 0, 0, 0};
 }
 
-// The tile's groups, one after the other, into the wave's columns [col0, col0 + CT*16) of s_acc ([R + 1][LDW]
+// The tile's groups, one after the other, into the wave's columns [col0, col0 + CT*16) of s_acc ([ROWS + 1][LDW]
 // 32-bit words, cleared by the caller, by clear() below while the first indices are on their way, or by the other
 // waves of the workgroup meanwhile: wait_clear then makes this wave meet them at that many barriers before its first
 // sum).
@@ -299,7 +299,7 @@ __device__ __forceinline__ void conv_wave_clear(uint32_t *s_acc, int LDW, int co
 // same slot of the next block.  Everything a block of four groups needs from its indices -- accumulator
 // addresses, byte offsets of the rows to gather -- is computed at the top of the block from eight lane permutes
 // issued together, so no group waits for a permute of its own.
-template <sph_dtype DT, int NS, int CT, bool MASKED, class Meta>
+template <sph_dtype DT, int NS, int CT, bool MASKED, int ROWS = R, class Meta>
 __device__ __forceinline__ void conv_wave_groups(const ConvArgs &a, int nwtot, const Meta &meta, int ngrp, uint32_t *s_acc,
                                                  int col0, int lane, bool clear, int wait_clear = 0)
 {
@@ -348,7 +348,7 @@ __device__ __forceinline__ void conv_wave_groups(const ConvArgs &a, int nwtot, c
     };
     auto acc_ptr = [&](int ow_blk, int u) -> uint32_t * {
         const int rl = __shfl(ow_blk, u * SPH_GROUP + (lane & 15), kWave);
-        return (uint32_t *)((char *)s_acc + (int)__umul24((unsigned)(rl >= 0 ? rl : R), (unsigned)(LDW * 4)) + acc_lane);
+        return (uint32_t *)((char *)s_acc + (int)__umul24((unsigned)(rl >= 0 ? rl : ROWS), (unsigned)(LDW * 4)) + acc_lane);
     };
     auto group_step = [&](int4v (&fw)[NS][CT], int4v (&fa)[NS], uint32_t *p, int k_next2, int row_next) {
         acc4 d[CT];
@@ -391,7 +391,7 @@ __device__ __forceinline__ void conv_wave_groups(const ConvArgs &a, int nwtot, c
     meta.load(0, lane, gi_n, ow_n, k_n);
     meta.load(kBlk, lane, gi_nn, ow_nn, k_nn);
     // clear the accumulator tile (and the scratch row) while the first indices are on their way
-    if (clear) conv_wave_clear<CT>(s_acc, LDW, col0, lane);
+    if (clear) conv_wave_clear<CT, ROWS>(s_acc, LDW, col0, lane);
     meta.finish(0, lane, gi_n, ow_n, k_n);
     // The first loads are issued in the order the loop issues them, pinned against the scheduler: the compiler
     // places one wait count per use for every path into the loop, and a start in another order would make every
