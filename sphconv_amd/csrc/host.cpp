@@ -128,6 +128,8 @@ public:
         if (seen) pinned().give(w);
     }
     int32_t *address() { return (int32_t *)w; }
+    // the word, to an owner who gives it back once the store has arrived; only where wait() has not returned
+    int64_t *leave() const { return w; }
     hipStream_t on() const { return st; }
     // both: the two 32-bit halves are written by one store; otherwise only the low half is written
     int64_t wait(bool both)
@@ -165,17 +167,32 @@ public:
 // ---- cells on the GPU that a count adds to --------------------------------------------------------
 // Zeros before and after a count, so a count in flight has cells of its own and the next one needs no launch that clears them.
 // Pages of 64 counts' cells (139 KB) for each device, as many as there were counts in flight at once; like the pinned words they
-// live as long as the process, and cells whose count nobody has seen end are not handed out again.
+// live as long as the process.  A count that nobody waited for (its layer did not run, or raised) leaves its cells with its word, and
+// both are handed out again once the word says that the count has ended.
 class CountCells {
     std::mutex m;
     std::vector<Tensor> pages;
     std::unordered_map<int, std::vector<uint64_t *>> free_;
+    struct Left { int device; uint64_t *cells; int64_t *word; };
+    std::vector<Left> left;
+    void collect()
+    {
+        size_t kept = 0;
+        for (const Left &l : left)
+            if (__atomic_load_n((int32_t *)l.word, __ATOMIC_ACQUIRE) == (int32_t)-1) left[kept++] = l;
+            else {
+                free_[l.device].push_back(l.cells);
+                pinned().give(l.word);
+            }
+        left.resize(kept);
+    }
 
 public:
     uint64_t *take(const OnDevice &here, const Tensor &like)
     {
         const int device = like.device().index();
         std::lock_guard<std::mutex> lock(m);
+        if (!left.empty()) collect();
         std::vector<uint64_t *> &f = free_[device];
         if (f.empty()) {
             const int words = sph_outcoords2_cell_words();
@@ -194,6 +211,11 @@ public:
     {
         std::lock_guard<std::mutex> lock(m);
         free_[device].push_back(c);
+    }
+    void leave(int device, uint64_t *c, int64_t *word)
+    {
+        std::lock_guard<std::mutex> lock(m);
+        left.push_back(Left{device, c, word});
     }
 };
 CountCells &count_cells()
@@ -392,6 +414,12 @@ struct OutCoords {
             bound = (long)most;
             fill(here, bound);
         }
+    }
+    OutCoords(const OutCoords &) = delete;
+    OutCoords &operator=(const OutCoords &) = delete;
+    ~OutCoords()
+    {
+        if (cells && !returned) count_cells().leave(z_ptr.device().index(), cells, total.leave());
     }
     // (on the stream of the count, which `here`'s device is that of)
     void fill(const OnDevice &here, long rows)

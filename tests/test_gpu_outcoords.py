@@ -93,3 +93,19 @@ def test_counts_in_flight_on_streams_and_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_counts_nobody_waits_for_give_their_cells_back():
+    args = (1, (8, 40, 12), (3, 3, 3), (2, 2, 2), (1, 1, 1))
+    scene = _scene(args[0], args[1], 0.3, 1)
+    want = _three(*scene, *args)
+    _ahead(*scene, *args).native.finish()    # the first page of cells is there
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    for _ in range(130):                     # more than two pages
+        left = _ahead(*scene, *args)
+        torch.cuda.synchronize()
+        del left
+    assert torch.cuda.memory_allocated() == before
+    got = _ahead(*scene, *args).native.finish()
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
