@@ -164,6 +164,10 @@ __device__ __forceinline__ void pair_groups(const ConvArgs &a, int nwtot, const 
     const __amdgpu_buffer_rsrc_t r_feat = __builtin_amdgcn_make_buffer_rsrc((void *)a.feat, 0, a.feat_rows * a.row_bytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t r_w = __builtin_amdgcn_make_buffer_rsrc((void *)a.wp, 0, a.book.KV * NS * wstep, kRsrcFlags);
     const int w_lane = (col0 / 16) * (kWave * 16) + lane * 16, chunk = (lane >> 4) * 16, acc_lane = (col0 + (lane >> 4) * 4) * 4;
+    if (total == 0) { // tiles without a pair (rows no output reaches): there is no last group to ask for in a group's place
+        conv_wave_clear<CT, kPairRows>(s_acc, LDW, col0, lane);
+        return;
+    }
     int4v x[D][NS], w[D][NS][CT];
     struct Entry { int gi, k; };
     auto entry = [&](int j) -> Entry { // (behind the last group: that one again)

@@ -18,6 +18,7 @@ GRIDS = {  # (grid, batch, share of the bins, kernel, stride)
     "strided": ((64, 512, 64), 1, 0.02, (3, 3, 3), (2, 2, 2)),
     "18 offsets": ((64, 512, 32), 2, 0.07, (2, 3, 3), (1, 1, 1)),
     "45 offsets": ((64, 512, 32), 2, 0.07, (5, 3, 3), (1, 1, 1)),
+    "empty pairs of tiles": ((64, 128, 32), 1, 0.5, (3, 3, 3), (4, 1, 1)),   # transposed: every fourth plane reaches no output
 }
 
 
@@ -32,7 +33,12 @@ def test_against_the_pairs_in_float64(grid):
         out = [(s + 2 * (k // 2) - k) // t + 1 for s, k, t in zip(shape, kernel, stride)]
         book = RuleBook.build(z_idx, z_ptr, batch, list(shape), out, list(kernel), list(stride), [k // 2 for k in kernel])
         rows = book.oz_idx.numel()
-    rows_in, kv, buf = z_idx.numel(), book.kv, book.grouped()
+    empty = grid == "empty pairs of tiles"
+    rows_in, kv, buf = z_idx.numel(), book.kv, book.grouped(transposed=empty)
+    if empty:
+        rows_in, rows = rows, rows_in
+        ngrp = buf.tile_ngrp[:buf.ntiles // 2 * 2].view(-1, 2)
+        assert bool((ngrp.sum(1) == 0).any()) and bool((ngrp.sum(1) > 0).any())
     assert buf.ntiles > 512 and rows_in <= rows
     if grid == "odd tiles":
         assert buf.ntiles % 2
