@@ -130,6 +130,8 @@ public:
     int32_t *address() { return (int32_t *)w; }
     // the word, to an owner who gives it back once the store has arrived; only where wait() has not returned
     int64_t *leave() const { return w; }
+    // no kernel was given its address
+    void unused() { seen = true; }
     hipStream_t on() const { return st; }
     // both: the two 32-bit halves are written by one store; otherwise only the low half is written
     int64_t wait(bool both)
@@ -167,8 +169,8 @@ public:
 // ---- cells on the GPU that a count adds to --------------------------------------------------------
 // Zeros before and after a count, so a count in flight has cells of its own and the next one needs no launch that clears them.
 // Pages of 64 counts' cells (139 KB) for each device, as many as there were counts in flight at once; like the pinned words they
-// live as long as the process.  A count that nobody waited for (its layer did not run, or raised) leaves its cells with its word, and
-// both are handed out again once the word says that the count has ended.
+// live as long as the process.  A count that nobody waited for (its layer did not run, or raised, the call that starts the count
+// itself among them) leaves its cells with its word, and both are handed out again once the word says that the count has ended.
 class CountCells {
     std::mutex m;
     std::vector<Tensor> pages;
@@ -223,6 +225,40 @@ CountCells &count_cells()
     static CountCells *p = new CountCells; // never destroyed, as the pinned words
     return *p;
 }
+
+// A count's cells, beside the word it reports to: given back with the count's end, whichever way its owner ends.
+class HeldCells {
+    HostWord &word;
+    uint64_t *cells = nullptr;
+    int device = 0;
+    bool adding = false; // a kernel may add to them
+
+public:
+    explicit HeldCells(HostWord &w) : word(w) {}
+    HeldCells(const HeldCells &) = delete;
+    HeldCells &operator=(const HeldCells &) = delete;
+    ~HeldCells()
+    {
+        if (!cells) return;
+        if (adding) count_cells().leave(device, cells, word.leave());
+        else {
+            count_cells().give(device, cells);
+            word.unused();
+        }
+    }
+    uint64_t *take(const OnDevice &here, const Tensor &like)
+    {
+        device = like.device().index();
+        return cells = count_cells().take(here, like);
+    }
+    void launched() { adding = true; }
+    // the word has arrived: all zeros again
+    void done()
+    {
+        if (cells) count_cells().give(device, cells);
+        cells = nullptr;
+    }
+};
 
 // ---- geometry and books -------------------------------------------------------------------------
 struct Geometry {
@@ -382,9 +418,10 @@ struct OutCoords {
     const Geometry *geom;
     py::object geom_owner;
     HostWord total;
-    uint64_t *cells = nullptr; // of a count in two launches
+    HeldCells cells{total}; // of a count in two launches (destroyed before the word)
+    bool two;
     long bound;
-    bool filled = false, returned = false;
+    bool filled = false;
     OutCoords(const OnDevice &here, Tensor zi, Tensor zp, py::object g)
         : z_idx(std::move(zi)), z_ptr(std::move(zp)), geom(g.cast<const Geometry *>()), geom_owner(g), total(here)
     {
@@ -393,7 +430,7 @@ struct OutCoords {
         if (n < 0) check(n);
         hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
         if (n > 0 && (hipStreamIsCapturing(here.stream, &recording) != hipSuccess || recording != hipStreamCaptureStatusNone)) n = 0;
-        const bool two = n > 0;
+        two = n > 0;
         if (!two) {
             n = sph_outcoords_scratch_ints(&q);
             if (n < 0) check(n);
@@ -405,8 +442,11 @@ struct OutCoords {
         for (int d = 0; d < 3; d++) most *= (q.K[d] + q.stride[d] - 1) / q.stride[d];
         most = std::min(most, (double)q.B * q.O[0] * q.O[1] * q.O[2]);
         if (two) {
-            cells = count_cells().take(here, z_ptr);
-            check(sph_outcoords2_count(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), rows, &q, ptr<int32_t>(scratch), cells, total.address(), total.on()));
+            const int32_t *zi = ptr<int32_t>(z_idx), *zp = ptr<int32_t>(z_ptr);
+            int32_t *sc = ptr<int32_t>(scratch);
+            const int rc = sph_outcoords2_count(zi, zp, rows, &q, sc, cells.take(here, z_ptr), total.address(), total.on());
+            if (rc != SPH_ERR_ARG) cells.launched(); // (also where a launch is said to have failed: such cells are not handed out again)
+            check(rc);
         } else
             check(sph_outcoords_count(ptr<int32_t>(z_idx), ptr<int32_t>(z_ptr), rows, &q, ptr<int32_t>(oz_ptr), ptr<int32_t>(scratch),
                                       total.address(), total.on()));
@@ -417,16 +457,12 @@ struct OutCoords {
     }
     OutCoords(const OutCoords &) = delete;
     OutCoords &operator=(const OutCoords &) = delete;
-    ~OutCoords()
-    {
-        if (cells && !returned) count_cells().leave(z_ptr.device().index(), cells, total.leave());
-    }
     // (on the stream of the count, which `here`'s device is that of)
     void fill(const OnDevice &here, long rows)
     {
         oz_idx = ints(rows, z_ptr);
         cols = ints(rows, z_ptr);
-        if (cells)
+        if (two)
             check(sph_outcoords2_fill(&geom->g, ptr<int32_t>(scratch), ptr<int32_t>(oz_ptr), ptr<int32_t>(oz_idx), (int)rows, ptr<int32_t>(cols),
                                       total.on()));
         else
@@ -439,10 +475,7 @@ struct OutCoords {
     std::tuple<Tensor, Tensor, Tensor> finish()
     {
         const long rows = (long)total.wait(false);
-        if (cells && !returned) { // all zeros again
-            count_cells().give(z_ptr.device().index(), cells);
-            returned = true;
-        }
+        cells.done();
         if (rows < 0 || (filled && rows > bound)) raise("the output coordinates of a strided layer are inconsistent");
         if (!filled) fill(OnDevice(z_ptr), rows);
         else if (rows < bound) {

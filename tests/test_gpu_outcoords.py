@@ -109,3 +109,35 @@ def test_counts_nobody_waits_for_give_their_cells_back():
     assert torch.cuda.memory_allocated() == before
     got = _ahead(*scene, *args).native.finish()
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_counts_whose_arrays_find_no_memory_give_their_cells_back():
+    """The count is on its way when the arrays of its rows (2 MB each) are asked for: a layer that raises there leaves nothing behind."""
+    args = (1, (32, 1024, 128), (3, 3, 3), (2, 2, 2), (1, 1, 1))
+    scene = _scene(args[0], args[1], 0.05, 3)
+    want = _three(*scene, *args)
+    _ahead(*scene, *args).native.finish()    # the first page of cells is there
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    raised, full = 0, []
+    try:                                     # no new memory, and none left in what there is for more than the small arrays
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / torch.cuda.get_device_properties(0).total_memory)
+        try:
+            while True:
+                full.append(torch.empty(2 << 20, dtype=torch.uint8, device=DEV))
+        except torch.OutOfMemoryError:
+            pass
+        before = torch.cuda.memory_allocated()
+        for _ in range(130):                 # more than two pages
+            try:
+                _ahead(*scene, *args)
+            except torch.OutOfMemoryError:
+                raised += 1
+            torch.cuda.synchronize()
+        after = torch.cuda.memory_allocated()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        del full
+    assert raised == 130 and after == before
+    got = _ahead(*scene, *args).native.finish()
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
