@@ -75,6 +75,17 @@ struct OnDevice {
     }
 };
 
+// The default stream (handle 0) cannot be recorded and is not asked: while another stream that waits for it is recorded, the question
+// alone is an error.  A stream that cannot say counts as recorded, and leaves no error for the next launch to report.
+bool being_recorded(hipStream_t st)
+{
+    if (!st) return false;
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 Tensor bytes(size_t n, const Tensor &like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte).requires_grad(false)); }
 Tensor ints(int64_t n, const Tensor &like) { return at::empty({n}, like.options().dtype(at::kInt).requires_grad(false)); }
 
@@ -190,6 +201,7 @@ class CountCells {
     }
 
 public:
+    // null: no page can be had just now (the stream that would clear it cannot be waited for)
     uint64_t *take(const OnDevice &here, const Tensor &like)
     {
         const int device = like.device().index();
@@ -200,8 +212,10 @@ public:
             const int words = sph_outcoords2_cell_words();
             Tensor page = at::zeros({64, words}, like.options().dtype(at::kLong).requires_grad(false));
             // another stream's count may be the first to use them
-            const hipError_t e = hipStreamSynchronize(here.stream);
-            if (e != hipSuccess) raise(std::string("clearing the cells of a count: ") + hipGetErrorString(e));
+            if (hipStreamSynchronize(here.stream) != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
             pages.push_back(page);
             for (int i = 63; i >= 0; i--) f.push_back((uint64_t *)page.data_ptr<int64_t>() + (int64_t)i * words);
         }
@@ -246,11 +260,13 @@ public:
             word.unused();
         }
     }
-    uint64_t *take(const OnDevice &here, const Tensor &like)
+    bool take(const OnDevice &here, const Tensor &like)
     {
         device = like.device().index();
-        return cells = count_cells().take(here, like);
+        cells = count_cells().take(here, like);
+        return cells != nullptr;
     }
+    uint64_t *get() const { return cells; }
     void launched() { adding = true; }
     // the word has arrived: all zeros again
     void done()
@@ -428,9 +444,7 @@ struct OutCoords {
         const sph_geom &q = geom->g;
         int n = sph_outcoords2_scratch_ints(&q);
         if (n < 0) check(n);
-        hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
-        if (n > 0 && (hipStreamIsCapturing(here.stream, &recording) != hipSuccess || recording != hipStreamCaptureStatusNone)) n = 0;
-        two = n > 0;
+        two = n > 0 && !being_recorded(here.stream) && cells.take(here, z_ptr);
         if (!two) {
             n = sph_outcoords_scratch_ints(&q);
             if (n < 0) check(n);
@@ -444,7 +458,7 @@ struct OutCoords {
         if (two) {
             const int32_t *zi = ptr<int32_t>(z_idx), *zp = ptr<int32_t>(z_ptr);
             int32_t *sc = ptr<int32_t>(scratch);
-            const int rc = sph_outcoords2_count(zi, zp, rows, &q, sc, cells.take(here, z_ptr), total.address(), total.on());
+            const int rc = sph_outcoords2_count(zi, zp, rows, &q, sc, cells.get(), total.address(), total.on());
             if (rc != SPH_ERR_ARG) cells.launched(); // (also where a launch is said to have failed: such cells are not handed out again)
             check(rc);
         } else

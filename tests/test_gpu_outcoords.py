@@ -141,3 +141,26 @@ def test_counts_whose_arrays_find_no_memory_give_their_cells_back():
     assert raised == 130 and after == before
     got = _ahead(*scene, *args).native.finish()
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_the_default_stream_while_another_records():
+    """The default stream cannot be recorded, and must not be asked: where a stream that waits for it is, the question is an error."""
+    args = (1, (8, 40, 12), (3, 3, 3), (2, 2, 2), (1, 1, 1))
+    scene = _scene(args[0], args[1], 0.3, 2)
+    want = _three(*scene, *args)
+    torch.cuda.synchronize()
+    hip = C.CDLL("libamdhip64.so")
+    other, graph = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(other), 0) == 0        # a blocking one
+    try:
+        assert hip.hipStreamBeginCapture(other, 2) == 0
+        try:
+            flying = [_ahead(*scene, *args) for _ in range(70)]        # more than a page of cells
+            all_got = [f.native.finish() for f in flying]
+        finally:
+            assert hip.hipStreamEndCapture(other, C.byref(graph)) == 0
+    finally:
+        if graph:
+            hip.hipGraphDestroy(graph)
+        hip.hipStreamDestroy(other)
+    assert all(torch.equal(x, y) for got in all_got for x, y in zip(got, want))
