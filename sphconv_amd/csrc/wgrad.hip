@@ -416,9 +416,10 @@ __global__ __launch_bounds__(256, 2) void wgrad_stage_kernel(WgradArgs a)
 // ---------------------------------------------------------------------------
 // wgrad, fast path (rows are whole 16-byte chunks).
 //
-// Work item = (offset k, chunk of up to 512 tiles, part of that chunk's groups at k, 64x64 block of [iC,oC]).  A submanifold
-// book has eight groups a tile at the centre offset and about one at the others, so eight workgroups share the centre's: the
-// grid is one round of workgroups of about the same number of groups, and each ends with one partial block.
+// Work item = (offset k, chunk of up to 192 tiles, part of that chunk's groups at k, 64x64 block of [iC,oC]).  A submanifold
+// book has eight groups a tile at the centre offset and about one at the others, so eight workgroups share the centre's; where no offset
+// stands out each has one.  The grid is one round of workgroups of about the same number of groups (on long books whole rounds), and
+// each ends with one partial block.
 // The workgroup's four waves take its batches (64 pairs; 16 for fp32) round robin and never synchronise until the end.
 // The contraction runs over pairs and memory has channels side by side, so both operands have to be turned; a wave does that
 // in its registers.  fp32: lane (m = lane % 16, q = lane / 16) loads channels MI m .. MI m + MI - 1 of pair 4 s + q for the
@@ -442,8 +443,15 @@ __global__ __launch_bounds__(256, 2) void wgrad_stage_kernel(WgradArgs a)
 // its pairs in 3.1 times fewer tiles stationary on the input rows, with groups more than twice as full (64->64 fp32 on
 // eight 64x512x512 scans, stride 2, with the kernel through LDS: 117 us from the forward book, 59 us from the transposed one with the
 // empty fours left out; 24->40 bf16: 52 -> 38 us).
+//
+// Where the kernel through LDS was the faster one still: long books of nearly full grids with 32 channels on a side in 16 bits, whose offsets
+// all have seven groups a tile and whose centre's workgroups have an eighth of the others' work (9002 tiles of 24 pairs a row, 32->64 f16
+// 403 : 476 us; of 11 pairs a row 242 : 246, of 3.7 127 : 102).  A book does not say how full its grid is before its groups are counted on the GPU.
 // ---------------------------------------------------------------------------
-constexpr int kWsPer = 8;      // most tiles of a chunk per lane
+constexpr int kWsMost = 192, kWsMostLight = 128; // most tiles of a chunk, and where a compute unit holds more than two workgroups
+constexpr int kWsPer = 4;      // most of a lane (even)
+constexpr int kWsParts = 8;    // most workgroups that share a chunk's groups at the centre offset
+static_assert(kWsMost <= kWsPer * kWave, "a chunk's tiles fit the lanes");
 constexpr int kWsLeast = 24;   // groups of a centre offset's share: six for every wave
 
 // f(0), f(1), ... until one says no
@@ -866,28 +874,40 @@ inline int wgrad_stage_chunks(int ntiles) { return ntiles < 1 ? 1 : sph_div_up(n
 inline size_t wgrad_wave_lds(int mi, int ni) { return (size_t)2 * mi * ni * kWave * 4 * sizeof(float) + 4 * kWsPer * kWave * sizeof(unsigned); }
 // Workgroups of wgrad_wave_kernel on a compute unit, by its registers (197 to 256, 141 to 194 for a side of 64 channels, 113 at most).
 inline int wgrad_wave_occupancy(bool f32, int mi, int ni) { return mi * ni >= 16 || !f32 ? 2 : (mi * ni >= 8 ? 3 : 4); }
-constexpr int kWsParts = 8;    // workgroups that share a chunk's groups at the centre offset
-// Chunks of a book's tiles: one round of workgroups of about the same number of groups each (a submanifold book has eight a tile at the
-// centre, about one at the others).  With whole chunks to an XCD (sixteen of them, six workgroups at the centre) 3 % fewer lines
-// come from memory, and the centre's workgroups last a third longer than the others: 32.9 : 29.0 us.
-// A small book's chunks are eight, or of 48 tiles (fp32: 16) if that is more, and in 16 bits of no fewer than eight tiles: each more
+// Does the middle offset hold far more pairs than the others?  The caller says so; a layer with as many rows out as in is taken for one too.
+inline bool wgrad_run(const WgradArgs &a) { return (a.book.middle_run != 0) || a.in_rows == a.out_rows; }
+struct WavePlan { int nchunk, nparts; };
+// Chunks of a book's tiles, and workgroups that share a chunk's groups at the centre offset: one round of workgroups of about the same number of
+// groups each.  A submanifold book has eight groups a tile at the centre and about one at the others, so eight share the centre's; of small
+// kernels (most of their offsets' pairs are there) four.  Where no offset stands out one: with eight the others' workgroups were four
+// times as long as the centre's and half the chip idle (2x2x2 stride 2, 64->64 f16, 998 tiles 20.4 us through LDS, 23.9 with eight, 19.0 with
+// one; fp32, transposed book of 16 611 tiles 264, 511, 237).
+// A round: with whole chunks to an XCD (sixteen of them, six workgroups at the centre) 3 % fewer lines come from memory, and the centre's
+// workgroups last a third longer than the others: 32.9 : 29.0 us.
+// An offset has at most 256 partial blocks in a round: few workgroups add up those of a small kernel (1x1x1, 2005 tiles, 32->64 f16: 504 blocks
+// 19.8 us, 252 17.3).
+// A small book's chunks are eight, or of 48 tiles for 27 offsets (fp32: 16) if that is more, and in 16 bits of no fewer than eight tiles: each more
 // writes a block for every offset and one for each of the centre's workgroups, and the sum of them then lasts longer than
-// the chunks' loads are shorter (608 tiles, 64->64 f16, nine offsets: 32 chunks 17.4 us, 19 16.2, 13 14.8; a full grid of 16 tiles,
+// the chunks' loads are shorter (608 tiles, 64->64 f16: 19 chunks 23 us, 13 20.5; nine offsets: 8 chunks 21, 38 18; a full grid of 16 tiles,
 // 27 offsets: 2 chunks 16.2, 1 chunk 20.0).  In fp32 a chunk's chain of products is longer (a full grid of 462 tiles, 64->64: 15 chunks
-// 125 us, 10 181; of 16 tiles: 8 chunks 16.3, 2 28.5; 608 tiles, 16->16, nine offsets: 38 chunks 13.2, 64 15.8).
-inline int wgrad_wave_chunks(int ntiles, int KV, int blocks, int occupancy, bool f32)
+// 125 us, 10 181; of 16 tiles: 8 chunks 16.3, 2 28.5).
+// A long book's chunks hold 192 tiles at most, 128 where a compute unit has three workgroups or four: the offsets of a longer chunk fall so far
+// behind each other that their rows are no longer in the XCD's L2 (64->64 f16, a full grid of 9002 tiles: chunks of 300 tiles 574 us, through LDS 537;
+// 32->32 fp32, stride 2, transposed book of 7057 tiles: chunks of 236 tiles 170, 96 tiles 143, through LDS 131).
+inline WavePlan wgrad_wave_plan(int ntiles, int KV, int blocks, int occupancy, bool f32, bool run)
 {
-    const int fit = 256 * occupancy / ((KV - 1 + kWsParts) * blocks), round = fit < 1 ? 1 : fit;
-    const int tiles = f32 ? 16 : 48;
+    const int nparts = !run ? 1 : (KV >= 16 ? kWsParts : kWsParts / 2);
+    const int slots = 256 / nparts, all = 256 * occupancy / ((KV - 1 + nparts) * blocks), fit = all < slots ? all : slots, round = fit < 1 ? 1 : fit;
+    const int of27 = (f32 ? 16 : 48) * KV / 27, least = run ? (f32 ? 8 : 16) : 4, tiles = of27 > least ? of27 : least;
     if (ntiles < tiles * round) {
         const int most = f32 ? ntiles : sph_div_up(ntiles, 8);
         const int n = sph_div_up(ntiles, tiles) < 8 ? 8 : sph_div_up(ntiles, tiles);
         const int r = n < round ? n : round, m = r < most ? r : most;
-        return m < 1 ? 1 : m;
+        return WavePlan{m < 1 ? 1 : m, nparts};
     }
     int n = round;
-    while (sph_div_up(ntiles, n) > kWsPer * kWave) n += round;
-    return n;
+    while (sph_div_up(ntiles, n) > (occupancy > 2 ? kWsMostLight : kWsMost)) n += round;
+    return WavePlan{n, nparts};
 }
 inline bool wgrad_wave_ok(sph_dtype dt, int iC, int oC)
 {
@@ -911,7 +931,8 @@ int launch_wgrad(const WgradArgs &a0, void *dw, bool f32_out, hipStream_t st)
         constexpr bool F32 = sizeof(elem) == 4;
         const int sb = wgrad_blocks(a.iC, a.oC);
         int mi = wgrad_tiles(a.iC), ni = wgrad_tiles(a.oC), slots, layout;
-        if (!F32 && mi * ni <= 4) {
+        // (books of four tiles or less: with 32 channels on one side this kernel's shorter way to its first product is 0.6 us of 9)
+        if (!F32 && (mi * ni <= 4 || (mi * ni == 8 && a.ntiles <= 4))) {
             a.nchunk = wgrad_stage_chunks(a.ntiles);
             // the centre offset's chain is what a small book's kernel lasts: eight workgroups share it there; on large
             // books four, which halves the partial blocks to write and add
@@ -927,11 +948,13 @@ int launch_wgrad(const WgradArgs &a0, void *dw, bool f32_out, hipStream_t st)
 #define SPH_WGRAD_CASE(M, N) \
     if (mi == M && ni == N) hipLaunchKernelGGL((wgrad_stage_kernel<DT, M, N>), grid, block, wgrad_stage_lds(M, N), st, a);
                 SPH_WGRAD_CASE(1, 1) SPH_WGRAD_CASE(1, 2) SPH_WGRAD_CASE(1, 4) SPH_WGRAD_CASE(2, 1) SPH_WGRAD_CASE(2, 2) SPH_WGRAD_CASE(4, 1)
+                SPH_WGRAD_CASE(2, 4) SPH_WGRAD_CASE(4, 2)
 #undef SPH_WGRAD_CASE
             }
         } else {
-            a.nchunk = wgrad_wave_chunks(a.ntiles, KV, sb, wgrad_wave_occupancy(F32, mi, ni), F32);
-            a.nparts = kWsParts;
+            const WavePlan plan = wgrad_wave_plan(a.ntiles, KV, sb, wgrad_wave_occupancy(F32, mi, ni), F32, wgrad_run(a));
+            a.nchunk = plan.nchunk;
+            a.nparts = plan.nparts;
             a.chunk_tiles = sph_div_up(a.ntiles, a.nchunk);
             slots = a.nchunk * a.nparts;
             layout = F32 ? kWsWords : kWsHalves;
@@ -982,8 +1005,13 @@ SPH_EXPORT size_t sph_wgrad_partial_elems(int KV, int iC, int oC, int out_rows)
     const int ntiles = sph_book_tiles(out_rows);
     const size_t general = (size_t)KV * wgrad_chunks(ntiles) * iC * oC;
     // whichever kernel and type takes it
-    const size_t wave = (size_t)KV * wgrad_wave_chunks(ntiles, KV, wgrad_blocks(iC, oC), 4, true) * kWsParts;
-    const size_t stage = (size_t)KV * wgrad_stage_chunks(ntiles) * kWsSlices, slots = wave > stage ? wave : stage;
+    size_t slots = (size_t)KV * wgrad_stage_chunks(ntiles) * kWsSlices;
+    for (int i = 0; i < 4; i++)
+        for (int occupancy = 2; occupancy <= 4; occupancy++) {
+            const WavePlan p = wgrad_wave_plan(ntiles, KV, wgrad_blocks(iC, oC), occupancy, i & 1, i & 2);
+            const size_t wave = (size_t)KV * p.nchunk * p.nparts;
+            slots = wave > slots ? wave : slots;
+        }
     const size_t blocks = (size_t)sph_div_up(iC, kWsBlock) * sph_div_up(oC, kWsBlock);
     const size_t fast = slots * blocks * kWsBlock * kWsBlock + slots; // 64x64 blocks + one flag word per slot
     return general > fast ? general : fast;

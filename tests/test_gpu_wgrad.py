@@ -29,7 +29,10 @@ GRIDS = {
     "sparse": ((40, 300, 30), 1, 0.02, (3, 3, 3), (1, 1, 1)),
     "strided": ((33, 201, 15), 2, 0.3, (3, 3, 3), (2, 2, 2)),
     "strided, one offset": ((33, 201, 15), 1, 0.3, (1, 1, 1), (2, 2, 2)),
+    "strided, 8 offsets": ((33, 201, 31), 2, 0.3, (2, 2, 2), (2, 2, 2)),
+    "strided, long": ((64, 512, 64), 1, 0.1, (3, 3, 3), (2, 2, 2)),
     "8 offsets": ((4, 91, 16), 1, 0.5, (2, 2, 2), (1, 1, 1)),
+    "1 offset": ((16, 301, 16), 1, 0.5, (1, 1, 1), (1, 1, 1)),
     "1100 tiles": ((16, 1101, 16), 1, 0.5, (3, 3, 3), (1, 1, 1)),
     "several tiles to a lane": ((64, 512, 20), 4, 0.5, (3, 3, 3), (1, 1, 1)),
 }
@@ -76,3 +79,9 @@ def test_against_the_pairs_in_float64(grid):
             assert bool(((d.double() - want).abs() <= 4 * n.sqrt() * 2.0 ** -24 * mag + 1e-30).all()), (dt, ic, oc)
         again = L.host().conv_wgrad(feat, grad, buf.native, False, True)
         assert torch.equal(again, got[0]), (dt, ic, oc)
+        # whether the middle offset is said to stand out decides how its groups are shared, not what comes out
+        said = buf.native.middle_run
+        buf.native.middle_run = 0 if said else L.RUN
+        d = L.host().conv_wgrad(feat, grad, buf.native, False, True)
+        buf.native.middle_run = said
+        assert bool(((d.double() - want).abs() <= 4 * n.sqrt() * 2.0 ** -24 * mag + 1e-30).all()), (dt, ic, oc)
