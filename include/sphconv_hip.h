@@ -78,7 +78,7 @@ typedef struct sph_geom {
     int32_t dil[3];
 } sph_geom;
 
-enum { SPH_RUN = 1, SPH_RUN_IN_FLIGHT = 2 }; /* values of sph_book.middle_run */
+enum { SPH_RUN = 1, SPH_RUN_IN_FLIGHT = 2, SPH_THIN = 4 }; /* values of sph_book.middle_run */
 
 typedef struct sph_book {
     int32_t *tile_ngrp;
@@ -103,7 +103,9 @@ typedef struct sph_book {
      * transposed book).  The kernels by groups then load that run's weight fragments once: helper waves take it on short
      * grids, the wave that begins a tile on long ones.  0 (also what a zero-initialised struct says): no assumption; results
      * are the same either way, up to the order of summation.  SPH_RUN_IN_FLIGHT says besides that the caller keeps three calls
-     * or more in flight on streams of their own: kernels that share the chip better are then taken up to larger grids. */
+     * or more in flight on streams of their own: kernels that share the chip better are then taken up to larger grids.
+     * SPH_THIN says that there is no such run and hardly more than one pair to a row (1.45 on average at most), as in a strided layer
+     * on scattered voxels: neighbouring tiles' groups can then be merged. */
     int32_t middle_run;
 } sph_book;
 

@@ -138,16 +138,14 @@ __global__ __launch_bounds__(128) void conv_wave_kernel(ConvArgs a, int nwtot)
     conv_wave_store<DT, CT>(a, nwtot, s_acc, col0, r0, nrows, lane, kWave);
 }
 
-// Two tiles at a time, for fp32 rows of 132 to 256 bytes into 33 to 64 columns, where a group of 16 pairs takes 64 matrix instructions of
+// Two tiles at a time, for fp32 rows of 196 to 256 bytes into 33 to 64 columns, where a group of 16 pairs takes 64 matrix instructions of
 // 32 cycles, empty slots or not.  At LiDAR sparsity a tile has about one group at an offset and five pairs in it: the last groups
 // of two neighbouring tiles at an offset are merged where their pairs fit one.  Two waves take 32 columns each of 256
 // accumulator rows, as much LDS for a wave as one that takes 64 columns of one tile.  A row's sum is in conv_wave_kernel's order.
-// Where merging would save less than a quarter of the groups, or the list has no room, each wave takes one tile as conv_wave_kernel does
-// (full grids: 64 -> 64 on 922 tiles of 24 pairs a row 241 : 234 us, 1021 tiles of 12 151 : 144).
+// Where merging would save less than a quarter of the groups, or the list has no room, each wave takes one tile as conv_wave_kernel does.
 // What bounds it: in conv_wave_kernel the matrix cores, 69 % of the time with two slots of three empty; here the rows and fragments,
 // 12 KB for a group and wave (a quarter more than half of what one wave with all columns loads), and two round trips more to make the list.
-// us, 64 -> 64: strided layer of eight 64x512x512 scans, 2848 tiles, 117.7 -> 96.4; submanifold, 1.6 pairs a row beside its own, 4048
-// tiles 185 -> 168, 1207 tiles 84.6 -> 74.8.  Rows and fragments requested as far ahead as conv_wave_groups does, two groups of 1024 cycles:
+// us, 64 -> 64: strided layer of eight 64x512x512 scans, 2848 tiles, 117.7 -> 96.4.  Rows and fragments requested as far ahead as conv_wave_groups does, two groups of 1024 cycles:
 // no gain (124); five 104 to 112, six 102 to 108 (behind 62 loads a wave cannot have more counted).
 constexpr int kPairRoom = 104;   // merged groups that fit the LDS beside the accumulators of two workgroups per compute unit
 constexpr int kPairRows = 2 * R;
@@ -880,13 +878,19 @@ int launch_conv_split(const ConvArgs &a, int nwtot, int ntiles, size_t lds, hipS
     return sph_check_launch("sph_conv_apply");
 }
 
-// Not below 513 tiles, where conv_wave_split_kernel shares a tile's groups between waves (64 -> 64, two tiles : those, 304 tiles 31.2 : 30.2,
-// 475 tiles 69 : 42), not for small kernels (9 offsets, 608 tiles 27.7 : 24.3, 2412 tiles 79 : 72: nothing to merge beside the middle's
-// full groups) and not where more rows are gathered than made (a strided layer's transposed book, 11 pairs to a group: 177 : 164).
+// Only for books that are said to be thin.  The list costs a pair of tiles its two round trips whether it then pays or not, and a workgroup of two
+// tiles is 5 % slower than two of one where it does not.  By pairs to a row, two tiles : one, 64 -> 64, 1100 to 4000 tiles: strided layers 1.0 to 1.25
+// pairs 0.78 to 0.92 of the time, 1.45 0.87 to 0.97, 1.6 0.92 to 1.04, 2 and more 1.04 to 1.13.  Submanifold layers, whose middle offset is full,
+// gain only from 1.35 to 2 pairs (0.86 to 0.98) and lose up to 0.3 below and 0.1 above; how many theirs are is not known before they are
+// counted on the GPU (the share of the grid's cells that is taken says 1.1 for 1.1 pairs where voxels lie anywhere, and for 1.6 where they
+// lie along surfaces).
+// Not below 641 tiles, where conv_wave_split_kernel shares a tile's groups between waves or the chip is not filled (64 -> 64, two tiles : those,
+// 304 tiles 31.2 : 30.2, 475 tiles 69 : 42; 606 tiles of stride 2x1x1 38.6 : 36.3, of stride 2x2x2 0.90), and not for smaller kernels, whose
+// offsets have more pairs each (18 offsets 1.03 to 1.10).
 inline bool pair_ok(const ConvArgs &a, int nwtot, int ntiles)
 {
-    return nwtot == 4 && a.book.KV >= 18 && a.book.KV <= kWave && a.feat_rows <= a.book.rows && a.book.tile_koff &&
-           (uintptr_t)a.book.grp_gather % 16 == 0 && ntiles > 512;
+    return nwtot == 4 && a.book.middle_run == SPH_THIN && a.book.KV >= 27 && a.book.KV <= kWave && a.book.tile_koff &&
+           (uintptr_t)a.book.grp_gather % 16 == 0 && ntiles > 640;
 }
 
 template <sph_dtype DT, int NS, int CT, bool MASKED>
@@ -899,7 +903,7 @@ int launch_conv_wave(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
     // (narrow layers on large grids keep the one-wave kernel: a group is one fragment load and one MFMA there,
     // and the helper waves' barriers cost a full chip more than the run saves: 16 -> 16 on 4912 tiles 22.6 / 25.8 us)
     constexpr bool kRunKernel = NS <= 2 && !(DT == SPH_F32 && NS == 2 && CT == 4);
-    const bool helpers = kRunKernel && waves == 1 && a.book.tile_koff && a.book.middle_run && (NS * CT >= 4 || ntiles <= 1024);
+    const bool helpers = kRunKernel && waves == 1 && a.book.tile_koff && book_has_run(&a.book) && (NS * CT >= 4 || ntiles <= 1024);
     if constexpr (DT == SPH_F32 && NS == 4 && CT == 4) {
         if (pair_ok(a, nwtot, ntiles)) {
             const size_t lds2 = pair_lds(nwtot);
@@ -950,7 +954,7 @@ int launch_conv_wave_ct(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st
         // (up to 64 output columns only: more would be four waves, beyond the kernel's launch bound).  A book with a
         // run at its middle offset takes one wave of 64 columns and two helper waves instead (36.7 -> 35.1 us).
         if constexpr (DT == SPH_I8)
-            if (ntiles > 1024 && nwtot <= 4 && !a.book.middle_run) return launch_conv_wave_m<DT, NS, 2>(a, nwtot, ntiles, st);
+            if (ntiles > 1024 && nwtot <= 4 && !book_has_run(&a.book)) return launch_conv_wave_m<DT, NS, 2>(a, nwtot, ntiles, st);
         return launch_conv_wave_m<DT, NS, 4>(a, nwtot, ntiles, st);
     }
 }

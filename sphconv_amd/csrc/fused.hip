@@ -166,7 +166,7 @@ int launch_fused(const FusedArgs &fa, int ntiles, hipStream_t st)
     // three workgroups of 256 threads per CU hold 768 tiles at once, four of 128 threads 1024 (and fp32 rows of 128
     // bytes into 64 columns do not fit the registers three workgroups leave a wave)
     if (!fa.small_wg) {
-        const int s = split_waves(DT, fa.c.row_bytes, fa.nwtot, fa.b.book.middle_run, ntiles, fused_acc(fa.nwtot), fused_region_b());
+        const int s = split_waves(DT, fa.c.row_bytes, fa.nwtot, book_has_run(&fa.b.book), ntiles, fused_acc(fa.nwtot), fused_region_b());
         if (s == 4) return launch_fused_nt<DT, NS, CT, MASKED, 256, 4>(fa, ntiles, st);
         if (s == 2) return launch_fused_nt<DT, NS, CT, MASKED, 256, 2>(fa, ntiles, st);
     }

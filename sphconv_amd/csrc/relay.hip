@@ -500,7 +500,7 @@ template <sph_dtype DT, int NS, int CT, int GPC>
 int relay_launch_m(const ConvArgs &a, int ntiles, hipStream_t st)
 {
     const bool masked = a.row_bytes < NS * 64;
-    if (a.book.middle_run)
+    if (book_has_run(&a.book))
         return masked ? relay_launch<DT, NS, CT, true, true, GPC>(a, ntiles, st) : relay_launch<DT, NS, CT, false, true, GPC>(a, ntiles, st);
     return masked ? relay_launch<DT, NS, CT, true, false, GPC>(a, ntiles, st) : relay_launch<DT, NS, CT, false, false, GPC>(a, ntiles, st);
 }

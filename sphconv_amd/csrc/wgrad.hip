@@ -446,7 +446,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_stage_kernel(WgradArgs a)
 //
 // Where the kernel through LDS was the faster one still: long books of nearly full grids with 32 channels on a side in 16 bits, whose offsets
 // all have seven groups a tile and whose centre's workgroups have an eighth of the others' work (9002 tiles of 24 pairs a row, 32->64 f16
-// 403 : 476 us; of 11 pairs a row 242 : 246, of 3.7 127 : 102).  A book does not say how full its grid is before its groups are counted on the GPU.
+// 403 : 476 us; of 11 pairs a row 242 : 253, of 3.7 128 : 104).  A book does not say how full its grid is before its groups are counted on the GPU.
 // ---------------------------------------------------------------------------
 constexpr int kWsMost = 192, kWsMostLight = 128; // most tiles of a chunk, and where a compute unit holds more than two workgroups
 constexpr int kWsPer = 4;      // most of a lane (even)
@@ -875,13 +875,13 @@ inline size_t wgrad_wave_lds(int mi, int ni) { return (size_t)2 * mi * ni * kWav
 // Workgroups of wgrad_wave_kernel on a compute unit, by its registers (197 to 256, 141 to 194 for a side of 64 channels, 113 at most).
 inline int wgrad_wave_occupancy(bool f32, int mi, int ni) { return mi * ni >= 16 || !f32 ? 2 : (mi * ni >= 8 ? 3 : 4); }
 // Does the middle offset hold far more pairs than the others?  The caller says so; a layer with as many rows out as in is taken for one too.
-inline bool wgrad_run(const WgradArgs &a) { return (a.book.middle_run != 0) || a.in_rows == a.out_rows; }
+inline bool wgrad_run(const WgradArgs &a) { return book_has_run(&a.book) || a.in_rows == a.out_rows; }
 struct WavePlan { int nchunk, nparts; };
 // Chunks of a book's tiles, and workgroups that share a chunk's groups at the centre offset: one round of workgroups of about the same number of
 // groups each.  A submanifold book has eight groups a tile at the centre and about one at the others, so eight share the centre's; of small
 // kernels (most of their offsets' pairs are there) four.  Where no offset stands out one: with eight the others' workgroups were four
-// times as long as the centre's and half the chip idle (2x2x2 stride 2, 64->64 f16, 998 tiles 20.4 us through LDS, 23.9 with eight, 19.0 with
-// one; fp32, transposed book of 16 611 tiles 264, 511, 237).
+// times as long as the centre's and half the chip idle (2x2x2 stride 2, 64->64 f16, 998 tiles 20.3 us through LDS, 23.9 with eight, 18.4 with
+// one; fp32, transposed book of 16 611 tiles 259, 511, 187).
 // A round: with whole chunks to an XCD (sixteen of them, six workgroups at the centre) 3 % fewer lines come from memory, and the centre's
 // workgroups last a third longer than the others: 32.9 : 29.0 us.
 // An offset has at most 256 partial blocks in a round: few workgroups add up those of a small kernel (1x1x1, 2005 tiles, 32->64 f16: 504 blocks

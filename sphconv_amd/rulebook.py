@@ -153,6 +153,8 @@ BY_ROW_MIN_PAIRS = 10.0
 # 412/413 (64->64): one line between the two.  The threshold of such books is this fraction of the one
 # above (where a book with groups and the table breaks even at 10.8: 298/297 and 653/670).
 BY_ROW_FORWARD_ONLY = 0.65
+# Pairs to a row up to which a strided layer's book is said to be thin (``SPH_THIN``).
+THIN_PAIRS = 1.45
 
 
 class RuleBook:
@@ -236,6 +238,15 @@ class RuleBook:
             return g.kv * self.out_rows / g.out_cells / g.steps
         return g.kv * self.in_rows / g.in_cells + self.cluster - 1.0
 
+    def _said(self, transposed: bool) -> int:
+        """What the book says of its pairs (``sph_book.middle_run``): a submanifold layer pairs every row with itself at
+        the middle offset; a strided layer's pairs are known (kernel volume / stride to an input row), and may be hardly more than
+        its rows."""
+        if self.subm:
+            return L.RUN
+        g = self._geometry
+        return L.THIN if g.kv * self.in_rows <= THIN_PAIRS * g.steps * (self.in_rows if transposed else self.out_rows) else 0
+
     def _rows_kernel_takes(self, weight, weight_transposed: bool) -> bool:
         """Whether ``sph_conv_apply`` can walk this layer by stationary row (rows of 16-byte multiples up
         to 128 bytes, 16-byte multiples out, a table that fits LDS): the conditions of the library."""
@@ -265,7 +276,7 @@ class RuleBook:
                 by_row = est >= BY_ROW_MIN_PAIRS * BY_ROW_FORWARD_ONLY
             groups = not (by_row and forward_only)
         buf = _Buffers(rows, self.kv, self.z_ptr.device, by_row, groups)
-        buf.native.middle_run = int(self.subm)       # every row pairs with itself at the middle offset
+        buf.native.middle_run = self._said(transposed)
         hint = self.row_cols if transposed else self.out_row_cols
         where = (self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, transposed, buf.native, hint)
         if weight is None:
@@ -283,7 +294,7 @@ class RuleBook:
         in fragment order for the forward pass and for dgrad; -> the two copies."""
         by_row = self._pairs_per_row(False) >= BY_ROW_MIN_PAIRS
         buf = _Buffers(self.out_rows, self.kv, self.z_ptr.device, by_row, True)
-        buf.native.middle_run = int(self.subm)
+        buf.native.middle_run = self._said(False)
         both = L.host().rules_build_pack(self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, False,
                                          buf.native, self.out_row_cols, weight, 2, self.mirrored(), L.dtype_code(dtype))
         self._fwd = buf
