@@ -160,8 +160,8 @@ void conv_rows_short_kernel(ConvArgs a, int nwtot)
 // stretch of the feature array (two where the rows straddle lines of the grid): three windows, brought by direct loads that are
 // all in flight at once, at multiples of a load's rows; the table is rewritten to places in LDS.  A row's 16-byte chunks lie
 // exchanged by its place (chunk ^ place), so that 16 rows' chunks, which the operands take together, lie in different banks; the
-// table holds places with that folded in, and an address is an exclusive or.  Empty slots point at a row of zeros.  A window
-// that finds no room leaves its offsets to gathers from the feature array.  The waves' sums meet in LDS, halves of the blocks
+// table holds places with that folded in, and an address is an exclusive or.  Empty slots point at a row of zeros.  The offsets of a window
+// that finds no room are left out, and follow from the feature array.  The waves' sums meet in LDS, halves of the blocks
 // first, then quarters.
 // Every offset's weight passes the compute unit's vector memory path once for NB * 16 rows (216 KiB at 64 -> 64), the rows
 // three times at most, where gathers bring each row 27 times: 290 KiB for 128 rows against 660.
@@ -170,7 +170,7 @@ void conv_rows_short_kernel(ConvArgs a, int nwtot)
 // on its SIMD), exchange 3.9 k, store 2.4 k; the one's products run beside the other's rest.  Blocks of 64 rows take the
 // weights twice: 165.
 template <sph_dtype DT, int NS, int CT, bool MASKED, int NB>
-__global__ __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(NB * CT >= 32 ? 2 : 2)))
+__global__ __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
 {
     typedef typename Traits<DT>::elem elem;
@@ -183,6 +183,7 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
     constexpr int TPR = 4 * kWave / RB;     // waves that share a row's entries while the table is read
     constexpr int TE = (kPhase + TPR - 1) / TPR; // entries of a thread and phase
     static_assert(RB >= kWave, "a wave reads whole offsets");
+    static_assert(W == 4 && kSplitKV <= 32, "every fourth bit of a word");
     extern __shared__ __attribute__((aligned(16))) char s_mem[];
     uint16_t *s_tab = (uint16_t *)s_mem;                       // [kSplitKV][16 rows][NB]
     char *s_win = s_mem + kSplitKV * RB * 2;                         // rows, chunks swizzled
@@ -367,37 +368,120 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    int k = wave;
+    // the wave's offsets of the phases in `mask`, one bit each, and the next of them
+    auto offsets_of = [&](int mask) {
+        unsigned m = 0;
+#pragma unroll
+        for (int p = 0; p < kPhases; p++) m |= mask >> p & 1 ? ((1u << kPhase) - 1) << (p * kPhase) : 0;
+        return m & (0x11111111u << wave);
+    };
+    auto next_of = [&](unsigned &left) {
+        const int k = left ? __builtin_ctz(left) : kSplitKV;
+        left &= left - 1;
+        return k;
+    };
+    unsigned left = offsets_of(ok_mask);
+    int k = next_of(left), kn = next_of(left);
+    if (ok_mask != 7) {
+        load_w(k, fw[0]);
+        load_w(kn, fw[1]);
+    }
     load_ix(k, ix0);
 #pragma unroll
     for (int j = 0; j < DX; j++) load_x(ix0, j, x[j]);
-    for (; k + W < kSplitKV; k += 2 * W) {
-        step(k + W, ix0, ix1, fw[0]);
-        load_w(k + 2 * W, fw[0]);
+    while (kn < kSplitKV) {
+        step(kn, ix0, ix1, fw[0]);
+        k = next_of(left);
+        load_w(k, fw[0]);
         __builtin_amdgcn_sched_barrier(0);
-        step(k + 2 * W, ix1, ix0, fw[1]);
-        load_w(k + 3 * W, fw[1]);
+        step(k, ix1, ix0, fw[1]);
+        kn = next_of(left);
+        load_w(kn, fw[1]);
         __builtin_amdgcn_sched_barrier(0);
     }
     if (k < kSplitKV) step(k, ix0, ix1, fw[0]);
     if (ok_mask != 7) {
-        // a window that found no room: its rows from the feature array
-#pragma unroll 1
-        for (int k = wave; k < kSplitKV; k += W) {
-            if (ok_mask >> (k / kPhase) & 1) continue;
-            load_w(k, fw[0]);
+        // Windows that found no room: their rows from the feature array, G blocks at a time and the next ones on their way, also into
+        // the next offset, whose part of the table is there an offset ahead.  Columns of 150 rows (two windows of three have no room),
+        // 5210 tiles, 64 -> 64 fp16: 1.05 of the time of conv_rows_kernel_w2, 32 -> 64 fp32 0.99.  With these offsets among the products
+        // above as well (rows of zeros) and an offset's loads waited for here before the next one's were asked for 1.31 and 1.39.
+        constexpr bool QUAD = NS == 2;     // as in conv_rows_short_kernel
+        constexpr int G = 2, U = NB / G, kTrRow = 80, kTrSet = SPH_GROUP * kTrRow;
+        static_assert(U % 2 == 0, "two units in flight, and an offset begins with the first");
+        if (QUAD) lds_barrier(); // the waves are through with the windows: each turns its rows in a part of them
+        char *tr = s_win + wave * (G * NS * kTrSet);
+        const int qrow = QUAD ? lane >> 2 : lane & 15, qchunk = (QUAD ? lane & 3 : lane >> 4) * 16;
+        auto load_id = [&](int k, int (&id)[NB]) {
 #pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const int id = tab[k * R + j * SPH_GROUP + (lane & 15)];
-                const unsigned off = (unsigned)id < (unsigned)a.feat_rows ? (unsigned)(id * rb + chunk * 16) : kNoRow;
-                int4v x[NS];
-                x[0] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(r_feat, live0 ? off : kNoRow, 0, 0));
-                if constexpr (NS == 2) x[1] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(r_feat, live1 ? off + 64 : kNoRow, 0, 0));
+            for (int j = 0; j < NB; j++) id[j] = tab[min(k, kSplitKV - 1) * R + j * SPH_GROUP + qrow];
+        };
+        auto gather = [&](int k, const int (&id)[NB], int u, int4v (&v)[G][NS]) {
+            const unsigned lim = k < kSplitKV ? a.feat_rows : 0;
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const unsigned off = (unsigned)id[u * G + g] < lim ? (unsigned)(id[u * G + g] * rb + qchunk) : kNoRow;
+#pragma unroll
+                for (int st = 0; st < NS; st++)
+                    v[g][st] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                                             r_feat, MASKED && st * 64 + qchunk >= rb ? kNoRow : off + st * 64, 0, 0));
+            }
+        };
+        unsigned rest = offsets_of(~ok_mask);
+        int k0 = next_of(rest), k1 = next_of(rest);
+        int id0[NB], id1[NB];
+        int4v v[2][G][NS];
+        if (k0 < kSplitKV) {
+            load_w(k0, fw[0]);
+            load_id(k0, id0);
+            load_id(k1, id1);
+#pragma unroll
+            for (int u = 0; u < 2; u++) gather(k0, id0, u, v[u]);
+        }
+        while (k0 < kSplitKV) {
+            const int k2 = next_of(rest);
+            int id2[NB];
+            if constexpr (NB < 8) load_id(k2, id2);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                int4v y[G][NS];
+                if constexpr (QUAD) { // (a wave's accesses of LDS keep their order)
+#pragma unroll
+                    for (int g = 0; g < G; g++)
+#pragma unroll
+                        for (int st = 0; st < NS; st++) *(int4v *)(tr + (g * NS + st) * kTrSet + (lane >> 2) * kTrRow + (lane & 3) * 16) = v[u & 1][g][st];
+                    asm volatile("" ::: "memory");
+                } else {
+#pragma unroll
+                    for (int g = 0; g < G; g++) y[g][0] = v[u & 1][g][0];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (u + 2 < U) gather(k0, id0, u + 2, v[u & 1]);
+                else gather(k1, id1, u + 2 - U, v[u & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (QUAD) {
+#pragma unroll
+                    for (int g = 0; g < G; g++)
+#pragma unroll
+                        for (int st = 0; st < NS; st++) y[g][st] = *(const int4v *)(tr + (g * NS + st) * kTrSet + (lane & 15) * kTrRow + (lane >> 4) * 16);
+                    asm volatile("" ::: "memory");
+                }
 #pragma unroll
                 for (int st = 0; st < NS; st++)
 #pragma unroll
-                    for (int c = 0; c < CT; c++) acc[j][c] = mfma_step<DT>(fw[0][st][c], x[st], acc[j][c]);
+                    for (int g = 0; g < G; g++)
+#pragma unroll
+                        for (int c = 0; c < CT; c++) acc[u * G + g][c] = mfma_step<DT>(fw[0][st][c], y[g][st], acc[u * G + g][c]);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            load_w(k1, fw[0]);
+#pragma unroll
+            for (int j = 0; j < NB; j++) id0[j] = id1[j];
+            if constexpr (NB < 8) {
+#pragma unroll
+                for (int j = 0; j < NB; j++) id1[j] = id2[j];
+            } else load_id(k2, id1);
+            k0 = k1;
+            k1 = k2;
         }
     }
 

@@ -93,6 +93,8 @@ GRIDS = {
     "300 tiles": ((12, 400, 16), 0.5, (3, 3, 3), (1, 1, 1)),
     "1100 tiles": ((16, 1101, 16), 0.5, (3, 3, 3), (1, 1, 1)),
     "deep": ((3, 19, 333), 0.97, (3, 3, 3), (1, 1, 1)),                 # columns longer than a tile: windows of 600 rows
+    "some windows": ((8, 100, 128), 0.6, (3, 3, 3), (1, 1, 1)),         # one or two of a tile's three find room
+    "deep, 600 tiles": ((8, 70, 333), 0.45, (3, 3, 3), (1, 1, 1)),
     "strided, 3 to a row": ((24, 700, 16), 0.45, (3, 3, 3), (2, 2, 2)),
     "strided, 7 to a row": ((33, 601, 15), 0.9, (3, 3, 3), (2, 2, 2)),
     "45 offsets": ((8, 200, 16), 0.4, (5, 3, 3), (1, 1, 1)),
