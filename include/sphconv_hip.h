@@ -78,7 +78,7 @@ typedef struct sph_geom {
     int32_t dil[3];
 } sph_geom;
 
-enum { SPH_RUN = 1, SPH_RUN_IN_FLIGHT = 2, SPH_THIN = 4 }; /* values of sph_book.middle_run */
+enum { SPH_RUN = 1, SPH_RUN_IN_FLIGHT = 2, SPH_THIN = 4, SPH_SHALLOW = 8 }; /* values of sph_book.middle_run */
 
 typedef struct sph_book {
     int32_t *tile_ngrp;
@@ -105,7 +105,8 @@ typedef struct sph_book {
      * are the same either way, up to the order of summation.  SPH_RUN_IN_FLIGHT says besides that the caller keeps three calls
      * or more in flight on streams of their own: kernels that share the chip better are then taken up to larger grids.
      * SPH_THIN says that there is no such run and hardly more than one pair to a row (1.45 on average at most), as in a strided layer
-     * on scattered voxels: neighbouring tiles' groups can then be merged. */
+     * on scattered voxels: neighbouring tiles' groups can then be merged.  SPH_SHALLOW may be added to any of them, and says that a column of
+     * the gathered side's grid holds 16 rows or fewer on average: what 64 rows gather at nine neighbouring offsets then lies close together. */
     int32_t middle_run;
 } sph_book;
 

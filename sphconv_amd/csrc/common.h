@@ -9,6 +9,10 @@
 
 #define SPH_EXPORT extern "C" __attribute__((visibility("default")))
 
+// what the caller says of a book's middle offset and pairs, and of its columns (sph_book.middle_run)
+static inline int book_says(const sph_book *b) { return b->middle_run & ~SPH_SHALLOW; }
+static inline int book_is_shallow(const sph_book *b) { return b->middle_run & SPH_SHALLOW; }
+
 void sph_set_error(const char *fmt, ...);
 
 #define SPH_REQUIRE(cond, code, ...)      \

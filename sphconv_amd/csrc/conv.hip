@@ -889,7 +889,7 @@ int launch_conv_split(const ConvArgs &a, int nwtot, int ntiles, size_t lds, hipS
 // offsets have more pairs each (18 offsets 1.03 to 1.10).
 inline bool pair_ok(const ConvArgs &a, int nwtot, int ntiles)
 {
-    return nwtot == 4 && a.book.middle_run == SPH_THIN && a.book.KV >= 27 && a.book.KV <= kWave && a.book.tile_koff &&
+    return nwtot == 4 && book_says(&a.book) == SPH_THIN && a.book.KV >= 27 && a.book.KV <= kWave && a.book.tile_koff &&
            (uintptr_t)a.book.grp_gather % 16 == 0 && ntiles > 640;
 }
 
@@ -959,17 +959,17 @@ int launch_conv_wave_ct(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st
     }
 }
 
-// Whether a layer of one K step goes through the window.  With up to 32 columns always, on grids of more than 1024 tiles (shorter
-// ones are faster with four waves per tile: 312 tiles, 32 -> 32 fp16, 17.2 : 19.2 us).  With 64 columns two waves of a tile have
-// only two waves of a SIMD beside them, and it depends.  Times with the window over times without, 3x3x3, 0.4 of the bins:
-//   tiles             260   400   600   800  1000  1100  1250  1500  1800  2000  3000  4000
-//   fp16 32 -> 64    0.92  0.91  0.74  0.62  0.64  0.96  0.95  0.96  0.84  0.95  0.80  0.84
-//   int8 64 -> 64    0.93  0.93  0.73  0.61  0.62  0.86  0.85  0.89  0.80  0.83  0.72  0.82
-//   fp32 16 -> 64    1.44  1.43  0.99  0.87  0.88  0.82  0.94  1.06  1.04  1.12  1.03  1.06   (5x3x3: 0.90 0.93 0.83 0.88 at the end)
-//   fp16, 3x3x1      1.09  1.16  0.94  0.78  0.81  1.43  1.43  1.42  1.24  1.35  1.26  1.35   (one phase: nothing overlaps its window)
-//   fp16, 2x2x2      1.29  1.30  1.15  0.92  0.93  1.49  1.52  1.56  1.40  1.43  1.37  1.54   (a phase costs nine offsets; 3x2x2 alike)
-//   fp16, stride 2   1.36  1.32  1.13        0.95        1.33        1.11  1.22  0.99  1.02   (3.2 gathered rows to a row: windows too small;
-//   stride 1,2,2     0.94  1.02  0.83        0.72        1.05        0.91  0.98  0.88  0.92    1.6 to a row: they fit)
+// Whether a layer of one K step that rows_hold.hip and rows_split.hip leave goes through the window.  With up to 32 columns on grids of
+// more than 1024 tiles; into 64 columns what arrives is 27 offsets in 16 bits and int8 on 961 to 1024 tiles and beyond 1900, and other kernels from 641
+// or 769 tiles on (win_first).  Two waves of a tile have only two waves of a SIMD beside them then, and it depends.  Times with the
+// window over times without, 3x3x3 but where said, 0.4 of the bins:
+//   tiles             800  1000  1100  1250  1500  1800  2000  3000  4000
+//   fp16 32 -> 64                                              0.80  0.84
+//   int8 64 -> 64                                              0.72  0.82
+//   fp32, 5x3x3                        0.90  0.93                    0.88
+//   fp16, 3x3x1      0.78  0.81  1.43  1.43  1.42  1.24  1.35  1.26  1.35   (one phase: nothing overlaps its window)
+//   fp16, 2x2x2      0.92  0.93  1.49  1.52  1.56  1.40  1.43  1.37  1.54   (a phase costs nine offsets; 3x2x2 alike)
+//   fp16, stride 2         0.95        1.33        1.11  1.22  0.99  1.02   (3.2 gathered rows to a row: windows too small)
 template <sph_dtype DT, int CT>
 bool win_ok(const ConvArgs &a, int ntiles)
 {
@@ -979,7 +979,7 @@ bool win_ok(const ConvArgs &a, int ntiles)
     if (DT == SPH_F32) return ntiles > 768 && (ntiles <= 1280 || a.book.KV > 4 * kWinPhase);
     // (without it 2048 tiles are on the chip at once: 2037 tiles, 6.9 pairs a row, fp16 32 -> 64 1.09, 16 -> 64 1.16; int8 1.04)
     if (DT != SPH_I8 && ntiles > 1920 && ntiles <= 2048) return false;
-    return ntiles > 256;
+    return true;
 }
 
 // One wave per tile instead of two (32 columns): with two 1536 tiles are on the chip at once, with one 2048.  us, one : two:

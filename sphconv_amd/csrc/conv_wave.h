@@ -82,7 +82,7 @@ __device__ __forceinline__ int4v mfma_step<SPH_I8>(int4v a, int4v b, int4v d)
 }
 
 // does the middle offset hold a run of full groups, by what the caller says?
-inline bool book_has_run(const sph_book *b) { return b->middle_run != 0 && b->middle_run != SPH_THIN; }
+inline bool book_has_run(const sph_book *b) { return book_says(b) != 0 && book_says(b) != SPH_THIN; }
 inline int book_has_groups(const sph_book *b) { return b->grp_k && b->grp_gather && b->grp_owner; }
 
 // the groups may be missing (all three arrays null) in a book that keeps its pairs by row

@@ -537,7 +537,7 @@ bool sph_relay_ok(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles)
     if (!a.aligned_in || !a.aligned_out || a.nsteps > 2 || nwtot > 4) return false;
     if (KV <= kRelayPart || KV > (kRelayStages - 1) * kRelayPart) return false;
     if ((double)ntiles * a.cap * SPH_GROUP * 4 >= 2147483648.0) return false; // 32-bit offsets into the book
-    return ntiles > relay_line(dt, a.nsteps, nwtot, a.book.middle_run == SPH_RUN_IN_FLIGHT);
+    return ntiles > relay_line(dt, a.nsteps, nwtot, book_says(&a.book) == SPH_RUN_IN_FLIGHT);
 }
 
 int sph_relay_launch(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)

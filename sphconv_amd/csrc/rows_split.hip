@@ -560,31 +560,47 @@ enum Way { kNone, kShort1, kShort2, kByOffset, kSplit4, kSplit8 };
 //     were asked for by quads, which took 64 -> 64 511 tiles of 7.2 to a row from 40 to 35)
 //   64 rows with windows (kSplit4) up to 256 tiles, 128 rows (kSplit8) beyond, 64 -> 64 fp16: 201 tiles 12.2 : 13.1 : plain 18.7; 400 tiles
 //     21.1 : 18.9 : 31; 1001 tiles 41.8 : 34.8 : 59.5; 3996 tiles 165 : 129 : 167.  fp32, whose matrix cores are the bound, up to 32 columns
-//     always (32 -> 32 3996 tiles 252 : 254 : 344), 64 up to 512 (700 tiles 97 : 94).  3.6 to a row 1399 tiles 71 : 79, 2000 tiles 103 : 90
+//     always (32 -> 32 3996 tiles 252 : 254 : 344), 64 up to 512 (700 tiles 97 : 94).  3.6 to a row 1399 tiles 71 : 79
 //   one K step: 32 -> 64 1401 tiles 33 : win 39, 2000 tiles 48 : 55, 2997 tiles 70 : 68; fp32 16 -> 64 3996 tiles 250 : 265; 32 -> 32 1001
 //     tiles 16 : plain 27, 1401 tiles 22 : win 19 (fp32 16 -> 32 51 : 54, 2000 tiles 72 : 69); 32 -> 64 3.6 to a row 4000 tiles 106 : 117;
 //     32 -> 32 3.6 to a row 511 tiles kByOffset 12 : split 15, 4000 tiles split 74 : win 88, 2.8 to a row 4000 tiles 64.5 : 64.9
+// Where the windows are not sure to find room the lines are those at which nothing measured is much slower than the kernels of conv.hip (twenty tile
+// counts from 20 to 10 000, 0.15 to 0.9 of the bins, columns of 4 to 51 rows, strides of one, two or three axes; columns of 150 rows are up to 1.3):
+//   fp32 into 64 columns, more than 1.3 to a row: an offset at a time 0.83 to 0.93, with windows 0.77 to 1.10; beyond 6000 tiles neither
+//   one K step, more than 2 to a row: rows shorter than 64 bytes (16 -> 64 f16 2.6 to 7 to a row, 1100 tiles 1.05, 1950 1.2 to 1.4 of plain, where
+//     columns hold 13 rows or fewer 0.7 to 0.9), fp32 16 -> 64 beyond 1900 tiles 1.06 to 1.15 (0.83 to 0.9)
+//   one K step, 64 columns, 961 to 1024 tiles: one round of conv_rows_win_kernel (995 tiles 1.05, int8 1.07 to 1.10 of it); int8 rows of 16 bytes
+//     and 16-bit ones of up to 48 from 1901 tiles on 1.04 to 1.10 of plain
+//   8 offsets, 45 offsets, 16 bits, one K step into 64 columns: 645 tiles 1.04 to 1.09, 990 tiles 1.10 of plain or the window kernel
+//   65 to 128 columns of other than 27 offsets: 512 tiles (9 offsets 64 -> 128 f16 520 tiles 0.93, 650 1.07, 1000 1.38 of plain)
+// int8 takes 16 bits' lines but for these (64 -> 64 against the window kernel: 300 to 960 tiles 0.58 to 0.9, 1100 to 1950 tiles 0.8 to 1.05).
 template <sph_dtype DT, int NS, int CT>
 Way pick_way(const ConvArgs &a, int nwtot, int ntiles)
 {
     const double to_a_row = (double)a.feat_rows / a.book.rows;
     const long T = (long)ntiles * sph_div_up(nwtot, CT);
     const int KV = a.book.KV;
-    const bool f32 = DT == SPH_F32;
+    const bool f32 = DT == SPH_F32, half = DT == SPH_F16 || DT == SPH_BF16;
     if (T <= 32) return kShort1;
     if (KV != kSplitKV) {
         if (T <= 64 && KV >= 16) return kShort2;
-        return T <= 1024 ? kByOffset : kNone;
+        return T <= (half && NS == 1 && nwtot == 4 && (KV <= 8 || KV > kSplitKV) ? 640 : 1024) ? kByOffset : kNone;
     }
     if (T <= (NS == 1 && CT <= 2 ? 128 : 64)) return kShort2;
     if (NS == 2) {
+        if (f32 && CT == 4 && to_a_row > 1.3 && T > 512) return T <= 6000 ? kByOffset : kNone;
         if (to_a_row <= 2.4) return f32 && (CT <= 2 || T <= 512) ? kSplit4 : (T <= 256 ? kSplit4 : kSplit8);
-        if (f32 ? CT <= 2 || T <= 1536 : T <= 1024) return kByOffset;
-        return !f32 && T <= 1400 && to_a_row <= 5 ? kSplit4 : kNone;
+        if (f32 || T <= 1024) return kByOffset;
+        return T <= 1400 && to_a_row <= 5 ? kSplit4 : kNone;
     }
-    if (CT == 4) return f32 || T <= 2048 || to_a_row > 2 || nwtot > 4 ? kSplit4 : kNone;
+    if (CT == 4) {
+        const bool brief = a.row_bytes < 64;
+        if (to_a_row > 2) return book_is_shallow(&a.book) || (!f32 && !brief) || T <= (f32 ? 1900 : nwtot > 4 ? 2048 : 1024) ? kSplit4 : kNone;
+        if (f32 || nwtot > 4) return kSplit4;
+        return T <= 960 || (T > 1024 && T <= (brief ? 1900 : 2048)) ? kSplit4 : kNone;
+    }
     if (to_a_row <= 2.4) return T <= (f32 ? 1536 : 1024) ? kSplit4 : kNone;
-    if (T <= 640) return kByOffset;
+    if (T <= (f32 && CT == 1 ? 1024 : 640)) return kByOffset;
     if (CT == 1) return T <= 1024 ? kSplit4 : kNone;
     return f32 || T <= 2048 || to_a_row > 3.3 ? kSplit4 : kNone;
 }
@@ -642,12 +658,14 @@ bool sph_rows_split_ok(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles)
 {
     if ((double)a.feat_rows * a.row_bytes >= 2147483648.0) return false; // lane offsets are 31-bit
     const int ct = nwtot < 4 ? nwtot : 4;
-    auto way = [&](auto f32) {
-        constexpr sph_dtype DT = decltype(f32)::value ? SPH_F32 : SPH_F16;
+    auto way = [&](auto type) {
+        constexpr sph_dtype DT = decltype(type)::value;
         if (a.nsteps == 1) return ct == 1 ? pick_way<DT, 1, 1>(a, nwtot, ntiles) : ct == 2 ? pick_way<DT, 1, 2>(a, nwtot, ntiles) : pick_way<DT, 1, 4>(a, nwtot, ntiles);
         return ct == 1 ? pick_way<DT, 2, 1>(a, nwtot, ntiles) : ct == 2 ? pick_way<DT, 2, 2>(a, nwtot, ntiles) : pick_way<DT, 2, 4>(a, nwtot, ntiles);
     };
-    return (dt == SPH_F32 ? way(std::true_type()) : way(std::false_type())) != kNone;
+    if (dt == SPH_F32) return way(std::integral_constant<sph_dtype, SPH_F32>()) != kNone;
+    if (dt == SPH_I8) return way(std::integral_constant<sph_dtype, SPH_I8>()) != kNone;
+    return way(std::integral_constant<sph_dtype, SPH_F16>()) != kNone;
 }
 
 int sph_rows_split_launch(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)

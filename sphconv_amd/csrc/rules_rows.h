@@ -351,7 +351,7 @@ inline void (*rows_kernel(const BuildArgs &a, int KV, int ntiles))(BuildArgs)
     constexpr int cube = TRANSPOSED ? 2 : 3;
     const int nl = rows_lines(a, TRANSPOSED), c = a.lines;
     if (KV == 27 && c == cube && nl == cube) {
-        if (!TRANSPOSED && a.book.middle_run == SPH_RUN_IN_FLIGHT && ntiles <= kRowFlightTiles)
+        if (!TRANSPOSED && book_says(&a.book) == SPH_RUN_IN_FLIGHT && ntiles <= kRowFlightTiles)
             return build_rows_kernel<false, 3, 3, 27, HINT, 2>;
         return build_rows_kernel<TRANSPOSED, cube, cube, 27, HINT>;
     }

@@ -75,13 +75,18 @@ class _Buffers:
         return int(((own >= 0) & used).sum().item())
 
 
+# Pairs to a row up to which a strided layer's book is said to be thin (``SPH_THIN``).
+THIN_PAIRS = 1.45
+# Rows to a column up to which a by-row book's gathered side is said to be shallow (``SPH_SHALLOW``).
+SHALLOW_ROWS = 16
+
 
 class _Geometry:
     """One convolution geometry: the C struct and what Python wants to know of it.  Made once per geometry and shared
     by every book that has it (a network meets a few dozen)."""
 
     __slots__ = ("native", "batch", "in_shape", "out_shape", "kernel", "stride", "padding", "dilation", "kv", "in_cells",
-                 "out_cells", "steps", "odd_same", "z_shape", "cluster", "key")
+                 "out_cells", "steps", "odd_same", "z_shape", "cluster", "key", "thin", "shallow")
 
     def __init__(self, batch, in_shape, out_shape, kernel, stride, padding, dilation):
         self.batch = batch
@@ -101,6 +106,9 @@ class _Geometry:
         for k, s in zip(kernel, stride):
             reach = [len(range(r, k, s)) for r in range(s)]
             self.cluster *= sum(c * c for c in reach) / max(sum(reach), 1)
+        # stationary rows from which a strided layer's book is thin, to an input row; rows up to which each side is shallow
+        self.thin = self.kv / (THIN_PAIRS * self.steps)
+        self.shallow = tuple(SHALLOW_ROWS * batch * s[0] * s[1] for s in (in_shape, out_shape))
         # odd kernel, stride 1, padding K//2: a submanifold book is then its own transpose, offsets mirrored
         self.odd_same = all(k % 2 == 1 for k in kernel) and self.steps == 1 and all(p == k // 2 for p, k in zip(padding, kernel))
         self.native = L.host().Geometry(batch, self.in_shape, self.out_shape, self.kernel, self.stride, self.padding,
@@ -153,8 +161,6 @@ BY_ROW_MIN_PAIRS = 10.0
 # 412/413 (64->64): one line between the two.  The threshold of such books is this fraction of the one
 # above (where a book with groups and the table breaks even at 10.8: 298/297 and 653/670).
 BY_ROW_FORWARD_ONLY = 0.65
-# Pairs to a row up to which a strided layer's book is said to be thin (``SPH_THIN``).
-THIN_PAIRS = 1.45
 
 
 class RuleBook:
@@ -238,14 +244,18 @@ class RuleBook:
             return g.kv * self.out_rows / g.out_cells / g.steps
         return g.kv * self.in_rows / g.in_cells + self.cluster - 1.0
 
-    def _said(self, transposed: bool) -> int:
+    def _said(self, transposed: bool, by_row: bool) -> int:
         """What the book says of its pairs (``sph_book.middle_run``): a submanifold layer pairs every row with itself at
         the middle offset; a strided layer's pairs are known (kernel volume / stride to an input row), and may be hardly more than
-        its rows."""
-        if self.subm:
-            return L.RUN
+        its rows; and of a by-row book how deep the gathered side's columns are."""
         g = self._geometry
-        return L.THIN if g.kv * self.in_rows <= THIN_PAIRS * g.steps * (self.in_rows if transposed else self.out_rows) else 0
+        if self.subm:
+            said = L.RUN
+        else:
+            said = L.THIN if g.thin * self.in_rows <= (self.in_rows if transposed else self.out_rows) else 0
+        if by_row and (self.out_rows if transposed else self.in_rows) <= g.shallow[transposed]:
+            said |= L.SHALLOW
+        return said
 
     def _rows_kernel_takes(self, weight, weight_transposed: bool) -> bool:
         """Whether ``sph_conv_apply`` can walk this layer by stationary row (rows of 16-byte multiples up
@@ -276,7 +286,7 @@ class RuleBook:
                 by_row = est >= BY_ROW_MIN_PAIRS * BY_ROW_FORWARD_ONLY
             groups = not (by_row and forward_only)
         buf = _Buffers(rows, self.kv, self.z_ptr.device, by_row, groups)
-        buf.native.middle_run = self._said(transposed)
+        buf.native.middle_run = self._said(transposed, by_row)
         hint = self.row_cols if transposed else self.out_row_cols
         where = (self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, transposed, buf.native, hint)
         if weight is None:
@@ -294,7 +304,7 @@ class RuleBook:
         in fragment order for the forward pass and for dgrad; -> the two copies."""
         by_row = self._pairs_per_row(False) >= BY_ROW_MIN_PAIRS
         buf = _Buffers(self.out_rows, self.kv, self.z_ptr.device, by_row, True)
-        buf.native.middle_run = self._said(False)
+        buf.native.middle_run = self._said(False, by_row)
         both = L.host().rules_build_pack(self.z_idx, self.z_ptr, self.oz_idx, self.oz_ptr, self._geometry.native, False,
                                          buf.native, self.out_row_cols, weight, 2, self.mirrored(), L.dtype_code(dtype))
         self._fwd = buf

@@ -4,6 +4,8 @@ three phases, the last tile's remainder, rows of every width -- against the sum 
 import pytest
 from test_gpu_rows_split import _book, _check
 
+from sphconv_amd import _lib as L
+
 pytestmark = pytest.mark.gpu
 
 # (grid, share of the bins, kernel, stride)
@@ -25,5 +27,6 @@ LAYERS = [("f16", 16, 32), ("f16", 32, 32), ("bf16", 24, 24), ("bf16", 8, 32), (
 def test_long_grids_against_the_table_in_float64(grid):
     rows_in, rows, kv, buf = _book(*GRIDS[grid], seed=len(grid))
     assert buf.ntiles > (1024 if "strided" in grid else 5000)
+    buf.native.middle_run = L.SHALLOW        # (which rows of 64 bytes have to say of their columns)
     for n, (dt, ic, oc) in enumerate(LAYERS):
         _check(rows_in, rows, kv, buf, dt, ic, oc, n, epilogue=n % 2 == 0)

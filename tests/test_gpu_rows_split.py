@@ -95,6 +95,7 @@ GRIDS = {
     "deep": ((3, 19, 333), 0.97, (3, 3, 3), (1, 1, 1)),                 # columns longer than a tile: windows of 600 rows
     "some windows": ((8, 100, 128), 0.6, (3, 3, 3), (1, 1, 1)),         # one or two of a tile's three find room
     "deep, 600 tiles": ((8, 70, 333), 0.45, (3, 3, 3), (1, 1, 1)),
+    "strided, 1.6 to a row": ((24, 1801, 16), 0.2, (3, 3, 3), (2, 2, 2)),
     "strided, 3 to a row": ((24, 700, 16), 0.45, (3, 3, 3), (2, 2, 2)),
     "strided, 7 to a row": ((33, 601, 15), 0.9, (3, 3, 3), (2, 2, 2)),
     "45 offsets": ((8, 200, 16), 0.4, (5, 3, 3), (1, 1, 1)),
@@ -102,7 +103,7 @@ GRIDS = {
     "8 offsets": ((4, 31, 16), 0.5, (2, 2, 2), (1, 1, 1)),
 }
 LAYERS = [("f16", 64, 64), ("bf16", 48, 40), ("f16", 32, 64), ("bf16", 24, 32), ("f16", 16, 16), ("f16", 64, 128), ("f32", 32, 32),
-          ("f32", 16, 64), ("f32", 4, 24), ("i8", 64, 64), ("i8", 128, 32), ("i8", 16, 48)]
+          ("f32", 16, 64), ("f32", 32, 64), ("f32", 4, 24), ("i8", 64, 64), ("i8", 128, 32), ("i8", 16, 48)]
 
 
 @pytest.mark.parametrize("grid", list(GRIDS))
