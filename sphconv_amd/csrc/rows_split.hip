@@ -368,38 +368,28 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // the wave's offsets of the phases in `mask`, one bit each, and the next of them
-    auto offsets_of = [&](int mask) {
-        unsigned m = 0;
-#pragma unroll
-        for (int p = 0; p < kPhases; p++) m |= mask >> p & 1 ? ((1u << kPhase) - 1) << (p * kPhase) : 0;
-        return m & (0x11111111u << wave);
-    };
-    auto next_of = [&](unsigned &left) {
-        const int k = left ? __builtin_ctz(left) : kSplitKV;
-        left &= left - 1;
-        return k;
-    };
-    unsigned left = offsets_of(ok_mask);
-    int k = next_of(left), kn = next_of(left);
-    if (ok_mask != 7) {
+    // The first run of phases whose windows have room; the others follow (a list of the offsets of any such phases made this loop 1 to 4 %
+    // slower where all have room).
+    const int fit0 = __builtin_ctz(ok_mask | 1 << kPhases), fit1 = fit0 + __builtin_ctz(~(ok_mask >> fit0));
+    auto from = [&](int p) { return p * kPhase + ((wave - p * kPhase) & (W - 1)); }; // the wave's first offset of a phase
+    const int kend = min(fit1, kPhases) * kPhase;
+    int k = from(fit0);
+    if (fit0) {
         load_w(k, fw[0]);
-        load_w(kn, fw[1]);
+        load_w(k + W, fw[1]);
     }
     load_ix(k, ix0);
 #pragma unroll
     for (int j = 0; j < DX; j++) load_x(ix0, j, x[j]);
-    while (kn < kSplitKV) {
-        step(kn, ix0, ix1, fw[0]);
-        k = next_of(left);
-        load_w(k, fw[0]);
+    for (; k + W < kend; k += 2 * W) {
+        step(k + W, ix0, ix1, fw[0]);
+        load_w(k + 2 * W, fw[0]);
         __builtin_amdgcn_sched_barrier(0);
-        step(k, ix1, ix0, fw[1]);
-        kn = next_of(left);
-        load_w(kn, fw[1]);
+        step(k + 2 * W, ix1, ix0, fw[1]);
+        load_w(k + 3 * W, fw[1]);
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (k < kSplitKV) step(k, ix0, ix1, fw[0]);
+    if (k < kend) step(k, ix0, ix1, fw[0]);
     if (ok_mask != 7) {
         // Windows that found no room: their rows from the feature array, G blocks at a time and the next ones on their way, also into
         // the next offset, whose part of the table is there an offset ahead.  Columns of 150 rows (two windows of three have no room),
@@ -426,7 +416,15 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
                                                              r_feat, MASKED && st * 64 + qchunk >= rb ? kNoRow : off + st * 64, 0, 0));
             }
         };
-        unsigned rest = offsets_of(~ok_mask);
+        unsigned rest = 0; // the wave's offsets there, one bit each
+#pragma unroll
+        for (int p = 0; p < kPhases; p++) rest |= p < fit0 || p >= fit1 ? ((1u << kPhase) - 1) << (p * kPhase) : 0;
+        rest &= 0x11111111u << wave;
+        auto next_of = [&](unsigned &left) {
+            const int k = left ? __builtin_ctz(left) : kSplitKV;
+            left &= left - 1;
+            return k;
+        };
         int k0 = next_of(rest), k1 = next_of(rest);
         int id0[NB], id1[NB];
         int4v v[2][G][NS];
