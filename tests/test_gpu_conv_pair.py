@@ -78,6 +78,32 @@ def test_against_the_pairs_in_float64(grid):
         assert torch.equal(got, ext._apply(feat, packed, ic, oc, buf, *args))
 
 
+def test_rows_that_are_not_numbers():
+    """A row of infinities or NaN reaches the outputs that it is paired with and no other row of the merged groups."""
+    shape, batch, keep, kernel, stride = GRIDS["27 offsets, thin"]
+    z_idx, z_ptr = _scene(shape, batch, keep, 7)
+    out = [(s + 2 * (k // 2) - k) // t + 1 for s, k, t in zip(shape, kernel, stride)]
+    book = RuleBook.build(z_idx, z_ptr, batch, list(shape), out, list(kernel), list(stride), [k // 2 for k in kernel])
+    buf = book.grouped()
+    buf.native.middle_run = L.THIN
+    assert buf.ntiles > 640
+    cap = buf.cap
+    used = (torch.arange(cap, device=DEV) < buf.tile_ngrp[:buf.ntiles, None]).repeat_interleave(16, 1)
+    gather, owner = (x.view(-1, cap * 16).long()[:buf.ntiles][used] for x in (buf.grp_gather, buf.grp_owner))
+    gather, owner = gather[owner >= 0], owner[owner >= 0]
+    rows_in, rows = z_idx.numel(), book.oz_idx.numel()
+    feat, weight = torch.randn((rows_in, 64), device=DEV), torch.randn((27, 64, 64), device=DEV)
+    is_bad = torch.zeros(rows_in, dtype=torch.bool, device=DEV)
+    is_bad[::97] = True
+    feat[::97] = float("nan")
+    feat[::194] = float("inf")
+    got = ext._apply(feat, ext._packed_weight(weight, False), 64, 64, buf, None, None, False)
+    hit = torch.zeros(rows, dtype=torch.bool, device=DEV)
+    hit[owner[is_bad[gather]]] = True
+    assert bool(hit.any()) and not bool(hit.all())
+    assert not bool(torch.isfinite(got)[hit].any()) and bool(torch.isfinite(got)[~hit].all())
+
+
 def test_which_books_are_thin():
     """Strided layers with up to 1.45 pairs to an output row say so in their forward book; denser ones, transposed books and
     submanifold ones say what they said."""

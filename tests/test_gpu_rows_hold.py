@@ -2,7 +2,7 @@
 windows that fit, tiles that straddle lines and columns too deep for a window (gathers from the array), kernels of one, two and
 three phases, the last tile's remainder, rows of every width -- against the sum over the book's own table in float64 (int8: exactly)."""
 import pytest
-from test_gpu_rows_split import _book, _check
+from test_gpu_rows_split import _book, _check, _check_bad_rows
 
 from sphconv_amd import _lib as L
 
@@ -30,3 +30,13 @@ def test_long_grids_against_the_table_in_float64(grid):
     buf.native.middle_run = L.SHALLOW        # (which rows of 64 bytes have to say of their columns)
     for n, (dt, ic, oc) in enumerate(LAYERS):
         _check(rows_in, rows, kv, buf, dt, ic, oc, n, epilogue=n % 2 == 0)
+
+
+@pytest.mark.parametrize("grid", ["subm", "deep"])
+def test_rows_that_are_not_numbers(grid):
+    """A row of infinities or NaN reaches the outputs that gather it and no other: not the empty slots that the window's row of
+    zeros stands for, and not the next unit of a wave."""
+    rows_in, rows, kv, buf = _book(*GRIDS[grid], seed=len(grid))
+    buf.native.middle_run = L.SHALLOW
+    for dt, ic, oc in (("f16", 32, 32), ("bf16", 24, 24), ("f32", 16, 20)):
+        _check_bad_rows(rows_in, rows, kv, buf, dt, ic, oc)

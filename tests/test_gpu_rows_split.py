@@ -84,6 +84,24 @@ def _check(rows_in, rows, kv, buf, dt, ic, oc, seed, epilogue):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
+def _check_bad_rows(rows_in, rows, kv, buf, dt, ic, oc):
+    table = buf.tile_nbr.permute(0, 2, 1).reshape(-1, kv)[:rows].long()
+    dtype = DTYPES[dt]
+    feat = torch.randn((rows_in, ic), device=DEV).to(dtype)
+    bad = torch.arange(0, rows_in, 997, device=DEV)
+    feat[bad] = float("nan")
+    feat[bad[::2]] = float("inf")
+    weight = torch.randn((kv, ic, oc), device=DEV).to(dtype)
+    out = torch.empty((rows, oc), device=DEV, dtype=dtype)
+    epi = L.Epilogue(None, None, 0)
+    L.check(L.lib().sph_conv_apply(L.dtype_code(dtype), feat.data_ptr(), rows_in, ic, ext._packed_weight(weight, False).data_ptr(), oc,
+                                   C.byref(buf.struct()), C.byref(epi), out.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    is_bad = torch.zeros(rows_in + 1, dtype=torch.bool, device=DEV)
+    is_bad[bad] = True
+    hit = is_bad[torch.where(table < 0, torch.full_like(table, rows_in), table)].any(1)
+    assert not bool(torch.isfinite(out)[hit].any()) and bool(torch.isfinite(out)[~hit].all()) and bool(hit.any()) and not bool(hit.all())
+
+
 # grids by the tiles they come to: (grid, share of the bins, kernel, stride)
 GRIDS = {
     "9 tiles": ((4, 40, 16), 0.45, (3, 3, 3), (1, 1, 1)),
@@ -125,6 +143,21 @@ def test_rows_in_two_places(dt, ic, oc):
         at = torch.randint(0, places, table.shape, generator=g, device=DEV, dtype=torch.int32)
         buf.tile_nbr.copy_(torch.where(table >= 0, table + at * far, table))
         _check(rows_in + far * (places - 1), rows, kv, buf, dt, ic, oc, places, epilogue=True)
+
+
+@pytest.mark.parametrize("phases", [(0,), (1,), (2,), (0, 2), (1, 2)])
+def test_phases_without_a_window(phases):
+    """Some of a kernel's three phases gather rows too far apart for a window, the others do not."""
+    rows_in, rows, kv, buf = _book((12, 400, 16), 0.5, (3, 3, 3), (1, 1, 1), seed=3)
+    table = buf.tile_nbr.clone()
+    g = torch.Generator(device=DEV).manual_seed(9)
+    at = torch.randint(0, 3, table.shape, generator=g, device=DEV, dtype=torch.int32)
+    for p in range(3):
+        if p not in phases:
+            at.view(-1, kv, L.TILE_ROWS)[:, 9 * p:9 * p + 9] = 0
+    buf.tile_nbr.copy_(torch.where(table >= 0, table + at * 3 * rows_in, table))
+    for n, (dt, ic, oc) in enumerate([("f16", 64, 64), ("f32", 32, 64), ("bf16", 24, 64), ("i8", 64, 32)]):
+        _check(7 * rows_in, rows, kv, buf, dt, ic, oc, n, epilogue=n % 2 == 0)
 
 
 def test_rows_that_are_not_numbers():

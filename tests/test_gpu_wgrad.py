@@ -85,3 +85,27 @@ def test_against_the_pairs_in_float64(grid):
         d = L.host().conv_wgrad(feat, grad, buf.native, False, True)
         buf.native.middle_run = said
         assert bool(((d.double() - want).abs() <= 4 * n.sqrt() * 2.0 ** -24 * mag + 1e-30).all()), (dt, ic, oc)
+
+
+@pytest.mark.parametrize("dt,ic,oc", [("f32", 4, 4), ("f16", 24, 40)])
+def test_rows_beyond_two_to_the_24(dt, ic, oc):
+    """Gathered rows at the end of an array of more than 2^24 (their offsets are 32-bit products then): what the same book gives where
+    they lie at the beginning, bit for bit, and not a number of the rows in front of them."""
+    z_idx, z_ptr = _scene((8, 200, 16), 1, 0.5, 3)
+    book = RuleBook.build_subm(z_idx, z_ptr, 1, [8, 200, 16], [3, 3, 3])
+    rows, far = z_idx.numel(), 1 << 24
+    g = torch.Generator(device=DEV).manual_seed(ic)
+    feat = torch.randn((rows, ic), generator=g, device=DEV).to(DTYPES[dt])
+    grad = torch.randn((rows, oc), generator=g, device=DEV).to(DTYPES[dt])
+    for transposed in (False, True):
+        buf = book.grouped(transposed)
+        assert buf.ntiles > 4
+        want = L.host().conv_wgrad(feat, grad, buf.native, transposed, True)
+        small = grad if transposed else feat
+        big = torch.full((far + rows, small.shape[1]), float("nan"), device=DEV, dtype=small.dtype)
+        big[far:] = small
+        kept = buf.grp_gather.clone()
+        buf.grp_gather.copy_(torch.where(kept >= 0, kept + far, kept))
+        got = L.host().conv_wgrad(*((feat, big) if transposed else (big, grad)), buf.native, transposed, True)
+        buf.grp_gather.copy_(kept)
+        assert torch.equal(got, want)
