@@ -12,7 +12,9 @@
 // stationary row (dense neighbourhoods), conv_rows_kernel_* walks (offset, block of 16
 // rows) steps with the accumulators in registers instead; with rows of up to 64 bytes and
 // up to 64 output columns conv_rows_win_kernel does so from a copy of the gathered rows
-// in LDS.
+// in LDS.  Before these, rows_hold.hip takes long grids of up to 32 columns, whose weight it
+// keeps in LDS, and rows_split.hip grids that do not fill the chip with a wave per tile and
+// rows that its larger windows hold.
 #include "common.h"
 #include "pack.h"
 #include "conv_wave.h"

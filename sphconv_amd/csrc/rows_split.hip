@@ -603,7 +603,8 @@ Way pick_way(const ConvArgs &a, int nwtot, int ntiles)
     return f32 || T <= 2048 || to_a_row > 3.3 ? kSplit4 : kNone;
 }
 
-// LDS of a workgroup of 64 rows: what four, three or two of them on a compute unit leave each, by the rows its windows should hold (about half
+// LDS of a workgroup of 64 rows: what four, three or two of them on a compute unit leave each (where their registers let as many be
+// there: up to 128 of a lane four, 168 three), by the rows its windows should hold (about half
 // of the gathered rows to a row lie on a window's line, and a column or two more on either side)
 template <int NS>
 int split4_lds(const ConvArgs &a)

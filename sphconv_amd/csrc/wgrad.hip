@@ -127,15 +127,16 @@ __global__ void wgrad_reduce_kernel(const float *partial, int KV, int nchunk, in
 // ---------------------------------------------------------------------------
 constexpr int kWsBlock = 64;   // channels per block side
 
-// Narrow layers of 16 bits (blocks of up to four tiles): through LDS.  A row is two to four lanes' loads of 16 bytes here; turning it
+// Narrow layers of 16 bits (blocks of up to four tiles; of eight on books of up to four tiles of rows): through LDS.  A row is two to four lanes' loads of 16 bytes here; turning it
 // in registers, as wgrad_wave_kernel does, takes pieces of 4 or 8 bytes, as many loads as a row of 64 channels (16->16 on 14 599
 // tiles 66 us here, 116 there; 32->32 118 : 130; 64->16 on 2 437 tiles 32 : 34; 24->40 the other way round, 173 : 137).
 // Work item = (offset k, chunk of 64 tiles, slice of 64 groups of that chunk's groups at
-// k, 64x64 block of [iC,oC]).  A chunk holds at most 64*8 groups per offset; four
-// workgroups are launched per (offset, chunk), workgroup h takes slices h and h+4, and
-// those whose first slice lies beyond the chunk's real group count exit at once (a
-// submanifold book has 8 groups per tile at the centre offset and about one elsewhere:
-// slicing by groups, not tiles, is what balances the grid).
+// k, 64x64 block of [iC,oC]).  A chunk holds at most 64*8 groups per offset.  Slicing by groups,
+// not tiles, is what balances the grid: a submanifold book has 8 groups per tile at the centre
+// offset and about one elsewhere.  nslice workgroups (8 or 4) share the centre offset, workgroup h
+// takes slices h, h + nslice, ..., and one takes the whole of every other offset; on small grids
+// (all_slices) every offset has nslice.  A workgroup whose first slice lies beyond the chunk's real
+// group count exits at once.
 // The four waves of the workgroup take the slice's batches (32 pairs) round
 // robin and never synchronise until the end: a wave gathers the batch's feature rows and
 // d_out rows with 16-byte loads into its own LDS area in natural [pair][channel] order,
@@ -147,7 +148,7 @@ constexpr int kWsBlock = 64;   // channels per block side
 constexpr int kWsTiles = 64;   // tiles per chunk (one lane each)
 constexpr int kWsSlice = 64;   // groups per slice
 constexpr int kWsSlices = 8;   // most workgroups per chunk at the centre offset (workgroup h takes slices h, h + nslice, ...);
-                               // WgradArgs::nslice = 8 on small books, 4 on large ones; one workgroup elsewhere
+                               // WgradArgs::nslice = 8 on books of up to 16 chunks, 4 on larger ones
 
 typedef short short4v __attribute__((ext_vector_type(4)));
 
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_stage_kernel(WgradArgs a)
     static_assert(E == 2, "16-bit types");
     constexpr int GPB = 2;                             // groups per batch: one MFMA super step of 32 pairs
     constexpr int PB = GPB * SPH_GROUP;                // pairs per batch
-    // MI, NI: 16-channel tiles of the block's two sides (1 or 2; narrower blocks are zero padded).
+    // MI, NI: 16-channel tiles of the block's two sides (1, 2 or 4, up to 8 together; narrower blocks are zero padded).
     // A batch of rows of MI tiles is MI 16-byte loads per lane.
     extern __shared__ __attribute__((aligned(16))) char s_raw[];
 
