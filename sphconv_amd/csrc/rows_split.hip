@@ -376,7 +376,9 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
     int k = from(fit0);
     if (fit0) {
         load_w(k, fw[0]);
+        __builtin_amdgcn_sched_barrier(0); // (in the loop's order: what it then waits for is counted)
         load_w(k + W, fw[1]);
+        __builtin_amdgcn_sched_barrier(0);
     }
     load_ix(k, ix0);
 #pragma unroll
