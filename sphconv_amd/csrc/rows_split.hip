@@ -403,6 +403,9 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
         if (QUAD) lds_barrier(); // the waves are through with the windows: each turns its rows in a part of them
         char *tr = s_win + wave * (G * NS * kTrSet);
         const int qrow = QUAD ? lane >> 2 : lane & 15, qchunk = (QUAD ? lane & 3 : lane >> 4) * 16;
+        unsigned qadd[NS]; // (a chunk beyond the row's end: out of range with any row added, which is below 2^31)
+#pragma unroll
+        for (int st = 0; st < NS; st++) qadd[st] = !MASKED || st * 64 + qchunk < rb ? st * 64 + qchunk : kNoRow;
         auto load_id = [&](int k, int (&id)[NB]) {
 #pragma unroll
             for (int j = 0; j < NB; j++) id[j] = tab[min(k, kSplitKV - 1) * R + j * SPH_GROUP + qrow];
@@ -411,11 +414,11 @@ void conv_rows_split_kernel(ConvArgs a, int nwtot, int cap_rows)
             const unsigned lim = k < kSplitKV ? a.feat_rows : 0;
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                const unsigned off = (unsigned)id[u * G + g] < lim ? (unsigned)(id[u * G + g] * rb + qchunk) : kNoRow;
 #pragma unroll
-                for (int st = 0; st < NS; st++)
-                    v[g][st] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
-                                                             r_feat, MASKED && st * 64 + qchunk >= rb ? kNoRow : off + st * 64, 0, 0));
+                for (int st = 0; st < NS; st++) {
+                    const unsigned off = (unsigned)id[u * G + g] < lim ? (unsigned)(id[u * G + g] * rb) + qadd[st] : kNoRow;
+                    v[g][st] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(r_feat, off, 0, 0));
+                }
             }
         };
         unsigned rest = 0; // the wave's offsets there, one bit each
