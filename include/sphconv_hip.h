@@ -78,7 +78,9 @@ typedef struct sph_geom {
     int32_t dil[3];
 } sph_geom;
 
-enum { SPH_RUN = 1, SPH_RUN_IN_FLIGHT = 2, SPH_THIN = 4, SPH_SHALLOW = 8 }; /* values of sph_book.middle_run */
+enum { SPH_RUN = 1, SPH_RUN_IN_FLIGHT = 2, SPH_THIN = 4 }; /* values of sph_book.middle_run */
+/* may be added to any of them: `rows` 1..4095, `stride` 1..127 (more count as the most) */
+#define SPH_PLANE(rows, stride) (((rows) < 4095 ? (rows) : 4095) << 8 | ((stride) < 127 ? (stride) : 127) << 20)
 
 typedef struct sph_book {
     int32_t *tile_ngrp;
@@ -105,8 +107,10 @@ typedef struct sph_book {
      * are the same either way, up to the order of summation.  SPH_RUN_IN_FLIGHT says besides that the caller keeps three calls
      * or more in flight on streams of their own: kernels that share the chip better are then taken up to larger grids.
      * SPH_THIN says that there is no such run and hardly more than one pair to a row (1.45 on average at most), as in a strided layer
-     * on scattered voxels: neighbouring tiles' groups can then be merged.  SPH_SHALLOW may be added to any of them, and says that a column of
-     * the gathered side's grid holds 16 rows or fewer on average: what 64 rows gather at nine neighbouring offsets then lies close together. */
+     * on scattered voxels: neighbouring tiles' groups can then be merged.  SPH_PLANE says of a book by row how far apart lies what a row gathers: `rows`
+     * of the gathered side, on average, from the first to the last column that a kernel's plane (offsets of one k0) reaches beside each
+     * other ((K1 - 1) * dilation columns' rows, 1 at least), and how many lines of the gathered grid, `stride`, the stationary side's next line
+     * moves on by (the first axis' stride; 1 in a transposed book).  Kernels that bring a plane's rows to LDS are then taken where they find room there. */
     int32_t middle_run;
 } sph_book;
 

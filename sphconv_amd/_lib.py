@@ -21,8 +21,14 @@ STATIC_MAX_COLUMNS = 1 << 20     # SPH_STATIC_MAX_COLUMNS of the header
 F32, F16, BF16, I8 = 0, 1, 2, 3
 ERR_ARG, ERR_UNSUPPORTED, ERR_LAUNCH = -1, -2, -3      # sph_status
 FUSED_WRITE_BOOK, FUSED_IN_FLIGHT = 1, 2               # flags of sph_rules_conv
-RUN, RUN_IN_FLIGHT, THIN, SHALLOW = 1, 2, 4, 8         # values of sph_book.middle_run
+RUN, RUN_IN_FLIGHT, THIN = 1, 2, 4                     # values of sph_book.middle_run
+SAID = 0xff                                            # ... without what SPH_PLANE adds
 _DTYPES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16, torch.int8: I8}
+
+
+def plane(rows, stride):
+    """SPH_PLANE of the header."""
+    return min(max(int(rows), 1), 4095) << 8 | min(stride, 127) << 20
 
 
 class SphconvError(RuntimeError):

@@ -9,9 +9,10 @@
 
 #define SPH_EXPORT extern "C" __attribute__((visibility("default")))
 
-// what the caller says of a book's middle offset and pairs, and of its columns (sph_book.middle_run)
-static inline int book_says(const sph_book *b) { return b->middle_run & ~SPH_SHALLOW; }
-static inline int book_is_shallow(const sph_book *b) { return b->middle_run & SPH_SHALLOW; }
+// what the caller says of a book's middle offset and pairs, and of a plane's rows (sph_book.middle_run; 0: not said)
+static inline int book_says(const sph_book *b) { return b->middle_run & 0xff; }
+static inline int book_plane_rows(const sph_book *b) { return b->middle_run >> 8 & 0xfff; }
+static inline int book_plane_stride(const sph_book *b) { const int s = b->middle_run >> 20 & 0x7f; return s ? s : 1; }
 
 void sph_set_error(const char *fmt, ...);
 

@@ -81,6 +81,13 @@ __device__ __forceinline__ int4v mfma_step<SPH_I8>(int4v a, int4v b, int4v d)
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, d, 0, 0, 0);
 }
 
+// Rows of the gathered side, on average, from the first to the last that `rows` neighbouring rows gather at a kernel plane's offsets: their own
+// stretch of a line and the lines beside it.
+inline double plane_window(const ConvArgs &a, int rows)
+{
+    return rows * ((double)a.feat_rows / a.book.rows) / book_plane_stride(&a.book) + book_plane_rows(&a.book);
+}
+
 // does the middle offset hold a run of full groups, by what the caller says?
 inline bool book_has_run(const sph_book *b) { return book_says(b) != 0 && book_says(b) != SPH_THIN; }
 inline int book_has_groups(const sph_book *b) { return b->grp_k && b->grp_gather && b->grp_owner; }

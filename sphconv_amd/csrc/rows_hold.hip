@@ -297,22 +297,28 @@ int launch(const ConvArgs &a, hipStream_t st)
 //   stride 1,2,2, f16 32 -> 32  1.43  1.35  1.16  1.53  1.52  1.44  1.44  1.39  1.35  1.37  1.48   (that of 128 rows fits)
 //   stride 1,2,2, f16 16 -> 32  1.00  0.95  0.85  1.03  1.01  0.95  0.95  0.91  0.84  0.84  0.87
 // 16 columns gain nothing (f16 16 -> 16 1.07 to 1.11 on the longest grids), 45 offsets leave room for eight waves (1.08).
-// Rows of 64 bytes only where the caller says that columns are shallow: nine offsets' rows, 64 and two columns more, have to find room
-// among 116, and a phase without a window is three round trips of gathers for every three offsets (13 rows a column 0.83 to 0.88, 21 rows 0.92 to
-// 0.95, 29 rows 1.68 to 1.84, 51 rows 1.41 to 1.54; a window for every three offsets of such a phase takes registers that
-// the usual one then misses: 29 rows 1.18 to 1.44, but 13 rows 1.08 to 1.13 where it was 0.88 to 0.93).
+// Rows of 64 bytes in 16 bits and int8 only where the caller says how far apart a plane's rows lie: those of 64 rows have to find room among 116
+// (7500 tiles, 97 rows 0.76 to 0.87, 103 rows 0.86 to 0.90, 114 rows 1.06 to 1.17, 138 rows 1.34 to 1.64, 184 rows 1.16 to 1.42), as a phase without a
+// window is three round trips of gathers for every three offsets; or those of 128 rows find none in the other kernel's window either (248 rows 1.16
+// to 1.41, 298 and more 0.81 to 0.91).  fp32, which waits for its matrix cores, gains in any case (0.75 to 0.96).  A window for every three offsets of a phase
+// without one takes registers that the usual one then misses: 29 rows a column 1.18 to 1.44, but 13 rows 1.08 to 1.13 where it was 0.88 to 0.93.
 // A round of the chip's 3072 waves (1536 tiles) that is mostly empty counts on short grids: strided layers on 1537 to 2303 tiles, and on 3073 to 3455, are
 // not taken in fp32 (4 -> 32 1.08 to 1.23), and from 1537 to 2047 not in 16 bits where columns are deep (29 rows 1.17 to 1.32; 8 and 13 rows 0.56
-// to 0.8).  Kernels of nine offsets or fewer are one phase, with nothing to work ahead of (8 offsets 1.06 to 1.28).
+// to 0.8; of stride 2 with two gathered rows to a row, 25 to 50 rows, 0.71 to 0.82).  Kernels of nine offsets or fewer are one phase, with nothing to work ahead of (8 offsets 1.06 to 1.28).
 bool sph_rows_hold_ok(sph_dtype dt, const ConvArgs &a, int nwtot, int ntiles)
 {
     if (a.nsteps != 1 || nwtot != CT || hold_lds(a.book.KV) > 160 * 1024 || (double)a.feat_rows * a.row_bytes >= 1073741824.0) return false;
     const double gathered = a.feat_rows / (double)a.book.rows; // to a row
-    if (a.row_bytes > 48 && (gathered > 1.25 || !book_is_shallow(&a.book))) return false;
+    const bool said = book_plane_rows(&a.book) > 0;
+    const double window = plane_window(a, kRows);
+    if (a.row_bytes > 48) {
+        if (gathered > 1.25) return false;
+        if (dt != SPH_F32 && !(said && (window <= 104 || plane_window(a, R) > 280))) return false;
+    }
     if (ntiles > 5000) return true;
     if (gathered <= 2 || ntiles <= 1024 || a.book.KV <= kPhase) return false;
     if (dt == SPH_F32) return ntiles <= 1536 || (ntiles >= 2304 && (ntiles <= 3072 || ntiles >= 3456));
-    return ntiles <= 1536 || ntiles >= 2048 || book_is_shallow(&a.book);
+    return ntiles <= 1536 || ntiles >= 2048 || (said && (window <= 170 || book_plane_rows(&a.book) <= 32));
 }
 
 int sph_rows_hold_launch(sph_dtype dt, const ConvArgs &a, hipStream_t st)

@@ -567,16 +567,52 @@ enum Way { kNone, kShort1, kShort2, kByOffset, kSplit4, kSplit8 };
 //   one K step: 32 -> 64 1401 tiles 33 : win 39, 2000 tiles 48 : 55, 2997 tiles 70 : 68; fp32 16 -> 64 3996 tiles 250 : 265; 32 -> 32 1001
 //     tiles 16 : plain 27, 1401 tiles 22 : win 19 (fp32 16 -> 32 51 : 54, 2000 tiles 72 : 69); 32 -> 64 3.6 to a row 4000 tiles 106 : 117;
 //     32 -> 32 3.6 to a row 511 tiles kByOffset 12 : split 15, 4000 tiles split 74 : win 88, 2.8 to a row 4000 tiles 64.5 : 64.9
-// Where the windows are not sure to find room the lines are those at which nothing measured is much slower than the kernels of conv.hip (twenty tile
-// counts from 20 to 10 000, 0.15 to 0.9 of the bins, columns of 4 to 51 rows, strides of one, two or three axes; columns of 150 rows are up to 1.3):
-//   fp32 into 64 columns, more than 1.3 to a row: an offset at a time 0.83 to 0.93, with windows 0.77 to 1.10; beyond 6000 tiles neither
-//   one K step, more than 2 to a row: rows shorter than 64 bytes (16 -> 64 f16 2.6 to 7 to a row, 1100 tiles 1.05, 1950 1.2 to 1.4 of plain, where
-//     columns hold 13 rows or fewer 0.7 to 0.9), fp32 16 -> 64 beyond 1900 tiles 1.06 to 1.15 (0.83 to 0.9)
-//   one K step, 64 columns, 961 to 1024 tiles: one round of conv_rows_win_kernel (995 tiles 1.05, int8 1.07 to 1.10 of it); int8 rows of 16 bytes
-//     and 16-bit ones of up to 48 from 1901 tiles on 1.04 to 1.10 of plain
+// Which windows find room decides between kSplit4, kSplit8 and the kernels without them (kByOffset; plain or win from 1025 tiles on).  A window holds a
+// plane's rows, which lie between its first and last column (sph_book.middle_run says how many), and the workgroup's own stretch of a line.
+// Times over those of the kernels before the windows came, 17 680 calls (500 to 9000 tiles, 0.3 to 0.8 of the bins, columns of 5 to 170 rows,
+// strides 1x1x1, 1x2x2, 2x2x2 and 2x1x1), by three, two, one of three with room: 64 -> 64 fp16 kSplit8 0.71 to 0.80, 0.83 to 0.97, 0.98 to 1.07; where
+// more than 1.9 are gathered to a row kSplit4's three 0.92, its two 1.10 to 1.18; 64 -> 128 the same, two 1.04 to 1.16.  One K step into 64
+// columns, more than 2 to a row: kSplit4 0.81 to 0.92, 0.87 to 1.03, 0.98 to 1.12, more than 5 to a row 0.9, 1.11, 1.22.  The lines by T beside that:
+//   fp32 two K steps into 32: an offset at a time 0.64 to 0.84 beyond 1152 tiles, windows 0.66 to 1.0 (into 16, up to 2048 tiles, 0.8 of the former);
+//     into 64: an offset at a time 0.78 to 0.95, windows 0.75 to 1.05 (three with room, 1300 to 5500 tiles, 0.76 to 0.90; 330 tiles 0.63, an offset at a time 0.78), beyond 6000 tiles 1.03, 0.96 to 1.11
+//   rows shorter than 64 bytes into 64 columns, 16 bits and int8, up to 2 to a row: kSplit4 0.55 to 0.95 (three with room, where conv_rows_win_kernel
+//     has room as well, 7000 tiles 0.99, 0.90 to 1.14; two, 1900 tiles and more 0.95 to 1.13); 2 to 5 to a row: three 0.65 to 0.97, two or one 0.73 to 0.98 up to
+//     1100 tiles, 1.0 to 1.19 beyond but for 2200 (0.86 to 0.92: a round of plain is 2048); more: an offset at a time 0.72 to 0.84 up to 800 tiles
+//   rows of 64 bytes into 64 columns, up to 2 to a row: 961 to 1024 tiles of submanifold books are one round of conv_rows_win_kernel (995 tiles 1.05, int8 1.07 to 1.10
+//     of it; strided 1000 tiles 0.70 to 0.80);
+//     1700 tiles 0.74 of it, 2000 0.8 to 0.97, 16 bits with fewer than three with room 1.07 to 1.18
+//   one K step into 16 and 32 columns: fp32 into 16, fewer than three with room, 700 and 1000 tiles: an offset at a time 1.03 to 1.05, windows to 1.15 (four waves of
+//     one tile were faster there); 16 bits into 32, up to 1024 tiles, three with room 0.64 (16 -> 32 0.75), an offset at a time 0.71, two or one with
+//     room 0.8 to 1.0; 16 -> 32 fp16, more than 2.4 to a row, 1700 tiles: 0.76, windows 1.00
+//   two blocks of columns: up to 1152 tiles of rows windows in any case (1040 tiles 0.75, neither 1.0), one K step beyond only where three have room to spare (1.0
+//     per row, columns of 60 and 70 rows 1.07 to 1.20)
+// Over 37 076 other calls (130 to 5500 tiles, 0.25 to 0.75 of the bins, 24 widths and types): 0.81 of the time before the windows, 234 calls more than 6 % and
+// 71 more than 10 % slower (1.31 at most); by T and the rows to a row alone 0.885, 6029, 4981 and 2.16.
 //   8 offsets, 45 offsets, 16 bits, one K step into 64 columns: 645 tiles 1.04 to 1.09, 990 tiles 1.10 of plain or the window kernel
 //   65 to 128 columns of other than 27 offsets: 512 tiles (9 offsets 64 -> 128 f16 520 tiles 0.93, 650 1.07, 1000 1.38 of plain)
-// int8 takes 16 bits' lines but for these (64 -> 64 against the window kernel: 300 to 960 tiles 0.58 to 0.9, 1100 to 1950 tiles 0.8 to 1.05).
+
+// LDS of a workgroup of 64 rows: what four, three or two of them on a compute unit leave each (where their registers let as many be
+// there: up to 128 of a lane four, 168 three), by the rows its windows should hold (about half
+// of the gathered rows to a row lie on a window's line, and a column or two more on either side)
+template <int NS>
+int split4_lds(const ConvArgs &a)
+{
+    const double to_a_row = (double)a.feat_rows / a.book.rows;
+    const double rows = kPhases * (64 * (to_a_row > 2 ? to_a_row / 2 : 1.0) + 32);
+    const double need = (rows * NS * 64 + kSplitKV * 64 * 2) / 1024;
+    return (NS == 2 && to_a_row > 1.5 ? 79 : need <= 39 ? 39 : need <= 52 ? 52 : 79) * 1024;
+}
+constexpr int kSplit8Lds = 79 * 1024;
+
+// Of the three windows of `rows` rows, on average, those that find room in so much LDS.
+template <int NS>
+int windows_with_room(const ConvArgs &a, int rows, int lds)
+{
+    const int cap_rows = (lds - kSplitKV * rows * 2) / (NS * 64);
+    const double window = plane_window(a, rows);
+    return kPhases * window <= cap_rows ? kPhases : 2 * window <= cap_rows ? 2 : 1;
+}
+
 template <sph_dtype DT, int NS, int CT>
 Way pick_way(const ConvArgs &a, int nwtot, int ntiles)
 {
@@ -590,34 +626,48 @@ Way pick_way(const ConvArgs &a, int nwtot, int ntiles)
         return T <= (half && NS == 1 && nwtot == 4 && (KV <= 8 || KV > kSplitKV) ? 640 : 1024) ? kByOffset : kNone;
     }
     if (T <= (NS == 1 && CT <= 2 ? 128 : 64)) return kShort2;
+    const int room4 = windows_with_room<NS>(a, 64, split4_lds<NS>(a)), room8 = NS == 2 ? windows_with_room<NS>(a, 128, kSplit8Lds) : 0;
+    const bool two_blocks = nwtot > 4, many = T > (two_blocks ? 2304 : 1024);
+    if (NS == 2 && f32) {
+        if (CT < 4) return to_a_row <= 2.4 && room4 == 3 && T <= (CT == 1 ? 2048 : 1152) ? kSplit4 : kByOffset;
+        if (to_a_row <= (T <= 384 ? 2.4 : 1.3) && room4 == 3 && (T <= 512 || T > 1024)) return T <= 512 ? kSplit4 : kSplit8;
+        return T <= 6000 ? kByOffset : kNone;
+    }
     if (NS == 2) {
-        if (f32 && CT == 4 && to_a_row > 1.3 && T > 512) return T <= 6000 ? kByOffset : kNone;
-        if (to_a_row <= 2.4) return f32 && (CT <= 2 || T <= 512) ? kSplit4 : (T <= 256 ? kSplit4 : kSplit8);
-        if (f32 || T <= 1024) return kByOffset;
-        return T <= 1400 && to_a_row <= 5 ? kSplit4 : kNone;
+        if (to_a_row > (CT == 4 ? 2.5 : 2.4)) {
+            if (T <= 1024) return kByOffset;
+            return to_a_row > 5 || T > 1400 ? kNone : room4 == 3 ? kSplit4 : kByOffset;
+        }
+        if (CT < 4 || !many) return T <= 256 ? kSplit4 : kSplit8;
+        if (room8 == 3) return kSplit8;
+        if (two_blocks) return kNone;
+        return to_a_row >= 1.9 && room4 == 3 ? kSplit4 : room8 == 2 ? kSplit8 : kNone;
+    }
+    if (CT == 4 && f32) {
+        if (T <= 1900 || (to_a_row <= 2 && (T <= 6000 || room4 == 3))) return kSplit4;
+        return T <= 6000 && (room4 == 3 || (room4 == 2 && to_a_row <= 5)) ? kSplit4 : kNone;
     }
     if (CT == 4) {
-        const bool brief = a.row_bytes < 64;
-        if (to_a_row > 2) return book_is_shallow(&a.book) || (!f32 && !brief) || T <= (f32 ? 1900 : nwtot > 4 ? 2048 : 1024) ? kSplit4 : kNone;
-        if (f32 || nwtot > 4) return kSplit4;
-        return T <= 960 || (T > 1024 && T <= (brief ? 1900 : 2048)) ? kSplit4 : kNone;
+        if (!two_blocks && a.row_bytes < 64) {
+            const bool win = plane_window(a, R) <= 255; // conv_rows_win_kernel's has room for a tile
+            if (to_a_row > 5) return T <= 768 ? kByOffset : kNone;
+            if (to_a_row > 2) return room4 == 3 || T <= 1152 || (T > 2048 && T <= 2304) ? kSplit4 : kNone;
+            return !win || T <= (room4 == 3 ? 6000 : 1700) ? kSplit4 : kNone;
+        }
+        const bool win_round = T > 960 && T <= 1024 && to_a_row <= 1.3 && book_plane_stride(&a.book) == 1;
+        if (!two_blocks && to_a_row <= 2) return !win_round && T <= (room4 == 3 || !half ? 2048 : 1900) ? kSplit4 : kNone;
+        if (!many) return kSplit4;
+        if (two_blocks) return to_a_row <= 4.5 && windows_with_room<NS>(a, 64, split4_lds<NS>(a) * 9 / 10) == 3 ? kSplit4 : kNone;
+        if (room4 == 3) return kSplit4;
+        return to_a_row <= 5 && (room4 == 2 || (T <= 2700 && book_plane_stride(&a.book) == 1)) ? kSplit4 : kNone;
     }
-    if (to_a_row <= 2.4) return T <= (f32 ? 1536 : 1024) ? kSplit4 : kNone;
-    if (T <= (f32 && CT == 1 ? 1024 : 640)) return kByOffset;
-    if (CT == 1) return T <= 1024 ? kSplit4 : kNone;
-    return f32 || T <= 2048 || to_a_row > 3.3 ? kSplit4 : kNone;
-}
-
-// LDS of a workgroup of 64 rows: what four, three or two of them on a compute unit leave each (where their registers let as many be
-// there: up to 128 of a lane four, 168 three), by the rows its windows should hold (about half
-// of the gathered rows to a row lie on a window's line, and a column or two more on either side)
-template <int NS>
-int split4_lds(const ConvArgs &a)
-{
-    const double to_a_row = (double)a.feat_rows / a.book.rows;
-    const double rows = kPhases * (64 * (to_a_row > 2 ? to_a_row / 2 : 1.0) + 32);
-    const double need = (rows * NS * 64 + kSplitKV * 64 * 2) / 1024;
-    return (NS == 2 && to_a_row > 1.5 ? 79 : need <= 39 ? 39 : need <= 52 ? 52 : 79) * 1024;
+    if (to_a_row <= 2.4) {
+        if (T > (f32 ? 1536 : 1024)) return kNone;
+        return room4 == 3 || (f32 && CT == 2) || many ? kSplit4 : kByOffset;
+    }
+    if (CT == 1) return T <= (f32 ? 1024 : 640) ? kByOffset : T <= 1024 ? kSplit4 : kNone;
+    if (f32) return T <= 640 ? kByOffset : kSplit4;
+    return T <= 2048 ? kByOffset : to_a_row > 3.3 ? kSplit4 : kNone;
 }
 
 template <sph_dtype DT, int NS, int CT, bool MASKED>
@@ -628,7 +678,7 @@ int launch_m(const ConvArgs &a, int nwtot, int ntiles, hipStream_t st)
     case kShort2: return launch_short<DT, NS, CT, MASKED, 2, 8, 4>(a, nwtot, st);
     case kSplit4: return launch_split<DT, NS, CT, MASKED, 4>(a, nwtot, st, split4_lds<NS>(a));
     case kSplit8:
-        if constexpr (NS == 2) return launch_split<DT, NS, CT, MASKED, 8>(a, nwtot, st, 79 * 1024);
+        if constexpr (NS == 2) return launch_split<DT, NS, CT, MASKED, 8>(a, nwtot, st, kSplit8Lds);
     default: return launch_short<DT, NS, CT, MASKED, 4, 4, 1>(a, nwtot, st);
     }
 }

@@ -77,8 +77,6 @@ class _Buffers:
 
 # Pairs to a row up to which a strided layer's book is said to be thin (``SPH_THIN``).
 THIN_PAIRS = 1.45
-# Rows to a column up to which a by-row book's gathered side is said to be shallow (``SPH_SHALLOW``).
-SHALLOW_ROWS = 16
 
 
 class _Geometry:
@@ -86,7 +84,7 @@ class _Geometry:
     by every book that has it (a network meets a few dozen)."""
 
     __slots__ = ("native", "batch", "in_shape", "out_shape", "kernel", "stride", "padding", "dilation", "kv", "in_cells",
-                 "out_cells", "steps", "odd_same", "z_shape", "cluster", "key", "thin", "shallow")
+                 "out_cells", "steps", "odd_same", "z_shape", "cluster", "key", "thin", "plane")
 
     def __init__(self, batch, in_shape, out_shape, kernel, stride, padding, dilation):
         self.batch = batch
@@ -106,9 +104,10 @@ class _Geometry:
         for k, s in zip(kernel, stride):
             reach = [len(range(r, k, s)) for r in range(s)]
             self.cluster *= sum(c * c for c in reach) / max(sum(reach), 1)
-        # stationary rows from which a strided layer's book is thin, to an input row; rows up to which each side is shallow
+        # stationary rows from which a strided layer's book is thin, to an input row; rows that lie between a kernel plane's
+        # first and last column, to a row of each side (``SPH_PLANE``)
         self.thin = self.kv / (THIN_PAIRS * self.steps)
-        self.shallow = tuple(SHALLOW_ROWS * batch * s[0] * s[1] for s in (in_shape, out_shape))
+        self.plane = tuple((kernel[1] - 1) * dilation[1] / max(batch * s[0] * s[1], 1) for s in (in_shape, out_shape))
         # odd kernel, stride 1, padding K//2: a submanifold book is then its own transpose, offsets mirrored
         self.odd_same = all(k % 2 == 1 for k in kernel) and self.steps == 1 and all(p == k // 2 for p, k in zip(padding, kernel))
         self.native = L.host().Geometry(batch, self.in_shape, self.out_shape, self.kernel, self.stride, self.padding,
@@ -247,14 +246,17 @@ class RuleBook:
     def _said(self, transposed: bool, by_row: bool) -> int:
         """What the book says of its pairs (``sph_book.middle_run``): a submanifold layer pairs every row with itself at
         the middle offset; a strided layer's pairs are known (kernel volume / stride to an input row), and may be hardly more than
-        its rows; and of a by-row book how deep the gathered side's columns are."""
+        its rows; and of a by-row book how far apart lies what a row gathers."""
         g = self._geometry
         if self.subm:
             said = L.RUN
         else:
             said = L.THIN if g.thin * self.in_rows <= (self.in_rows if transposed else self.out_rows) else 0
-        if by_row and (self.out_rows if transposed else self.in_rows) <= g.shallow[transposed]:
-            said |= L.SHALLOW
+        if by_row:
+            if transposed:
+                said |= L.plane(self.out_rows * g.plane[1] + 0.999, 1)
+            else:
+                said |= L.plane(self.in_rows * g.plane[0] + 0.999, g.stride[0])
         return said
 
     def _rows_kernel_takes(self, weight, weight_transposed: bool) -> bool:

@@ -114,7 +114,7 @@ def test_which_books_are_thin():
         buf, back = book.grouped(), book.grouped(transposed=True)
         pairs = buf.num_pairs() / book.out_rows
         assert (pairs < 1.3) == (keep < 0.1)
-        said[keep] = tuple(b.native.middle_run & ~L.SHALLOW for b in (buf, back))
+        said[keep] = tuple(b.native.middle_run & L.SAID for b in (buf, back))
     assert said == {0.005: (L.THIN, 0), 0.5: (0, 0)}
     subm = RuleBook.build_subm(z_idx, z_ptr, 1, [32, 64, 32], [3, 3, 3])
-    assert subm.grouped().native.middle_run & ~L.SHALLOW == L.RUN
+    assert subm.grouped().native.middle_run & L.SAID == L.RUN

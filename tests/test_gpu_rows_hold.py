@@ -27,7 +27,7 @@ LAYERS = [("f16", 16, 32), ("f16", 32, 32), ("bf16", 24, 24), ("bf16", 8, 32), (
 def test_long_grids_against_the_table_in_float64(grid):
     rows_in, rows, kv, buf = _book(*GRIDS[grid], seed=len(grid))
     assert buf.ntiles > (1024 if "strided" in grid else 5000)
-    buf.native.middle_run = L.SHALLOW        # (which rows of 64 bytes have to say of their columns)
+    buf.native.middle_run = L.plane(32, 1)   # (that columns are shallow, which rows of 64 bytes have to say)
     for n, (dt, ic, oc) in enumerate(LAYERS):
         _check(rows_in, rows, kv, buf, dt, ic, oc, n, epilogue=n % 2 == 0)
 
@@ -37,6 +37,6 @@ def test_rows_that_are_not_numbers(grid):
     """A row of infinities or NaN reaches the outputs that gather it and no other: not the empty slots that the window's row of
     zeros stands for, and not the next unit of a wave."""
     rows_in, rows, kv, buf = _book(*GRIDS[grid], seed=len(grid))
-    buf.native.middle_run = L.SHALLOW
+    buf.native.middle_run = L.plane(32, 1)
     for dt, ic, oc in (("f16", 32, 32), ("bf16", 24, 24), ("f32", 16, 20)):
         _check_bad_rows(rows_in, rows, kv, buf, dt, ic, oc)
