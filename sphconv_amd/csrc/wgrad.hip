@@ -435,7 +435,8 @@ __global__ __launch_bounds__(256, 2) void wgrad_stage_kernel(WgradArgs a)
 // one of four SIMDs, and some 150 vector instructions for the exchange and the addresses; the rows come from L2 (2.3 times
 // each at fourteen pairs to a row).  Through LDS, as wgrad_stage_kernel below 64 channels, a row was written, read back and waited for
 // on top: 64x64 f16 on eight 64x512x32 scans (2 412 tiles) 42 -> 29 us and the sum of the partials 7.7 -> 6.0, fewer of them; 64x64 fp32
-// on the strided layer of eight 64x512x512 scans 61 -> 45; 24->40 bf16 on eight ragged grids 38 -> 30.
+// on the strided layer of eight 64x512x512 scans 61 -> 40; 24->40 bf16 on eight ragged grids 38 -> 27 (45 and 31 with
+// workgroups kept for a centre that these books have not).
 // Loads stand between the matrix instructions: in one burst all waves of the chip ask at the same time and then all wait
 // (43 : 33 us).  A wave that has no batch left leaves the unrolled pipeline instead of skipping its stages: behind a skipped
 // load the compiler cannot tell how many are on their way and waits for all of them.
